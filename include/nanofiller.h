@@ -478,11 +478,10 @@ enum {
    * depend on it; nanofiller_amd/autotune.py picks it per workload): */
   NF_OPT_WAVES_OLD = 10,     /* waves per CU, reject vs accepted (0: default 16)     */
   NF_OPT_WAVES_NEW = 11,     /* waves per CU, reject vs same-round (0: default 16)   */
-  NF_OPT_PART_SHIFT = 12,    /* reject vs accepted: a dense cell is dealt over
-                                1 << shift work items in launches with few cells per
-                                wave (-1: default 1)                                    */
+  NF_OPT_PART_SHIFT = 12,    /* reject vs accepted: a dense cell is dealt over at most
+                                1 << shift work items (-1: by the cell's cost)         */
   NF_OPT_SPLIT_MIN = 13,     /* probes per work item of a dealt cell, at least
-                                (0: default 32)                                         */
+                                (0: by the cell's cost; either option set: 1 and 32)   */
   NF_OPT_TEST_ALL_PAIRS = 14 /* 1: the reject-vs-accepted pass tests every pair within
                                 reach, so that the pair-test count is the oracle's;
                                 0 (default): a proposal leaves its stencil walk once an

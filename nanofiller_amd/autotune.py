@@ -43,11 +43,11 @@ from . import configs
 # option keys of a tile entry in cell_tuning.json
 TILE_KEYS = {"waves_old": NF_OPT_WAVES_OLD, "waves_new": NF_OPT_WAVES_NEW, "part_shift": NF_OPT_PART_SHIFT,
              "split_min": NF_OPT_SPLIT_MIN}
-TILE_DEFAULTS = {"cell_factor": 1.0, "waves_old": 16, "waves_new": 16, "part_shift": 1, "split_min": 32}
+TILE_DEFAULTS = {"cell_factor": 1.0, "waves_old": 16, "waves_new": 16, "part_shift": -1, "split_min": 0}
 # cell_factor scales the library's default generation cell edge (0.85 of a
 # typical pair reach; 1.18 makes it one reach), passed as cell_size = -f
 TILE_CHOICES = {"cell_factor": [0.85, 1.0, 1.18, 1.35], "waves_old": [8, 12, 16], "waves_new": [8, 12, 16],
-                "part_shift": [0, 1, 2], "split_min": [16, 32, 64]}
+                "part_shift": [-1, 0, 1, 2], "split_min": [0, 16, 32, 64]}
 
 
 def _gen_ms(params, tiles: dict, repeats: int) -> float:

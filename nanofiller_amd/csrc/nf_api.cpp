@@ -433,7 +433,7 @@ static void release_gen(nf_handle* h) {
   void* ptrs[] = {b.desc, b.st, b.ri, b.slot_base, b.stencil, b.agg, b.mesh, b.cell_inst, b.oP, b.oD,
                   b.oid, b.ostart, b.ocount, b.ohl, b.bP, b.bD, b.sP, b.sD, b.scell, b.srk,
                   b.surv, b.srank, b.pP, b.pD, b.pslot, b.palive, b.pcount, b.pstart, b.phl,
-                  b.order, b.aP, b.aD, b.aslot, b.aidx, b.acount, b.astart, b.queues, b.scan_tmp};
+                  b.items, b.qcnt, b.aP, b.aD, b.aslot, b.aidx, b.acount, b.astart, b.queues, b.scan_tmp};
   for (void* p : ptrs) dfree(h, p);
   b = GenBuffers();
 }
@@ -542,7 +542,8 @@ extern "C" int nf_create_batch(const nf_params* ps, int n, nf_handle** out) {
   ALLOC(b.palive, b.T_cap);
   ALLOC(b.pcount, b.total_cells);
   ALLOC(b.pstart, b.total_cells + 1);
-  ALLOC(b.order, b.total_cells);
+  ALLOC(b.items, b.total_cells * pair_items_max(b.total_cells));
+  ALLOC(b.qcnt, QUEUES_PER_KERNEL);
   ALLOC(b.aP, b.T_cap);
   ALLOC(b.aD, b.T_cap);
   ALLOC(b.aslot, b.T_cap);

@@ -103,7 +103,7 @@ enum { Q_OLD = 0, Q_NEW = 1, Q_CNT = 2, Q_REC = 3, Q_N = 4 };
 
 // Device buffers of a generation batch.
 // Launch shape of the generation's pair passes (0 / -1: the built-in
-// choice of pair_grid, pair_part_shift and pair_split_min).
+// choice of pair_grid and of the work list's costs).
 struct PairTiles {
   uint32_t waves_old = 0;  // waves per CU, reject vs accepted rods
   uint32_t waves_new = 0;  // waves per CU, reject vs same-round proposals
@@ -146,7 +146,8 @@ struct GenBuffers {
   uint32_t* palive = nullptr;
   uint32_t* pcount = nullptr;  // total_cells
   uint32_t* pstart = nullptr;  // total_cells + 1
-  uint32_t* order = nullptr;   // total_cells: work order of a pair pass
+  uint2* items = nullptr;      // total_cells * pair_items_max: work list of a pair pass
+  uint32_t* qcnt = nullptr;    // QUEUES_PER_KERNEL: items in each queue's part of the list
   // survivors of the reject-vs-accepted pass, compacted per cell
   float4* aP = nullptr;
   float4* aD = nullptr;
@@ -225,10 +226,12 @@ struct PairArgs {
   InstState* st;
   const uint32_t* cell_inst;
   uint32_t ncells_total;
-  uint32_t part_shift;  // work items per cell: 1 << part_shift (pair_part_shift)
-  uint32_t split_min;   // probes per part of a split cell, at least (pair_split_min)
+  uint32_t split_min;   // the handle's own split: probes per item of a cell, at least (0: by cost)
+  uint32_t npmax;       // work items per cell, at most
   uint32_t test_all;    // reject vs accepted: test every pair within reach (NF_OPT_TEST_ALL_PAIRS)
-  uint32_t* order;      // ncells_total: work order of the cells (filled by launch_pair; nullptr: none)
+  uint2* items;         // work list of the pass (filled by launch_pair; nullptr: one item per cell)
+  uint32_t* qcnt;       // items per queue
+  int n_inst;
   const int4* stencil;
   uint32_t st_off, st_n;  // used when desc == nullptr (contacts)
   // probes
@@ -320,12 +323,8 @@ void launch_pair(int mode, int prec, const PairArgs& a, hipStream_t s, const Pai
 // rounds: same-round pass 1.72 ms per generation at 16 per CU, 1.82 at 12;
 // with the earlier, smaller rounds 12 per CU had been best).
 int pair_grid(int mode);
-// Work items per cell of a pair pass, as a shift: each dense cell's stencil
-// walk is dealt over 1 << shift items, so that dense cells do not hold a
-// launch back.  launch_pair applies it to launches with fewer than 16 cells
-// per wave of the grid.
-int pair_part_shift(int mode);
-int pair_split_min(int mode);
+// Work items of one cell of a generation pass, at most (sizes the work list).
+uint32_t pair_items_max(uint64_t ncells);
 
 // ---- launchers (nf_seg.hip) ----
 void launch_seg_cross(int prec, const SegCrossArgs& a, hipStream_t s);

@@ -1,7 +1,8 @@
 // nf_pair.hip - the cell-pair engine.
 //
-// One 64-lane wavefront (one workgroup) per home cell, taken from 64 work
-// queues (eight per XCD, each counter on its own cache line).  The home
+// One 64-lane wavefront (one workgroup) per work item, a home cell or a part
+// of one (k_items), taken from 64 work queues (eight per XCD, each counter on
+// its own cache line).  The home
 // cell's probes are taken 64 at a time, one per lane, and read by the
 // other lanes with readlane.  The stencil, sorted by minimum cell-to-cell
 // distance, is looked up 64 offsets at a time (one round trip), and the
@@ -325,8 +326,8 @@ __device__ __forceinline__ void screen_batch(const PairArgs& a, const CellGeom& 
 // taken in stencil (lane) order with readlane.  All other fields are
 // wave-uniform.
 struct StencilCursor {
-  uint32_t sb;              // next stencil block (first offset)
-  uint32_t step;            // offsets from one block of this work item to its next
+  uint32_t sb;              // next stencil block (first offset of this work item)
+  uint32_t nst;             // stencil parts of the cell: the item's offsets lie nst apart
   unsigned long long mask;  // relevant cells of the block not yet taken
   uint32_t cS, cN, cM;      // per lane: the lane's cell of the block
   uint32_t start;           // current neighbour cell: first index, rod count, staged so far
@@ -342,7 +343,7 @@ __device__ void refill_cells(const PairArgs& a, const CellGeom& g, PairLds& L, S
                              int c0, int c1, int c2, float chunk_hl, float rr_chunk2) {
   const int lane = threadIdx.x;
   while (!c.last) {
-    const uint32_t si = c.sb + (uint32_t)lane;
+    const uint32_t si = c.sb + (uint32_t)lane * c.nst;
     const bool valid = si < g.st_n;
     const int4 so = g.st[min(si, g.st_n - 1u)];
     const float md2 = __int_as_float(so.w);
@@ -375,8 +376,8 @@ __device__ void refill_cells(const PairArgs& a, const CellGeom& g, PairLds& L, S
     c.cS = st0;
     c.cN = n;
     c.cM = (uint32_t)pack_img(img[0], img[1], img[2]) | (same ? 0x80000000u : 0u);
-    const bool stop = (__ballot(beyond) != 0ull) || (c.sb + c.step >= g.st_n);
-    c.sb += c.step;
+    const bool stop = (__ballot(beyond) != 0ull) || (c.sb + WAVE * c.nst >= g.st_n);
+    c.sb += WAVE * c.nst;
     c.mask = mk;
     if (stop) c.last = true;
     if (mk != 0ull) return;
@@ -498,16 +499,16 @@ __device__ __forceinline__ void probe_loop(const PairArgs& a, const CellGeom& g,
 // count or cut is queued.  The probe's part of rr'' is computed per lane,
 // the slot's part is staged with the slot (Q.w).
 //
-// A cell is 1 << part_shift work items (parts).  A cell with more than
-// split_min probes uses np = min(parts, ceil(probes / split_min)) of them:
-// part k < np walks the stencil blocks k, k + np, k + 2 np, ... (64 offsets
-// each), so the parts partition the pairs of the cell and a dense cell is
-// worked on by several waves at once; parts k >= np return at once.
-// The probe bytes, counted per probe, belong to part 0.
+// A work item is one probe chunk group and one stencil part of a cell
+// (k_items): the cell's probes are dealt into nch equal chunks of at most 64;
+// the item takes the chunks cg, cg + ncg, ... and the stencil offsets sp,
+// sp + nst, ..., so the ncg * nst items of a cell partition its pairs and a
+// dense cell is worked on by several waves at once.  Interleaved offsets
+// give every part near and far cells alike.  The probe bytes, counted per
+// probe, belong to part sp = 0.
 template <int MODE, int PREC>
-__device__ void process_cell(const PairArgs& a, const CellGeom& g, uint32_t gc, uint32_t part,
-                             PairLds& L, Acc& acc) {
-  constexpr bool GEN = (MODE == PM_GEN_OLD || MODE == PM_GEN_NEW);
+__device__ void process_cell(const PairArgs& a, const CellGeom& g, uint32_t gc, uint32_t cg, uint32_t ncg,
+                             uint32_t sp, uint32_t nst, PairLds& L, Acc& acc) {
   const int lane = threadIdx.x;
   // an instance without proposals (finished, or planned none) or without
   // accepted rods (its first round) has no pairs: its cells would walk their
@@ -516,8 +517,8 @@ __device__ void process_cell(const PairArgs& a, const CellGeom& g, uint32_t gc, 
   uint32_t pc = uni(g.hCount[gc]);
   if (MODE == PM_GEN_OLD && g.inv) pc = min(pc, g.cap);  // accepted cells hold at most cap rods
   if (pc == 0) return;
-  const uint32_t np = min(1u << a.part_shift, (pc + a.split_min - 1u) / a.split_min);
-  if (part >= np) return;
+  const uint32_t nch = (pc + WAVE - 1u) / WAVE;
+  const uint32_t csz = (pc + nch - 1u) / nch;  // probes per chunk
   const uint32_t ps = uni(g.hStart[gc]);
   const uint32_t lc = gc - g.cell_base;
   const int c0 = (int)(lc % (uint32_t)g.nc[0]);
@@ -525,8 +526,8 @@ __device__ void process_cell(const PairArgs& a, const CellGeom& g, uint32_t gc, 
   const int c2 = (int)(lc / ((uint32_t)g.nc[0] * (uint32_t)g.nc[1]));
   const float pad_r = g.R_max + 16.0f * g.ew;
 
-  for (uint32_t pb = 0; pb < pc; pb += WAVE) {
-    const uint32_t G = min((uint32_t)WAVE, pc - pb);
+  for (uint32_t pb = cg * csz; pb < pc; pb += ncg * csz) {
+    const uint32_t G = min(csz, pc - pb);
     // lane l holds probe l of the chunk (clamped loads, every lane loads)
     const bool inrange = (uint32_t)lane < G;
     const uint32_t pidx = ps + pb + min((uint32_t)lane, G - 1u);
@@ -541,15 +542,16 @@ __device__ void process_cell(const PairArgs& a, const CellGeom& g, uint32_t gc, 
     // probes taking part, as a wave-uniform mask; the prefilter reads each
     // probe from its lane's registers
     unsigned long long pmask = __ballot(have);
-    if (pmask == 0ull) continue;  // every probe of the chunk already cut: nothing to stage
     const float chunk_hl = unif(wave_max(have ? P1.w : 0.0f));
-    if (part == 0u) acc.bytes += (unsigned long long)G * 36ull;
+    if (sp == 0u) acc.bytes += (unsigned long long)G * 36ull;
     const float rr_chunk = (chunk_hl + g.hl_max) * 1.000001f + g.R_max + CELL_MARGIN;
     const float rr_chunk2 = rr_chunk * rr_chunk;
     uint32_t qn = 0;   // wave-uniform queue lengths: prefiltered pairs,
     uint32_t q2n = 0;  // and pairs waiting for the full test
-    StencilCursor cur{part * (uint32_t)WAVE, np * (uint32_t)WAVE, 0ull, 0u, 0u, 0u, 0u, 0u, 0u, 0u,
-                      false, false};
+    StencilCursor cur{sp, nst, 0ull, 0u, 0u, 0u, 0u, 0u, 0u, 0u, false, false};
+    // several parts walk for this chunk's proposals: each tells the others of
+    // its cuts through the alive flags
+    const bool share = MODE == PM_GEN_OLD && !g.inv && !a.test_all && nst > 1u;
     __syncthreads();
 
     while (!cur.done) {
@@ -590,6 +592,10 @@ __device__ void process_cell(const PairArgs& a, const CellGeom& g, uint32_t gc, 
         x0 = g.nX[src0];
         x1 = g.nX[src1];
       }
+      // the proposals that the cell's other parts have cut meanwhile
+      uint32_t alive = 1u;
+      if (share)
+        alive = __hip_atomic_load(&a.alive_out[pidx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       L.bP[lane] = p0;
       L.bD[lane] = d0;
       L.bX[lane] = x0;
@@ -618,6 +624,10 @@ __device__ void process_cell(const PairArgs& a, const CellGeom& g, uint32_t gc, 
         const bool o0 = v0 && ((m0 & 0x80000000u) != 0u || src0 - qlo < G);
         const bool o1 = v1 && ((m1 & 0x80000000u) != 0u || src1 - qlo < G);
         ord = __ballot(o0 || o1) != 0ull;
+      }
+      if (share) {
+        pmask &= __ballot(alive != 0u);
+        if (pmask == 0ull) break;
       }
       __syncthreads();
       // ---- prefilter every (probe, slot) pair, queue the survivors
@@ -656,7 +666,10 @@ __device__ void process_cell(const PairArgs& a, const CellGeom& g, uint32_t gc, 
         // stencil is sorted by distance, so near a jammed state most
         // proposals leave after their first batches.  The decisions are
         // unchanged; the pair-test count is then the pairs evaluated.
-        pmask = __ballot(have && L.hit[lane] == 0u);
+        const bool cut = have && L.hit[lane] != 0u;
+        if (share && cut && ((pmask >> lane) & 1ull))
+          __hip_atomic_store(&a.alive_out[pidx], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        pmask &= ~__ballot(cut);
         if (pmask == 0ull) break;
       }
     }
@@ -669,6 +682,24 @@ __device__ void process_cell(const PairArgs& a, const CellGeom& g, uint32_t gc, 
     }
     __syncthreads();
   }
+}
+
+// Reject-vs-accepted pass: an instance's proposals of this round and accepted
+// rods.  Accepted-major (inv) when the accepted rods outnumber the proposals
+// four to one: fewer, denser probe chunks stage the sparser set (the pair set
+// and every decision are the same).  Below that ratio the proposals are the
+// probes, so that cut ones can leave their walk early.  idle: no pairs.
+struct OldRoles {
+  uint32_t nacc, nprop;
+  bool inv, idle;
+};
+__device__ __forceinline__ OldRoles old_roles(const PairArgs& a, uint32_t inst, const InstDesc& d) {
+  OldRoles r;
+  r.nacc = a.st[inst].n_acc;
+  r.nprop = a.prStart[d.cell_base + d.ncells] - a.prStart[d.cell_base];
+  r.inv = r.nacc > 4u * r.nprop;
+  r.idle = r.nprop == 0u || r.nacc == 0u;
+  return r;
 }
 
 template <int MODE, int PREC>
@@ -725,28 +756,50 @@ __global__ void __launch_bounds__(PAIR_THREADS, 4) k_pair(PairArgs a) {
   // vector load of the 64 counters finds the first queue with work left.
   const int sub0 = (blockIdx.x >> 3) & 7;
   const int my_q = (((xcd + (threadIdx.x >> 3)) & 7) << 3) | ((sub0 + (int)threadIdx.x) & 7);
-  // queue q: the parts of cells [W q / 64, W (q + 1) / 64) (k_order's ranges)
-  const uint32_t my_qb = (uint32_t)(((uint64_t)W * (uint32_t)my_q) / QUEUES_PER_KERNEL) << a.part_shift;
-  const uint32_t my_qe = (uint32_t)(((uint64_t)W * (uint32_t)(my_q + 1)) / QUEUES_PER_KERNEL) << a.part_shift;
+  // queue q: the items of cells [W q / 64, W (q + 1) / 64), from k_items's
+  // list, or (no list) the cells themselves, one item each
+  const uint32_t my_c0 = (uint32_t)(((uint64_t)W * (uint32_t)my_q) / QUEUES_PER_KERNEL);
+  const uint32_t my_c1 = (uint32_t)(((uint64_t)W * (uint32_t)(my_q + 1)) / QUEUES_PER_KERNEL);
+  const uint32_t my_qb = a.items ? my_c0 * a.npmax : my_c0;
+  const uint32_t my_qn = a.items ? a.qcnt[my_q] : my_c1 - my_c0;
+  // the first pre items of each queue belong to its own waves, one each: a
+  // short launch needs no queue grab to begin
+  const uint32_t pre = gridDim.x / QUEUES_PER_KERNEL;
+  const uint32_t rank = blockIdx.x / QUEUES_PER_KERNEL;
+  bool first = rank < pre;
   for (;;) {
-    const uint32_t seen =
-        __hip_atomic_load(&a.qctr[my_q * QSTRIDE], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const unsigned long long open = __ballot(seen < my_qe - my_qb);
-    if (open == 0ull) break;
-    const int pick = (int)__builtin_ctzll(open);  // uniform
+    int pick = 0;  // uniform
+    if (!first) {
+      const uint32_t seen =
+          __hip_atomic_load(&a.qctr[my_q * QSTRIDE], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const unsigned long long open = __ballot(seen + pre < my_qn);
+      if (open == 0ull) break;
+      pick = (int)__builtin_ctzll(open);
+    }
     const int q = __builtin_amdgcn_readlane(my_q, pick);
     const uint32_t qb = uni((uint32_t)__builtin_amdgcn_readlane((int)my_qb, pick));
-    const uint32_t qe = uni((uint32_t)__builtin_amdgcn_readlane((int)my_qe, pick));
+    const uint32_t qn = uni((uint32_t)__builtin_amdgcn_readlane((int)my_qn, pick));
     for (;;) {
-      // lane 0 takes the next item; readfirstlane makes it a scalar, so the
-      // loop exit below is uniform
-      uint32_t old = 0u;
-      if (l0) old = atomicAdd(&a.qctr[q * QSTRIDE], 1u);
-      const uint32_t item = uni(old);
-      if (item >= qe - qb) break;
-      const uint32_t ci = (qb + item) >> a.part_shift;
-      const uint32_t gc = a.order ? uni(a.order[ci]) : ci;
-      const uint32_t part = (qb + item) & ((1u << a.part_shift) - 1u);
+      uint32_t item = rank;
+      if (!first) {
+        // lane 0 takes the next item; readfirstlane makes it a scalar, so the
+        // loop exit below is uniform
+        uint32_t old = 0u;
+        if (l0) old = atomicAdd(&a.qctr[q * QSTRIDE], 1u);
+        item = uni(old) + pre;
+      }
+      first = false;
+      if (item >= qn) break;
+      uint32_t gc = qb + item, cg = 0u, ncg = 1u, sp = 0u, nst = 1u;
+      if (a.items) {
+        const uint2 w = a.items[qb + item];
+        gc = uni(w.x);
+        const uint32_t code = uni(w.y);
+        cg = code & 0xFFu;
+        ncg = (code >> 8) & 0xFFu;
+        sp = (code >> 16) & 0xFFu;
+        nst = code >> 24;
+      }
       if (GEN) {
         const uint32_t inst = uni(a.cell_inst[gc]);
         if (inst != cur_inst) {
@@ -772,15 +825,9 @@ __global__ void __launch_bounds__(PAIR_THREADS, 4) k_pair(PairArgs a) {
           g.state = &a.st[inst];
           cur_inst = inst;
           if (MODE == PM_GEN_OLD) {
-            // accepted-major when the instance's accepted rods outnumber
-            // this round's proposals four to one: fewer, denser probe chunks
-            // stage the sparser set (the pair set and every decision are the
-            // same).  Below that ratio the proposals are the probes, so that
-            // cut ones can leave their walk early.
-            const uint32_t nacc = uni(a.st[inst].n_acc);
-            const uint32_t nprop = uni(a.prStart[d.cell_base + d.ncells]) - uni(a.prStart[d.cell_base]);
-            g.inv = nacc > 4u * nprop;
-            g.idle = nprop == 0u || nacc == 0u;
+            const OldRoles r = old_roles(a, inst, d);
+            g.inv = uni(r.inv ? 1u : 0u) != 0u;
+            g.idle = uni(r.idle ? 1u : 0u) != 0u;
             g.hP = g.inv ? a.nbP : a.prP;
             g.hD = g.inv ? a.nbD : a.prD;
             g.hX = g.inv ? a.nbX : a.prX;
@@ -798,71 +845,154 @@ __global__ void __launch_bounds__(PAIR_THREADS, 4) k_pair(PairArgs a) {
           }
         }
       }
-      process_cell<MODE, PREC>(a, g, gc, part, L, acc);
+      process_cell<MODE, PREC>(a, g, gc, cg, ncg, sp, nst, L, acc);
     }
   }
   if (!GEN || cur_inst != 0xFFFFFFFFu) flush<GEN>(a, g, acc, MODE);
 }
 
-// Work order of a pair pass: within each of the 64 queue ranges of cells,
-// the cells by decreasing estimated cost, so that each queue starts with its
-// costliest cells and the launch ends on light ones.  The cost of a cell is
-// the rods around (its probe and neighbour counts) times the volume its
-// stencil walk covers, (h + H)^3, h the cell's longest rod (half length) and
-// H the instance's longest half length plus a cell edge; two buckets per
-// octave.  One workgroup per range; the order inside a bucket is arbitrary,
-// as every result of a pair pass is independent of the order of its work.
-constexpr int ORDER_BUCKETS = 32;
-constexpr int ORDER_THREADS = 256;
-__device__ __forceinline__ uint32_t order_bucket(const PairArgs& a, uint32_t c) {
-  const InstDesc& d = a.desc[a.cell_inst[c]];
-  const float h = fmaxf(a.prHl[c], a.nbHl[c]) + d.hl_max + d.edge[0];
-  const float w = (float)(a.prCount[c] + a.nbCount[c]) * h * h * h;
-  // (bits >> 22) = 2 * biased exponent + first mantissa bit; bucket 0: w >= 2^13
-  const int k = 283 - (int)(__float_as_uint(w) >> 22);
-  return (uint32_t)min(max(k, 0), ORDER_BUCKETS - 1);
+// Work list of a generation pass: per queue range of cells, the items of its
+// cells that hold probes (and whose instance has pairs), costliest first, so
+// that each queue starts with its costliest items and the launch ends on
+// light ones.
+//
+// A cell's cost is its probes times the rods its walk is expected to stage:
+// the volume of the walk (a cube of edge two reaches plus a cell edge, less
+// its corners) times the mean of the cell's own neighbour density and the
+// instance's.  A cell is dealt over ceil(cost / share) items: share is the
+// launch's whole cost over ITEMS_PER_WAVE items per wave of the grid, but at
+// least ITEM_FULL pairs, so that an item's own overhead (queue grab, probe
+// loads, stencil look-up) stays small, or, where that would leave waves
+// without an item, one wave's part of the cost down to ITEM_MIN pairs.
+// Chunks of probes are dealt first: they share no staging anyway.  Two cost
+// buckets per octave; the order inside a bucket is arbitrary, as every result
+// of a pair pass is independent of the order of its work.
+//
+// What bounds a launch over few cells is the longest cell on one wave: 125
+// cells of 160 rods kept 125 to 250 of the 4096 waves busy.  Measured on
+// MI355X against one item per cell (at most two for the reject-vs-accepted
+// pass), whole generations: 20,000 rods on 1 um cells, FP64, 10.2 -> 3.9 ms;
+// 2,000 rods 1.84 -> 0.72 ms; 32 uneven packings 244 -> 153 ms, where empty
+// cells had also been taken one by one; 500,000 and 4M rods unchanged.
+// 2, 8 and 16 items per wave: the 32 packings 156, 164 and 191 ms.
+constexpr int ITEM_BUCKETS = 48;
+constexpr int ITEM_THREADS = 512;
+constexpr float ITEMS_PER_WAVE = 4.0f;
+constexpr float ITEM_MIN = 4096.0f, ITEM_FULL = 16384.0f;
+
+struct ItemPlan {
+  uint32_t ncg, nst, bucket;
+};
+
+// Walk volume of a cell whose longest probe has half length h, over the box.
+__device__ __forceinline__ float walk_share(const InstDesc& d, float h) {
+  float v = 0.8f;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const float e = 2.0f * (h + d.hl_max + d.R_max) + d.edge[k];
+    v *= e / d.boxf[k];
+  }
+  return v;
 }
 
-__global__ void __launch_bounds__(ORDER_THREADS) k_order(PairArgs a) {
-  __shared__ uint32_t slot[ORDER_BUCKETS];
+template <int MODE>
+__device__ __forceinline__ bool item_plan(const PairArgs& a, uint32_t c, float share, ItemPlan* o) {
+  const uint32_t inst = a.cell_inst[c];
+  const InstDesc& d = a.desc[inst];
+  uint32_t pc, nb, total;
+  float h;
+  if (MODE == PM_GEN_OLD) {
+    const OldRoles r = old_roles(a, inst, d);
+    if (r.idle) return false;
+    pc = min(r.inv ? a.nbCount[c] : a.prCount[c], r.inv ? d.cap : 0xFFFFFFFFu);
+    nb = r.inv ? a.prCount[c] : a.nbCount[c];
+    total = r.inv ? r.nprop : r.nacc;
+    h = r.inv ? a.nbHl[c] : a.prHl[c];
+  } else {
+    pc = nb = a.prCount[c];
+    total = a.prStart[d.cell_base + d.ncells] - a.prStart[d.cell_base];
+    h = a.prHl[c];
+  }
+  if (pc == 0u) return false;
+  float w = (float)pc * walk_share(d, h) * 0.5f * ((float)total + (float)nb * (float)d.ncells);
+  if (MODE == PM_GEN_NEW) w *= 0.5f;  // half stencil
+  const uint32_t np = (uint32_t)fminf(ceilf(w / share), (float)a.npmax);
+  const uint32_t nch = (pc + WAVE - 1u) / WAVE;
+  o->ncg = max(1u, min(nch, np));
+  const uint32_t st_n = MODE == PM_GEN_NEW ? d.hst_n : d.st_n;
+  o->nst = max(1u, min(np / o->ncg, min(st_n, 255u)));
+  if (a.split_min != 0u) {
+    // the handle's own split (NF_OPT_PART_SHIFT, NF_OPT_SPLIT_MIN): at most
+    // npmax stencil parts of at least split_min probes each
+    o->ncg = 1u;
+    o->nst = max(1u, min(a.npmax, (pc + a.split_min - 1u) / a.split_min));
+  }
+  w /= (float)(o->ncg * o->nst);
+  // (bits >> 22) = 2 * biased exponent + first mantissa bit; bucket 0: w >= 2^24
+  const int k = 2 * (127 + 24) - (int)(__float_as_uint(w) >> 22);
+  o->bucket = (uint32_t)min(max(k, 0), ITEM_BUCKETS - 1);
+  return true;
+}
+
+template <int MODE>
+__global__ void __launch_bounds__(ITEM_THREADS) k_items(PairArgs a, float waves) {
+  __shared__ uint32_t slot[ITEM_BUCKETS];
+  __shared__ float part[ITEM_THREADS / WAVE];
   const uint32_t r = blockIdx.x;
   const uint32_t c0 = (uint32_t)(((uint64_t)a.ncells_total * r) / QUEUES_PER_KERNEL);
   const uint32_t c1 = (uint32_t)(((uint64_t)a.ncells_total * (r + 1u)) / QUEUES_PER_KERNEL);
-  if (threadIdx.x < ORDER_BUCKETS) slot[threadIdx.x] = 0u;
-  __syncthreads();
-  for (uint32_t c = c0 + threadIdx.x; c < c1; c += ORDER_THREADS) atomicAdd(&slot[order_bucket(a, c)], 1u);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t sum = c0;
-    for (int k = 0; k < ORDER_BUCKETS; ++k) {
-      const uint32_t t = slot[k];
-      slot[k] = sum;
-      sum += t;
+  if (threadIdx.x < ITEM_BUCKETS) slot[threadIdx.x] = 0u;
+  // the launch's whole cost, from the instances' totals
+  float sum = 0.0f;
+  for (int i = threadIdx.x; i < a.n_inst; i += ITEM_THREADS) {
+    const InstDesc& d = a.desc[i];
+    if (MODE == PM_GEN_OLD) {
+      const OldRoles o = old_roles(a, (uint32_t)i, d);
+      if (!o.idle) sum += (float)o.nacc * (float)o.nprop * walk_share(d, d.hl_max);
+    } else {
+      const float n = (float)(a.prStart[d.cell_base + d.ncells] - a.prStart[d.cell_base]);
+      sum += 0.5f * n * n * walk_share(d, d.hl_max);
     }
   }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, WAVE);
+  if ((threadIdx.x & (WAVE - 1)) == 0) part[threadIdx.x / WAVE] = sum;
   __syncthreads();
-  for (uint32_t c = c0 + threadIdx.x; c < c1; c += ORDER_THREADS)
-    a.order[atomicAdd(&slot[order_bucket(a, c)], 1u)] = c;
+  sum = 0.0f;
+  for (int k = 0; k < ITEM_THREADS / WAVE; ++k) sum += part[k];
+  const float share = fmaxf(sum / (waves * ITEMS_PER_WAVE), fminf(fmaxf(sum / waves, ITEM_MIN), ITEM_FULL));
+  ItemPlan p;
+  for (uint32_t c = c0 + threadIdx.x; c < c1; c += ITEM_THREADS)
+    if (item_plan<MODE>(a, c, share, &p)) atomicAdd(&slot[p.bucket], p.ncg * p.nst);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint32_t at = 0;
+    for (int k = 0; k < ITEM_BUCKETS; ++k) {
+      const uint32_t t = slot[k];
+      slot[k] = at;
+      at += t;
+    }
+    a.qcnt[r] = at;
+  }
+  __syncthreads();
+  uint2* out = a.items + (uint64_t)c0 * a.npmax;
+  for (uint32_t c = c0 + threadIdx.x; c < c1; c += ITEM_THREADS) {
+    if (!item_plan<MODE>(a, c, share, &p)) continue;
+    uint32_t at = atomicAdd(&slot[p.bucket], p.ncg * p.nst);
+    for (uint32_t sp = 0; sp < p.nst; ++sp)
+      for (uint32_t cg = 0; cg < p.ncg; ++cg)
+        out[at++] = make_uint2(c, cg | (p.ncg << 8) | (sp << 16) | (p.nst << 24));
+  }
+}
+
+// Items per cell at most: about 2^19 list entries in all, between 2 and 64
+// per cell.
+uint32_t pair_items_max(uint64_t ncells) {
+  const uint64_t k = ((uint64_t)1 << 19) / (ncells ? ncells : 1);
+  return (uint32_t)(k < 2 ? 2 : (k > 64 ? 64 : k));
 }
 
 static int g_cus = 0;
-
-// Two parts per cell for the reject-vs-accepted pass, whose
-// agglomerate-dense cells otherwise end a launch alone; none for the
-// same-round and contact passes.  Used only when a launch has fewer than 16
-// cells per wave (launch_pair): with more, dense cells are spread over many
-// items per wave anyway, and the grabs of empty parts cost more than they
-// save.  Measured on MI355X (500k-rod generation, 12k cells, with the
-// dense-first order of k_order): reject-vs-accepted pass 2.72 ms with two
-// parts of at least 32 probes, 2.77 with 24, 2.97 with four parts;
-// same-round pass 1.80 ms unsplit, 1.91-2.06 split.  The 256-packing batch
-// (1M+ cells): 301 ms unsplit, 312 split.
-int pair_part_shift(int mode) { return mode == PM_GEN_OLD ? 1 : 0; }
-
-int pair_split_min(int mode) {
-  (void)mode;
-  return 32;
-}
 
 int pair_grid(int mode) {
   if (g_cus == 0) {
@@ -884,16 +1014,18 @@ void launch_pair(int mode, int prec, const PairArgs& args, hipStream_t s, const 
   const int cus = pair_grid(mode) / 16;
   const dim3 grid(waves ? (uint32_t)cus * waves : (uint32_t)pair_grid(mode)), block(PAIR_THREADS);
   PairArgs a = args;
-  // launches with few cells per wave: costliest cells first (under 64 per
-  // wave), dense cells split (under 16 per wave)
-  const bool small = a.ncells_total < 16u * grid.x;
-  const int ps = (t && mode == PM_GEN_OLD && t->part_shift >= 0) ? t->part_shift : pair_part_shift(mode);
-  a.part_shift = small ? (uint32_t)ps : 0u;
-  if (a.ncells_total < 64u * grid.x && a.order != nullptr)
-    hipLaunchKernelGGL(k_order, dim3(QUEUES_PER_KERNEL), dim3(ORDER_THREADS), 0, s, a);
-  else
-    a.order = nullptr;
-  a.split_min = (t && t->split_min) ? t->split_min : (uint32_t)pair_split_min(mode);
+  if (a.items != nullptr) {
+    a.npmax = pair_items_max(a.ncells_total);
+    a.split_min = 0u;
+    if (t && mode == PM_GEN_OLD && (t->part_shift >= 0 || t->split_min != 0u)) {
+      a.split_min = t->split_min ? t->split_min : 32u;
+      a.npmax = min(a.npmax, 1u << (t->part_shift >= 0 ? t->part_shift : 1));
+    }
+    if (mode == PM_GEN_OLD)
+      hipLaunchKernelGGL(k_items<PM_GEN_OLD>, dim3(QUEUES_PER_KERNEL), dim3(ITEM_THREADS), 0, s, a, (float)grid.x);
+    else
+      hipLaunchKernelGGL(k_items<PM_GEN_NEW>, dim3(QUEUES_PER_KERNEL), dim3(ITEM_THREADS), 0, s, a, (float)grid.x);
+  }
   a.test_all = (t && mode == PM_GEN_OLD) ? t->test_all : 0u;
 #define NF_LAUNCH(M, P) hipLaunchKernelGGL((k_pair<M, P>), grid, block, 0, s, a)
   if (prec == NF_PREC_FP64) {
