@@ -42,7 +42,7 @@ SOURCES = [
     "nf_noalloc.hip",
     "nf_reduce.hip",
 ]
-HEADERS = ["nf_common.h", "nf_internal.h", "nf_host.h", "nf_seg.h"]
+HEADERS = ["nf_common.h", "nf_internal.h", "nf_host.h", "nf_seg.h", "nf_line.h"]
 ARCH = os.environ.get("NF_OFFLOAD_ARCH", "gfx950")
 
 

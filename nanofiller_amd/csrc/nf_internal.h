@@ -228,7 +228,6 @@ struct PairArgs {
   uint32_t ncells_total;
   uint32_t split_min;   // the handle's own split: probes per item of a cell, at least (0: by cost)
   uint32_t npmax;       // work items per cell, at most
-  uint32_t test_all;    // reject vs accepted: test every pair within reach (NF_OPT_TEST_ALL_PAIRS)
   uint2* items;         // work list of the pass (filled by launch_pair; nullptr: one item per cell)
   uint32_t* qcnt;       // items per queue
   int n_inst;

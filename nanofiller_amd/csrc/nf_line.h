@@ -1,0 +1,72 @@
+// nf_line.h - the line filter of the generation passes: a pair of rods whose
+// infinite axes certainly stay apart cannot overlap.
+//
+// With p and q the centres from a common origin, u1 and u2 the directions and
+// v = u1 x u2, the distance of the two lines is |w.v| / |v|, w = p - q, and
+// never exceeds the segments' (Lumelsky 1985).  From the lines' moments
+// m = centre x direction,
+//   w.v = m1.u2 + m2.u1   and   |v|^2 = 1 - (u1.u2)^2,
+// so with t = w.v / R and c = u1.u2 (moments stored over R)
+//   t^2 + c^2 - 1 - slack >= 0
+// drops the pair: 11 FMAs and one multiplication, no root, no quotient, and
+// each rod's side depends on the rod alone.
+//
+// Margins.  R exceeds the cut distance by its roundings and by the FP64
+// algorithm's error bound (1e-12 S^2 in the squared distance, see pair_f32).
+// A pair that may be cut lies within reach, so with S = |p| + hl1 + hl2 + R
+// over all pairs of the pass both centres are below S.  The error of w.v:
+// w's components are each off by less than 4 ew (ew bounds the rounding of a
+// shifted centre; centre, shift and origin give 2 ew per rod), together less
+// than 8 ew |v|; the moments' products and sums, each below 2 S, take 4
+// roundings per component and the six-term sum 6 more of values below 4 S:
+// below 64 u S.  So |t| is off by less than Et = (8 ew + 64 u S) / R, which
+// raises t^2 by less than 2 Et + Et^2 where |t| <= 1; c^2 and the directions'
+// own norms (within 4 u of 1) are off by less than 24 u.  The slack takes
+// 64 u for these and the three last roundings.
+#pragma once
+
+#include "nf_common.h"
+
+namespace nf {
+
+struct LineFilter {
+  float scale;  // 1 / R, rounded down
+  float slack;
+};
+
+struct LineSide {
+  float ux, uy, uz;  // direction
+  float mx, my, mz;  // moment over R
+};
+
+// R_max: largest cut distance; S: see above.
+NF_HD LineFilter line_filter(float R_max, float ew, float S) {
+  const float R2 = fmaf(R_max * 1.00002f, R_max, 2e-12f * S * S);
+  LineFilter f;
+  f.scale = recip(sqrt_up(R2)) * (1.0f - 4.0f * U32);
+  const float Et = (8.0f * ew + 64.0f * U32 * S) * f.scale;
+  f.slack = fmaf(Et, Et, 2.0f * Et) * 1.001f + 64.0f * U32;
+  return f;
+}
+
+// (x, y, z): the centre from the common origin.
+NF_HD LineSide line_side(const LineFilter& f, float x, float y, float z, const float4 D) {
+  LineSide s;
+  s.ux = D.x;
+  s.uy = D.y;
+  s.uz = D.z;
+  s.mx = f.scale * fmaf(y, D.z, -(z * D.y));
+  s.my = f.scale * fmaf(z, D.x, -(x * D.z));
+  s.mz = f.scale * fmaf(x, D.y, -(y * D.x));
+  return s;
+}
+
+// Negative when the lines may come within R; b = -1 - slack.
+NF_HD float line_apart(const LineSide& p, const LineSide& q, float b) {
+  const float t =
+      fmaf(p.ux, q.mx, fmaf(p.uy, q.my, fmaf(p.uz, q.mz, fmaf(p.mx, q.ux, fmaf(p.my, q.uy, p.mz * q.uz)))));
+  const float c = fmaf(p.ux, q.ux, fmaf(p.uy, q.uy, p.uz * q.uz));
+  return fmaf(t, t, fmaf(c, c, b));
+}
+
+}  // namespace nf

@@ -8,7 +8,7 @@
 // distance, is looked up 64 offsets at a time (one round trip), and the
 // neighbour cells that can reach the chunk are packed into a 128-slot
 // staging buffer (two slots per lane).  Every (probe, slot) pair passes a
-// conservative centre-distance prefilter; survivors queue in LDS, go
+// conservative filter; survivors queue in LDS, go
 // through the rigorous FP32 screen 64 at a time, and those the screen
 // cannot settle get the full FP32-band / FP64 test 64 at a time, so each
 // expensive step runs on dense work.
@@ -28,6 +28,7 @@
 //                                        CONTACT_RECORD in one pass (appended, unsorted)
 //                                        (src/core_cell_interaction_kernel.cu:70-315)
 #include "nf_internal.h"
+#include "nf_line.h"
 
 namespace nf {
 
@@ -59,6 +60,7 @@ struct CellGeom {
   const int4* st;
   uint32_t st_n;
   float ew, hl_max, R_max;
+  float edge[3];
   double sf64, sep64;
   float sf32, sep32;
   uint32_t cap;
@@ -144,14 +146,17 @@ __device__ __forceinline__ void flush(const PairArgs& a, const CellGeom& g, Acc&
 }
 
 // LDS of one wave (under 10 KB, so 16 waves fit a CU): the probe chunk, the
-// staged neighbour rods and the two pair queues.
+// staged neighbour rods and the two pair queues.  The probes still in the
+// walk sit at the front, in lane order (compact_probes).
 constexpr int SLOTS = 2 * WAVE;
-constexpr int QCAP = 3 * WAVE;
+constexpr int QCAP = 2 * WAVE;   // fewer than 64 wait between pushes of up to 64
+constexpr int PUNROLL = 4;       // probes per trip of the filter loop
 struct PairLds {
   float4 sP[WAVE], sD[WAVE];  // probes of the chunk
+  float4 pf[WAVE];            // filter: direction, x of the moment (every pair: 2 (P - o), 2 rp)
+  float2 pg[WAVE];            // filter: y and z of the moment (every pair: |P - o|^2 - rp^2 - slack)
   uint32_t sX[WAVE];
-  uint32_t hit[WAVE];          // per probe: overlaps something (generation)
-  uint32_t dummy[WAVE];        // sink of branch-free stores
+  uint32_t hit[WAVE];           // per probe: overlaps something (generation)
   float4 bP[SLOTS], bD[SLOTS];  // staged neighbour rods
   uint32_t bX[SLOTS];           // rod id (0xFFFFFFFF: not a candidate)
   uint32_t bM[SLOTS];           // image code | same cell << 31
@@ -406,98 +411,180 @@ __device__ __forceinline__ void next_cell(const PairArgs& a, const CellGeom& g, 
   c.off = 0u;
 }
 
-// Prefilter of one (probe, slot) pair, the slot's data in registers:
-// centre distance against the pair's own reach bound rp + Q2.w (the probe's
-// part from its lane, the slot's staged with the slot), and the
-// pass-specific pair filters.  Unfilled slots sit at 1e30, so the
-// distance test drops them.  Keeps every pair the full test could count or
-// cut (see process_cell).  ORD: the batch holds slots the ordering below
-// can drop (else it keeps every pair, and is left out).
-template <int MODE, bool ORD>
-__device__ __forceinline__ bool prefilter(const float4 P1, float rp, uint32_t X1, uint32_t qprobe,
-                                          const float4 Q2, uint32_t xj, uint32_t qa, uint32_t qb) {
-  constexpr bool CNT = (MODE == PM_CNT);
-  const float wx = P1.x - Q2.x, wy = P1.y - Q2.y, wz = P1.z - Q2.z;
-  const float w2 = fmaf(wz, wz, fmaf(wy, wy, wx * wx));
-  const float rr = rp + Q2.w;  // the pair's own reach bound
-  bool f = w2 <= rr * rr;
-  // half-stencil passes (contacts, same-round): a slot of the home cell only
-  // after the probe's index; another cell (an image may map back to the home
-  // cell) never the probe itself
-  if ((CNT || MODE == PM_GEN_NEW) && ORD) f = f && (qprobe < qa || qprobe > qb);
-  return f;
+// Constants of the filter for one home cell.
+struct Filter {
+  float3 o;       // origin: the cell's centre
+  LineFilter ln;  // nf_line.h (every pair: slack 64 u S^2, see process_cell)
+};
+
+// A slot's side of the filter: its line, or, where every pair within reach is
+// tested, its centre (u), the reach part rq (mx) and rq^2 - |centre|^2 (b).
+struct SlotPre {
+  LineSide l;
+  float b;  // -1 - slack; an unfilled slot is apart from everything
+};
+
+// Shifts a pair's verdict into the word: 1 when the lines may come within the
+// cut distance, or (every pair) the centres within reach.
+template <bool ALL>
+__device__ __forceinline__ uint32_t may_cut(const float4 f, const float2 h, const SlotPre& q, uint32_t word) {
+  float d;
+  if (ALL)
+    d = h.x - fmaf(f.w, q.l.mx, fmaf(f.z, q.l.uz, fmaf(f.y, q.l.uy, fmaf(f.x, q.l.ux, q.b))));
+  else
+    d = line_apart(LineSide{f.x, f.y, f.z, f.w, h.x, h.y}, q.l, q.b);
+  return __builtin_amdgcn_alignbit(word, __float_as_uint(d), 31u);
 }
 
-// Appends the prefilter results of every lane for one probe (both slot
-// halves) to the first queue, screening 64 at a time when enough wait.
-template <int MODE, int PREC, bool TWO>
-__device__ __forceinline__ void push_pairs(const PairArgs& a, const CellGeom& g, PairLds& L,
-                                           bool f0, bool f1, uint32_t pp, uint32_t& qn,
-                                           uint32_t& q2n, Acc& acc) {
-  const int lane = threadIdx.x;
-  const unsigned long long m0 = __ballot(f0);
-  const uint32_t n0 = (uint32_t)__popcll(m0);
-  if (f0) L.qE[qn + lane_prefix(m0)] = pp | ((uint32_t)lane << 8);
-  qn += n0;
-  if (TWO) {
-    const unsigned long long m1 = __ballot(f1);
-    if (f1) L.qE[qn + lane_prefix(m1)] = pp | ((uint32_t)(lane + WAVE) << 8);
-    qn += (uint32_t)__popcll(m1);
+template <bool ALL>
+__device__ __forceinline__ SlotPre slot_pre(const float4 P, const float4 D, const float3 sh, const Filter& F,
+                                            bool valid) {
+  SlotPre q;
+  const float x = (P.x + sh.x) - F.o.x, y = (P.y + sh.y) - F.o.y, z = (P.z + sh.z) - F.o.z;
+  if (ALL) {
+    const float r = (P.w * 1.000001f) * 1.000006f;
+    q.l = LineSide{valid ? x : 0.0f, valid ? y : 0.0f, valid ? z : 0.0f, r, 0.0f, 0.0f};
+    q.b = valid ? fmaf(r, r, -fmaf(z, z, fmaf(y, y, x * x))) : -3e38f;
+  } else {
+    q.l = line_side(F.ln, x, y, z, D);
+    q.b = valid ? -1.0f - F.ln.slack : 3e38f;
   }
-  while (qn >= (uint32_t)WAVE) {
-    __syncthreads();
-    screen_batch<MODE, PREC>(a, g, L, qn - WAVE, WAVE, q2n, acc);
-    qn -= WAVE;
+  return q;
+}
+
+// Appends the pairs of one word of probes (bit k: probe base + k) with the
+// lane's slot to the first queue, screening 64 at a time when enough wait.
+template <int MODE, int PREC>
+__device__ __forceinline__ void push_pairs(const PairArgs& a, const CellGeom& g, PairLds& L, uint32_t word,
+                                           uint32_t base, uint32_t slot, uint32_t& qn, uint32_t& q2n, Acc& acc) {
+  for (;;) {
+    const bool f = word != 0u;
+    const unsigned long long m = __ballot(f);
+    if (m == 0ull) return;
+    const uint32_t k = base + (uint32_t)__builtin_ctz(word | 0x80000000u);
+    word &= word - 1u;
+    if (f) L.qE[qn + lane_prefix(m)] = k | (slot << 8);
+    qn += (uint32_t)__popcll(m);
+    if (qn >= (uint32_t)WAVE) {
+      __syncthreads();
+      screen_batch<MODE, PREC>(a, g, L, qn - WAVE, WAVE, q2n, acc);
+      qn -= WAVE;
+    }
   }
 }
 
-// Prefilter of every (probe, slot) pair of one staged batch, looping over
-// the probes of the mask (read from their lanes' registers); TWO: the batch
-// fills the second slot of the lanes too.  rp_l is the probe part of the
-// lane's own probe's reach bound; the slot part sits in Q.w.
-template <int MODE, int PREC, bool TWO, bool ORD>
-__device__ __forceinline__ void probe_loop(const PairArgs& a, const CellGeom& g, PairLds& L,
-                                           unsigned long long pmask, const float4 P1, uint32_t X1,
-                                           float rp_l, uint32_t qbase, const float4 Q0, uint32_t x0,
-                                           uint32_t qa0, uint32_t qb0, const float4 Q1, uint32_t x1,
-                                           uint32_t qa1, uint32_t qb1, uint32_t& qn, uint32_t& q2n,
-                                           Acc& acc) {
-  for (unsigned long long pm = pmask; pm != 0ull; pm &= pm - 1ull) {
-    const int pl = (int)__builtin_ctzll(pm);
-    const float4 Pp = make_float4(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(P1.x), pl)),
-                                  __int_as_float(__builtin_amdgcn_readlane(__float_as_int(P1.y), pl)),
-                                  __int_as_float(__builtin_amdgcn_readlane(__float_as_int(P1.z), pl)),
-                                  0.0f);
-    const uint32_t Xp = (uint32_t)__builtin_amdgcn_readlane((int)X1, pl);
-    const float rp = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rp_l), pl));
-    const uint32_t qprobe = qbase + (uint32_t)pl;
-    const bool f0 = prefilter<MODE, ORD>(Pp, rp, Xp, qprobe, Q0, x0, qa0, qb0);
-    const bool f1 = TWO && prefilter<MODE, ORD>(Pp, rp, Xp, qprobe, Q1, x1, qa1, qb1);
-    push_pairs<MODE, PREC, TWO>(a, g, L, f0, f1, (uint32_t)pl, qn, q2n, acc);
+// Filter of every (probe, slot) pair of one staged batch, the lanes spanning
+// the slots (one each, or two when the batch fills the second half), the
+// probes read from LDS by all lanes at once.  A lane gathers the verdicts of
+// 32 probes in one word per slot and only then turns to the pairs that
+// passed, so the loop is 13 VALU instructions per 64 pairs without a branch,
+// ballot or queue write.  keep0, keep1: the pairs that the pass's ordering
+// allows (half-stencil passes).
+template <int MODE, int PREC, bool ALL, bool TWO>
+__device__ __forceinline__ void probe_loop(const PairArgs& a, const CellGeom& g, PairLds& L, uint32_t nprobe,
+                                           const SlotPre& Q0, const SlotPre& Q1, unsigned long long keep0,
+                                           unsigned long long keep1, uint32_t& qn, uint32_t& q2n, Acc& acc) {
+  constexpr bool ORD = (MODE == PM_CNT || MODE == PM_GEN_NEW);
+  const uint32_t lane = threadIdx.x;
+  for (uint32_t w = 0; w < nprobe; w += 32u) {
+    uint32_t m0 = 0u, m1 = 0u;
+    // the first probe ends in bit 0
+    const uint32_t n = min(32u, nprobe - w);
+    int k = (int)((n + PUNROLL - 1u) & ~(uint32_t)(PUNROLL - 1));
+    while (k > 0) {
+      k -= PUNROLL;
+      const uint32_t at = w + (uint32_t)k;
+#pragma unroll
+      for (int u = PUNROLL - 1; u >= 0; --u) {
+        const float4 f = L.pf[at + (uint32_t)u];
+        const float2 h = L.pg[at + (uint32_t)u];
+        m0 = may_cut<ALL>(f, h, Q0, m0);
+        if (TWO) m1 = may_cut<ALL>(f, h, Q1, m1);
+      }
+    }
+    const uint32_t some = n < 32u ? (1u << n) - 1u : ~0u;  // the rows past the last probe
+    m0 &= some;
+    m1 &= some;
+    if (ORD) {
+      m0 &= (uint32_t)(keep0 >> w);
+      m1 &= (uint32_t)(keep1 >> w);
+    }
+    push_pairs<MODE, PREC>(a, g, L, m0, w, lane, qn, q2n, acc);
+    if (TWO) push_pairs<MODE, PREC>(a, g, L, m1, w, lane + WAVE, qn, q2n, acc);
   }
+}
+
+// Writes the probes of the mask (one per lane) to the front of the chunk's
+// LDS tables, in lane order.  Returns the lane's place among them.
+template <bool ALL>
+__device__ __forceinline__ uint32_t compact_probes(const CellGeom& g, PairLds& L, unsigned long long pmask,
+                                                   const float4 P1, const float4 D1, uint32_t X1, const Filter& F) {
+  const uint32_t lane = threadIdx.x;
+  const uint32_t at = lane_prefix(pmask);
+  if ((pmask >> lane) & 1ull) {
+    const float x = P1.x - F.o.x, y = P1.y - F.o.y, z = P1.z - F.o.z;
+    L.sP[at] = P1;
+    L.sD[at] = D1;
+    L.sX[at] = X1;
+    L.hit[at] = 0u;
+    if (ALL) {
+      const float rp = (P1.w * 1.000001f + (g.R_max + 16.0f * g.ew)) * 1.000006f;
+      L.pf[at] = make_float4(2.0f * x, 2.0f * y, 2.0f * z, 2.0f * rp);
+      L.pg[at] = make_float2(fmaf(z, z, fmaf(y, y, x * x)) - fmaf(rp, rp, F.ln.slack), 0.0f);
+    } else {
+      const LineSide l = line_side(F.ln, x, y, z, D1);
+      L.pf[at] = make_float4(l.ux, l.uy, l.uz, l.mx);
+      L.pg[at] = make_float2(l.my, l.mz);
+    }
+  }
+  return at;
+}
+
+// The pairs that the ordering of a half-stencil pass keeps for one slot, bit
+// k the probe of index lo + k: of the home cell's rods only the later ones of
+// a probe, elsewhere (an image may map back to the home cell) never the probe
+// itself.
+__device__ __forceinline__ unsigned long long ordered(uint32_t src, uint32_t meta, uint32_t lo) {
+  const uint32_t k = src - lo;  // wraps past 2^32 below lo
+  if (meta & 0x80000000u) return src <= lo ? 0ull : (k >= 64u ? ~0ull : (1ull << k) - 1ull);
+  return k >= 64u ? ~0ull : ~(1ull << k);
 }
 
 // One home cell.  For each chunk of up to 64 probes: walk the sorted
 // stencil and pack the rods of consecutive relevant neighbour cells into a
 // 128-slot staging buffer (two slots per lane, both loads in flight
-// together, no lanes wasted on sparse cells); then loop over the chunk's
-// probes (read by broadcast from LDS) with the lanes spanning the slots,
-// keep the pairs that pass a conservative centre-distance prefilter in an
-// LDS queue (ballot + lane prefix), screen them 64 at a time (reach band,
-// line distance) and run the full test on the survivors 64 at a time, so
-// every expensive step runs on dense work.
+// together, no lanes wasted on sparse cells); then run the chunk's probes
+// (read by broadcast from LDS) through a conservative filter with the lanes
+// spanning the slots, keep the pairs that pass in an LDS queue, screen them
+// 64 at a time (reach band, line distance) and run the full test on the
+// survivors 64 at a time, so every expensive step runs on dense work.
 //
-// Prefilter: the full test first rejects pairs whose FP32 centre distance
+// What bounds the pass is VALU issue.  The filter is the distance of the two
+// axes' lines (nf_line.h), which leaves about one pair in a hundred; a
+// centre-distance filter leaves the fifth of the staged pairs that are within
+// reach, each of which then cost some 90 instructions of gather and screen.
+// Same-round pass of 4M uniform rods, MI355X: 1.65 -> 1.06 ms; 2,000 rods
+// 0.10 -> 0.036 ms, 500,000 log-normal rods in agglomerates 0.49 -> 0.44 ms.
+//
+// Every pair within reach (ALL: the contact pass, and the generation passes
+// that count pair tests as the oracle does): the full test first rejects pairs whose FP32 centre distance
 // w2 exceeds rr^2 by more than its error band, rr = (hl1 + hl2) * 1.000001
-// + R.  The prefilter keeps every pair with w2' <= rr''^2, where
+// + R.  The filter keeps every pair with w2' <= rr''^2, where
 // rr'' = (hl1 * 1.000001 + R_max + 16 ew) * 1.000006 + (hl2 * 1.000001) * 1.000006
 // is rr' = hl1 * 1.000001 + hl2 * 1.000001 + R_max + 16 ew >= rr + 16 ew
 // scaled by 1.000006 less a few float roundings (below 1e-7 relative), so
-// rr''^2 >= rr'^2 * 1.00001; and w' = P1 - (P2 + shift) differs from the
-// full test's ((P1 - P2) - shift) by a few roundings of coordinates bounded
-// by box + reach, i.e. by less than 6 ew.  So every pair the full test would
-// count or cut is queued.  The probe's part of rr'' is computed per lane,
-// the slot's part is staged with the slot (Q.w).
+// rr''^2 >= rr'^2 * 1.00001.  The probe's part rp of rr'' is computed per
+// lane, the slot's part rq is staged with the slot.  Centres are taken from
+// an origin o in the home cell: p = P1 - o and q = (P2 + shift) - o are each
+// within 2 ew of the exact differences, so w' = p - q differs from the full
+// test's ((P1 - P2) - shift) by less than 8 ew.  The test is
+//   2 p.q + 2 rp rq + (rq^2 - |q|^2) - (|p|^2 - rp^2) >= 0,
+// four FMAs.  For a pair that has to pass, |q| <= |p| + rp + rq, so with
+// S = |p| + rp + rq every term and partial sum is below 4 S^2; the two
+// brackets take five roundings of values below S^2 each, the chain one
+// subtraction and four FMAs of values below 4 S^2: 30 u S^2 in all.  The
+// slack in the probe's bracket is 64 u S^2 with S bounded over the cell.
+// So with ALL every pair the full test would count or cut is queued.
 //
 // A work item is one probe chunk group and one stencil part of a cell
 // (k_items): the cell's probes are dealt into nch equal chunks of at most 64;
@@ -506,7 +593,7 @@ __device__ __forceinline__ void probe_loop(const PairArgs& a, const CellGeom& g,
 // dense cell is worked on by several waves at once.  Interleaved offsets
 // give every part near and far cells alike.  The probe bytes, counted per
 // probe, belong to part sp = 0.
-template <int MODE, int PREC>
+template <int MODE, int PREC, bool ALL>
 __device__ void process_cell(const PairArgs& a, const CellGeom& g, uint32_t gc, uint32_t cg, uint32_t ncg,
                              uint32_t sp, uint32_t nst, PairLds& L, Acc& acc) {
   const int lane = threadIdx.x;
@@ -524,7 +611,15 @@ __device__ void process_cell(const PairArgs& a, const CellGeom& g, uint32_t gc, 
   const int c0 = (int)(lc % (uint32_t)g.nc[0]);
   const int c1 = (int)((lc / (uint32_t)g.nc[0]) % (uint32_t)g.nc[1]);
   const int c2 = (int)(lc / ((uint32_t)g.nc[0] * (uint32_t)g.nc[1]));
-  const float pad_r = g.R_max + 16.0f * g.ew;
+  // the filter's origin (the home cell's centre), scale and slack
+  Filter F;
+  F.o = make_float3(((float)c0 + 0.5f) * g.edge[0], ((float)c1 + 0.5f) * g.edge[1], ((float)c2 + 0.5f) * g.edge[2]);
+  const float Smax = 0.51f * (g.edge[0] + g.edge[1] + g.edge[2]) + 2.0f * CELL_MARGIN +
+                     2.00002f * (g.hl_max + g.R_max + 16.0f * g.ew);
+  if (ALL)
+    F.ln = LineFilter{0.0f, 64.0f * U32 * Smax * Smax};
+  else
+    F.ln = line_filter(g.R_max, g.ew, Smax);
 
   for (uint32_t pb = cg * csz; pb < pc; pb += ncg * csz) {
     const uint32_t G = min(csz, pc - pb);
@@ -535,23 +630,20 @@ __device__ void process_cell(const PairArgs& a, const CellGeom& g, uint32_t gc, 
     const float4 D1 = g.hD[pidx];
     const uint32_t X1 = g.hX[pidx];
     const bool have = inrange;
-    L.sP[lane] = P1;
-    L.sD[lane] = D1;
-    L.sX[lane] = X1;
-    L.hit[lane] = 0u;
-    // probes taking part, as a wave-uniform mask; the prefilter reads each
-    // probe from its lane's registers
+    // probes still in the walk, as a wave-uniform mask
     unsigned long long pmask = __ballot(have);
     const float chunk_hl = unif(wave_max(have ? P1.w : 0.0f));
     if (sp == 0u) acc.bytes += (unsigned long long)G * 36ull;
     const float rr_chunk = (chunk_hl + g.hl_max) * 1.000001f + g.R_max + CELL_MARGIN;
     const float rr_chunk2 = rr_chunk * rr_chunk;
-    uint32_t qn = 0;   // wave-uniform queue lengths: prefiltered pairs,
+    uint32_t qn = 0;   // wave-uniform queue lengths: filtered pairs,
     uint32_t q2n = 0;  // and pairs waiting for the full test
     StencilCursor cur{sp, nst, 0ull, 0u, 0u, 0u, 0u, 0u, 0u, 0u, false, false};
     // several parts walk for this chunk's proposals: each tells the others of
     // its cuts through the alive flags
-    const bool share = MODE == PM_GEN_OLD && !g.inv && !a.test_all && nst > 1u;
+    const bool share = MODE == PM_GEN_OLD && !g.inv && !ALL && nst > 1u;
+    uint32_t at = compact_probes<ALL>(g, L, pmask, P1, D1, X1, F);
+    unsigned long long listed = pmask;  // the probes in the LDS tables
     __syncthreads();
 
     while (!cur.done) {
@@ -605,49 +697,28 @@ __device__ void process_cell(const PairArgs& a, const CellGeom& g, uint32_t gc, 
       L.bX[lane + WAVE] = x1;
       L.bM[lane + WAVE] = m1;
       const float3 s0 = shift_f32(g, m0), s1 = shift_f32(g, m1);
-      const float far = 1e30f;  // unfilled slots: out of every reach
-      // w: the slot's part of the pair reach bound (see the prefilter note)
-      const float4 Q0 = v0 ? make_float4(p0.x + s0.x, p0.y + s0.y, p0.z + s0.z, (p0.w * 1.000001f) * 1.000006f)
-                           : make_float4(far, far, far, 0.0f);
-      const float4 Q1 = v1 ? make_float4(p1.x + s1.x, p1.y + s1.y, p1.z + s1.z, (p1.w * 1.000001f) * 1.000006f)
-                           : make_float4(far, far, far, 0.0f);
-      // contacts: keep slot iff qprobe < qa || qprobe > qb (home cell: only
-      // later indices; elsewhere: anything but the probe itself)
-      const uint32_t qa0 = src0, qa1 = src1;
-      const uint32_t qb0 = (m0 & 0x80000000u) ? 0xFFFFFFFFu : src0;
-      const uint32_t qb1 = (m1 & 0x80000000u) ? 0xFFFFFFFFu : src1;
-      // the ordering can only drop a pair whose slot is of the home cell, or
-      // is one of the chunk's probes (through an image)
-      bool ord = false;
+      const SlotPre Q0 = slot_pre<ALL>(p0, d0, s0, F, v0), Q1 = slot_pre<ALL>(p1, d1, s1, F, v1);
+      unsigned long long keep0 = ~0ull, keep1 = ~0ull;
       if (MODE == PM_CNT || MODE == PM_GEN_NEW) {
-        const uint32_t qlo = ps + pb;
-        const bool o0 = v0 && ((m0 & 0x80000000u) != 0u || src0 - qlo < G);
-        const bool o1 = v1 && ((m1 & 0x80000000u) != 0u || src1 - qlo < G);
-        ord = __ballot(o0 || o1) != 0ull;
+        keep0 = ordered(src0, m0, ps + pb);
+        keep1 = ordered(src1, m1, ps + pb);
       }
       if (share) {
         pmask &= __ballot(alive != 0u);
         if (pmask == 0ull) break;
       }
-      __syncthreads();
-      // ---- prefilter every (probe, slot) pair, queue the survivors
-      // each lane's own probe part of the pair reach bound
-      const float rp_l = (P1.w * 1.000001f + pad_r) * 1.000006f;
-      if (ord) {
-        if (fill > (uint32_t)WAVE)
-          probe_loop<MODE, PREC, true, true>(a, g, L, pmask, P1, X1, rp_l, ps + pb, Q0, x0, qa0, qb0,
-                                             Q1, x1, qa1, qb1, qn, q2n, acc);
-        else
-          probe_loop<MODE, PREC, false, true>(a, g, L, pmask, P1, X1, rp_l, ps + pb, Q0, x0, qa0, qb0,
-                                              Q1, x1, qa1, qb1, qn, q2n, acc);
-      } else {
-        if (fill > (uint32_t)WAVE)
-          probe_loop<MODE, PREC, true, false>(a, g, L, pmask, P1, X1, rp_l, ps + pb, Q0, x0, qa0, qb0,
-                                              Q1, x1, qa1, qb1, qn, q2n, acc);
-        else
-          probe_loop<MODE, PREC, false, false>(a, g, L, pmask, P1, X1, rp_l, ps + pb, Q0, x0, qa0,
-                                               qb0, Q1, x1, qa1, qb1, qn, q2n, acc);
+      // probes have left the walk: the others move up
+      if (MODE == PM_GEN_OLD && pmask != listed) {
+        at = compact_probes<ALL>(g, L, pmask, P1, D1, X1, F);
+        listed = pmask;
       }
+      __syncthreads();
+      // ---- filter every (probe, slot) pair, queue the survivors
+      const uint32_t np = (uint32_t)__popcll(listed);
+      if (fill > (uint32_t)WAVE)
+        probe_loop<MODE, PREC, ALL, true>(a, g, L, np, Q0, Q1, keep0, keep1, qn, q2n, acc);
+      else
+        probe_loop<MODE, PREC, ALL, false>(a, g, L, np, Q0, Q1, keep0, keep1, qn, q2n, acc);
       // ---- drain both queues before the slots are restaged
       if (qn > 0) {
         __syncthreads();
@@ -660,26 +731,21 @@ __device__ void process_cell(const PairArgs& a, const CellGeom& g, uint32_t gc, 
         q2n = 0;
       }
       __syncthreads();
-      if (MODE == PM_GEN_OLD && !g.inv && !a.test_all) {
+      if (MODE == PM_GEN_OLD && !g.inv && !ALL) {
         // a proposal once cut is rejected whatever else it overlaps: cut
         // proposals leave the walk, which ends when none is left.  The
         // stencil is sorted by distance, so near a jammed state most
         // proposals leave after their first batches.  The decisions are
         // unchanged; the pair-test count is then the pairs evaluated.
-        const bool cut = have && L.hit[lane] != 0u;
-        if (share && cut && ((pmask >> lane) & 1ull))
+        const bool cut = ((listed >> lane) & 1ull) && L.hit[at] != 0u;
+        if (cut && ((pmask >> lane) & 1ull))
           __hip_atomic_store(&a.alive_out[pidx], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         pmask &= ~__ballot(cut);
         if (pmask == 0ull) break;
       }
     }
-    if (MODE == PM_GEN_OLD && !g.inv) {
-      // branch-free result store: lanes without a result write a private
-      // LDS slot instead
-      const bool hitp = have && L.hit[lane] != 0u;
-      uint32_t* dst = hitp ? &a.alive_out[pidx] : &L.dummy[lane];
-      *dst = 0u;
-    }
+    // every pair tested: the cut proposals' flags now
+    if (MODE == PM_GEN_OLD && !g.inv && ALL && have && L.hit[at] != 0u) a.alive_out[pidx] = 0u;
     __syncthreads();
   }
 }
@@ -702,7 +768,7 @@ __device__ __forceinline__ OldRoles old_roles(const PairArgs& a, uint32_t inst, 
   return r;
 }
 
-template <int MODE, int PREC>
+template <int MODE, int PREC, bool ALL>
 __global__ void __launch_bounds__(PAIR_THREADS, 4) k_pair(PairArgs a) {
   __shared__ PairLds L;
   constexpr bool GEN = (MODE == PM_GEN_OLD || MODE == PM_GEN_NEW);
@@ -722,6 +788,7 @@ __global__ void __launch_bounds__(PAIR_THREADS, 4) k_pair(PairArgs a) {
       g.boxf[d] = a.boxf[d];
       g.nc[d] = a.ncell[d];
       g.rnc[d] = 1.0f / (float)a.ncell[d];
+      g.edge[d] = a.boxf[d] / (float)a.ncell[d];
     }
     g.cell_base = 0;
     g.st = a.stencil + a.st_off;
@@ -810,6 +877,7 @@ __global__ void __launch_bounds__(PAIR_THREADS, 4) k_pair(PairArgs a) {
             g.boxf[dd] = d.boxf[dd];
             g.nc[dd] = d.ncell[dd];
             g.rnc[dd] = 1.0f / (float)d.ncell[dd];
+            g.edge[dd] = d.edge[dd];
           }
           g.cell_base = d.cell_base;
           g.st = a.stencil + (MODE == PM_GEN_NEW ? d.hst_off : d.st_off);
@@ -845,7 +913,7 @@ __global__ void __launch_bounds__(PAIR_THREADS, 4) k_pair(PairArgs a) {
           }
         }
       }
-      process_cell<MODE, PREC>(a, g, gc, cg, ncg, sp, nst, L, acc);
+      process_cell<MODE, PREC, ALL>(a, g, gc, cg, ncg, sp, nst, L, acc);
     }
   }
   if (!GEN || cur_inst != 0xFFFFFFFFu) flush<GEN>(a, g, acc, MODE);
@@ -1026,21 +1094,27 @@ void launch_pair(int mode, int prec, const PairArgs& args, hipStream_t s, const 
     else
       hipLaunchKernelGGL(k_items<PM_GEN_NEW>, dim3(QUEUES_PER_KERNEL), dim3(ITEM_THREADS), 0, s, a, (float)grid.x);
   }
-  a.test_all = (t && mode == PM_GEN_OLD) ? t->test_all : 0u;
-#define NF_LAUNCH(M, P) hipLaunchKernelGGL((k_pair<M, P>), grid, block, 0, s, a)
+  const bool all = t && t->test_all;
+#define NF_LAUNCH(M, P, A) hipLaunchKernelGGL((k_pair<M, P, A>), grid, block, 0, s, a)
+#define NF_LAUNCH_ALL(M, P) \
+  if (all)                  \
+    NF_LAUNCH(M, P, true);  \
+  else                      \
+    NF_LAUNCH(M, P, false)
   if (prec == NF_PREC_FP64) {
     switch (mode) {
-      case PM_GEN_OLD: NF_LAUNCH(PM_GEN_OLD, NF_PREC_FP64); break;
-      case PM_GEN_NEW: NF_LAUNCH(PM_GEN_NEW, NF_PREC_FP64); break;
-      default: NF_LAUNCH(PM_CNT, NF_PREC_FP64); break;
+      case PM_GEN_OLD: NF_LAUNCH_ALL(PM_GEN_OLD, NF_PREC_FP64); break;
+      case PM_GEN_NEW: NF_LAUNCH_ALL(PM_GEN_NEW, NF_PREC_FP64); break;
+      default: NF_LAUNCH(PM_CNT, NF_PREC_FP64, true); break;
     }
   } else {
     switch (mode) {
-      case PM_GEN_OLD: NF_LAUNCH(PM_GEN_OLD, NF_PREC_FP32_RECHECK); break;
-      case PM_GEN_NEW: NF_LAUNCH(PM_GEN_NEW, NF_PREC_FP32_RECHECK); break;
-      default: NF_LAUNCH(PM_CNT, NF_PREC_FP32_RECHECK); break;
+      case PM_GEN_OLD: NF_LAUNCH_ALL(PM_GEN_OLD, NF_PREC_FP32_RECHECK); break;
+      case PM_GEN_NEW: NF_LAUNCH_ALL(PM_GEN_NEW, NF_PREC_FP32_RECHECK); break;
+      default: NF_LAUNCH(PM_CNT, NF_PREC_FP32_RECHECK, true); break;
     }
   }
+#undef NF_LAUNCH_ALL
 #undef NF_LAUNCH
 }
 
