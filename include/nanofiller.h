@@ -96,7 +96,7 @@ typedef struct nf_gen_stats {
   int32_t status;         /* NF_STATUS_*                                   */
   uint64_t candidates;    /* Philox candidate slots drawn                  */
   uint64_t proposals;     /* candidates that passed the density test       */
-  uint64_t pair_tests;    /* capsule predicate evaluations (pairs in reach)*/
+  uint64_t pair_tests;    /* pairs examined (NF_OPT_TEST_ALL_PAIRS: in reach) */
   uint64_t rechecks;      /* FP32 results inside the error band, redone FP64*/
   uint64_t rejected_old;  /* proposals overlapping an accepted rod         */
   uint64_t rejected_new;  /* proposals overlapping a higher-priority one   */

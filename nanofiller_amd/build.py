@@ -27,6 +27,7 @@ SOURCES = [
     "nf_scan.hip",
     "nf_gen.hip",
     "nf_pair.hip",
+    "nf_walk.hip",
     "nf_seg.hip",
     "nf_post.hip",
     "nf_net.hip",

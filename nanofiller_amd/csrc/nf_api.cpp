@@ -330,6 +330,55 @@ std::vector<int4> build_stencil(const int32_t nc[3], const double box[3], double
 // ===========================================================================
 // lifecycle
 // ===========================================================================
+// Crossing lists of an instance (nf_walk.hip).  Fine cells of 1.5 times the
+// mean spacing of the rods, between a sixteenth and two thirds of a typical
+// rod: 1, 1.5 and 2 times gave 54.7, 52.7 and 56.4 ms of kernels for 32 uneven
+// packings, 2.03, 1.89 and 1.91 ms for 500,000 rods (smaller cells: fewer
+// pairs, more entries to make).
+//
+// Which packings: entering a rod costs some seven device-scope atomics, the
+// cell-pair engine a number of staged pairs that grows with crowding (rods
+// per excluded volume), with the spread of the lengths (its cells are as wide
+// as the longest) and with the rounds.  Whole generations of constant-length
+// rods at 0.5 / 1 / 1.5 rods per excluded volume, cells of one reach against
+// lists: 200,000 rods 0.97 / 1.53 / 2.03 against 0.94 / 1.32 / 1.79 ms, 1M
+// 1.77 / 2.86 / 4.40 against 2.21 / 3.26 / 4.38 ms, 4M 4.7 / 7.9 / 12.6
+// against 7.1 / 10.7 / 15.1 ms; at 0.25 200,000 rods 0.55 against 0.62 ms.
+// Log-normal lengths, 1M rods: 3.2 / 6.8 / 11.6 against 2.4 / 3.5 / 4.5 ms.
+//
+// peak: densest point over the mean.
+static void plan_fine(const nf_params& p, InstDesc& d, double peak) {
+  FineGrid& g = d.fine;
+  const double V = p.box[0] * p.box[1] * p.box[2];
+  const double crowd = (double)p.n_rods * excluded_volume(p.len, p.radius) / V;
+  if (p.len_law == NF_LEN_CONST &&
+      ((p.n_rods > 300000u && crowd < 1.6) || (p.n_rods > 100000u && crowd < 0.4)))
+    return;
+  const double r = 0.50001 * (double)d.R_max + 16.0 * (double)d.ew;
+  double E = 1.5 * std::cbrt(V / (double)p.n_rods);
+  E = std::min(std::max(E, p.len / 16.0), p.len / 1.5);
+  E = std::max(E, 4.0 * r);
+  uint64_t cells = 1;
+  for (int a = 0; a < 3; ++a) {
+    // one wrap per axis; a grid that uses the whole box
+    if (!((double)d.hl_max * 1.0001 + r < 0.999 * p.box[a])) return;
+    const double n = std::min(std::max(std::floor(p.box[a] / E), 1.0), 1024.0);
+    g.n[a] = (int32_t)n;
+    g.e[a] = (float)(p.box[a] / n);
+    g.ie[a] = (float)(n / p.box[a]);
+    cells *= (uint64_t)g.n[a];
+  }
+  if (cells > (1ull << ENTRY_BITS) || p.max_batch > (1u << ENTRY_BITS)) return;
+  g.r = (float)r;
+  // rods crossing a cell: a rod of length l crosses about 2 (3/4 l / E + 1)
+  const double lam = peak * (double)p.n_rods / (double)cells * 2.0 * (0.75 * p.len / E + 1.0);
+  const double first = std::min((double)p.max_batch, 1.25 * (double)p.n_rods) / (double)p.n_rods;
+  auto room = [](double l) { return (uint32_t)std::min(4.0 * std::ceil((1.15 * l + 6.0 * std::sqrt(l) + 10.0) / 4.0), 65532.0); };
+  g.capA = room(lam);
+  g.capP = room(lam * first);
+  g.on = 1u;
+}
+
 static int plan_instance(const nf_params& p, InstDesc& d, std::vector<double>& agg,
                          std::vector<int4>& stencil) {
   std::memset(&d, 0, sizeof(d));
@@ -425,6 +474,7 @@ static int plan_instance(const nf_params& p, InstDesc& d, std::vector<double>& a
   d.sep32 = (float)p.sep;
   const double Lmax = std::max(p.box[0], std::max(p.box[1], p.box[2]));
   d.ew = (float)(5.9604644775390625e-8 * (Lmax + reach) * 1.01);
+  plan_fine(p, d, peak);
   return NF_OK;
 }
 
@@ -433,7 +483,8 @@ static void release_gen(nf_handle* h) {
   void* ptrs[] = {b.desc, b.st, b.ri, b.slot_base, b.stencil, b.agg, b.mesh, b.cell_inst, b.oP, b.oD,
                   b.oid, b.ostart, b.ocount, b.ohl, b.bP, b.bD, b.sP, b.sD, b.scell, b.srk,
                   b.surv, b.srank, b.pP, b.pD, b.pslot, b.palive, b.pcount, b.pstart, b.phl,
-                  b.items, b.qcnt, b.aP, b.aD, b.aslot, b.aidx, b.acount, b.astart, b.queues, b.scan_tmp};
+                  b.items, b.qcnt, b.aP, b.aD, b.aslot, b.aidx, b.acount, b.astart, b.queues, b.scan_tmp,
+                  b.fcountA, b.fcountP, b.flistA, b.flistP, b.sdst, b.oR, b.aR};
   for (void* p : ptrs) dfree(h, p);
   b = GenBuffers();
 }
@@ -448,6 +499,58 @@ void nf::release_contacts(nf_handle* h) {
                   c.nd_cel_gap, c.nd_cel_side};
   for (void* p : ptrs) dfree(h, p);
   c = ContactBuffers();
+}
+
+// Offsets and device memory of the crossing lists of the instances that have
+// them (desc: to be uploaded afterwards).
+constexpr uint32_t LIST_CAP_MAX = 8192;
+constexpr uint64_t LIST_ENTRIES_MAX = (uint64_t)1 << 32;  // 16 GiB
+static int layout_lists(nf_handle* h) {
+  GenBuffers& b = h->gb;
+  void* old[] = {b.fcountA, b.fcountP, b.flistA, b.flistP, b.oR, b.aR};
+  for (void* p : old) dfree(h, p);
+  b.fcountA = b.fcountP = b.flistA = b.flistP = nullptr;
+  b.oR = b.aR = nullptr;
+  b.total_fine = b.total_listA = b.total_listP = 0;
+  b.walk = b.cellwise = false;
+  for (InstDesc& d : h->desc) {
+    FineGrid& g = d.fine;
+    if (!g.on) {
+      b.cellwise = true;
+      continue;
+    }
+    const uint64_t cells = (uint64_t)g.n[0] * g.n[1] * g.n[2];
+    // entries name a cell slot of the instance in ENTRY_BITS bits; lists far
+    // longer than planned (one crowded spot) or past the memory set aside go
+    // without
+    if ((uint64_t)d.ncells * d.cap > (1ull << ENTRY_BITS) || g.capA > LIST_CAP_MAX || g.capP > LIST_CAP_MAX ||
+        b.total_listA + b.total_listP + cells * ((uint64_t)g.capA + g.capP) > LIST_ENTRIES_MAX ||
+        b.total_fine + cells > 0xFFFFFFF0ull) {
+      g.on = 0u;
+      b.cellwise = true;
+      continue;
+    }
+    g.base = (uint32_t)b.total_fine;
+    g.offA = b.total_listA;
+    g.offP = b.total_listP;
+    b.total_fine += cells;
+    b.total_listA += cells * g.capA;
+    b.total_listP += cells * g.capP;
+    b.walk = true;
+  }
+  if (!b.walk) return NF_OK;
+  int rc = dalloc(h, &b.fcountA, b.total_fine);
+  if (rc == NF_OK) rc = dalloc(h, &b.fcountP, b.total_fine);
+  if (rc == NF_OK) rc = dalloc(h, &b.flistA, b.total_listA);
+  if (rc == NF_OK) rc = dalloc(h, &b.flistP, b.total_listP);
+  if (rc == NF_OK) rc = dalloc(h, &b.oR, 2 * b.total_old);
+  if (rc == NF_OK) rc = dalloc(h, &b.aR, 2 * b.T_cap);
+  if (rc == NF_E_NOMEM) {
+    // the packings do not need the lists
+    for (InstDesc& d : h->desc) d.fine.on = 0u;
+    return layout_lists(h);
+  }
+  return rc;
 }
 
 extern "C" int nf_create_batch(const nf_params* ps, int n, nf_handle** out) {
@@ -552,8 +655,10 @@ extern "C" int nf_create_batch(const nf_params* ps, int n, nf_handle** out) {
   ALLOC(b.astart, b.total_cells + 1);
   ALLOC(b.phl, b.total_cells);
   ALLOC(b.queues, Q_N * QWORDS);
+  ALLOC(b.sdst, b.T_cap);
   ALLOC(b.scan_tmp, std::max(scan_tmp_words(b.total_cells), scan_tmp_words(b.T_cap)));
 #undef ALLOC
+  if (rc == NF_OK) rc = layout_lists(h);
   if (rc != NF_OK) {
     std::string m = h->err;
     nf_destroy(h);
@@ -598,7 +703,11 @@ extern "C" int nf_create_batch(const nf_params* ps, int n, nf_handle** out) {
   }
   h->n_rods.assign(n, 0);
   h->planned_cap.resize(n);
-  for (int i = 0; i < n; ++i) h->planned_cap[i] = h->desc[i].cap;
+  h->planned_list.resize(n);
+  for (int i = 0; i < n; ++i) {
+    h->planned_cap[i] = h->desc[i].cap;
+    h->planned_list[i] = {h->desc[i].fine.capA, h->desc[i].fine.capP};
+  }
   *out = h;
   return NF_OK;
 }
@@ -705,6 +814,7 @@ static int reset_generation(nf_handle* h) {
   HIPCHK(h, hipMemsetAsync(b.ri, 0, sizeof(RoundInfo), h->stream));
   fill_u32(b.ocount, 0u, b.total_cells, h->stream);
   fill_u32((uint32_t*)b.ohl, 0u, b.total_cells, h->stream);
+  if (b.walk) fill_u32(b.fcountA, 0u, b.total_fine, h->stream);
   HIPCHK(h, hipGetLastError());
   HIPCHK(h, sync_stream(h->stream, "generation reset"));
   return NF_OK;
@@ -797,6 +907,8 @@ static int relayout_old(nf_handle* h, const std::vector<uint32_t>& caps) {
   if (rc == NF_OK) rc = dalloc(h, &b.oid, std::max<uint64_t>(off, 1));
   if (rc != NF_OK) return rc;
   b.total_old = off;
+  rc = layout_lists(h);
+  if (rc != NF_OK) return rc;
   std::vector<uint32_t> ostart(b.total_cells);
   for (int i = 0; i < n; ++i) {
     const InstDesc& d = h->desc[i];
@@ -811,28 +923,36 @@ static int relayout_old(nf_handle* h, const std::vector<uint32_t>& caps) {
   return NF_OK;
 }
 
-// The planned slots per cell scaled by scale (at least one, at most what
+static uint32_t scaled_list(uint32_t cap, double scale) {
+  return (uint32_t)(4.0 * std::max(1.0, std::min(std::ceil(cap * scale / 4.0), LIST_CAP_MAX / 4.0)));
+}
+
+// The planned slots per cell and list lengths scaled by scale (at least one, at most what
 // cannot overflow: the instance's target + 16).
 static int scale_slots(nf_handle* h, double scale) {
   std::vector<uint32_t> caps(h->desc.size());
   for (size_t i = 0; i < caps.size(); ++i) {
     const double c = std::ceil((double)h->planned_cap[i] * scale);
     caps[i] = (uint32_t)std::max(1.0, std::min(c, (double)h->desc[i].n_target + 16.0));
+    FineGrid& g = h->desc[i].fine;
+    if (!g.on) continue;
+    g.capA = scaled_list(h->planned_list[i].first, scale);
+    g.capP = scaled_list(h->planned_list[i].second, scale);
   }
   return relayout_old(h, caps);
 }
 
-static int generate_once(nf_handle* h, nf_gen_stats* stats, std::vector<int>* overflowed);
+static int generate_once(nf_handle* h, nf_gen_stats* stats, std::vector<std::pair<int, uint32_t>>* overflowed);
 
-// Generation with slot growth: an instance whose cell slots overflowed is
-// generated again from the start with twice the slots per cell (the packing
-// is the same; only its storage was too small), up to the capacity that
+// Generation with growth: an instance whose cell slots or crossing lists
+// overflowed is generated again from the start with twice the room (the
+// packing is the same; only its storage was too small), up to the slots that
 // cannot overflow.
 extern "C" int nf_generate(nf_handle* h, nf_gen_stats* stats) {
   if (!h) return fail(nullptr, NF_E_INVALID, "null handle");
   uint32_t growths = 0;
   for (;;) {
-    std::vector<int> over;
+    std::vector<std::pair<int, uint32_t>> over;  // instance, what ran out of room (OVER_*)
     const int rc = generate_once(h, stats, &over);
     if (rc != NF_E_OVERFLOW || over.empty()) {
       if (stats)
@@ -842,22 +962,29 @@ extern "C" int nf_generate(nf_handle* h, nf_gen_stats* stats) {
     std::vector<uint32_t> caps(h->desc.size());
     bool grew = false;
     for (size_t i = 0; i < caps.size(); ++i) caps[i] = h->desc[i].cap;
-    for (int i : over) {
-      const uint32_t lim = h->desc[i].n_target + 16u;
-      const uint32_t c = (uint32_t)std::min<uint64_t>(2ull * caps[i], lim);
-      grew = grew || c > caps[i];
-      caps[i] = c;
+    for (const auto& [i, bits] : over) {
+      if (bits & OVER_SLOTS) {
+        const uint32_t lim = h->desc[i].n_target + 16u;
+        const uint32_t c = (uint32_t)std::min<uint64_t>(2ull * caps[i], lim);
+        grew = grew || c > caps[i];
+        caps[i] = c;
+      }
+      // lists double too; past LIST_CAP_MAX the instance goes without them
+      FineGrid& g = h->desc[i].fine;
+      if (bits & OVER_LISTS_A) g.capA *= 2u;
+      if (bits & OVER_LISTS_P) g.capP *= 2u;
+      grew = grew || (bits & (OVER_LISTS_A | OVER_LISTS_P)) != 0u;
     }
     if (!grew) return rc;
     const int r2 = relayout_old(h, caps);
     if (r2 != NF_OK) return r2;
     ++growths;
-    trace("generate: cell slots overflowed, regenerating with %u slots per cell (instance %d)", caps[over[0]],
-          over[0]);
+    trace("generate: out of room (%u), regenerating with %u slots per cell (instance %d)", over[0].second,
+          caps[over[0].first], over[0].first);
   }
 }
 
-static int generate_once(nf_handle* h, nf_gen_stats* stats, std::vector<int>* overflowed) {
+static int generate_once(nf_handle* h, nf_gen_stats* stats, std::vector<std::pair<int, uint32_t>>* overflowed) {
   h->err.clear();
   const int prec = h->params[0].precision;
   for (auto& p : h->params)
@@ -946,7 +1073,7 @@ static int generate_once(nf_handle* h, nf_gen_stats* stats, std::vector<int>* ov
     h->n_rods[i] = st[i].n_acc;
     if (st[i].status == NF_STATUS_OVERFLOW) {
       status_rc = NF_E_OVERFLOW;
-      overflowed->push_back(i);
+      overflowed->push_back({i, st[i].overflow});
     }
     if (stats) {
       nf_gen_stats& s = stats[i];

@@ -54,13 +54,18 @@ __global__ void __launch_bounds__(GEN_THREADS) k_ctl_begin(const InstDesc* __res
                                                            uint32_t* __restrict__ queues, int n_inst,
                                                            uint32_t* __restrict__ pcount,
                                                            uint32_t* __restrict__ phl,
-                                                           uint64_t ncells) {
+                                                           uint64_t ncells,
+                                                           uint32_t* __restrict__ fcount,
+                                                           uint64_t nfine) {
   // every thread: clear the per-cell proposal counts and longest proposals
   for (uint64_t c = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; c < ncells;
        c += (uint64_t)gridDim.x * blockDim.x) {
     pcount[c] = 0u;
     phl[c] = 0u;
   }
+  // and the lengths of the survivors' crossing lists
+  for (uint64_t c = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; c < nfine; c += (uint64_t)gridDim.x * blockDim.x)
+    fcount[c] = 0u;
   // the first wave: the controller
   if (blockIdx.x != 0 || threadIdx.x >= WAVE) return;
   const int lane = threadIdx.x;
@@ -191,7 +196,8 @@ __global__ void __launch_bounds__(GEN_THREADS) k_alive_scatter(const uint32_t* _
                                                                uint32_t* __restrict__ astart,
                                                                uint32_t* __restrict__ acount,
                                                                uint32_t* __restrict__ surv,
-                                                               uint64_t ncells) {
+                                                               uint64_t ncells,
+                                                               float4* __restrict__ aR) {
   const uint64_t P = pstart[ncells];  // proposals of this round, all instances
   const uint64_t n = P > ncells + 1 ? P : ncells + 1;
   for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n;
@@ -200,9 +206,14 @@ __global__ void __launch_bounds__(GEN_THREADS) k_alive_scatter(const uint32_t* _
       const uint32_t g = pslot[k];
       if (palive[k]) {
         const uint32_t dst = aidx[k];
-        aP[dst] = pP[k];
-        aD[dst] = pD[k];
+        const float4 P = pP[k], D = pD[k];
+        aP[dst] = P;
+        aD[dst] = D;
         aslot[dst] = g;
+        if (aR) {
+          aR[2ull * dst] = P;
+          aR[2ull * dst + 1u] = make_float4(D.x, D.y, D.z, __uint_as_float(g));
+        }
       } else {
         surv[g] = 0u;
       }
@@ -236,7 +247,9 @@ __global__ void __launch_bounds__(GEN_THREADS) k_commit(const InstDesc* __restri
                                                         float* __restrict__ ohl,
                                                         float4* __restrict__ oP,
                                                         float4* __restrict__ oD,
-                                                        uint32_t* __restrict__ oid) {
+                                                        uint32_t* __restrict__ oid,
+                                                        uint32_t* __restrict__ sdst,
+                                                        float4* __restrict__ oR) {
   const uint32_t T = ri->T;
   for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < T; g += gridDim.x * blockDim.x) {
     if (!surv[g]) continue;
@@ -244,6 +257,7 @@ __global__ void __launch_bounds__(GEN_THREADS) k_commit(const InstDesc* __restri
     const InstDesc& d = desc[inst];
     const uint32_t n_acc = st[inst].n_acc;
     const uint32_t r = srank[g] - srank[slot_base[inst]];
+    sdst[g] = 0xFFFFFFFFu;
     if (r >= d.n_target - n_acc) continue;
     const uint32_t id = n_acc + r;
     const float4 P = sP[g], D = sD[g];
@@ -256,6 +270,11 @@ __global__ void __launch_bounds__(GEN_THREADS) k_commit(const InstDesc* __restri
       oP[dst] = P;
       oD[dst] = D;
       oid[dst] = id;
+      sdst[g] = dst;
+      if (oR) {
+        oR[2ull * dst] = P;
+        oR[2ull * dst + 1u] = D;
+      }
       atomicMax((unsigned int*)&ohl[c], __float_as_uint(P.w));
     } else {
       // no slot: give the count back, so that once this kernel ends every
@@ -263,7 +282,7 @@ __global__ void __launch_bounds__(GEN_THREADS) k_commit(const InstDesc* __restri
       // instances of a batch read a cell's first `count` slots), and stop
       // the instance (the host generates it again with more slots)
       atomicSub(&ocount[c], 1u);
-      atomicOr(&st[inst].overflow, 1u);
+      atomicOr(&st[inst].overflow, (uint32_t)OVER_SLOTS);
     }
   }
 }
@@ -345,9 +364,12 @@ static int gen_grid(uint64_t n) {
 void launch_round(GenBuffers& b, int prec, int diag, hipStream_t s, hipEvent_t* ev) {
   const int n = b.n_inst;
   if (ev) (void)hipEventRecord(ev[0], s);
-  hipLaunchKernelGGL(k_ctl_begin, dim3(gen_grid(b.total_cells)), dim3(GEN_THREADS), 0, s, b.desc,
-                     b.st, b.ri, b.slot_base, b.queues, n, b.pcount, (uint32_t*)b.phl,
-                     (uint64_t)b.total_cells);
+  // crossing lists, unless every pair within reach has to be tested
+  const bool walk = b.walk && !b.tiles.test_all;
+  const bool cells = b.cellwise || !walk;
+  hipLaunchKernelGGL(k_ctl_begin, dim3(gen_grid(std::max(b.total_cells, walk ? b.total_fine : 0))),
+                     dim3(GEN_THREADS), 0, s, b.desc, b.st, b.ri, b.slot_base, b.queues, n, b.pcount,
+                     (uint32_t*)b.phl, (uint64_t)b.total_cells, b.fcountP, walk ? b.total_fine : (uint64_t)0);
   if (ev) (void)hipEventRecord(ev[1], s);
   hipLaunchKernelGGL(k_gen, dim3(gen_grid(b.T_cap + 1)), dim3(GEN_THREADS), 0, s, b.desc, b.st,
                      b.ri, b.slot_base, n, b.T_cap, b.sP, b.sD, b.scell, b.srk, b.surv, b.palive,
@@ -384,7 +406,33 @@ void launch_round(GenBuffers& b, int prec, int diag, hipStream_t s, hipEvent_t* 
   a.nbHl = b.ohl;
   a.qctr = b.queues + Q_OLD * QWORDS;
   a.alive_out = b.palive;
-  launch_pair(PM_GEN_OLD, prec, a, s, &b.tiles);
+  a.skip_walk = walk ? 1u : 0u;
+  WalkArgs w{};
+  w.desc = b.desc;
+  w.ri = b.ri;
+  w.st = b.st;
+  w.cell_inst = b.cell_inst;
+  w.scell = b.scell;
+  w.ncells = b.total_cells;
+  w.n_inst = n;
+  w.prP = b.pP;
+  w.prD = b.pD;
+  w.prX = b.pslot;
+  w.prStart = b.pstart;
+  w.rods = b.oR;
+  w.fcountA = b.fcountA;
+  w.fcountP = b.fcountP;
+  w.flistA = b.flistA;
+  w.flistP = b.flistP;
+  w.sdst = b.sdst;
+  w.slot_base = b.slot_base;
+  w.srank = b.srank;
+  w.alive_out = b.palive;
+  w.surv = b.surv;
+  w.diag = diag;
+  w.qctr = b.queues + Q_WALK_OLD * QWORDS;
+  if (walk) launch_walk(PM_GEN_OLD, prec, w, s);
+  if (cells) launch_pair(PM_GEN_OLD, prec, a, s, &b.tiles);
   if (ev) (void)hipEventRecord(ev[4], s);
   // stage 2: survivors vs higher-priority survivors, over the survivors
   // compacted per cell (a cell's longest rod stays that of all its
@@ -392,7 +440,7 @@ void launch_round(GenBuffers& b, int prec, int diag, hipStream_t s, hipEvent_t* 
   scan_u32(b.palive, b.aidx, b.T_cap, b.scan_tmp, s);
   hipLaunchKernelGGL(k_alive_scatter, dim3(gen_grid(std::max(b.T_cap, b.total_cells + 1))),
                      dim3(GEN_THREADS), 0, s, b.pstart, b.pP, b.pD, b.pslot, b.palive, b.aidx, b.aP,
-                     b.aD, b.aslot, b.astart, b.acount, b.surv, (uint64_t)b.total_cells);
+                     b.aD, b.aslot, b.astart, b.acount, b.surv, (uint64_t)b.total_cells, walk ? b.aR : (float4*)nullptr);
   a.prP = b.aP;
   a.prD = b.aD;
   a.prX = b.aslot;
@@ -408,12 +456,23 @@ void launch_round(GenBuffers& b, int prec, int diag, hipStream_t s, hipEvent_t* 
   a.qctr = b.queues + Q_NEW * QWORDS;
   a.alive_out = nullptr;
   a.surv = b.surv;
-  launch_pair(PM_GEN_NEW, prec, a, s, &b.tiles);
+  w.rods = b.aR;
+  w.prP = b.aP;
+  w.prD = b.aD;
+  w.prX = b.aslot;
+  w.prStart = b.astart;
+  w.qctr = b.queues + Q_WALK_NEW * QWORDS;
+  if (walk) {
+    launch_enter(false, w, b.T_cap, s);
+    launch_walk(PM_GEN_NEW, prec, w, s);
+  }
+  if (cells) launch_pair(PM_GEN_NEW, prec, a, s, &b.tiles);
   if (ev) (void)hipEventRecord(ev[5], s);
   scan_u32(b.surv, b.srank, b.T_cap, b.scan_tmp, s);
   hipLaunchKernelGGL(k_commit, dim3(gen_grid(b.T_cap)), dim3(GEN_THREADS), 0, s, b.desc, b.st,
                      b.ri, b.slot_base, n, b.sP, b.sD, b.scell, b.surv, b.srank, b.bP, b.bD,
-                     b.ostart, b.ocount, b.ohl, b.oP, b.oD, b.oid);
+                     b.ostart, b.ocount, b.ohl, b.oP, b.oD, b.oid, b.sdst, walk ? b.oR : (float4*)nullptr);
+  if (walk) launch_enter(true, w, b.T_cap, s);
   if (ev) (void)hipEventRecord(ev[6], s);
   hipLaunchKernelGGL(k_ctl_end, dim3(1), dim3(WAVE), 0, s, b.desc, b.st, b.ri,
                      b.slot_base, b.srank, b.pstart, b.astart, n);

@@ -30,6 +30,7 @@ struct nf_handle {
   int device = 0;
   std::vector<uint32_t> n_rods;  // current rod count per instance
   std::vector<uint32_t> planned_cap;  // cell slots per instance as planned (NF_OPT_SLOT_SCALE scales them)
+  std::vector<std::pair<uint32_t, uint32_t>> planned_list;  // and entries per crossing list (accepted, survivors)
   std::vector<double> milestones;  // volume fractions (percent) of the state dumps, ascending
   std::string milestone_dir;       // where nf_generate writes them
   bool generated = false;

@@ -16,6 +16,20 @@ namespace nf {
 constexpr int WAVE = 64;
 constexpr float CELL_MARGIN = 1e-4f;  // rods may sit this far outside their cell
 
+constexpr uint32_t ENTRY_BITS = 26;  // of a crossing list's entry: the rod's index
+
+// Fine grid of an instance's crossing lists (nf_walk.hip).  A rod reaches
+// less than one box edge past the box, so one wrap per axis finds its cells.
+struct FineGrid {
+  int32_t n[3];
+  float e[3], ie[3];    // cell edge and its inverse
+  float r;              // half the cut distance, with the margins of the cell arithmetic
+  uint32_t base;        // first fine cell of the instance
+  uint32_t capA, capP;  // entries per list: accepted rods, a round's survivors (multiples of 4)
+  uint32_t on;          // 0: the instance has no lists (the cell-pair engine tests its pairs)
+  uint64_t offA, offP;  // first entry of the instance's lists
+};
+
 // Per-instance constant descriptor (device array, read by every kernel).
 struct InstDesc {
   SampleDesc smp;
@@ -37,12 +51,16 @@ struct InstDesc {
   float hl_max;           // max half length of any rod of this instance
   float R_max;            // max hard-core distance
   uint32_t pad;
+  FineGrid fine;
 };
+
+// What ran out of room (InstState::overflow).
+enum { OVER_SLOTS = 1, OVER_LISTS_A = 2, OVER_LISTS_P = 4 };
 
 // Per-instance dynamic state (device), updated by the round controller.
 struct InstState {
   uint32_t n_acc, round, M, status;
-  uint32_t mprev, aprev, stall, overflow;
+  uint32_t mprev, aprev, stall, overflow;  // overflow: OVER_* bits
   unsigned long long candidates, proposals, pair_tests, rechecks, rej_old, rej_new;
   double max_dd;  // diagnostic max |d32 - d64|
   unsigned long long tile_bytes;      // probe + tile bytes streamed by the reject-vs-accepted kernel
@@ -99,7 +117,7 @@ __device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v)
 constexpr int QUEUES_PER_KERNEL = 64;
 constexpr int QSTRIDE = 32;
 constexpr int QWORDS = QUEUES_PER_KERNEL * QSTRIDE;  // words per launch
-enum { Q_OLD = 0, Q_NEW = 1, Q_CNT = 2, Q_REC = 3, Q_N = 4 };
+enum { Q_OLD = 0, Q_NEW = 1, Q_WALK_OLD = 2, Q_WALK_NEW = 3, Q_N = 4 };
 
 // Device buffers of a generation batch.
 // Launch shape of the generation's pair passes (0 / -1: the built-in
@@ -158,6 +176,17 @@ struct GenBuffers {
   float* phl = nullptr;
   uint32_t* queues = nullptr;  // Q_N * QWORDS
   uint32_t* scan_tmp = nullptr;
+  // crossing lists of the instances that have them (walk: some do; cellwise:
+  // some do not)
+  uint32_t* fcountA = nullptr;  // total_fine
+  uint32_t* fcountP = nullptr;
+  uint32_t* flistA = nullptr;
+  uint32_t* flistP = nullptr;
+  float4* oR = nullptr;         // 2 total_old: accepted rods by cell slot, centre and direction
+  float4* aR = nullptr;         // 2 T_cap: survivors of the first pass, the slot in the direction's w
+  uint32_t* sdst = nullptr;     // T_cap: cell slot of an accepted candidate
+  uint64_t total_fine = 0, total_listA = 0, total_listP = 0;
+  bool walk = false, cellwise = true;
   uint64_t total_cells = 0, total_old = 0, T_cap = 0, total_rods = 0;
   int n_inst = 0;
 };
@@ -228,6 +257,7 @@ struct PairArgs {
   uint32_t ncells_total;
   uint32_t split_min;   // the handle's own split: probes per item of a cell, at least (0: by cost)
   uint32_t npmax;       // work items per cell, at most
+  uint32_t skip_walk;   // leave out the instances with crossing lists
   uint2* items;         // work list of the pass (filled by launch_pair; nullptr: one item per cell)
   uint32_t* qcnt;       // items per queue
   int n_inst;
@@ -269,6 +299,37 @@ struct PairArgs {
   float hl_max, R_max;
   unsigned long long* ctr;  // [0] pair tests, [1] rechecks, [2] max dd bits, [3] tile bytes
   int diag;                 // record max |d32-d64| over full tests
+};
+
+// Arguments of the crossing-list passes (nf_walk.hip).
+struct WalkArgs {
+  const InstDesc* desc;
+  const RoundInfo* ri;
+  InstState* st;
+  const uint32_t* cell_inst;
+  const int32_t* scell;
+  uint64_t ncells;
+  int n_inst;
+  // probes, in cell order
+  const float4* prP;
+  const float4* prD;
+  const uint32_t* prX;      // slot
+  const uint32_t* prStart;  // ncells + 1
+  // rods that the lists' entries name, centre and direction side by side
+  // (survivors: the slot in the direction's w)
+  const float4* rods;
+  uint32_t* fcountA;
+  uint32_t* fcountP;
+  uint32_t* flistA;
+  uint32_t* flistP;
+  // entering accepted rods: their cell slots, the round's slot ranks
+  const uint32_t* sdst;
+  const uint32_t* slot_base;
+  const uint32_t* srank;
+  uint32_t* alive_out;
+  uint32_t* surv;
+  uint32_t* qctr;  // eight chunk counters, QSTRIDE words apart
+  int diag;
 };
 
 enum PairMode { PM_GEN_OLD = 0, PM_GEN_NEW = 1, PM_CNT = 2 };
@@ -324,6 +385,12 @@ void launch_pair(int mode, int prec, const PairArgs& a, hipStream_t s, const Pai
 int pair_grid(int mode);
 // Work items of one cell of a generation pass, at most (sizes the work list).
 uint32_t pair_items_max(uint64_t ncells);
+
+// ---- launchers (nf_walk.hip) ----
+// Enters the round's accepted rods (rods: candidate slots) or the survivors
+// of the first pass in their lists.
+void launch_enter(bool accepted, const WalkArgs& a, uint64_t rods, hipStream_t s);
+void launch_walk(int mode, int prec, const WalkArgs& a, hipStream_t s);
 
 // ---- launchers (nf_seg.hip) ----
 void launch_seg_cross(int prec, const SegCrossArgs& a, hipStream_t s);

@@ -69,4 +69,13 @@ NF_HD float line_apart(const LineSide& p, const LineSide& q, float b) {
   return fmaf(t, t, fmaf(c, c, b));
 }
 
+// The same with the origin at the first rod's centre, whose moment is then
+// zero: u1s its direction times scale, (x, y, z) the second rod's centre.
+NF_HD float line_apart_from(const float3 u1s, float x, float y, float z, const float4 D1, const float4 D2, float b) {
+  const float mx = fmaf(y, D2.z, -(z * D2.y)), my = fmaf(z, D2.x, -(x * D2.z)), mz = fmaf(x, D2.y, -(y * D2.x));
+  const float t = fmaf(u1s.x, mx, fmaf(u1s.y, my, u1s.z * mz));
+  const float c = fmaf(D1.x, D2.x, fmaf(D1.y, D2.y, D1.z * D2.z));
+  return fmaf(t, t, fmaf(c, c, b));
+}
+
 }  // namespace nf

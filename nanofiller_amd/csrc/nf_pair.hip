@@ -764,7 +764,7 @@ __device__ __forceinline__ OldRoles old_roles(const PairArgs& a, uint32_t inst, 
   r.nacc = a.st[inst].n_acc;
   r.nprop = a.prStart[d.cell_base + d.ncells] - a.prStart[d.cell_base];
   r.inv = r.nacc > 4u * r.nprop;
-  r.idle = r.nprop == 0u || r.nacc == 0u;
+  r.idle = r.nprop == 0u || r.nacc == 0u || (a.skip_walk && d.fine.on);
   return r;
 }
 
@@ -977,6 +977,7 @@ __device__ __forceinline__ bool item_plan(const PairArgs& a, uint32_t c, float s
     total = r.inv ? r.nprop : r.nacc;
     h = r.inv ? a.nbHl[c] : a.prHl[c];
   } else {
+    if (a.skip_walk && d.fine.on) return false;
     pc = nb = a.prCount[c];
     total = a.prStart[d.cell_base + d.ncells] - a.prStart[d.cell_base];
     h = a.prHl[c];
@@ -1018,6 +1019,7 @@ __global__ void __launch_bounds__(ITEM_THREADS) k_items(PairArgs a, float waves)
       const OldRoles o = old_roles(a, (uint32_t)i, d);
       if (!o.idle) sum += (float)o.nacc * (float)o.nprop * walk_share(d, d.hl_max);
     } else {
+      if (a.skip_walk && d.fine.on) continue;
       const float n = (float)(a.prStart[d.cell_base + d.ncells] - a.prStart[d.cell_base]);
       sum += 0.5f * n * n * walk_share(d, d.hl_max);
     }
