@@ -34,7 +34,8 @@ struct FineGrid {
 struct InstDesc {
   SampleDesc smp;
   float boxf[3];
-  int32_t ncell[3];
+  int32_t ncell[3];      // cells of the passes
+  int32_t grid[3];       // the generation's cell grid as state files and expand name it
   double cell_scale[3];  // ncell / box, for cell assignment
   float edge[3];         // cell edge
   uint32_t cell_base;    // first global cell of this instance

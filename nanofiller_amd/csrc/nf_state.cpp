@@ -105,7 +105,7 @@ extern "C" int nf_save_state(nf_handle* h, const char* path) {
   uint32_t got = 0;
   int rc = nf_get_rods(h, h->post_inst, rods.data(), n, &got);
   if (rc != NF_OK) return rc;
-  const int32_t ext[3] = {d.ncell[0], d.ncell[1], d.ncell[2]};
+  const int32_t ext[3] = {d.grid[0], d.grid[1], d.grid[2]};
   const uint64_t G = (uint64_t)ext[0] * ext[1] * ext[2];
   // cell of every rod, as the reference's key: floor(x * ext / L) per axis
   std::vector<uint32_t> key(got), occ(G, 0);
@@ -223,7 +223,7 @@ extern "C" int nf_expand(nf_handle* h, int dir, nf_handle** out) {
   int rc = contact_bounds(h, n, P, D, &hlmax, &amax);
   if (rc != NF_OK) return rc;
   const double L = p.box[k];
-  const double E = L / (double)d.ncell[k];
+  const double E = L / (double)d.grid[k];
   const double reach = 2.0 * (double)hlmax + p.contact_gap;
   const double B = std::ceil(reach / E) * E;
   if (!(B <= L)) return fail(h, NF_E_INVALID, "expand: the buffer (rod length + contact gap) is wider than the box");

@@ -116,3 +116,16 @@ def test_options_and_graph_keep_the_packing():
         for _ in range(3):
             pk.generate()
             np.testing.assert_array_equal(pk.rods().view(np.uint32), r0.view(np.uint32))
+
+
+def test_state_file_names_the_planned_grid(tmp_path):
+    """The passes of a large packing of one length run on wider cells; the
+    state file still names the grid of the default cell edge."""
+    p = _params(**LARGE["350,000 rods on cells"])
+    with nf.Packing(p) as pk:
+        pk.generate()
+        pk.save_state(str(tmp_path / "s.bin"))
+    hd = nf.read_state_header(str(tmp_path / "s.bin"))
+    reach = p.len * 1.000001 + 2.0 * p.radius
+    assert hd["ext"] == (int(p.box[0] / (0.85 * reach)),) * 3
+    assert hd["n_rods"] == 350000
