@@ -491,7 +491,9 @@ enum {
 /* Candidate pairs of nf_contacts.  Both give the same contact list.
  * FOOTPRINT: each rod binned into the fine cells its capsule (radius
  * a + gap/2) can touch; rods sharing a cell are tested, each contact
- * reported by the cell holding the midpoint of its closest points.
+ * reported by the cell holding the midpoint of its closest points (lists of
+ * the rods crossing each cell, or home cells of 1..4 fine cells a side,
+ * whichever suits the packing; NF_OPT_FOOTPRINT_* ask for the latter).
  * CELLS: the cell-pair engine of the generator over a centre cell list; its
  * capsule-test count is the number of pairs within centre reach (the
  * reference's stencil count). */

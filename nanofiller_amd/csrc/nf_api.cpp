@@ -186,7 +186,7 @@ double nf::default_cell_edge(double reach_typ, double density, double factor) {
   return e;
 }
 
-static double excluded_volume(double L, double a) {
+double nf::excluded_volume(double L, double a) {
   const double D = 2.0 * a;
   const double PI = 3.14159265358979323846;
   return 0.5 * PI * D * L * L + 2.0 * PI * D * D * L + (4.0 * PI / 3.0) * D * D * D;

@@ -1,8 +1,8 @@
 // nf_contacts.cpp - host orchestration of contact detection and histograms
 // on the packing of instance 0.
 //
-// Contacts: bin -> one pair pass that appends every contact to an unsorted
-// list -> CSR over I (count, scan, scatter) -> canonical row sort -> contact
+// Contacts: bin -> one pair pass (crossing lists, footprints on home cells, or
+// cell pairs) that appends every contact to an unsorted list -> CSR over I (count, scan, scatter) -> canonical row sort -> contact
 // areas.  This replaces the COUNT and RECORD passes of get_contact_counts /
 // get_contact_arrays (src/get_contact_arrays.cu:12-140); a pass whose list
 // overflows the append buffer is repeated once at the exact size.
@@ -21,22 +21,29 @@ using namespace nf;
 namespace nf {
 
 // Reach bounds of the contact rods: the instance's bounds after generation,
-// else the largest half length and radius of the rods (copied once).
-int contact_bounds(nf_handle* h, uint32_t n, const float4* P, const float4* D, float* hlmax, float* amax) {
+// else the largest half length and radius of the rods (one device reduction).
+// dev: how far the squares of the directions are from 1 (0 for generated
+// rods, whose directions are rounded unit vectors).
+int contact_bounds(nf_handle* h, uint32_t n, const float4* P, const float4* D, float* hlmax, float* amax,
+                   float* dev) {
   *hlmax = h->desc[h->post_inst].hl_max;
   *amax = (float)h->params[h->post_inst].radius;
+  if (dev) *dev = 0.0f;
   if (h->generated) return NF_OK;
-  std::vector<float4> hP(n), hD(n);
-  if (n) {
-    HIPCHK(h, hipMemcpy(hP.data(), P, sizeof(float4) * n, hipMemcpyDeviceToHost));
-    HIPCHK(h, hipMemcpy(hD.data(), D, sizeof(float4) * n, hipMemcpyDeviceToHost));
-  }
-  *hlmax = 0.0f;
-  *amax = 0.0f;
-  for (uint32_t i = 0; i < n; ++i) {
-    *hlmax = std::max(*hlmax, hP[i].w);
-    *amax = std::max(*amax, hD[i].w);
-  }
+  uint32_t* out = nullptr;
+  int rc = dalloc(h, &out, 4);
+  if (rc != NF_OK) return rc;
+  float v[3] = {0.0f, 0.0f, 0.0f};
+  fill_u32(out, 0u, 4, h->stream);
+  launch_rod_bounds(P, D, n, out, h->stream);
+  hipError_t e = hipMemcpyAsync(v, out, sizeof(v), hipMemcpyDeviceToHost, h->stream);
+  if (e == hipSuccess) e = sync_stream(h->stream, "rod bounds");
+  if (e == hipSuccess) e = hipGetLastError();
+  dfree(h, out);
+  if (e != hipSuccess) return fail(h, NF_E_HIP, std::string("rod bounds: ") + hipGetErrorString(e));
+  *hlmax = v[0];
+  *amax = v[1];
+  if (dev) *dev = v[2];
   return NF_OK;
 }
 
@@ -192,9 +199,52 @@ static void footprint_cells(nf_handle* h, uint32_t n, double* edge, int* fine) {
   *fine = f < 1 ? 1 : (f > 4 ? 4 : f);
 }
 
-// One contact pass with the given engine.  Returns 1 (not an NF_ status)
-// when the footprint engine found a home cell with too many survivors.
-static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, bool cells) {
+// Ways of a contact pass.
+enum ContactWay {
+  WAY_LISTS,  // crossing lists (nf_walk.hip)
+  WAY_SEG,    // footprints on home cells (nf_seg.hip)
+  WAY_CELLS   // cell pairs (nf_pair.hip)
+};
+
+// Crossing lists of the contact rods: fine cells of 1.5 times the mean spacing
+// as in generation, at least four radii wide (a_max + gap / 2).  False when
+// the rods do not suit them: directions far from unit length, rods that reach
+// past a box edge, radii that do not fit fine cells.
+static bool contact_fine(nf_handle* h, uint32_t n, float dev, double gap, double ew, FineGrid* f, SegGrid* g) {
+  const ContactBuffers& c = h->cb;
+  const nf_params& p = h->params[h->post_inst];
+  if (n == 0 || !(dev <= 1e-3f)) return false;
+  const double V = p.box[0] * p.box[1] * p.box[2];
+  const double typ = p.len_law == NF_LEN_LOGNORMAL ? p.len : 2.0 * (double)c.hl_max;
+  double E = std::min(std::max(1.5 * std::cbrt(V / (double)n), typ / 16.0), typ / 1.5);
+  *g = seg_grid(p.box, E, (double)c.a_max, gap, ew);
+  if (4.0 * (double)g->r > E) {
+    E = 4.0 * (double)g->r;
+    if (E > typ / 1.5) return false;
+    *g = seg_grid(p.box, E, (double)c.a_max, gap, ew);
+  }
+  for (int a = 0; a < 3; ++a) {
+    if (!((double)c.hl_max * 1.002 + (double)g->r < 0.999 * p.box[a])) return false;
+    f->n[a] = g->nc[a];
+    f->e[a] = g->h[a];
+    f->ie[a] = g->inv_h[a];
+  }
+  if ((uint64_t)g->nc[0] * g->nc[1] * g->nc[2] > (1ull << ENTRY_BITS) || n > (1u << ENTRY_BITS)) return false;
+  f->r = g->r;
+  f->base = 0u;
+  f->offA = 0u;
+  // the plan's density peak; a list that is too short ends the pass
+  const double peak = p.den_law == NF_DEN_AGGLOM ? p.agg_peak : (p.den_law == NF_DEN_MESH ? 3.0 : 1.0);
+  const double lam = peak * (double)n / (double)g->ncells * 2.0 * (0.75 * typ / E + 1.0);
+  f->capA = (uint32_t)std::min(4.0 * std::ceil((1.15 * lam + 6.0 * std::sqrt(lam) + 10.0) / 4.0), 8192.0);
+  return (uint64_t)g->ncells * f->capA <= (1ull << 32);
+}
+
+// One contact pass.  Returns 1 (not an NF_ status) when its way does not
+// suit the rods: a crossing list too short, a home cell with too many
+// survivors, rods outside what the way takes.
+static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, ContactWay way) {
+  const bool cells = way == WAY_CELLS;
   ContactBuffers& c = h->cb;
   const nf_params& p = h->params[h->post_inst];
   const InstDesc& d = h->desc[h->post_inst];
@@ -206,8 +256,8 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, bo
   release_contacts(h);
   c.n_rods = n;
   c.gap_cut = gap;
-  float hlmax = 0.0f, amax = 0.0f;
-  int rc = contact_bounds(h, n, P, D, &hlmax, &amax);
+  float hlmax = 0.0f, amax = 0.0f, dev = 0.0f;
+  int rc = contact_bounds(h, n, P, D, &hlmax, &amax, &dev);
   if (rc != NF_OK) return rc;
   c.hl_max = hlmax;
   c.a_max = amax;
@@ -215,6 +265,11 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, bo
   const double reach = contact_reach(c);
   const double Lmax = std::max(p.box[0], std::max(p.box[1], p.box[2]));
   const double ew = 5.9604644775390625e-8 * (Lmax + reach) * 1.01;
+  WalkArgs wa{};
+  if (way == WAY_LISTS && !contact_fine(h, n, dev, gap, ew, &wa.cnt.fine, &wa.cnt.g)) return 1;
+  float4* lrods = nullptr;
+  uint32_t *lcount = nullptr, *llist = nullptr;
+  bool lown = false;  // the lists are this pass's own (else the generation's, idle here)
   unsigned long long* ctr = nullptr;
   uint32_t* tmp = nullptr;
   uint32_t* queues = nullptr;
@@ -231,8 +286,14 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, bo
     dfree(h, ctr);
     dfree(h, tmp);
     dfree(h, queues);
+    dfree(h, lrods);
+    if (lown) {
+      dfree(h, lcount);
+      dfree(h, llist);
+    }
     ctr = nullptr;
-    tmp = queues = nullptr;
+    tmp = queues = lcount = llist = nullptr;
+    lrods = nullptr;
   };
   if (rc != NF_OK) {
     free_scratch();
@@ -245,7 +306,7 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, bo
   PairArgs a{};
   SegCrossArgs xa{};
   // ---- bin: centre cell list
-  if (cells) {
+  if (cells || way == WAY_LISTS) {
     rc = build_contact_cells(h);
   } else {
     double edge = 0.0;
@@ -298,6 +359,45 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, bo
     a.R_max = (float)Rmax * 1.000001f;
     a.ctr = ctr;
     a.diag = h->opt_diag;
+  } else if (way == WAY_LISTS) {
+    WalkContacts& w = wa.cnt;
+    const uint64_t entries = (uint64_t)w.g.ncells * w.fine.capA;
+    rc = dalloc(h, &lrods, 2 * (uint64_t)n);
+    if (h->gb.walk && h->gb.total_fine >= w.g.ncells && h->gb.total_listA >= entries) {
+      lcount = h->gb.fcountA;  // cleared again before the next generation
+      llist = h->gb.flistA;
+    } else {
+      lown = true;
+      if (rc == NF_OK) rc = dalloc(h, &lcount, w.g.ncells);
+      if (rc == NF_OK) rc = dalloc(h, &llist, entries);
+    }
+    if (rc != NF_OK) {
+      free_scratch();
+      return rc == NF_E_NOMEM ? 1 : rc;
+    }
+    for (int k = 0; k < 3; ++k) {
+      w.x.box[k] = p.box[k];
+      w.x.boxf[k] = (float)p.box[k];
+    }
+    w.x.gap64 = gap;
+    w.x.gap32 = (float)gap;
+    w.x.ew = (float)ew;
+    w.x.diag = h->opt_diag;
+    w.ln = line_filter((float)Rmax * 1.000001f, (float)ew, 2.0001f * (hlmax + (float)Rmax) + 32.0f * (float)ew, dev);
+    w.n = n;
+    w.cP = c.cP;
+    w.cD = c.cD;
+    w.cid = c.cid;
+    w.rods = lrods;
+    w.overflow = (uint32_t*)(ctr + 6);
+    w.ctr = ctr;
+    wa.fcountA = lcount;
+    wa.flistA = llist;
+    wa.qctr = queues;
+    fill_u32(lcount, 0u, w.g.ncells, s);
+    launch_enter_contacts(wa, s);
+    c.fp_edge = (double)w.g.h[0];
+    c.fp_fine = 1;
   } else {
     // the claim grid is the cell list's grid
     for (int k = 0; k < 3; ++k) {
@@ -385,6 +485,16 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, bo
       a.outGap64 = appG64;
       a.outImg = appImg;
       launch_pair(PM_CNT, prec, a, s);
+    } else if (way == WAY_LISTS) {
+      WalkContacts& w = wa.cnt;
+      w.app_n = (uint32_t*)(ctr + 4);
+      w.app_cap = (uint32_t)cap;
+      w.outI = appI;
+      w.outJ = appJ;
+      w.outGap = appG;
+      w.outGap64 = appG64;
+      w.outImg = appImg;
+      launch_walk(PM_CNT, prec, wa, s);
     } else {
       xa.app_n = (uint32_t*)(ctr + 4);
       xa.app_cap = (uint32_t)cap;
@@ -396,14 +506,15 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, bo
       launch_seg_cross(prec, xa, s);
     }
     hipEventRecord(ev[2], s);
-    trace("contacts: %u rods, %s pass launched", n, cells ? "cell-pair" : "footprint");
+    trace("contacts: %u rods, %s pass launched", n,
+          cells ? "cell-pair" : (way == WAY_LISTS ? "crossing-list" : "footprint"));
     uint32_t over = 0;
     HIPCHK(h, hipMemcpyAsync(&total, (uint32_t*)(ctr + 4), sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     HIPCHK(h, hipMemcpyAsync(&over, (uint32_t*)(ctr + 6), sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     HIPCHK(h, sync_stream(s, "contact pair pass"));
     HIPCHK(h, hipGetLastError());
     if (over) {
-      trace("contacts: a home cell has more survivors than fit; cell-pair engine instead");
+      trace("contacts: more rods cross a cell than fit; another engine instead");
       free_all();
       return 1;
     }
@@ -463,10 +574,34 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, bo
   return NF_OK;
 }
 
+// Crossing lists where they are the faster way.  A whole call, home cells
+// against lists, MI355X: 20,000 rods 0.41 / 0.35 ms (a home cell's work runs on
+// one wave, and there are few), 2,000 0.46 / 0.30; 100,000 rods of one length
+// 0.41 / 0.47, 1M 1.0 / 1.2, 4M 3.1 / 3.9 (entering pays an atomic per rod and
+// cell); at two to four rods per excluded volume 200,000 0.81 / 0.74, 500,000
+// 1.28 / 1.25, 800,000 1.72 / 1.96.  Log-normal lengths, one rod per excluded
+// volume, 300,000 rods 0.73 / 0.64, 600,000 0.97 / 0.90, 1M 1.24 / 1.25; at a
+// quarter 0.49 / 0.52.  In FP64 home cells evaluate every candidate in full,
+// the lists only what the line filter leaves: 800,000 rods at one to four per
+// excluded volume 3.5..7.2 / 1.5..3.4, 600,000 at a half 0.75 / 1.0 ms.
+static bool lists_suit(const nf_handle* h, int prec) {
+  const nf_params& p = h->params[h->post_inst];
+  const uint32_t n = h->n_rods[h->post_inst];
+  const double crowd = (double)n * excluded_volume(p.len, p.radius) / (p.box[0] * p.box[1] * p.box[2]);
+  if (n <= 60000u) return true;
+  if (p.len_law == NF_LEN_LOGNORMAL && crowd >= 0.4 && n <= 800000u) return true;
+  if (prec == NF_PREC_FP64) return crowd >= 0.8 && n <= 1000000u;
+  return crowd >= 1.8 && n <= 400000u;
+}
+
 int contacts_run(nf_handle* h, double gap, uint64_t* n_out, int prec, unsigned long long*) {
-  const bool cells = h->opt_contact_engine == NF_ENGINE_CELLS;
-  int rc = contacts_pass(h, gap, n_out, prec, cells);
-  if (rc == 1) rc = contacts_pass(h, gap, n_out, prec, true);
+  if (h->opt_contact_engine == NF_ENGINE_CELLS) return contacts_pass(h, gap, n_out, prec, WAY_CELLS);
+  int rc = 1;
+  // (home cells or fine cells asked for by size are the footprint pass's)
+  if (h->opt_footprint_fine == 0 && h->opt_footprint_occ == 0 && lists_suit(h, prec))
+    rc = contacts_pass(h, gap, n_out, prec, WAY_LISTS);
+  if (rc == 1) rc = contacts_pass(h, gap, n_out, prec, WAY_SEG);
+  if (rc == 1) rc = contacts_pass(h, gap, n_out, prec, WAY_CELLS);
   return rc;
 }
 

@@ -63,9 +63,13 @@ void release_contacts(nf_handle* h);
 // stencil): built by the cell engine of nf_contacts, or on demand by the
 // node network.
 int build_contact_cells(nf_handle* h);
-// Largest half length and radius of instance 0's n rods at P, D: the
-// generation's bounds after nf_generate, else scanned (one host copy).
-int contact_bounds(nf_handle* h, uint32_t n, const float4* P, const float4* D, float* hlmax, float* amax);
+// Largest half length and radius of the post-processing instance's n rods at
+// P, D (and how far the squares of their directions are from 1): the
+// generation's bounds after nf_generate, else reduced on the device.
+int contact_bounds(nf_handle* h, uint32_t n, const float4* P, const float4* D, float* hlmax, float* amax,
+                   float* dev = nullptr);
+// Mean excluded volume of two isotropic capsules of length L and radius a.
+double excluded_volume(double L, double a);
 // Default cell edge for a typical pair reach and a mean rod density.
 double default_cell_edge(double reach_typ, double density, double factor);
 // Neighbour offsets of a home block of bx cells along x (offsets from its

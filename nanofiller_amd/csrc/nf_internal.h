@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "nf_common.h"
+#include "nf_line.h"
 #include "nf_seg.h"
 
 namespace nf {
@@ -302,6 +303,29 @@ struct PairArgs {
   int diag;                 // record max |d32-d64| over full tests
 };
 
+// A contact pass over crossing lists: probes and listed rods are the n rods of
+// a cell list.
+struct WalkContacts {
+  FineGrid fine;  // its r, base, capA, offA; lists and lengths in flistA, fcountA
+  SegGrid g;      // the same cells for the reporting rule
+  SegCtx x;
+  LineFilter ln;
+  uint32_t n;
+  const float4* cP;
+  const float4* cD;
+  const uint32_t* cid;
+  float4* rods;        // 2 n: centre and direction side by side (filled by launch_enter_contacts)
+  uint32_t* overflow;  // set when a list is too short
+  uint32_t* app_n;
+  uint32_t app_cap;
+  uint32_t* outI;
+  uint32_t* outJ;
+  float* outGap;
+  double* outGap64;
+  int32_t* outImg;
+  unsigned long long* ctr;  // [0] capsule tests, [1] rechecks, [2] max dd bits, [3] bytes
+};
+
 // Arguments of the crossing-list passes (nf_walk.hip).
 struct WalkArgs {
   const InstDesc* desc;
@@ -331,6 +355,7 @@ struct WalkArgs {
   uint32_t* surv;
   uint32_t* qctr;  // eight chunk counters, QSTRIDE words apart
   int diag;
+  WalkContacts cnt;
 };
 
 enum PairMode { PM_GEN_OLD = 0, PM_GEN_NEW = 1, PM_CNT = 2 };
@@ -392,6 +417,7 @@ uint32_t pair_items_max(uint64_t ncells);
 // of the first pass in their lists.
 void launch_enter(bool accepted, const WalkArgs& a, uint64_t rods, hipStream_t s);
 void launch_walk(int mode, int prec, const WalkArgs& a, hipStream_t s);
+void launch_enter_contacts(const WalkArgs& a, hipStream_t s);
 
 // ---- launchers (nf_seg.hip) ----
 void launch_seg_cross(int prec, const SegCrossArgs& a, hipStream_t s);
@@ -418,6 +444,9 @@ void launch_bin_rods(const BinPlan& bp, const float4* P, const float4* D, uint32
                      const double scale[3], uint32_t* M, uint32_t* scan_tmp, float4* tP, float4* tD,
                      uint32_t* tid, float4* oP, float4* oD, uint32_t* oid, uint32_t* start, uint32_t* count,
                      float* hl, hipStream_t s);
+// out[0..2] (cleared): largest half length, radius and |u|^2 - 1 of the rods, as
+// the bits of non-negative floats.
+void launch_rod_bounds(const float4* P, const float4* D, uint32_t n, uint32_t* out, hipStream_t s);
 void launch_expand_flags(const float4* P, uint32_t n, int k, double L, double B, uint32_t* below, uint32_t* above,
                          hipStream_t s);
 void launch_expand_scatter(const float4* P, const float4* D, uint32_t n, int k, double L, double B,

@@ -21,8 +21,11 @@
 // roundings per component and the six-term sum 6 more of values below 4 S:
 // below 64 u S.  So |t| is off by less than Et = (8 ew + 64 u S) / R, which
 // raises t^2 by less than 2 Et + Et^2 where |t| <= 1; c^2 and the directions'
-// own norms (within 4 u of 1) are off by less than 24 u.  The slack takes
-// 64 u for these and the three last roundings.
+// own norms (their squares within 4 u of 1) are off by less than 24 u.  The
+// slack takes 64 u for these and the three last roundings.  Rods of another
+// source may have directions less exact: with squares within dev of 1,
+// |v|^2 = |u1|^2 |u2|^2 - c^2 exceeds 1 - c^2 by at most 2 dev + dev^2, and
+// lengths, moments and |t| grow by less than a factor 1 + dev.
 #pragma once
 
 #include "nf_common.h"
@@ -39,13 +42,14 @@ struct LineSide {
   float mx, my, mz;  // moment over R
 };
 
-// R_max: largest cut distance; S: see above.
-NF_HD LineFilter line_filter(float R_max, float ew, float S) {
+// R_max: largest cut distance; S: see above; dev: at most 1e-3.
+NF_HD LineFilter line_filter(float R_max, float ew, float S, float dev = 0.0f) {
+  S = S * (1.0f + dev);
   const float R2 = fmaf(R_max * 1.00002f, R_max, 2e-12f * S * S);
   LineFilter f;
   f.scale = recip(sqrt_up(R2)) * (1.0f - 4.0f * U32);
   const float Et = (8.0f * ew + 64.0f * U32 * S) * f.scale;
-  f.slack = fmaf(Et, Et, 2.0f * Et) * 1.001f + 64.0f * U32;
+  f.slack = fmaf(Et, Et, 2.0f * Et) * (1.001f + 2.0f * dev) + 64.0f * U32 + 2.1f * dev;
   return f;
 }
 

@@ -15,6 +15,11 @@
 // evaluation are those of nf_pair.hip), so a packing does not depend on which
 // engine tests its pairs.
 //
+// nf_contacts reads contacts from the same lists, all rods entered with half
+// the contact distance: a pair is taken up by the rod further on in the cell
+// list and reported in the one cell that holds the midpoint of its closest
+// points (nf_seg.h's rule).
+//
 // What bounds them: the walk is VALU issue (75% busy on 32 jamming packings;
 // its rods come from L2, 92% hits), entering is the rate of device-scope
 // atomics, about 30 G/s.  Whole generations on MI355X, cell-pair engine with
@@ -160,6 +165,21 @@ __global__ void __launch_bounds__(ENTER_THREADS) k_enter_accepted(WalkArgs a) {
   }
 }
 
+// The rods of a contact pass, all of a cell list; also side by side in rods.
+__global__ void __launch_bounds__(ENTER_THREADS) k_enter_contacts(WalkArgs a) {
+  const WalkContacts& c = a.cnt;
+  for (uint64_t t = (uint64_t)blockIdx.x * ENTER_THREADS + threadIdx.x; t < (uint64_t)c.n * ENTER_LANES;
+       t += (uint64_t)gridDim.x * ENTER_THREADS) {
+    const uint32_t k = (uint32_t)(t / ENTER_LANES);
+    const float4 P = c.cP[k], D = c.cD[k];
+    if ((threadIdx.x & (ENTER_LANES - 1)) == 0u) {
+      c.rods[2ull * k] = P;
+      c.rods[2ull * k + 1u] = D;
+    }
+    enter(c.fine, a.fcountA, a.flistA, c.fine.offA, c.fine.capA, P, D, k, c.overflow, 1u);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // The walk.  A wave holds 64 >> sb probes, 1 << sb lanes each (more lanes per
 // probe where the launch has few).  The lanes list the cells their probe
@@ -181,7 +201,8 @@ struct WalkLds {
   uint16_t len[WSEG][WAVE];   // entries in its list
   float4 sP[WAVE], sD[WAVE];  // the wave's probes
   uint32_t hit[WAVE];
-  uint32_t qe[WQ], qp[WQ];    // queued pairs: rod; probe | image << 8
+  uint32_t qe[WQ], qp[WQ];    // queued pairs: rod; probe | image << 8 (contacts: entry; probe)
+  uint32_t qc[WQ];            // contacts: the cell they met in, with the probe's image
 };
 
 struct WalkAcc {
@@ -232,13 +253,45 @@ __device__ __forceinline__ void walk_full(const WalkArgs& a, const InstDesc& d, 
   if (cut) L.hit[p] = 1u;
 }
 
+// One queued pair of a contact pass (valid lanes only): the screen, band and
+// reporting rule of the footprint pass (nf_seg.h); appends a contact.
+__device__ __forceinline__ uint32_t crossing_translate(uint32_t image) {
+  return seg_pack(1 - (int)(image & 3u), 1 - (int)((image >> 2) & 3u), 1 - (int)((image >> 4) & 3u));
+}
+
+template <int PREC>
+__device__ __forceinline__ void walk_contact(const WalkContacts& c, WalkLds& L, uint32_t e, bool valid,
+                                             WalkAcc& acc) {
+  const uint32_t ent = L.qe[e], p = L.qp[e], cell = L.qc[e];
+  const float4 P1 = L.sP[p], D1 = L.sD[p];
+  const uint32_t k = L.hit[p];
+  if (!valid) return;
+  const uint32_t idx = ent & ENT_MASK;
+  const float4 P2 = c.rods[2ull * idx], D2 = c.rods[2ull * idx + 1u];
+  const uint32_t m1 = crossing_translate(cell >> ENT_BITS), m2 = crossing_translate(ent >> ENT_BITS);
+  const int code = seg_screen<PREC>(c.x, P1, D1, m1, P2, D2, m2, acc.tests);
+  if (code == 0) return;
+  SegHit hit;
+  if (!seg_full<PREC>(c.x, c.g, c.cid[k], P1, D1, m1, c.cid[idx], P2, D2, m2, cell & ENT_MASK, code, acc.tests,
+                      acc.rech, acc.maxdd, &hit))
+    return;
+  const uint32_t pos = atomicAdd(c.app_n, 1u);
+  if (pos >= c.app_cap) return;
+  c.outI[pos] = hit.I;
+  c.outJ[pos] = hit.J;
+  c.outGap[pos] = (float)hit.gap;
+  c.outGap64[pos] = hit.gap;
+  c.outImg[pos] = hit.img;
+}
+
 template <int MODE, int PREC>
 __global__ void __launch_bounds__(WAVE, 4) k_walk(WalkArgs a) {
   __shared__ WalkLds L;
-  if (wuni(a.ri->T) == 0u) return;
+  constexpr bool CNT = MODE == PM_CNT;
+  if (!CNT && wuni(a.ri->T) == 0u) return;
   if (MODE == PM_GEN_OLD && wuni(a.ri->old) == 0u) return;
   const uint32_t lane = threadIdx.x;
-  const uint32_t total = wuni(a.prStart[a.ncells]);
+  const uint32_t total = CNT ? a.cnt.n : wuni(a.prStart[a.ncells]);
   // lanes per probe: more where that leaves a wave fewer than two turns
   int sb = 0;
   while (sb < 3 && ((uint64_t)total << sb) < (uint64_t)gridDim.x * (2u * WAVE)) ++sb;
@@ -271,12 +324,24 @@ __global__ void __launch_bounds__(WAVE, 4) k_walk(WalkArgs a) {
   const float4* rods = nullptr;
   LineFilter ln = {0.0f, 0.0f};
   float lb = 0.0f;
+  if (CNT) {
+    cap = a.cnt.fine.capA;
+    count = a.fcountA + a.cnt.fine.base;
+    list = a.flistA + a.cnt.fine.offA;
+    rods = a.cnt.rods;
+    ln = a.cnt.ln;
+    lb = -1.0f - ln.slack;
+  }
+  unsigned long long bytes = 0;
   bool started = false;
   uint32_t kills = 0;
   auto flush_queue = [&]() {
     if (qn == 0u) return;
     __syncthreads();
-    walk_full<PREC>(a, *d, rods, L, min(lane, qn - 1u), lane < qn, acc);
+    if (CNT)
+      walk_contact<PREC>(a.cnt, L, min(lane, qn - 1u), lane < qn, acc);
+    else
+      walk_full<PREC>(a, *d, rods, L, min(lane, qn - 1u), lane < qn, acc);
     qn = 0u;
     __syncthreads();
   };
@@ -294,7 +359,15 @@ __global__ void __launch_bounds__(WAVE, 4) k_walk(WalkArgs a) {
     double v = acc.maxdd;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, WAVE));
-    if (lane == 0u) {
+    if (CNT) {
+      const unsigned long long wb = wave_sum_u64(bytes);
+      if (lane == 0u) {
+        if (wt) atomicAdd(&a.cnt.ctr[0], wt);
+        if (wr) atomicAdd(&a.cnt.ctr[1], wr);
+        if (v > 0.0) atomicMax(&a.cnt.ctr[2], (unsigned long long)__double_as_longlong(v));
+        atomicAdd(&a.cnt.ctr[3], wb);
+      }
+    } else if (lane == 0u) {
       InstState& st = a.st[inst];
       if (wt) atomicAdd(&st.pair_tests, wt);
       if (wr) atomicAdd(&st.rechecks, wr);
@@ -316,7 +389,7 @@ __global__ void __launch_bounds__(WAVE, 4) k_walk(WalkArgs a) {
       const bool hand = cur < part_end, swap = lv == 0ull && cur == part_end && (open || cur < end);
       if (again || hand || swap) {
         flush_queue();  // the idle probes' verdicts
-        const bool hit = idle && have && L.hit[pl] != 0u;
+        const bool hit = !CNT && idle && have && L.hit[pl] != 0u;
         const bool cont = idle && have && (mm & group) != 0ull && !hit;
         if (idle && have && !cont) {
           if (hit && sub == 0u) verdict();
@@ -351,6 +424,10 @@ __global__ void __launch_bounds__(WAVE, 4) k_walk(WalkArgs a) {
               }
               if (!open) break;
             }
+            if (CNT) {
+              part_end = end;
+              break;
+            }
             const uint32_t i0 = a.n_inst == 1 ? 0u : wuni(a.cell_inst[a.scell[a.prX[cur]]]);
             const InstDesc* di = a.desc + i0;
             part_end = min(end, wuni(a.prStart[di->cell_base + di->ncells]));
@@ -379,16 +456,16 @@ __global__ void __launch_bounds__(WAVE, 4) k_walk(WalkArgs a) {
         const bool fresh = need && rank < part_end - cur;
         if (fresh) {
           k = cur + rank;
-          P1 = a.prP[k];
-          D1 = a.prD[k];
-          slot = a.prX[k];
+          P1 = CNT ? rods[2ull * k] : a.prP[k];
+          D1 = CNT ? rods[2ull * k + 1u] : a.prD[k];
+          slot = CNT ? k : a.prX[k];
           u1 = make_float3(ln.scale * D1.x, ln.scale * D1.y, ln.scale * D1.z);
           c0 = 0u;
           have = true;
           if (sub == 0u) {
             L.sP[pl] = P1;
             L.sD[pl] = D1;
-            L.hit[pl] = 0u;
+            L.hit[pl] = CNT ? k : 0u;
           }
         }
         cur += min((uint32_t)__popcll(nm), part_end - cur);
@@ -396,7 +473,7 @@ __global__ void __launch_bounds__(WAVE, 4) k_walk(WalkArgs a) {
         // four loads in flight; empty lists leave
         if (fresh || cont) {
           uint32_t ns = 0, ord = 0;
-          crossed_cells(d->fine, P1, D1, [&](uint32_t c, uint32_t image) {
+          crossed_cells(CNT ? a.cnt.fine : d->fine, P1, D1, [&](uint32_t c, uint32_t image) {
             const uint32_t o = ord++;
             if ((o & ((1u << sb) - 1u)) != sub) return;
             const uint32_t at = (o >> sb) - c0;  // wraps below c0
@@ -464,9 +541,10 @@ __global__ void __launch_bounds__(WAVE, 4) k_walk(WalkArgs a) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           const uint32_t im = ent[u] >> ENT_BITS;
-          P2[u].x += (float)rel_img(pi, im, 0) * d->boxf[0];
-          P2[u].y += (float)rel_img(pi, im, 1) * d->boxf[1];
-          P2[u].z += (float)rel_img(pi, im, 2) * d->boxf[2];
+          const float* bf = CNT ? a.cnt.x.boxf : d->boxf;
+          P2[u].x += (float)rel_img(pi, im, 0) * bf[0];
+          P2[u].y += (float)rel_img(pi, im, 1) * bf[1];
+          P2[u].z += (float)rel_img(pi, im, 2) * bf[2];
         }
       }
 #pragma unroll
@@ -475,8 +553,13 @@ __global__ void __launch_bounds__(WAVE, 4) k_walk(WalkArgs a) {
                  line_apart_from(u1, P2[u].x - P1.x, P2[u].y - P1.y, P2[u].z - P1.z, D1, D2[u], lb) < 0.0f;
         // same-round pass: only an earlier slot rejects the probe
         if (MODE == PM_GEN_NEW) may[u] = may[u] && __float_as_uint(D2[u].w) < slot;
+        // contacts: each pair from the rod further on in the cell list
+        if (CNT) may[u] = may[u] && (ent[u] & ENT_MASK) < k;
       }
-      acc.tests += min(m, 4u);
+      if (CNT)
+        bytes += 36ull * min(m, 4u);
+      else
+        acc.tests += min(m, 4u);
       pos += 4u;
     }
     bool ran = false;
@@ -487,29 +570,38 @@ __global__ void __launch_bounds__(WAVE, 4) k_walk(WalkArgs a) {
       if (may[u]) {
         const uint32_t at = qn + wprefix(m);
         const uint32_t im = ent[u] >> ENT_BITS, pi = cell >> ENT_BITS;
-        L.qe[at] = ent[u] & ENT_MASK;
-        L.qp[at] = pl | (uint32_t)(rel_img(pi, im, 0) + 2) << 8 | (uint32_t)(rel_img(pi, im, 1) + 2) << 11 |
-                   (uint32_t)(rel_img(pi, im, 2) + 2) << 14;
+        if (CNT) {
+          L.qe[at] = ent[u];
+          L.qp[at] = pl;
+          L.qc[at] = cell;
+        } else {
+          L.qe[at] = ent[u] & ENT_MASK;
+          L.qp[at] = pl | (uint32_t)(rel_img(pi, im, 0) + 2) << 8 | (uint32_t)(rel_img(pi, im, 1) + 2) << 11 |
+                     (uint32_t)(rel_img(pi, im, 2) + 2) << 14;
+        }
       }
       qn += (uint32_t)__popcll(m);
       if (qn >= (uint32_t)WAVE) {
         __syncthreads();
-        walk_full<PREC>(a, *d, rods, L, qn - WAVE + lane, true, acc);
+        if (CNT)
+          walk_contact<PREC>(a.cnt, L, qn - WAVE + lane, true, acc);
+        else
+          walk_full<PREC>(a, *d, rods, L, qn - WAVE + lane, true, acc);
         qn -= WAVE;
         __syncthreads();
         ran = true;
       }
     }
-    if (qn >= QFLUSH) {
+    if (!CNT && qn >= QFLUSH) {
       flush_queue();
       ran = true;
     }
     // a proposal once cut is rejected whatever else it overlaps
-    if (ran) live = live && L.hit[pl] == 0u;
+    if (!CNT && ran) live = live && L.hit[pl] == 0u;
   }
-  if (d == nullptr) return;
+  if (!CNT && d == nullptr) return;
   flush_queue();
-  if (have && sub == 0u && L.hit[pl] != 0u) verdict();
+  if (!CNT && have && sub == 0u && L.hit[pl] != 0u) verdict();
   flush_stats();
 }
 
@@ -527,9 +619,18 @@ void launch_enter(bool accepted, const WalkArgs& a, uint64_t rods, hipStream_t s
     hipLaunchKernelGGL(k_enter_survivors, dim3(enter_grid(rods)), dim3(ENTER_THREADS), 0, s, a);
 }
 
+void launch_enter_contacts(const WalkArgs& a, hipStream_t s) {
+  hipLaunchKernelGGL(k_enter_contacts, dim3(enter_grid(a.cnt.n)), dim3(ENTER_THREADS), 0, s, a);
+}
+
 void launch_walk(int mode, int prec, const WalkArgs& a, hipStream_t s) {
   const dim3 grid(pair_grid(mode)), block(WAVE);
-  if (mode == PM_GEN_OLD) {
+  if (mode == PM_CNT) {
+    if (prec == NF_PREC_FP64)
+      hipLaunchKernelGGL((k_walk<PM_CNT, NF_PREC_FP64>), grid, block, 0, s, a);
+    else
+      hipLaunchKernelGGL((k_walk<PM_CNT, NF_PREC_FP32_RECHECK>), grid, block, 0, s, a);
+  } else if (mode == PM_GEN_OLD) {
     if (prec == NF_PREC_FP64)
       hipLaunchKernelGGL((k_walk<PM_GEN_OLD, NF_PREC_FP64>), grid, block, 0, s, a);
     else
