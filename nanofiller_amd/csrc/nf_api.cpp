@@ -95,7 +95,8 @@ void trace(const char* fmt, ...) {
   va_end(ap);
 }
 
-hipError_t sync_stream(hipStream_t s, const char* what) {
+template <class Query>
+static hipError_t poll(Query query, const char* what) {
   static double limit = -1.0;
   if (limit < 0.0) {
     const char* e = std::getenv("NF_SYNC_TIMEOUT_S");
@@ -104,7 +105,7 @@ hipError_t sync_stream(hipStream_t s, const char* what) {
   }
   const auto t0 = std::chrono::steady_clock::now();
   for (;;) {
-    const hipError_t e = hipStreamQuery(s);
+    const hipError_t e = query();
     if (e != hipErrorNotReady) return e;
     const double el = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     if (el > limit) {
@@ -114,6 +115,14 @@ hipError_t sync_stream(hipStream_t s, const char* what) {
     }
     std::this_thread::sleep_for(std::chrono::microseconds(el < 0.01 ? 2 : 200));
   }
+}
+
+hipError_t sync_stream(hipStream_t s, const char* what) {
+  return poll([&] { return hipStreamQuery(s); }, what);
+}
+
+hipError_t sync_event(hipEvent_t ev, const char* what) {
+  return poll([&] { return hipEventQuery(ev); }, what);
 }
 
 // Returns a block to the handle's pool.  The handle's stream is drained
@@ -734,6 +743,7 @@ extern "C" void nf_destroy(nf_handle* h) {
   for (auto& kv : h->pool) (void)hipFree(kv.second);
   for (auto& e : h->ev)
     if (e) (void)hipEventDestroy(e);
+  if (h->cg_host) (void)hipHostFree(h->cg_host);
   if (h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
 }

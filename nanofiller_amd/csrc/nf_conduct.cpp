@@ -1,7 +1,9 @@
 // nf_conduct.cpp - host side of the DC conductance solve on the network of
 // the last nf_network call (see nf_solve.hip): reduced system, conjugate
 // gradients with a convergence check every CG_CHECK iterations, currents and
-// rod potentials.
+// rod potentials.  The check itself runs on the device; on a long solve the
+// next iterations are queued before its verdict is read, and do nothing if it
+// was the last.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -14,7 +16,10 @@
 using namespace nf;
 
 namespace {
-constexpr uint32_t CG_CHECK = 16;  // iterations queued between host convergence checks
+constexpr uint32_t CG_CHECK = 16;  // iterations between convergence checks
+// Iterations from which one batch is queued ahead: a converged solve then has
+// 32 launches that do nothing (60 us), against 8 us of waiting per check.
+constexpr uint32_t CG_AHEAD = 128;
 }
 
 extern "C" int nf_conductance(nf_handle* h, double tol, uint32_t max_iter, nf_conductance_info* info,
@@ -28,12 +33,13 @@ extern "C" int nf_conductance(nf_handle* h, double tol, uint32_t max_iter, nf_co
   uint32_t *flag = nullptr, *act = nullptr, *rl = nullptr, *idx = nullptr, *off = nullptr,
            *tmp = nullptr, *crow = nullptr, *ccol = nullptr;
   double *cval = nullptr, *dinv = nullptr, *bsrc = nullptr, *bsnk = nullptr, *x = nullptr,
-         *r = nullptr, *z = nullptr, *pv = nullptr, *q = nullptr, *part = nullptr, *vdev = nullptr;
+         *r = nullptr, *pv = nullptr, *q = nullptr, *part = nullptr, *vdev = nullptr;
+  double2* zp = nullptr;
   CgScal* scal = nullptr;
   uint32_t *acto = nullptr, *rlo = nullptr, *idxo = nullptr, *offo = nullptr;
   auto release = [&]() {
     void* ptrs[] = {flag, act, rl,   idx, off, tmp,  crow, ccol, cval, dinv, bsrc, bsnk,
-                    x,    r,   z,    pv,  q,   part, vdev, scal, acto, rlo,  idxo, offo};
+                    x,    r,   zp,   pv,  q,   part, vdev, scal, acto, rlo,  idxo, offo};
     for (void* p : ptrs) dfree(h, p);
   };
   const uint64_t n1 = (uint64_t)n + 1;
@@ -46,7 +52,7 @@ extern "C" int nf_conductance(nf_handle* h, double tol, uint32_t max_iter, nf_co
   ALLOC(idx, n1);
   ALLOC(off, n1);
   ALLOC(tmp, scan_tmp_words(n1));
-  ALLOC(part, 2 * CG_MAX_BLOCKS);
+  ALLOC(part, 3 * CG_MAX_BLOCKS);
   ALLOC(scal, 1);
   if (rc != NF_OK) {
     release();
@@ -114,41 +120,71 @@ extern "C" int nf_conductance(nf_handle* h, double tol, uint32_t max_iter, nf_co
     ALLOC(bsnk, m);
     ALLOC(x, m);
     ALLOC(r, m);
-    ALLOC(z, m);
+    ALLOC(zp, m);
     ALLOC(pv, m);
     ALLOC(q, m);
     if (rc != NF_OK) {
       release();
       return rc;
     }
+    if (!h->cg_host) {
+      if (hipError_t e = hipHostMalloc((void**)&h->cg_host, 2 * sizeof(CgScal), hipHostMallocDefault); e != hipSuccess) {
+        h->cg_host = nullptr;
+        release();
+        return fail(h, NF_E_NOMEM, std::string("conductance scalars: ") + hipGetErrorString(e));
+      }
+    }
     launch_cs_fill(c.nrow, c.ncol, c.nval, n, act, idx, off, crow, ccol, cval, dinv, bsrc, bsnk, s);
     fill_u32(crow + m, nnz, 1, s);
-    CgArgs a{m, crow, ccol, cval, dinv, bsrc, bsnk, x, r, z, pv, q, part, scal};
+    CgArgs a{m, 0, 0, crow, ccol, cval, dinv, bsrc, bsnk, x, r, pv, q, zp,
+             part, part + CG_MAX_BLOCKS, part + 2 * CG_MAX_BLOCKS, scal};
+    cg_grids(a);
+    struct Check {
+      uint32_t it;     // iterations before it
+      CgScal* host;    // pinned copy of the scalars
+      hipEvent_t done;
+    };
+    Check slot[2] = {{0, h->cg_host, h->ev[2]}, {0, h->cg_host + 1, h->ev[3]}};
+    uint32_t pending = 0, newest = 0;
     hipEventRecord(h->ev[0], s);
-    launch_cg_init(a, s);
+    // queues what leads to the next check (init for the first), the check and the copy of its verdict
+    auto queue = [&](uint32_t it, uint32_t count, Check& c) -> hipError_t {
+      if (count == 0)
+        launch_cg_init(a, tol, s);
+      else
+        launch_cg_iterations(a, it, count, tol, s);
+      c.it = it + count;
+      hipError_t e = hipMemcpyAsync(c.host, scal, sizeof(CgScal), hipMemcpyDeviceToHost, s);
+      if (e == hipSuccess) e = hipEventRecord(c.done, s);
+      ++pending;
+      return e;
+    };
     uint32_t it = 0;
     CgScal hs{};
-    bool conv = false;
+    hipError_t e = queue(0, 0, slot[0]);
     for (;;) {
-      if (hipError_t e_ = hipMemcpyAsync(&hs, scal, sizeof(CgScal), hipMemcpyDeviceToHost, s); e_ != hipSuccess) {
-      release();
-      return fail(h, NF_E_HIP, std::string("conductance copy: ") + hipGetErrorString(e_));
-    }
-      if (hipError_t e = sync_stream(s, "conductance iterations"); e != hipSuccess) {
+      Check& oldest = slot[newest ^ (pending - 1u)];
+      const uint32_t last = slot[newest].it;
+      if (e == hipSuccess && pending == 1 && last >= CG_AHEAD && last < max_iter) {
+        newest ^= 1u;
+        e = queue(last, std::min(CG_CHECK, max_iter - last), slot[newest]);
+      }
+      if (e == hipSuccess) e = sync_event(oldest.done, "conductance iterations");
+      if (e != hipSuccess) {
         release();
         return fail(h, NF_E_HIP, std::string("conductance iterations: ") + hipGetErrorString(e));
       }
-      const double res = hs.bb > 0.0 ? std::sqrt(std::max(hs.rr, 0.0) / hs.bb) : 0.0;
-      out.residual = res;
-      if (res <= tol) {
-        conv = true;
-        break;
+      --pending;
+      hs = *oldest.host;
+      it = oldest.it;
+      out.residual = hs.res;
+      if (hs.done || it >= max_iter) break;
+      if (pending == 0) {
+        newest ^= 1u;
+        e = queue(it, std::min(CG_CHECK, max_iter - it), slot[newest]);
       }
-      if (it >= max_iter || !std::isfinite(res)) break;
-      const uint32_t k = std::min(CG_CHECK, max_iter - it);
-      for (uint32_t j = 0; j < k; ++j) launch_cg_iteration(a, s);
-      it += k;
     }
+    const bool conv = hs.done == CG_CONVERGED;
     launch_cg_current(a, s);
     hipEventRecord(h->ev[1], s);
     if (hipError_t e_ = hipMemcpyAsync(&hs, scal, sizeof(CgScal), hipMemcpyDeviceToHost, s); e_ != hipSuccess) {

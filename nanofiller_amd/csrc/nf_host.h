@@ -44,6 +44,7 @@ struct nf_handle {
   uint64_t contact_hint = 0;                      // contacts found by the last call (append capacity)
   nf_network_info net_info = {};
   std::vector<uint32_t> reduce_ids;  // old id of every rod kept by the last nf_reduce
+  nf::CgScal* cg_host = nullptr;  // pinned: scalars of nf_conductance's last two checks
   float net_ms = 0.0f;  // device time of the last nf_network call
 };
 
@@ -55,6 +56,7 @@ int fail(nf_handle* h, int code, const std::string& msg);
 // Waits for the stream with a wall-clock limit (NF_SYNC_TIMEOUT_S, default
 // 120 s); prints progress when NF_TRACE is set.
 hipError_t sync_stream(hipStream_t s, const char* what);
+hipError_t sync_event(hipEvent_t ev, const char* what);
 void trace(const char* fmt, ...);
 int dalloc_bytes(nf_handle* h, void** p, size_t bytes);
 void dfree(nf_handle* h, void* p);

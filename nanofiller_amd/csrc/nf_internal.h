@@ -484,24 +484,30 @@ void launch_vdw(const float4* P, const float4* D, uint32_t n, const uint32_t* ro
 
 // ---- conductance solve (nf_solve.hip) ----
 constexpr int CG_MAX_BLOCKS = 1024;
+constexpr uint32_t CG_CONVERGED = 1u, CG_BROKEN = 2u;
 // Device scalars of the conjugate-gradient solve.
 struct CgScal {
-  double rz, pq, alpha, beta, rr, bb;  // r.z, p.Ap, step, direction update, r.r, b.b
-  double isrc, isnk;                   // currents into the source and out to the sink
+  double rz[2];       // r.z of even and odd iterations
+  double bb, res;     // b.b, relative residual at the last check
+  double isrc, isnk;  // currents into the source and out to the sink
+  uint32_t done, pad;
 };
 struct CgArgs {
-  uint32_t m;  // unknowns
+  uint32_t m;   // unknowns
+  uint32_t nb, ns;  // blocks of the vector kernels and of the product (cg_grids)
   const uint32_t* crow;
   const uint32_t* ccol;
   const double* cval;
   const double* dinv;
   const double* bsrc;  // source couplings (right-hand side)
   const double* bsnk;  // sink couplings
-  double *x, *r, *z, *p, *q;
-  double* part;  // 2 * CG_MAX_BLOCKS block partials
+  double *x, *r, *p, *q;
+  double2* zp;       // preconditioned residual and last direction
+  // CG_MAX_BLOCKS block sums each; part_rr follows part_rz
+  double *part_pq, *part_rz, *part_rr;
   CgScal* scal;
 };
-int cg_grid(uint64_t m);
+void cg_grids(CgArgs& a);
 void launch_cs_flag(const uint32_t* nrow, const uint32_t* ncol, const uint32_t* labels, uint32_t n,
                     uint32_t* flag, hipStream_t s);
 void launch_cs_active(const uint32_t* nrow, const uint32_t* ncol, const uint32_t* labels,
@@ -519,8 +525,9 @@ void launch_cs_potential(uint32_t n, const uint32_t* labels, const uint32_t* fla
 void launch_cs_order(uint32_t n, const uint32_t* ord, const uint32_t* act, const uint32_t* rl, uint32_t* acto,
                      uint32_t* rlo, const uint32_t* idxo, const uint32_t* offo, uint32_t* idx, uint32_t* off,
                      int stage, hipStream_t s);
-void launch_cg_init(const CgArgs& a, hipStream_t s);
-void launch_cg_iteration(const CgArgs& a, hipStream_t s);
+void launch_cg_init(const CgArgs& a, double tol, hipStream_t s);
+// Iterations it .. it + count - 1, then a check of the residual.
+void launch_cg_iterations(const CgArgs& a, uint32_t it, uint32_t count, double tol, hipStream_t s);
 void launch_cg_current(const CgArgs& a, hipStream_t s);
 
 // ---- node-level segment network (nf_nodes.hip) ----

@@ -15,9 +15,15 @@
 // conjugate gradients in FP64.
 //
 // Every reduction is a fixed-order tree over fixed per-block ranges, so a
-// solve is bit-reproducible on one device and grid.  The kernels stream the
-// reduced CSR and five vectors per iteration and are bound by HBM bandwidth
-// (or, on small systems, by launch latency).
+// solve is bit-reproducible on one device and grid.  An iteration is two
+// kernels: the product (which also forms the new direction and the sum p.Ap)
+// and the update (x, r, z and the sums r.z, r.r); each block of the next
+// kernel adds up the block sums of the one before, so no launch serves a
+// scalar alone.  On systems that stay in the caches the chain of dependent
+// loads and the launches bound an iteration, on larger ones the CSR and the
+// vectors that it streams.
+#include <algorithm>
+
 #include "nf_internal.h"
 
 namespace nf {
@@ -26,18 +32,66 @@ namespace {
 
 constexpr int NT = 256;
 
+// x of the lane that the DPP control names, 0 where there is none.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_f64(double x) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xF, false);
+  return __longlong_as_double(((long long)hi << 32) | (uint32_t)lo);
+}
+
+// Sum over a wave in a fixed order, in lane 63 (shuffles through LDS took
+// three times as long, and an iteration waits for five sums in a row).
+__device__ __forceinline__ double wave_sum_last(double v) {
+  v += dpp_f64<0xB1, 0xF>(v);   // lane ^ 1
+  v += dpp_f64<0x4E, 0xF>(v);   // lane ^ 2
+  v += dpp_f64<0x141, 0xF>(v);  // the other quad of eight lanes
+  v += dpp_f64<0x140, 0xF>(v);  // the other eight of a row of 16
+  v += dpp_f64<0x142, 0xA>(v);  // row before, into rows 1 and 3
+  v += dpp_f64<0x143, 0xC>(v);  // rows 0 and 1, into rows 2 and 3
+  return v;
+}
+
+// Sums over a block of NW waves, valid in every thread: the waves' sums in
+// order.  sh[NW] is written once per call.
+template <int NW = NT / WAVE>
 __device__ __forceinline__ double block_sum(double v, double* sh) {
-  // wave sums in a fixed butterfly order, then the waves' sums in order
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
-  const int w = threadIdx.x / WAVE, l = threadIdx.x % WAVE;
-  if (l == 0) sh[w] = v;
+  v = wave_sum_last(v);
+  if (threadIdx.x % WAVE == WAVE - 1) sh[threadIdx.x / WAVE] = v;
   __syncthreads();
   double t = 0.0;
-  if (threadIdx.x == 0)
-    for (int k = 0; k < NT / WAVE; ++k) t += sh[k];
+#pragma unroll
+  for (int k = 0; k < NW; ++k) t += sh[k];
+  return t;
+}
+
+template <int NW = NT / WAVE>
+__device__ __forceinline__ double2 block_sum2(double v, double w, double2* sh) {
+  v = wave_sum_last(v);
+  w = wave_sum_last(w);
+  if (threadIdx.x % WAVE == WAVE - 1) sh[threadIdx.x / WAVE] = make_double2(v, w);
   __syncthreads();
-  return t;  // valid in thread 0
+  double2 t = make_double2(0.0, 0.0);
+#pragma unroll
+  for (int k = 0; k < NW; ++k) {
+    t.x += sh[k].x;
+    t.y += sh[k].y;
+  }
+  return t;
+}
+
+// This thread's share of at most CG_MAX_BLOCKS block sums of an earlier
+// kernel: loads without a branch, so that they go out with the caller's.
+template <int NW = NT / WAVE>
+__device__ __forceinline__ double part_share(const double* __restrict__ part, uint32_t nb) {
+  constexpr uint32_t STEP = NW * WAVE;
+  double w[CG_MAX_BLOCKS / STEP], v = 0.0;
+#pragma unroll
+  for (uint32_t q = 0; q < CG_MAX_BLOCKS / STEP; ++q) w[q] = part[min(threadIdx.x + q * STEP, nb - 1u)];
+#pragma unroll
+  for (uint32_t q = 0; q < CG_MAX_BLOCKS / STEP; ++q) v += threadIdx.x + q * STEP < nb ? w[q] : 0.0;
+  return v;
 }
 
 // Marks the components coupled to the source (bit 0) and the sink (bit 1):
@@ -137,133 +191,171 @@ __global__ void __launch_bounds__(NT) k_cs_from_order(uint32_t n, const uint32_t
   }
 }
 
-// x = 0, r = b, z = D^-1 r, p = z; partials of r.z and b.b.
-__global__ void __launch_bounds__(NT) k_cg_init(uint32_t m, const double* __restrict__ b,
-                                                const double* __restrict__ dinv,
-                                                double* __restrict__ x, double* __restrict__ r,
-                                                double* __restrict__ z, double* __restrict__ p,
-                                                double* __restrict__ part) {
-  __shared__ double sh[NT / WAVE];
+// x = 0, r = b, (z, p) = (D^-1 r, 0); partials of r.z and b.b.
+__global__ void __launch_bounds__(NT) k_cg_init(CgArgs a) {
+  __shared__ double2 sh[NT / WAVE];
   double rz = 0.0, bb = 0.0;
-  for (uint32_t k = blockIdx.x * NT + threadIdx.x; k < m; k += gridDim.x * NT) {
-    const double bk = b[k], zk = dinv[k] * bk;
-    x[k] = 0.0;
-    r[k] = bk;
-    z[k] = zk;
-    p[k] = zk;
+  for (uint32_t k = blockIdx.x * NT + threadIdx.x; k < a.m; k += gridDim.x * NT) {
+    const double bk = a.bsrc[k], zk = a.dinv[k] * bk;
+    a.x[k] = 0.0;
+    a.r[k] = bk;
+    a.zp[k] = make_double2(zk, 0.0);
     rz += bk * zk;
     bb += bk * bk;
   }
-  const double s1 = block_sum(rz, sh);
-  const double s2 = block_sum(bb, sh);
+  const double2 t = block_sum2(rz, bb, sh);
   if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = s1;
-    part[2 * blockIdx.x + 1] = s2;
+    a.part_rz[blockIdx.x] = t.x;
+    a.part_rr[blockIdx.x] = t.y;
   }
 }
 
-// q = A p; partial of p.q.  Four lanes per row: lane j of a row sums its
-// entries j, j + 4, ... (consecutive lanes read consecutive entries, so the
-// column and value loads coalesce across the rows of a wave), then the four
-// lane sums combine in a fixed butterfly, so the result is reproducible.
-constexpr int SPMV_LANES = 4;
+// p = z + beta p and q = A p; partial of p.q.  z and the last direction lie
+// side by side, so a column costs one 16-byte gather and the direction needs
+// no pass of its own; it is written for the update kernel, not over the last
+// one, which other rows still read.
+//
+// Two lanes per row, lane j summing its entries j, j + 2, ...; the lane sums
+// combine in a fixed order, so the result is reproducible.  A row's chain of
+// dependent loads (offsets, column, gather) bounds it, not the bytes: the first
+// eight entries and the block sums that beta needs are fetched side by side,
+// and every row of 262,000 is in flight at once.  178,000 unknowns with 3.9
+// entries a row: 7.2 us, and the update 5.8, where product, direction, update
+// and two scalars had been launches of 9.9, 3.5, 4.3 and 3.1 us each; 3120
+// iterations 64 -> 37..43 ms.  One or four lanes per row: 7.2, 8.7 us.
+constexpr int SPMV_LANES = 2, SPMV_AHEAD = 8 / SPMV_LANES;  // entries of a row fetched at once: 8
+constexpr int SPMV_NT = 512;
+constexpr int SPMV_ROWS = SPMV_NT / SPMV_LANES;
 
-__global__ void __launch_bounds__(NT) k_cg_spmv(uint32_t m, const uint32_t* __restrict__ crow,
-                                                const uint32_t* __restrict__ ccol,
-                                                const double* __restrict__ cval,
-                                                const double* __restrict__ p, double* __restrict__ q,
-                                                double* __restrict__ part) {
-  __shared__ double sh[NT / WAVE];
-  const uint32_t sub = threadIdx.x & (SPMV_LANES - 1);
-  const uint32_t rows_per_block = NT / SPMV_LANES;
-  double pq = 0.0;
-  // block-uniform loop over row groups, so the shuffles run with every lane
-  for (uint32_t k0 = blockIdx.x * rows_per_block; k0 < m; k0 += gridDim.x * rows_per_block) {
-    const uint32_t k = k0 + threadIdx.x / SPMV_LANES;
-    double s = 0.0;
-    if (k < m) {
-      const uint32_t e1 = crow[k + 1];
-      for (uint32_t e = crow[k] + sub; e < e1; e += SPMV_LANES) s += cval[e] * p[ccol[e]];
-    }
-    s += __shfl_xor(s, 1, WAVE);
-    s += __shfl_xor(s, 2, WAVE);
-    if (k < m && sub == 0u) {
-      q[k] = s;
-      pq += p[k] * s;
-    }
+struct SpmvRow {
+  uint32_t e0, e1;
+  double v[SPMV_AHEAD];
+  double2 w[SPMV_AHEAD], own;
+};
+
+__device__ __forceinline__ void spmv_fetch(const CgArgs& a, uint32_t k, uint32_t sub, SpmvRow& r) {
+  const uint32_t kr = min(k, a.m - 1u);
+  uint32_t c[SPMV_AHEAD];
+  r.e0 = a.crow[kr] + sub;
+  r.e1 = a.crow[kr + 1u];  // (a row holds its diagonal at least)
+#pragma unroll
+  for (int q = 0; q < SPMV_AHEAD; ++q) {
+    const uint32_t e = min(r.e0 + q * SPMV_LANES, r.e1 - 1u);
+    c[q] = a.ccol[e];
+    r.v[q] = a.cval[e];
   }
-  const double t = block_sum(pq, sh);
-  if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = t;
-    part[2 * blockIdx.x + 1] = 0.0;
-  }
+  r.own = a.zp[kr];
+#pragma unroll
+  for (int q = 0; q < SPMV_AHEAD; ++q) r.w[q] = a.zp[c[q]];
 }
 
-// One block: sums the nb partial pairs in block order.  which = 0: init
-// (rz, bb); 1: alpha = rz / pq; 2: beta = rz' / rz, rz = rz', rr;
-// 3: source and sink currents.
-__global__ void __launch_bounds__(NT) k_cg_scalar(const double* __restrict__ part, int nb, int which,
-                                                  CgScal* __restrict__ sc) {
-  __shared__ double sh[NT / WAVE];
-  double a = 0.0, c = 0.0;
-  for (int k = threadIdx.x; k < nb; k += NT) {
-    a += part[2 * k];
-    c += part[2 * k + 1];
+// Writes p and q of the row; returns the lane's share of p.q.
+__device__ __forceinline__ double spmv_row(const CgArgs& a, uint32_t k, uint32_t sub, double beta, const SpmvRow& r) {
+  double s = 0.0;
+#pragma unroll
+  for (int q = 0; q < SPMV_AHEAD; ++q)
+    if (r.e0 + q * SPMV_LANES < r.e1) s += r.v[q] * (r.w[q].x + beta * r.w[q].y);
+  for (uint32_t e = r.e0 + SPMV_AHEAD * SPMV_LANES; e < r.e1; e += SPMV_LANES) {
+    const double2 t = a.zp[a.ccol[e]];
+    s += a.cval[e] * (t.x + beta * t.y);
   }
-  const double sa = block_sum(a, sh);
-  const double sb = block_sum(c, sh);
-  if (threadIdx.x != 0) return;
-  if (which == 0) {
-    sc->rz = sa;
-    sc->bb = sb;
-    sc->rr = sb;
-  } else if (which == 1) {
-    sc->pq = sa;
-    sc->alpha = sa != 0.0 ? sc->rz / sa : 0.0;
-  } else if (which == 3) {
-    sc->isrc = sa;
-    sc->isnk = sb;
-  } else {
-    sc->beta = sc->rz != 0.0 ? sa / sc->rz : 0.0;
-    sc->rz = sa;
-    sc->rr = sb;
-  }
+#pragma unroll
+  for (int o = 1; o < SPMV_LANES; o <<= 1) s += __shfl_xor(s, o, WAVE);
+  if (k >= a.m || sub != 0u) return 0.0;
+  const double pk = r.own.x + beta * r.own.y;
+  a.p[k] = pk;
+  a.q[k] = s;
+  return pk * s;
 }
 
-// x += alpha p, r -= alpha q, z = D^-1 r; partials of r.z and r.r.
-__global__ void __launch_bounds__(NT) k_cg_update(uint32_t m, const CgScal* __restrict__ sc,
-                                                  const double* __restrict__ dinv,
-                                                  const double* __restrict__ p,
-                                                  const double* __restrict__ q,
-                                                  double* __restrict__ x, double* __restrict__ r,
-                                                  double* __restrict__ z,
-                                                  double* __restrict__ part) {
+__global__ void __launch_bounds__(SPMV_NT) k_cg_spmv(CgArgs a, uint32_t it) {
+  constexpr int NW = SPMV_NT / WAVE;
+  __shared__ double sh[NW], sh_pq[NW];
+  const uint32_t sub = threadIdx.x % SPMV_LANES;
+  uint32_t k = blockIdx.x * SPMV_ROWS + threadIdx.x / SPMV_LANES;
+  SpmvRow row;
+  const uint32_t done = a.scal->done;
+  double old = a.scal->rz[(it + 1u) & 1u];
+  double share = part_share<NW>(a.part_rz, a.nb);
+  spmv_fetch(a, k, sub, row);
+  asm volatile("" : "+v"(old));  // (fetched here, not behind the sum)
+  const double rz = block_sum<NW>(share, sh);
+  if (done) return;
+  const double beta = it && old != 0.0 ? rz / old : 0.0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) a.scal->rz[it & 1u] = rz;
+  double pq = spmv_row(a, k, sub, beta, row);
+  // block-uniform loop over row groups, so the sums run with every lane
+  for (uint32_t k0 = (blockIdx.x + gridDim.x) * SPMV_ROWS; k0 < a.m; k0 += gridDim.x * SPMV_ROWS) {
+    k += gridDim.x * SPMV_ROWS;
+    spmv_fetch(a, k, sub, row);
+    pq += spmv_row(a, k, sub, beta, row);
+  }
+  const double t = block_sum<NW>(pq, sh_pq);
+  if (threadIdx.x == 0) a.part_pq[blockIdx.x] = t;
+}
+
+// x += alpha p, r -= alpha q, (z, p) = (D^-1 r, p); partials of r.z and r.r.
+__global__ void __launch_bounds__(NT) k_cg_update(CgArgs a, uint32_t it) {
   __shared__ double sh[NT / WAVE];
-  const double alpha = sc->alpha;
+  __shared__ double2 sh2[NT / WAVE];
+  uint32_t k = blockIdx.x * NT + threadIdx.x;
+  // the first elements are on their way while alpha is summed
+  const uint32_t kr = min(k, a.m - 1u);
+  const uint32_t done = a.scal->done;
+  double rz0 = a.scal->rz[it & 1u];
+  double pk = a.p[kr], qk = a.q[kr], xk = a.x[kr], r0 = a.r[kr], dk = a.dinv[kr];
+  double share = part_share(a.part_pq, a.ns);
+  asm volatile("" : "+v"(rz0));  // (fetched here, not behind the sum)
+  const double pq = block_sum(share, sh);
+  if (done) return;
+  const double alpha = pq != 0.0 ? rz0 / pq : 0.0;
   double rz = 0.0, rr = 0.0;
-  for (uint32_t k = blockIdx.x * NT + threadIdx.x; k < m; k += gridDim.x * NT) {
-    x[k] += alpha * p[k];
-    const double rk = r[k] - alpha * q[k];
-    const double zk = dinv[k] * rk;
-    r[k] = rk;
-    z[k] = zk;
+  while (k < a.m) {
+    a.x[k] = xk + alpha * pk;
+    const double rk = r0 - alpha * qk;
+    const double zk = dk * rk;
+    a.r[k] = rk;
+    a.zp[k] = make_double2(zk, pk);
     rz += rk * zk;
     rr += rk * rk;
+    k += gridDim.x * NT;
+    if (k < a.m) {
+      pk = a.p[k];
+      qk = a.q[k];
+      xk = a.x[k];
+      r0 = a.r[k];
+      dk = a.dinv[k];
+    }
   }
-  const double s1 = block_sum(rz, sh);
-  const double s2 = block_sum(rr, sh);
+  const double2 t = block_sum2(rz, rr, sh2);
   if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = s1;
-    part[2 * blockIdx.x + 1] = s2;
+    a.part_rz[blockIdx.x] = t.x;
+    a.part_rr[blockIdx.x] = t.y;
   }
 }
 
-// p = z + beta p.
-__global__ void __launch_bounds__(NT) k_cg_dir(uint32_t m, const CgScal* __restrict__ sc,
-                                               const double* __restrict__ z,
-                                               double* __restrict__ p) {
-  const double beta = sc->beta;
-  for (uint32_t k = blockIdx.x * NT + threadIdx.x; k < m; k += gridDim.x * NT) p[k] = z[k] + beta * p[k];
+// One block: relative residual after `it` iterations.  From convergence on
+// (or a residual that is no number) the queued iterations do nothing.
+__global__ void __launch_bounds__(NT) k_cg_check(CgArgs a, uint32_t it, double tol) {
+  __shared__ double sh[NT / WAVE];
+  CgScal* sc = a.scal;
+  if (it && sc->done) return;
+  const double rr = block_sum(part_share(a.part_rr, a.nb), sh);
+  if (threadIdx.x != 0) return;
+  const double bb = it ? sc->bb : rr;
+  const double res = bb > 0.0 ? sqrt_cr((rr > 0.0 ? rr : 0.0) / bb) : 0.0;
+  sc->bb = bb;
+  sc->res = res;
+  sc->done = res <= tol ? CG_CONVERGED : (res < __longlong_as_double(0x7FF0000000000000ll) ? 0u : CG_BROKEN);
+}
+
+// One block: source and sink currents.
+__global__ void __launch_bounds__(NT) k_cg_currents(CgArgs a) {
+  __shared__ double2 sh[NT / WAVE];
+  const double2 t = block_sum2(part_share(a.part_rz, a.nb), part_share(a.part_rr, a.nb), sh);
+  if (threadIdx.x != 0) return;
+  a.scal->isrc = t.x;
+  a.scal->isnk = t.y;
 }
 
 // Partials of the source current sum bs (1 - x) and the sink current sum bk x.
@@ -271,17 +363,16 @@ __global__ void __launch_bounds__(NT) k_cg_current(uint32_t m, const double* __r
                                                    const double* __restrict__ bk,
                                                    const double* __restrict__ x,
                                                    double* __restrict__ part) {
-  __shared__ double sh[NT / WAVE];
+  __shared__ double2 sh[NT / WAVE];
   double is = 0.0, ik = 0.0;
   for (uint32_t k = blockIdx.x * NT + threadIdx.x; k < m; k += gridDim.x * NT) {
     is += bs[k] * (1.0 - x[k]);
     ik += bk[k] * x[k];
   }
-  const double s1 = block_sum(is, sh);
-  const double s2 = block_sum(ik, sh);
+  const double2 t = block_sum2(is, ik, sh);
   if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = s1;
-    part[2 * blockIdx.x + 1] = s2;
+    part[blockIdx.x] = t.x;
+    part[CG_MAX_BLOCKS + blockIdx.x] = t.y;
   }
 }
 
@@ -314,7 +405,11 @@ int grid_for(uint64_t n, int cap) {
 
 }  // namespace
 
-int cg_grid(uint64_t m) { return grid_for(m, CG_MAX_BLOCKS); }
+void cg_grids(CgArgs& a) {
+  auto grid = [&](uint32_t per) { return std::min<uint32_t>((a.m + per - 1u) / per, CG_MAX_BLOCKS); };
+  a.nb = grid(NT);
+  a.ns = grid(SPMV_ROWS);
+}
 
 void launch_cs_flag(const uint32_t* nrow, const uint32_t* ncol, const uint32_t* labels, uint32_t n,
                     uint32_t* flag, hipStream_t s) {
@@ -352,29 +447,22 @@ void launch_cs_order(uint32_t n, const uint32_t* ord, const uint32_t* act, const
                        idx, off);
 }
 
-void launch_cg_init(const CgArgs& a, hipStream_t s) {
-  const int g = cg_grid(a.m);
-  hipLaunchKernelGGL(k_cg_init, dim3(g), dim3(NT), 0, s, a.m, a.bsrc, a.dinv, a.x, a.r, a.z, a.p,
-                     a.part);
-  hipLaunchKernelGGL(k_cg_scalar, dim3(1), dim3(NT), 0, s, a.part, g, 0, a.scal);
+void launch_cg_init(const CgArgs& a, double tol, hipStream_t s) {
+  hipLaunchKernelGGL(k_cg_init, dim3(a.nb), dim3(NT), 0, s, a);
+  hipLaunchKernelGGL(k_cg_check, dim3(1), dim3(NT), 0, s, a, 0u, tol);
 }
 
-void launch_cg_iteration(const CgArgs& a, hipStream_t s) {
-  const int g = cg_grid(a.m);
-  CgScal* sc = a.scal;
-  hipLaunchKernelGGL(k_cg_spmv, dim3(g), dim3(NT), 0, s, a.m, a.crow, a.ccol, a.cval, a.p, a.q,
-                     a.part);
-  hipLaunchKernelGGL(k_cg_scalar, dim3(1), dim3(NT), 0, s, a.part, g, 1, sc);
-  hipLaunchKernelGGL(k_cg_update, dim3(g), dim3(NT), 0, s, a.m, sc, a.dinv, a.p, a.q, a.x, a.r, a.z,
-                     a.part);
-  hipLaunchKernelGGL(k_cg_scalar, dim3(1), dim3(NT), 0, s, a.part, g, 2, sc);
-  hipLaunchKernelGGL(k_cg_dir, dim3(g), dim3(NT), 0, s, a.m, sc, a.z, a.p);
+void launch_cg_iterations(const CgArgs& a, uint32_t it, uint32_t count, double tol, hipStream_t s) {
+  for (uint32_t j = it; j < it + count; ++j) {
+    hipLaunchKernelGGL(k_cg_spmv, dim3(a.ns), dim3(SPMV_NT), 0, s, a, j);
+    hipLaunchKernelGGL(k_cg_update, dim3(a.nb), dim3(NT), 0, s, a, j);
+  }
+  hipLaunchKernelGGL(k_cg_check, dim3(1), dim3(NT), 0, s, a, it + count, tol);
 }
 
 void launch_cg_current(const CgArgs& a, hipStream_t s) {
-  const int g = cg_grid(a.m);
-  hipLaunchKernelGGL(k_cg_current, dim3(g), dim3(NT), 0, s, a.m, a.bsrc, a.bsnk, a.x, a.part);
-  hipLaunchKernelGGL(k_cg_scalar, dim3(1), dim3(NT), 0, s, a.part, g, 3, a.scal);
+  hipLaunchKernelGGL(k_cg_current, dim3(a.nb), dim3(NT), 0, s, a.m, a.bsrc, a.bsnk, a.x, a.part_rz);
+  hipLaunchKernelGGL(k_cg_currents, dim3(1), dim3(NT), 0, s, a);
 }
 
 }  // namespace nf
