@@ -793,8 +793,10 @@ extern "C" int nf_centre_distance(nf_handle* h, int32_t bins, double width, int6
   hipStream_t s = h->stream;
   const float4* P = h->gb.bP + h->desc[h->post_inst].rod_off;
   const float4* D = h->gb.bD + h->desc[h->post_inst].rod_off;
-  // grid: edge about rmax (half stencil of +-1 cells), finer when crowded
-  const double edge = default_cell_edge(rmax, (double)n / (p.box[0] * p.box[1] * p.box[2]), 1.0);
+  // grid: edge just over rmax and the stencil's margin (half stencil of +-1
+  // cells; at rmax itself a box of whole edges has cells two away in it, three
+  // times the candidates), finer when crowded
+  const double edge = default_cell_edge(rmax + 1.01 * (double)CELL_MARGIN, (double)n / (p.box[0] * p.box[1] * p.box[2]), 1.0);
   int32_t nc[3];
   double scale[3];
   uint64_t ncells = 1;
@@ -807,7 +809,18 @@ extern "C" int nf_centre_distance(nf_handle* h, int32_t bins, double width, int6
     ncells *= (uint64_t)nc[a];
   }
   if (ncells > (1ull << 26)) return fail(h, NF_E_INVALID, "statistics grid too large");
+  // the half stencil as runs of cells along x
   std::vector<int4> st = build_stencil(nc, p.box, rmax, true);
+  std::sort(st.begin(), st.end(), [](const int4& a, const int4& b) {
+    return a.z != b.z ? a.z < b.z : (a.y != b.y ? a.y < b.y : a.x < b.x);
+  });
+  std::vector<int4> runs;
+  for (const int4& o : st) {
+    if (!runs.empty() && runs.back().z == o.y && runs.back().w == o.z && runs.back().y + 1 == o.x)
+      runs.back().y = o.x;
+    else
+      runs.push_back(make_int4(o.x, o.x, o.y, o.z));
+  }
   std::vector<double> e2(bins + 1);
   for (int k = 0; k <= bins; ++k) e2[k] = ((double)k * width) * ((double)k * width);
   float4* cP = nullptr;
@@ -816,7 +829,7 @@ extern "C" int nf_centre_distance(nf_handle* h, int32_t bins, double width, int6
   float* chl = nullptr;
   int4* dst = nullptr;
   double* de2 = nullptr;
-  unsigned long long* out = nullptr;
+  unsigned long long *out = nullptr, *part = nullptr;
   int rc = NF_OK;
   const uint64_t n1 = std::max<uint64_t>(n, 1);
   if (rc == NF_OK) rc = dalloc(h, &cP, n1);
@@ -825,12 +838,13 @@ extern "C" int nf_centre_distance(nf_handle* h, int32_t bins, double width, int6
   if (rc == NF_OK) rc = dalloc(h, &cstart, ncells + 1);
   if (rc == NF_OK) rc = dalloc(h, &ccount, ncells);
   if (rc == NF_OK) rc = dalloc(h, &chl, ncells);
-  if (rc == NF_OK) rc = dalloc(h, &dst, st.size());
+  if (rc == NF_OK) rc = dalloc(h, &dst, runs.size());
+  if (rc == NF_OK) rc = dalloc(h, &part, (size_t)CENT_BLOCKS * (bins + 3));
   if (rc == NF_OK) rc = dalloc(h, &de2, (size_t)bins + 1);
   if (rc == NF_OK) rc = dalloc(h, &out, (size_t)bins + 3);
   BinScratch bs;
   auto release = [&]() {
-    void* w[] = {cP, cD, cid, cstart, ccount, chl, dst, de2, out};
+    void* w[] = {cP, cD, cid, cstart, ccount, chl, dst, de2, part, out};
     for (void* q : w) dfree(h, q);
     free_bin_scratch(h, &bs);
   };
@@ -838,7 +852,7 @@ extern "C" int nf_centre_distance(nf_handle* h, int32_t bins, double width, int6
     release();
     return rc;
   }
-  hipError_t e = hipMemcpyAsync(dst, st.data(), sizeof(int4) * st.size(), hipMemcpyHostToDevice, s);
+  hipError_t e = hipMemcpyAsync(dst, runs.data(), sizeof(int4) * runs.size(), hipMemcpyHostToDevice, s);
   if (e == hipSuccess)
     e = hipMemcpyAsync(de2, e2.data(), sizeof(double) * e2.size(), hipMemcpyHostToDevice, s);
   if (e != hipSuccess) {
@@ -855,8 +869,8 @@ extern "C" int nf_centre_distance(nf_handle* h, int32_t bins, double width, int6
   const double Lmax = std::max(p.box[0], std::max(p.box[1], p.box[2]));
   const float ew = (float)(5.9604644775390625e-8 * (Lmax + rmax) * 1.01);
   const float rf = (float)rmax + 8.0f * ew;
-  launch_cent(cP, cid, cstart, ccount, dst, (uint32_t)st.size(), nc, p.box, de2, bins,
-              rf * rf * 1.00001f, out, s);
+  launch_cent(cP, cid, cstart, ccount, dst, (uint32_t)runs.size(), n, nc, p.box, de2, bins, width,
+              rf * rf * 1.00001f, part, out, s);
   std::vector<unsigned long long> hout((size_t)bins + 3);
   e = hipMemcpyAsync(hout.data(), out, sizeof(unsigned long long) * hout.size(), hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = sync_stream(s, "centre distance");

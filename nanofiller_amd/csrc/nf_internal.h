@@ -474,9 +474,11 @@ void launch_selftest_pairs(const float* ra, const float* rb, const double* sh, u
                            double sep_or_gap, double soft_frac, float ew, int32_t* out_screen, int32_t* out_dec,
                            int32_t* out_within, hipStream_t s);
 constexpr int CENT_BINS_MAX = 1024;
+constexpr int CENT_BLOCKS = 2048;  // part holds CENT_BLOCKS x (bins + 3) words
 void launch_cent(const float4* P, const uint32_t* X, const uint32_t* start, const uint32_t* count,
-                 const int4* st, uint32_t st_n, const int32_t nc[3], const double box[3],
-                 const double* e2, int bins, float r2f, unsigned long long* out, hipStream_t s);
+                 const int4* runs, uint32_t n_runs, uint32_t n, const int32_t nc[3], const double box[3],
+                 const double* e2, int bins, double width, float r2f, unsigned long long* part,
+                 unsigned long long* out, hipStream_t s);
 void launch_vdw(const float4* P, const float4* D, uint32_t n, const uint32_t* rowptr,
                 const uint32_t* J, const int32_t* img, const double box[3], double dlim, double A,
                 double B, double* rowsum, double* bsum, double* out, unsigned long long* pairs,

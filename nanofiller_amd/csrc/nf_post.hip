@@ -316,12 +316,25 @@ void launch_csr_scatter(const uint32_t* I, const uint32_t* J, const float* gap, 
 // every unordered pair of distinct rods over all periodic images with centre
 // distance below bins * width, binned by comparing d^2 with the squared bin
 // edges, plus exact fixed-point sums of round(d 2^24) and round(d^2 2^16).
-// One workgroup (one wave) per home cell over a half stencil; each neighbour
-// cell streams through LDS in 64-rod tiles; the FP64 distance is evaluated
-// with the lower id first and the image applied to the higher id, so every
-// bin decision matches a sequential evaluation.
+// The FP64 distance is evaluated with the lower id first and the image applied
+// to the higher id, so every bin decision matches a sequential evaluation.
+//
+// A wave takes an item: some rods of one cell against one run of neighbour
+// cells.  Cells along x follow each other in the cell list, so the half stencil
+// is a few runs (five at an edge of rmax) and a run's rods are loaded 64 at a
+// time, one per lane, whatever the single cells hold; the probes are uniform
+// and come through scalar loads.  Of the candidates 15 % are pairs: an FP32
+// test with a safe margin picks them, a queue in LDS collects 64 before the
+// FP64 distance, bin and sums are evaluated, so those run with every lane.  A
+// block keeps its counts and sums and writes them once; a second kernel adds
+// the blocks' (atomics on the few lines of the result had cost as much as the
+// pairs: 12 ns each on one line).  300,000 rods, 20 M pairs in 64 bins:
+// 1313 -> 213 + 9 us, bound by FP32 and FP64 instruction issue; two or four
+// probes to a look at the queue took 227 and 242 (its room costs occupancy).
 // ---------------------------------------------------------------------------
 constexpr int CENT_MAX_BINS = 1024;
+constexpr int CENT_THREADS = 256;
+constexpr int CENT_QUEUE = 2 * WAVE;
 
 // wave-uniform copies (SGPR) of values every lane already agrees on, so the
 // loops that hold barriers have scalar trip counts
@@ -330,121 +343,173 @@ __device__ __forceinline__ uint32_t uni_u32(uint32_t v) {
 }
 
 struct CentArg {
-  const float4* P;       // compact cell list (positions, half length)
-  const uint32_t* X;     // rod ids
+  const uint32_t* X;  // rod ids
   const uint32_t* start;
   const uint32_t* count;
-  const int4* st;
-  uint32_t st_n;
+  const int4* runs;  // first and last x offset, y and z offset
+  uint32_t n_runs, chunks, chunk;  // a cell's rods in `chunks` shares of `chunk` at a time
   int32_t nc[3];
   double box[3];
   const double* e2;      // bins + 1 squared edges
   int bins;
   float r2f;             // FP32 prefilter bound
-  unsigned long long* out;  // bins counts, then pairs, sum_q, sum2_q
+  float inv_width;
 };
 
-__global__ void __launch_bounds__(WAVE) k_cent(CentArg a) {
-  __shared__ float4 tP[WAVE];
-  __shared__ uint32_t tX[WAVE];
+struct CentQueue {
+  uint32_t p[CENT_QUEUE], q[CENT_QUEUE], img[CENT_QUEUE];
+};
+
+struct CentAcc {
+  unsigned long long cnt, sq, s2q;
+};
+
+// The pair of queue entry k: its bin and its fixed-point sums.
+__device__ void cent_pair(const float4* __restrict__ P, const CentArg& a, const CentQueue& L, uint32_t k,
+                          const double* e2, uint32_t* hist, CentAcc& acc) {
+  const uint32_t p = L.p[k], q = L.q[k], code = L.img[k];
+  if (p == q) return;  // a rod and its own image
+  const bool swap = a.X[p] > a.X[q];
+  const float4 Pa = swap ? P[q] : P[p], Pb = swap ? P[p] : P[q];
+  const int s = swap ? -1 : 1;
+  const double ux = (double)(s * ((int)(code & 1023u) - 512)) * a.box[0];
+  const double uy = (double)(s * ((int)((code >> 10) & 1023u) - 512)) * a.box[1];
+  const double uz = (double)(s * ((int)(code >> 20) - 512)) * a.box[2];
+  const double dx = ((double)Pa.x - (double)Pb.x) - ux;
+  const double dy = ((double)Pa.y - (double)Pb.y) - uy;
+  const double dz = ((double)Pa.z - (double)Pb.z) - uz;
+  const double d2 = dx * dx + dy * dy + dz * dz;
+  if (!(d2 < e2[a.bins])) return;
+  // a first guess in FP32, then the edges themselves decide
+  const float df = (float)d2, rf = __builtin_amdgcn_rsqf(df);
+  int b = (int)fminf(df * rf * a.inv_width, (float)(a.bins - 1));
+  while (b > 0 && e2[b] > d2) --b;
+  while (e2[b + 1] <= d2) ++b;
+  atomicAdd(&hist[b], 1u);
+  ++acc.cnt;
+  // round(d 2^24): one Newton step on the FP32 root is good to 2^-44 of d,
+  // which settles the rounding unless the value lies within 2^-42 of a half
+  const double y0 = d2 * (double)rf;
+  const double y = fma(fma(-y0, y0, d2), 0.5 * (double)rf, y0);
+  const double v = y * 16777216.0 + 0.5;
+  double w = floor(v);
+  const double f = v - w, g = v * 2.2737367544323206e-13;
+  if (!(f > g && f < 1.0 - g)) w = floor(sqrt_cr(d2) * 16777216.0 + 0.5);
+  acc.sq += (unsigned long long)w;
+  acc.s2q += (unsigned long long)floor(d2 * 65536.0 + 0.5);
+}
+
+__global__ void __launch_bounds__(CENT_THREADS) k_cent(const float4* __restrict__ P, CentArg a,
+                                                       unsigned long long* __restrict__ part) {
+  __shared__ double e2[CENT_MAX_BINS + 1];
   __shared__ uint32_t hist[CENT_MAX_BINS];
-  const int lane = threadIdx.x;
-  for (int k = lane; k < a.bins; k += WAVE) hist[k] = 0u;
+  __shared__ CentQueue queue[CENT_THREADS / WAVE];
+  __shared__ unsigned long long tot[3];
+  for (int k = threadIdx.x; k <= a.bins; k += CENT_THREADS) {
+    e2[k] = a.e2[k];
+    if (k < a.bins) hist[k] = 0u;
+  }
+  if (threadIdx.x < 3) tot[threadIdx.x] = 0ull;
   __syncthreads();
-  unsigned long long cnt = 0, sq = 0, s2q = 0;
-  const uint32_t ncells = (uint32_t)a.nc[0] * (uint32_t)a.nc[1] * (uint32_t)a.nc[2];
-  const double e2max = a.e2[a.bins];
-  for (uint32_t cell = blockIdx.x; cell < ncells; cell += gridDim.x) {
+  const uint32_t lane = threadIdx.x % WAVE, wave = uni_u32(threadIdx.x / WAVE);
+  CentQueue& L = queue[wave];
+  CentAcc acc = {0ull, 0ull, 0ull};
+  uint32_t qn = 0u;
+  const uint32_t per_cell = a.n_runs * a.chunks;
+  const uint64_t items = (uint64_t)a.nc[0] * (uint64_t)a.nc[1] * (uint64_t)a.nc[2] * per_cell;
+  for (uint64_t t = blockIdx.x * (CENT_THREADS / WAVE) + wave; t < items; t += gridDim.x * (CENT_THREADS / WAVE)) {
+    const uint32_t cell = uni_u32((uint32_t)(t / per_cell)), part_of = uni_u32((uint32_t)(t % per_cell));
+    const uint32_t c = part_of % a.chunks;
+    const int4 run = a.runs[part_of / a.chunks];
     const uint32_t pc = uni_u32(a.count[cell]), ps = uni_u32(a.start[cell]);
+    if (c * a.chunk >= pc) continue;
     const int c0 = (int)(cell % (uint32_t)a.nc[0]);
-    const int c1 = (int)((cell / (uint32_t)a.nc[0]) % (uint32_t)a.nc[1]);
-    const int c2 = (int)(cell / ((uint32_t)a.nc[0] * (uint32_t)a.nc[1]));
-    for (uint32_t pb = 0; pb < pc; pb += WAVE) {
-      const bool valid = pb + (uint32_t)lane < pc;
-      const uint32_t pi = ps + min(pb + (uint32_t)lane, pc - 1u);
-      const float4 P1 = a.P[pi];
-      const uint32_t X1 = a.X[pi];
-      for (uint32_t si = 0; si < a.st_n; ++si) {
-        const int4 so = a.st[si];
-        const int raw[3] = {c0 + so.x, c1 + so.y, c2 + so.z};
-        int img[3], m[3];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          int mm = raw[d] % a.nc[d];
-          if (mm < 0) mm += a.nc[d];
-          img[d] = (raw[d] - mm) / a.nc[d];
-          m[d] = mm;
-        }
-        const uint32_t nc = (uint32_t)(m[0] + a.nc[0] * (m[1] + a.nc[1] * m[2]));
-        const uint32_t n = uni_u32(a.count[nc]), ns = uni_u32(a.start[nc]);
-        const bool same = so.x == 0 && so.y == 0 && so.z == 0;
-        const double sx = (double)img[0] * a.box[0], sy = (double)img[1] * a.box[1],
-                     sz = (double)img[2] * a.box[2];
-        const float fx = (float)sx, fy = (float)sy, fz = (float)sz;
-        for (uint32_t tb = 0; tb < n; tb += WAVE) {
-          const uint32_t tn = min((uint32_t)WAVE, n - tb);
-          const uint32_t q = ns + tb + min((uint32_t)lane, tn - 1u);
-          tP[lane] = a.P[q];
-          tX[lane] = a.X[q];
-          __syncthreads();
-          if (valid) {
-            for (uint32_t j = 0; j < tn; ++j) {
-              if (same && tb + j <= pb + (uint32_t)lane) continue;
-              const uint32_t xj = tX[j];
-              if (xj == X1) continue;  // a rod and its own image
-              const float4 P2 = tP[j];
-              const float wx = (P1.x - P2.x) - fx, wy = (P1.y - P2.y) - fy, wz = (P1.z - P2.z) - fz;
-              if (fmaf(wz, wz, fmaf(wy, wy, wx * wx)) > a.r2f) continue;
-              const bool swap = X1 > xj;
-              const float4 Pa = swap ? P2 : P1, Pb = swap ? P1 : P2;
-              const double ux = swap ? -sx : sx, uy = swap ? -sy : sy, uz = swap ? -sz : sz;
-              const double dx = ((double)Pa.x - (double)Pb.x) - ux;
-              const double dy = ((double)Pa.y - (double)Pb.y) - uy;
-              const double dz = ((double)Pa.z - (double)Pb.z) - uz;
-              const double d2 = dx * dx + dy * dy + dz * dz;
-              if (!(d2 < e2max)) continue;
-              int lo = 0, hi = a.bins;
-              while (hi - lo > 1) {
-                const int mid = (lo + hi) >> 1;
-                if (a.e2[mid] <= d2)
-                  lo = mid;
-                else
-                  hi = mid;
-              }
-              atomicAdd(&hist[lo], 1u);
-              ++cnt;
-              sq += (unsigned long long)floor(sqrt_cr(d2) * 16777216.0 + 0.5);
-              s2q += (unsigned long long)floor(d2 * 65536.0 + 0.5);
+    const int c1 = (int)((cell / (uint32_t)a.nc[0]) % (uint32_t)a.nc[1]) + run.z;
+    const int c2 = (int)(cell / ((uint32_t)a.nc[0] * (uint32_t)a.nc[1])) + run.w;
+    const int i1 = floor_div(c1, a.nc[1]), i2 = floor_div(c2, a.nc[2]);
+    const uint32_t row = (uint32_t)a.nc[0] * (uint32_t)((c1 - i1 * a.nc[1]) + a.nc[1] * (c2 - i2 * a.nc[2]));
+    const float fy = (float)((double)i1 * a.box[1]), fz = (float)((double)i2 * a.box[2]);
+    for (int x = c0 + run.x; x <= c0 + run.y;) {
+      // the part of the run in one image of the box
+      const int i0 = floor_div(x, a.nc[0]), m0 = x - i0 * a.nc[0];
+      const int len = min(c0 + run.y - x + 1, a.nc[0] - m0);
+      const uint32_t last = row + (uint32_t)(m0 + len - 1);
+      const uint32_t q0 = uni_u32(a.start[row + (uint32_t)m0]);
+      const uint32_t q1 = uni_u32(a.start[last]) + uni_u32(a.count[last]);
+      const bool own = run.z == 0 && run.w == 0 && x == c0;  // each pair of the cell's own rods once
+      const float fx = (float)((double)i0 * a.box[0]);
+      const uint32_t code = (uint32_t)(i0 + 512) | ((uint32_t)(i1 + 512) << 10) | ((uint32_t)(i2 + 512) << 20);
+      for (uint32_t tb = q0; tb < q1; tb += WAVE) {
+        const uint32_t q = tb + lane;
+        const float4 P2 = P[min(q, q1 - 1u)];
+        const float tx = q < q1 ? P2.x + fx : 3e38f, ty = P2.y + fy, tz = P2.z + fz;
+        for (uint32_t pb = c * a.chunk; pb < pc; pb += a.chunks * a.chunk) {
+          const uint32_t pe = min(pb + a.chunk, pc);
+          for (uint32_t j = pb; j < pe; ++j) {
+            const float4 P1 = P[ps + j];
+            const float wx = P1.x - tx, wy = P1.y - ty, wz = P1.z - tz;
+            bool hit = fmaf(wz, wz, fmaf(wy, wy, wx * wx)) <= a.r2f;
+            if (own) hit = hit && q > ps + j;
+            const unsigned long long m = __ballot(hit);
+            if (m == 0ull) continue;
+            if (hit) {
+              const uint32_t at = qn + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                                 __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+              L.p[at] = ps + j;
+              L.q[at] = q;
+              L.img[at] = code;
+            }
+            qn += (uint32_t)__popcll(m);
+            if (qn >= (uint32_t)WAVE) {
+              __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+              qn -= WAVE;
+              cent_pair(P, a, L, qn + lane, e2, hist, acc);
+              __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             }
           }
-          __syncthreads();
         }
       }
+      x += len;
     }
   }
-  __syncthreads();
-  for (int k = lane; k < a.bins; k += WAVE)
-    if (hist[k]) atomicAdd(&a.out[k], (unsigned long long)hist[k]);
-  cnt = wave_sum_u64(cnt);
-  sq = wave_sum_u64(sq);
-  s2q = wave_sum_u64(s2q);
-  if (lane == 0) {
-    atomicAdd(&a.out[a.bins + 0], cnt);
-    atomicAdd(&a.out[a.bins + 1], sq);
-    atomicAdd(&a.out[a.bins + 2], s2q);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  if (lane < qn) cent_pair(P, a, L, lane, e2, hist, acc);
+  acc.cnt = wave_sum_u64(acc.cnt);
+  acc.sq = wave_sum_u64(acc.sq);
+  acc.s2q = wave_sum_u64(acc.s2q);
+  if (lane == 0u) {
+    atomicAdd(&tot[0], acc.cnt);
+    atomicAdd(&tot[1], acc.sq);
+    atomicAdd(&tot[2], acc.s2q);
   }
+  __syncthreads();
+  part += (uint64_t)blockIdx.x * (a.bins + 3);
+  for (int k = threadIdx.x; k < a.bins + 3; k += CENT_THREADS) part[k] = k < a.bins ? hist[k] : tot[k - a.bins];
+}
+
+// Adds the blocks' counts and sums: a lane per word, a wave per share of the blocks.
+__global__ void __launch_bounds__(CENT_THREADS) k_cent_total(const unsigned long long* __restrict__ part, uint32_t nb,
+                                                             uint32_t words, unsigned long long* __restrict__ out) {
+  const uint32_t k = blockIdx.x * WAVE + threadIdx.x % WAVE;
+  if (k >= words) return;
+  unsigned long long s = 0;
+#pragma unroll 4
+  for (uint32_t b = blockIdx.y * (CENT_THREADS / WAVE) + threadIdx.x / WAVE; b < nb;
+       b += gridDim.y * (CENT_THREADS / WAVE))
+    s += part[(uint64_t)b * words + k];
+  if (s) atomicAdd(&out[k], s);
 }
 
 void launch_cent(const float4* P, const uint32_t* X, const uint32_t* start, const uint32_t* count,
-                 const int4* st, uint32_t st_n, const int32_t nc[3], const double box[3],
-                 const double* e2, int bins, float r2f, unsigned long long* out, hipStream_t s) {
+                 const int4* runs, uint32_t n_runs, uint32_t n, const int32_t nc[3], const double box[3],
+                 const double* e2, int bins, double width, float r2f, unsigned long long* part,
+                 unsigned long long* out, hipStream_t s) {
   CentArg a;
-  a.P = P;
   a.X = X;
   a.start = start;
   a.count = count;
-  a.st = st;
-  a.st_n = st_n;
+  a.runs = runs;
+  a.n_runs = n_runs;
   for (int d = 0; d < 3; ++d) {
     a.nc[d] = nc[d];
     a.box[d] = box[d];
@@ -452,9 +517,18 @@ void launch_cent(const float4* P, const uint32_t* X, const uint32_t* start, cons
   a.e2 = e2;
   a.bins = bins;
   a.r2f = r2f;
-  a.out = out;
-  const uint64_t ncells = (uint64_t)nc[0] * nc[1] * nc[2];
-  hipLaunchKernelGGL(k_cent, dim3(grid_for(ncells, 1)), dim3(WAVE), 0, s, a);
+  a.inv_width = (float)(1.0 / width);
+  // shares of 32 probes, of fewer where cells and runs alone leave the chip idle
+  const uint64_t cr = (uint64_t)nc[0] * nc[1] * nc[2] * n_runs;
+  const uint64_t mean = (uint64_t)n / ((uint64_t)nc[0] * nc[1] * nc[2]) + 1;
+  a.chunk = 32;
+  while (a.chunk > 4 && cr * ((mean + a.chunk - 1) / a.chunk) < 16384) a.chunk /= 2;
+  a.chunks = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((mean + a.chunk - 1) / a.chunk, 65536 / std::min<uint64_t>(cr, 65536)));
+  const int blocks = std::min(grid_for(cr * a.chunks, CENT_THREADS / WAVE), CENT_BLOCKS);
+  hipLaunchKernelGGL(k_cent, dim3(blocks), dim3(CENT_THREADS), 0, s, P, a, part);
+  const uint32_t words = (uint32_t)bins + 3;
+  hipLaunchKernelGGL(k_cent_total, dim3((words + WAVE - 1) / WAVE, 64), dim3(CENT_THREADS), 0, s, part,
+                     (uint32_t)blocks, words, out);
 }
 
 // ---------------------------------------------------------------------------
