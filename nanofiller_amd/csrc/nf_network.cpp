@@ -71,8 +71,8 @@ extern "C" int nf_network(nf_handle* h, nf_network_info* info) {
   ALLOC(a.rowcnt, (uint64_t)n + 3);
   ALLOC(a.summary, NET_SUMMARY);
   ALLOC(a.tmp, scan_tmp_words((uint64_t)n + 2));
-  ALLOC(a.cg, n1);
-  ALLOC(a.bsum, n1 / 1024 + 2);
+  ALLOC(a.cg, 2 * n1);
+  ALLOC(a.bsum, 2 * (n1 / 1024 + 1));
 #undef ALLOC
   auto release_work = [&]() {
     void* w[] = {a.lowcnt, a.lowstart, a.lowfill, a.lcol, a.limg, a.lg, a.fsrc, a.fsnk,
