@@ -34,7 +34,7 @@ SOURCES = [
     "nf_solve.hip",
     "nf_nodes.hip",
     "nf_api.cpp",
-    "nf_contacts.cpp",
+    "nf_contacts.cpp", "nf_copy.cpp",
     "nf_network.cpp",
     "nf_io.cpp",
     "nf_state.cpp",

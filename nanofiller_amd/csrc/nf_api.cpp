@@ -47,6 +47,45 @@ static size_t size_class(size_t bytes) {
 
 constexpr size_t POOL_CAP = (size_t)16 << 30;  // freed bytes kept per handle
 
+constexpr size_t SLAB_FROM = (size_t)1 << 20, SLAB_TO = (size_t)32 << 20, SLAB_LARGEST = (size_t)256 << 20;
+
+static bool in_slab(const nf_handle* h, const void* p) {
+  for (const auto& s : h->slabs)
+    if ((const char*)p >= s.p && (const char*)p < s.p + s.size) return true;
+  return false;
+}
+
+// A block cut from the newest slab, or from a new one twice its size; null if
+// there is no memory for one.
+static void* slab_block(nf_handle* h, size_t cls) {
+  if (h->slabs.empty() || h->slabs.back().size - h->slabs.back().used < cls) {
+    const size_t size = h->slabs.empty() ? SLAB_TO : std::min(2 * h->slabs.back().size, SLAB_LARGEST);
+    void* p = nullptr;
+    if (hipMalloc(&p, size) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    h->slabs.push_back({(char*)p, size, 0});
+  }
+  auto& s = h->slabs.back();
+  void* q = s.p + s.used;
+  s.used += cls;
+  return q;
+}
+
+// Gives the pool's blocks back to the device, but for those cut from slabs.
+static void trim_pool(nf_handle* h) {
+  for (auto it = h->pool.begin(); it != h->pool.end();) {
+    if (in_slab(h, it->second)) {
+      ++it;
+      continue;
+    }
+    (void)hipFree(it->second);
+    h->pool_bytes -= it->first;
+    it = h->pool.erase(it);
+  }
+}
+
 int dalloc_bytes(nf_handle* h, void** p, size_t bytes) {
   *p = nullptr;
   if (bytes == 0) bytes = 16;
@@ -58,12 +97,11 @@ int dalloc_bytes(nf_handle* h, void** p, size_t bytes) {
     h->pool.erase(it);
     h->pool_bytes -= cls;
   } else {
-    hipError_t e = hipMalloc(&q, cls);
+    if (cls >= SLAB_FROM && cls <= SLAB_TO) q = slab_block(h, cls);
+    hipError_t e = q ? hipSuccess : hipMalloc(&q, cls);
     if (e != hipSuccess && !h->pool.empty()) {
       // give the cached blocks back and try once more
-      for (auto& kv : h->pool) (void)hipFree(kv.second);
-      h->pool.clear();
-      h->pool_bytes = 0;
+      trim_pool(h);
       e = hipMalloc(&q, cls);
     }
     if (e != hipSuccess)
@@ -113,7 +151,11 @@ static hipError_t poll(Query query, const char* what) {
       std::fflush(stderr);
       return hipErrorLaunchTimeOut;
     }
-    std::this_thread::sleep_for(std::chrono::microseconds(el < 0.01 ? 2 : 200));
+    // (a sleep of 2 us lasts 60: short waits spin)
+    if (el < 0.002)
+      std::this_thread::yield();
+    else
+      std::this_thread::sleep_for(std::chrono::microseconds(el < 0.01 ? 2 : 200));
   }
 }
 
@@ -138,7 +180,7 @@ void dfree(nf_handle* h, void* p) {
   const size_t cls = it->second;
   h->allocs.erase(it);
   if (h->stream) (void)hipStreamSynchronize(h->stream);
-  if (h->pool_bytes + cls > POOL_CAP) {
+  if (h->pool_bytes + cls > POOL_CAP && !in_slab(h, p)) {
     (void)hipFree(p);
     return;
   }
@@ -739,11 +781,13 @@ extern "C" void nf_destroy(nf_handle* h) {
   if (h->graph) (void)hipGraphExecDestroy(h->graph);
   release_contacts(h);
   release_gen(h);
-  for (auto& kv : h->allocs) (void)hipFree(kv.first);
-  for (auto& kv : h->pool) (void)hipFree(kv.second);
+  trim_pool(h);
+  for (auto& kv : h->allocs)
+    if (!in_slab(h, kv.first)) (void)hipFree(kv.first);
+  for (auto& s : h->slabs) (void)hipFree(s.p);
   for (auto& e : h->ev)
     if (e) (void)hipEventDestroy(e);
-  if (h->cg_host) (void)hipHostFree(h->cg_host);
+  release_pinned(h);
   if (h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
 }
@@ -1021,8 +1065,9 @@ static int generate_once(nf_handle* h, nf_gen_stats* stats, std::vector<std::pai
   }
   double kern[8] = {0};
   RoundInfo ri{};
-  RoundInfo* ri_host = nullptr;
-  HIPCHK(h, hipHostMalloc((void**)&ri_host, sizeof(RoundInfo), hipHostMallocDefault));
+  PinnedScalars* pinned = pinned_scalars(h);
+  if (!pinned) return fail(h, NF_E_NOMEM, "generation: no pinned memory");
+  RoundInfo* ri_host = &pinned->ri;
   uint32_t max_rounds = 0;
   for (auto& p : h->params) max_rounds = std::max(max_rounds, p.max_rounds);
   const auto t0 = std::chrono::steady_clock::now();
@@ -1051,7 +1096,7 @@ static int generate_once(nf_handle* h, nf_gen_stats* stats, std::vector<std::pai
       }
       ++launched;
     }
-    if (e == hipSuccess) e = hipMemcpyAsync(ri_host, h->gb.ri, sizeof(RoundInfo), hipMemcpyDeviceToHost, h->stream);
+    launch_to_pinned(h->gb.ri, sizeof(RoundInfo), ri_host, h->stream);
     if (e == hipSuccess) e = sync_stream(h->stream, "generation round");
     if (e != hipSuccess) break;
     ri = *ri_host;
@@ -1059,10 +1104,7 @@ static int generate_once(nf_handle* h, nf_gen_stats* stats, std::vector<std::pai
           ri.rounds, ri.running, ri.T);
     if (!h->milestones.empty()) {
       const int mrc = milestone_check(h, &next_ms);
-      if (mrc != NF_OK) {
-        (void)hipHostFree(ri_host);
-        return mrc;
-      }
+      if (mrc != NF_OK) return mrc;
     }
     if (ri.running == 0 || launched > max_rounds + 2) break;
     // next batch: the rounds the controller expects to need at the last
@@ -1072,7 +1114,6 @@ static int generate_once(nf_handle* h, nf_gen_stats* stats, std::vector<std::pai
     if (next_ms < h->milestones.size()) batch = 1;
   }
   const auto t1 = std::chrono::steady_clock::now();
-  (void)hipHostFree(ri_host);
   if (e == hipSuccess && h->opt_profile) {
     const int cls[7] = {NF_K_CONTROL, NF_K_GEN, NF_K_BIN, NF_K_REJECT_OLD, NF_K_REJECT_NEW,
                         NF_K_COMMIT, NF_K_CONTROL};
@@ -1087,7 +1128,8 @@ static int generate_once(nf_handle* h, nf_gen_stats* stats, std::vector<std::pai
   if (e != hipSuccess) return fail(h, NF_E_HIP, std::string("generation: ") + hipGetErrorString(e));
   const double wall = std::chrono::duration<double, std::milli>(t1 - t0).count();
   std::vector<InstState> st(h->gb.n_inst);
-  HIPCHK(h, hipMemcpy(st.data(), h->gb.st, sizeof(InstState) * st.size(), hipMemcpyDeviceToHost));
+  const HostPart st_part = {st.data(), h->gb.st, sizeof(InstState) * st.size()};
+  HIPCHK(h, to_host(h, &st_part, 1));
   int status_rc = NF_OK;
   for (int i = 0; i < h->gb.n_inst; ++i) {
     h->n_rods[i] = st[i].n_acc;
@@ -1130,23 +1172,8 @@ extern "C" int nf_get_rods(nf_handle* h, int inst, float* rods, uint32_t cap, ui
   if (n) *n = cnt;
   if (!rods) return NF_OK;
   if (cap < cnt) return fail(h, NF_E_CAPACITY, "rod buffer too small");
-  std::vector<float4> P(cnt), D(cnt);
   const uint32_t off = h->desc[inst].rod_off;
-  if (cnt) {
-    HIPCHK(h, hipMemcpy(P.data(), h->gb.bP + off, sizeof(float4) * cnt, hipMemcpyDeviceToHost));
-    HIPCHK(h, hipMemcpy(D.data(), h->gb.bD + off, sizeof(float4) * cnt, hipMemcpyDeviceToHost));
-  }
-  for (uint32_t i = 0; i < cnt; ++i) {
-    float* r = rods + 8 * (size_t)i;
-    r[0] = P[i].x;
-    r[1] = P[i].y;
-    r[2] = P[i].z;
-    r[3] = D[i].x;
-    r[4] = D[i].y;
-    r[5] = D[i].z;
-    r[6] = 2.0f * P[i].w;
-    r[7] = D[i].w;
-  }
+  HIPCHK(h, rods_to_host(h, h->gb.bP + off, h->gb.bD + off, cnt, rods));
   return NF_OK;
 }
 
@@ -1154,21 +1181,15 @@ extern "C" int nf_set_rods(nf_handle* h, int inst, const float* rods, uint32_t n
   if (!h || inst < 0 || inst >= (int)h->params.size()) return fail(h, NF_E_INVALID, "bad instance");
   if (n > h->desc[inst].n_target) return fail(h, NF_E_CAPACITY, "more rods than the instance target");
   if (n && !rods) return fail(h, NF_E_INVALID, "null rods");
-  std::vector<float4> P(n), D(n);
   for (uint32_t i = 0; i < n; ++i) {
     const float* r = rods + 8 * (size_t)i;
     if (!(r[6] > 0.0f) || !(r[7] > 0.0f)) return fail(h, NF_E_INVALID, "rod length and radius must be > 0");
     for (int a = 0; a < 3; ++a)
       if (!(r[a] >= 0.0f && r[a] < (float)h->params[inst].box[a]))
         return fail(h, NF_E_INVALID, "rod centre outside the box");
-    P[i] = make_float4(r[0], r[1], r[2], 0.5f * r[6]);
-    D[i] = make_float4(r[3], r[4], r[5], r[7]);
   }
   const uint32_t off = h->desc[inst].rod_off;
-  if (n) {
-    HIPCHK(h, hipMemcpy(h->gb.bP + off, P.data(), sizeof(float4) * n, hipMemcpyHostToDevice));
-    HIPCHK(h, hipMemcpy(h->gb.bD + off, D.data(), sizeof(float4) * n, hipMemcpyHostToDevice));
-  }
+  HIPCHK(h, rods_to_device(h, rods, n, h->gb.bP + off, h->gb.bD + off));
   h->n_rods[inst] = n;
   h->generated = false;
   h->cb.valid = false;

@@ -127,12 +127,10 @@ extern "C" int nf_conductance(nf_handle* h, double tol, uint32_t max_iter, nf_co
       release();
       return rc;
     }
-    if (!h->cg_host) {
-      if (hipError_t e = hipHostMalloc((void**)&h->cg_host, 2 * sizeof(CgScal), hipHostMallocDefault); e != hipSuccess) {
-        h->cg_host = nullptr;
-        release();
-        return fail(h, NF_E_NOMEM, std::string("conductance scalars: ") + hipGetErrorString(e));
-      }
+    PinnedScalars* pinned = pinned_scalars(h);
+    if (!pinned) {
+      release();
+      return fail(h, NF_E_NOMEM, "conductance: no pinned memory");
     }
     launch_cs_fill(c.nrow, c.ncol, c.nval, n, act, idx, off, crow, ccol, cval, dinv, bsrc, bsnk, s);
     fill_u32(crow + m, nnz, 1, s);
@@ -144,20 +142,18 @@ extern "C" int nf_conductance(nf_handle* h, double tol, uint32_t max_iter, nf_co
       CgScal* host;    // pinned copy of the scalars
       hipEvent_t done;
     };
-    Check slot[2] = {{0, h->cg_host, h->ev[2]}, {0, h->cg_host + 1, h->ev[3]}};
+    Check slot[2] = {{0, &pinned->cg[0], h->ev[2]}, {0, &pinned->cg[1], h->ev[3]}};
     uint32_t pending = 0, newest = 0;
     hipEventRecord(h->ev[0], s);
-    // queues what leads to the next check (init for the first), the check and the copy of its verdict
+    // queues what leads to the next check (init for the first) and the check, which leaves its verdict in c.host
     auto queue = [&](uint32_t it, uint32_t count, Check& c) -> hipError_t {
       if (count == 0)
-        launch_cg_init(a, tol, s);
+        launch_cg_init(a, tol, c.host, s);
       else
-        launch_cg_iterations(a, it, count, tol, s);
+        launch_cg_iterations(a, it, count, tol, c.host, s);
       c.it = it + count;
-      hipError_t e = hipMemcpyAsync(c.host, scal, sizeof(CgScal), hipMemcpyDeviceToHost, s);
-      if (e == hipSuccess) e = hipEventRecord(c.done, s);
       ++pending;
-      return e;
+      return hipEventRecord(c.done, s);
     };
     uint32_t it = 0;
     CgScal hs{};
@@ -185,16 +181,13 @@ extern "C" int nf_conductance(nf_handle* h, double tol, uint32_t max_iter, nf_co
       }
     }
     const bool conv = hs.done == CG_CONVERGED;
-    launch_cg_current(a, s);
+    launch_cg_current(a, pinned->cg, s);  // (after whatever is queued: both slots are free by then)
     hipEventRecord(h->ev[1], s);
-    if (hipError_t e_ = hipMemcpyAsync(&hs, scal, sizeof(CgScal), hipMemcpyDeviceToHost, s); e_ != hipSuccess) {
-      release();
-      return fail(h, NF_E_HIP, std::string("conductance copy: ") + hipGetErrorString(e_));
-    }
     if (hipError_t e = sync_stream(s, "conductance currents"); e != hipSuccess) {
       release();
       return fail(h, NF_E_HIP, std::string("conductance currents: ") + hipGetErrorString(e));
     }
+    hs = pinned->cg[0];
     hipEventElapsedTime(&solve_ms, h->ev[0], h->ev[1]);
     out.iterations = it;
     out.converged = conv ? 1 : 0;
@@ -209,11 +202,8 @@ extern "C" int nf_conductance(nf_handle* h, double tol, uint32_t max_iter, nf_co
       return rc;
     }
     launch_cs_potential(n, c.labels, flag, act, idx, x, vdev, s);
-    if (hipError_t e_ = hipMemcpyAsync(potentials, vdev, sizeof(double) * n, hipMemcpyDeviceToHost, s); e_ != hipSuccess) {
-      release();
-      return fail(h, NF_E_HIP, std::string("conductance copy: ") + hipGetErrorString(e_));
-    }
-    if (hipError_t e = sync_stream(s, "conductance potentials"); e != hipSuccess) {
+    const HostPart part = {potentials, vdev, sizeof(double) * n};
+    if (hipError_t e = to_host(h, &part, 1); e != hipSuccess) {
       release();
       return fail(h, NF_E_HIP, std::string("conductance potentials: ") + hipGetErrorString(e));
     }

@@ -621,13 +621,12 @@ extern "C" int nf_get_contacts(nf_handle* h, uint32_t* row_ptr, uint32_t* col, f
   ContactBuffers& c = h->cb;
   if (!c.valid) return fail(h, NF_E_STATE, "no contacts computed");
   if ((col || gap || image) && cap < c.n_contacts) return fail(h, NF_E_CAPACITY, "contact buffer too small");
-  if (row_ptr)
-    HIPCHK(h, hipMemcpy(row_ptr, c.rowptr, sizeof(uint32_t) * ((size_t)c.n_rods + 1), hipMemcpyDeviceToHost));
-  if (c.n_contacts) {
-    if (col) HIPCHK(h, hipMemcpy(col, c.J, sizeof(uint32_t) * c.n_contacts, hipMemcpyDeviceToHost));
-    if (gap) HIPCHK(h, hipMemcpy(gap, c.gap, sizeof(float) * c.n_contacts, hipMemcpyDeviceToHost));
-    if (image) HIPCHK(h, hipMemcpy(image, c.img, sizeof(int32_t) * c.n_contacts, hipMemcpyDeviceToHost));
-  }
+  const size_t nc = c.n_contacts;
+  const HostPart parts[4] = {{row_ptr, c.rowptr, row_ptr ? sizeof(uint32_t) * ((size_t)c.n_rods + 1) : 0},
+                             {col, c.J, col ? sizeof(uint32_t) * nc : 0},
+                             {gap, c.gap, gap ? sizeof(float) * nc : 0},
+                             {image, c.img, image ? sizeof(int32_t) * nc : 0}};
+  HIPCHK(h, to_host(h, parts, 4));
   return NF_OK;
 }
 
@@ -636,8 +635,8 @@ extern "C" int nf_get_contact_gap64(nf_handle* h, double* gap64, uint64_t cap) {
   ContactBuffers& c = h->cb;
   if (!c.valid) return fail(h, NF_E_STATE, "no contacts computed");
   if (cap < c.n_contacts) return fail(h, NF_E_CAPACITY, "buffer too small");
-  if (c.n_contacts && gap64)
-    HIPCHK(h, hipMemcpy(gap64, c.gap64, sizeof(double) * c.n_contacts, hipMemcpyDeviceToHost));
+  const HostPart part = {gap64, c.gap64, gap64 ? sizeof(double) * c.n_contacts : 0};
+  HIPCHK(h, to_host(h, &part, 1));
   return NF_OK;
 }
 
@@ -646,8 +645,8 @@ extern "C" int nf_get_contact_area(nf_handle* h, double* area, uint64_t cap) {
   ContactBuffers& c = h->cb;
   if (!c.valid) return fail(h, NF_E_STATE, "no contacts computed");
   if (cap < c.n_contacts) return fail(h, NF_E_CAPACITY, "buffer too small");
-  if (c.n_contacts && area)
-    HIPCHK(h, hipMemcpy(area, c.area, sizeof(double) * c.n_contacts, hipMemcpyDeviceToHost));
+  const HostPart part = {area, c.area, area ? sizeof(double) * c.n_contacts : 0};
+  HIPCHK(h, to_host(h, &part, 1));
   return NF_OK;
 }
 

@@ -1,5 +1,5 @@
 // nf_host.h - host-side handle layout and helpers shared by the library's
-// C++ translation units (nf_api.cpp, nf_contacts.cpp, nf_io.cpp).
+// C++ translation units (nf_api.cpp, nf_contacts.cpp, nf_copy.cpp, ...).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -10,6 +10,14 @@
 #include <vector>
 
 #include "nf_internal.h"
+
+namespace nf {
+// Scalars that a queued kernel's result is awaited in.
+struct PinnedScalars {
+  RoundInfo ri;   // of the generation's last round
+  CgScal cg[2];   // of the conductance solve's last two checks
+};
+}  // namespace nf
 
 // Options of nf_set_option() (declared in nanofiller.h).
 struct nf_handle {
@@ -39,12 +47,23 @@ struct nf_handle {
   std::unordered_map<void*, size_t> allocs;
   std::multimap<size_t, void*> pool;
   size_t pool_bytes = 0;
+  // blocks of 1 to 32 MB are cut from larger ones (one hipMalloc of that size
+  // takes 0.3 ms, and a packing needs a dozen); given back with the handle
+  struct Slab {
+    char* p;
+    size_t size, used;
+  };
+  std::vector<Slab> slabs;
   unsigned long long cb_stats[6] = {0, 0, 0, 0, 0, 0};  // contact pair tests, rechecks, max dd bits
   float cb_ms[4] = {0, 0, 0, 0};                  // contact kernel times: bin, pair pass, CSR build, row sort
   uint64_t contact_hint = 0;                      // contacts found by the last call (append capacity)
   nf_network_info net_info = {};
   std::vector<uint32_t> reduce_ids;  // old id of every rod kept by the last nf_reduce
-  nf::CgScal* cg_host = nullptr;  // pinned: scalars of nf_conductance's last two checks
+  // pinned host memory of the handle, made when first needed (nf_copy.cpp)
+  char* pin = nullptr;
+  size_t pin_bytes = 0;
+  hipEvent_t pin_ev[8] = {};
+  nf::PinnedScalars* pin_scal = nullptr;
   float net_ms = 0.0f;  // device time of the last nf_network call
 };
 
@@ -61,6 +80,18 @@ void trace(const char* fmt, ...);
 int dalloc_bytes(nf_handle* h, void** p, size_t bytes);
 void dfree(nf_handle* h, void* p);
 void release_contacts(nf_handle* h);
+// Device arrays to the caller's memory, on the handle's stream; waits for it.
+struct HostPart {
+  void* dst;
+  const void* src;
+  size_t bytes;
+};
+hipError_t to_host(nf_handle* h, const HostPart* parts, size_t n_parts);
+// Rods as nf_get_rods gives and nf_set_rods takes them.
+hipError_t rods_to_host(nf_handle* h, const float4* P, const float4* D, uint32_t n, float* rods);
+hipError_t rods_to_device(nf_handle* h, const float* rods, uint32_t n, float4* P, float4* D);
+PinnedScalars* pinned_scalars(nf_handle* h);
+void release_pinned(nf_handle* h);
 // Centre cell list of the contact rods (edge about one pair reach, sorted
 // stencil): built by the cell engine of nf_contacts, or on demand by the
 // node network.

@@ -446,6 +446,10 @@ void launch_bin_rods(const BinPlan& bp, const float4* P, const float4* D, uint32
                      float* hl, hipStream_t s);
 // out[0..2] (cleared): largest half length, radius and |u|^2 - 1 of the rods, as
 // the bits of non-negative floats.
+// bytes (a multiple of 4) of device memory to pinned host memory.
+void launch_to_pinned(const void* src, size_t bytes, void* dst, hipStream_t s);
+// rods[2 i], rods[2 i + 1]: rod i as eight floats (centre, direction, length, radius).
+void launch_pack_rods(const float4* P, const float4* D, uint32_t n, float4* rods, hipStream_t s);
 void launch_rod_bounds(const float4* P, const float4* D, uint32_t n, uint32_t* out, hipStream_t s);
 void launch_expand_flags(const float4* P, uint32_t n, int k, double L, double B, uint32_t* below, uint32_t* above,
                          hipStream_t s);
@@ -527,10 +531,11 @@ void launch_cs_potential(uint32_t n, const uint32_t* labels, const uint32_t* fla
 void launch_cs_order(uint32_t n, const uint32_t* ord, const uint32_t* act, const uint32_t* rl, uint32_t* acto,
                      uint32_t* rlo, const uint32_t* idxo, const uint32_t* offo, uint32_t* idx, uint32_t* off,
                      int stage, hipStream_t s);
-void launch_cg_init(const CgArgs& a, double tol, hipStream_t s);
+// (host: pinned copy of the scalars at the check that ends the launches)
+void launch_cg_init(const CgArgs& a, double tol, CgScal* host, hipStream_t s);
 // Iterations it .. it + count - 1, then a check of the residual.
-void launch_cg_iterations(const CgArgs& a, uint32_t it, uint32_t count, double tol, hipStream_t s);
-void launch_cg_current(const CgArgs& a, hipStream_t s);
+void launch_cg_iterations(const CgArgs& a, uint32_t it, uint32_t count, double tol, CgScal* host, hipStream_t s);
+void launch_cg_current(const CgArgs& a, CgScal* host, hipStream_t s);
 
 // ---- node-level segment network (nf_nodes.hip) ----
 enum NodeFlag { NODE_KEPT = 0, NODE_SCREENED = 1, NODE_CROSSING = 2 };

@@ -139,13 +139,10 @@ extern "C" int nf_get_network(nf_handle* h, uint32_t* labels, uint32_t* row_ptr,
   if (!c.net_valid) return fail(h, NF_E_STATE, "no network computed");
   if ((col || val) && cap < c.nnz) return fail(h, NF_E_CAPACITY, "network buffer too small");
   const uint32_t n = c.n_rods;
-  if (labels && n)
-    HIPCHK(h, hipMemcpy(labels, c.labels, sizeof(uint32_t) * n, hipMemcpyDeviceToHost));
-  if (row_ptr)
-    HIPCHK(h, hipMemcpy(row_ptr, c.nrow, sizeof(uint32_t) * ((size_t)n + 3), hipMemcpyDeviceToHost));
-  if (c.nnz) {
-    if (col) HIPCHK(h, hipMemcpy(col, c.ncol, sizeof(uint32_t) * c.nnz, hipMemcpyDeviceToHost));
-    if (val) HIPCHK(h, hipMemcpy(val, c.nval, sizeof(double) * c.nnz, hipMemcpyDeviceToHost));
-  }
+  const HostPart parts[4] = {{labels, c.labels, labels ? sizeof(uint32_t) * n : 0},
+                             {row_ptr, c.nrow, row_ptr ? sizeof(uint32_t) * ((size_t)n + 3) : 0},
+                             {col, c.ncol, col ? sizeof(uint32_t) * c.nnz : 0},
+                             {val, c.nval, val ? sizeof(double) * c.nnz : 0}};
+  HIPCHK(h, to_host(h, parts, 4));
   return NF_OK;
 }

@@ -244,8 +244,9 @@ extern "C" int nf_get_nodes(nf_handle* h, uint32_t* rod, double* t, uint64_t cap
   if (!c.nd_valid) return fail(h, NF_E_STATE, "no node network built");
   if (cap < c.nd_nodes) return fail(h, NF_E_CAPACITY, "node buffer too small");
   if (c.nd_nodes == 0) return NF_OK;
-  if (rod) HIPCHK(h, hipMemcpy(rod, c.nd_node_rod, sizeof(uint32_t) * c.nd_nodes, hipMemcpyDeviceToHost));
-  if (t) HIPCHK(h, hipMemcpy(t, c.nd_node_t, sizeof(double) * c.nd_nodes, hipMemcpyDeviceToHost));
+  const HostPart parts[2] = {{rod, c.nd_node_rod, rod ? sizeof(uint32_t) * c.nd_nodes : 0},
+                             {t, c.nd_node_t, t ? sizeof(double) * c.nd_nodes : 0}};
+  HIPCHK(h, to_host(h, parts, 2));
   return NF_OK;
 }
 
@@ -257,10 +258,11 @@ extern "C" int nf_get_segments(nf_handle* h, uint32_t* na, uint32_t* nb, double*
   const uint64_t m = c.nd_segments;
   if (cap < m) return fail(h, NF_E_CAPACITY, "segment buffer too small");
   if (m == 0) return NF_OK;
-  if (na) HIPCHK(h, hipMemcpy(na, c.nd_seg_a, sizeof(uint32_t) * m, hipMemcpyDeviceToHost));
-  if (nb) HIPCHK(h, hipMemcpy(nb, c.nd_seg_b, sizeof(uint32_t) * m, hipMemcpyDeviceToHost));
-  if (L) HIPCHK(h, hipMemcpy(L, c.nd_seg_L, sizeof(double) * m, hipMemcpyDeviceToHost));
-  if (A) HIPCHK(h, hipMemcpy(A, c.nd_seg_A, sizeof(double) * m, hipMemcpyDeviceToHost));
+  const HostPart parts[4] = {{na, c.nd_seg_a, na ? sizeof(uint32_t) * m : 0},
+                             {nb, c.nd_seg_b, nb ? sizeof(uint32_t) * m : 0},
+                             {L, c.nd_seg_L, L ? sizeof(double) * m : 0},
+                             {A, c.nd_seg_A, A ? sizeof(double) * m : 0}};
+  HIPCHK(h, to_host(h, parts, 4));
   return NF_OK;
 }
 
@@ -274,9 +276,10 @@ extern "C" int nf_get_node_edges(nf_handle* h, uint32_t* na, uint32_t* nb, uint3
   if (!na && !nb && !contact) return NF_OK;
   if (cap < m) return fail(h, NF_E_CAPACITY, "edge buffer too small");
   if (m == 0) return NF_OK;
-  if (na) HIPCHK(h, hipMemcpy(na, c.nd_ce_a, sizeof(uint32_t) * m, hipMemcpyDeviceToHost));
-  if (nb) HIPCHK(h, hipMemcpy(nb, c.nd_ce_b, sizeof(uint32_t) * m, hipMemcpyDeviceToHost));
-  if (contact) HIPCHK(h, hipMemcpy(contact, c.nd_ce_k, sizeof(uint32_t) * m, hipMemcpyDeviceToHost));
+  const HostPart parts[3] = {{na, c.nd_ce_a, na ? sizeof(uint32_t) * m : 0},
+                             {nb, c.nd_ce_b, nb ? sizeof(uint32_t) * m : 0},
+                             {contact, c.nd_ce_k, contact ? sizeof(uint32_t) * m : 0}};
+  HIPCHK(h, to_host(h, parts, 3));
   return NF_OK;
 }
 
@@ -290,8 +293,9 @@ extern "C" int nf_get_node_electrodes(nf_handle* h, uint32_t* node, double* gap,
   if (!node && !gap && !side) return NF_OK;
   if (cap < m) return fail(h, NF_E_CAPACITY, "electrode buffer too small");
   if (m == 0) return NF_OK;
-  if (node) HIPCHK(h, hipMemcpy(node, c.nd_cel_node, sizeof(uint32_t) * m, hipMemcpyDeviceToHost));
-  if (gap) HIPCHK(h, hipMemcpy(gap, c.nd_cel_gap, sizeof(double) * m, hipMemcpyDeviceToHost));
-  if (side) HIPCHK(h, hipMemcpy(side, c.nd_cel_side, sizeof(int32_t) * m, hipMemcpyDeviceToHost));
+  const HostPart parts[3] = {{node, c.nd_cel_node, node ? sizeof(uint32_t) * m : 0},
+                             {gap, c.nd_cel_gap, gap ? sizeof(double) * m : 0},
+                             {side, c.nd_cel_side, side ? sizeof(int32_t) * m : 0}};
+  HIPCHK(h, to_host(h, parts, 3));
   return NF_OK;
 }

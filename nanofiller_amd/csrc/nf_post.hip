@@ -833,6 +833,37 @@ void launch_rod_bounds(const float4* P, const float4* D, uint32_t n, uint32_t* o
   hipLaunchKernelGGL(k_rod_bounds, dim3(g > 1024 ? 1024 : g), dim3(256), 0, s, P, D, n, out);
 }
 
+__global__ void __launch_bounds__(256) k_to_pinned(const uint32_t* __restrict__ src, uint64_t words,
+                                                   uint64_t quads, uint32_t* __restrict__ dst) {
+  const uint64_t step = (uint64_t)gridDim.x * 256u;
+  const uint64_t t = blockIdx.x * 256u + threadIdx.x;
+  for (uint64_t k = t; k < quads; k += step) ((uint4*)dst)[k] = ((const uint4*)src)[k];
+  for (uint64_t k = 4 * quads + t; k < words; k += step) dst[k] = src[k];
+}
+
+void launch_to_pinned(const void* src, size_t bytes, void* dst, hipStream_t s) {
+  const uint64_t words = bytes / 4;
+  if (words == 0) return;
+  const uint64_t quads = ((uintptr_t)src | (uintptr_t)dst) % 16 == 0 ? words / 4 : 0;
+  hipLaunchKernelGGL(k_to_pinned, dim3(grid_for(words - 3 * quads, 256)), dim3(256), 0, s, (const uint32_t*)src, words,
+                     quads, (uint32_t*)dst);
+}
+
+// Rods as eight floats each, a lane per half so that a wave writes whole lines:
+// `rods` is pinned host memory, and the bus bounds it.
+__global__ void __launch_bounds__(256) k_pack_rods(const float4* __restrict__ P, const float4* __restrict__ D,
+                                                   uint32_t n, float4* __restrict__ rods) {
+  for (uint32_t t = blockIdx.x * 256u + threadIdx.x; t < 2u * n; t += gridDim.x * 256u) {
+    const float4 p = P[t >> 1], d = D[t >> 1];
+    rods[t] = (t & 1u) ? make_float4(d.y, d.z, 2.0f * p.w, d.w) : make_float4(p.x, p.y, p.z, d.x);
+  }
+}
+
+void launch_pack_rods(const float4* P, const float4* D, uint32_t n, float4* rods, hipStream_t s) {
+  if (n == 0) return;
+  hipLaunchKernelGGL(k_pack_rods, dim3(grid_for(2ull * n, 256)), dim3(256), 0, s, P, D, n, rods);
+}
+
 // ---------------------------------------------------------------------------
 // expand: periodic copies of the rods near the two faces normal to axis k.
 // A rod whose centre lies within B of the far face (x >= L - B) gets a copy

@@ -347,26 +347,30 @@ __global__ void __launch_bounds__(NT) k_cg_update(CgArgs a, uint32_t it) {
 
 // One block: relative residual after `it` iterations.  From convergence on
 // (or a residual that is no number) the queued iterations do nothing.
-__global__ void __launch_bounds__(NT) k_cg_check(CgArgs a, uint32_t it, double tol) {
+__global__ void __launch_bounds__(NT) k_cg_check(CgArgs a, uint32_t it, double tol, CgScal* host) {
   __shared__ double sh[NT / WAVE];
   CgScal* sc = a.scal;
-  if (it && sc->done) return;
-  const double rr = block_sum(part_share(a.part_rr, a.nb), sh);
-  if (threadIdx.x != 0) return;
-  const double bb = it ? sc->bb : rr;
-  const double res = bb > 0.0 ? sqrt_cr((rr > 0.0 ? rr : 0.0) / bb) : 0.0;
-  sc->bb = bb;
-  sc->res = res;
-  sc->done = res <= tol ? CG_CONVERGED : (res < __longlong_as_double(0x7FF0000000000000ll) ? 0u : CG_BROKEN);
+  if (it == 0 || !sc->done) {
+    const double rr = block_sum(part_share(a.part_rr, a.nb), sh);
+    if (threadIdx.x != 0) return;
+    const double bb = it ? sc->bb : rr;
+    const double res = bb > 0.0 ? sqrt_cr((rr > 0.0 ? rr : 0.0) / bb) : 0.0;
+    sc->bb = bb;
+    sc->res = res;
+    sc->done = res <= tol ? CG_CONVERGED : (res < __longlong_as_double(0x7FF0000000000000ll) ? 0u : CG_BROKEN);
+  }
+  if (threadIdx.x == 0) *host = *sc;
 }
 
 // One block: source and sink currents.
-__global__ void __launch_bounds__(NT) k_cg_currents(CgArgs a) {
+__global__ void __launch_bounds__(NT) k_cg_currents(CgArgs a, CgScal* host) {
   __shared__ double2 sh[NT / WAVE];
   const double2 t = block_sum2(part_share(a.part_rz, a.nb), part_share(a.part_rr, a.nb), sh);
   if (threadIdx.x != 0) return;
-  a.scal->isrc = t.x;
-  a.scal->isnk = t.y;
+  CgScal c = *a.scal;
+  c.isrc = t.x;
+  c.isnk = t.y;
+  *host = c;
 }
 
 // Partials of the source current sum bs (1 - x) and the sink current sum bk x.
@@ -458,22 +462,22 @@ void launch_cs_order(uint32_t n, const uint32_t* ord, const uint32_t* act, const
                        idx, off);
 }
 
-void launch_cg_init(const CgArgs& a, double tol, hipStream_t s) {
+void launch_cg_init(const CgArgs& a, double tol, CgScal* host, hipStream_t s) {
   hipLaunchKernelGGL(k_cg_init, dim3(a.nb), dim3(NT), 0, s, a);
-  hipLaunchKernelGGL(k_cg_check, dim3(1), dim3(NT), 0, s, a, 0u, tol);
+  hipLaunchKernelGGL(k_cg_check, dim3(1), dim3(NT), 0, s, a, 0u, tol, host);
 }
 
-void launch_cg_iterations(const CgArgs& a, uint32_t it, uint32_t count, double tol, hipStream_t s) {
+void launch_cg_iterations(const CgArgs& a, uint32_t it, uint32_t count, double tol, CgScal* host, hipStream_t s) {
   for (uint32_t j = it; j < it + count; ++j) {
     hipLaunchKernelGGL(k_cg_spmv, dim3(a.ns), dim3(SPMV_NT), 0, s, a, j);
     hipLaunchKernelGGL(k_cg_update, dim3(a.nb), dim3(NT), 0, s, a, j);
   }
-  hipLaunchKernelGGL(k_cg_check, dim3(1), dim3(NT), 0, s, a, it + count, tol);
+  hipLaunchKernelGGL(k_cg_check, dim3(1), dim3(NT), 0, s, a, it + count, tol, host);
 }
 
-void launch_cg_current(const CgArgs& a, hipStream_t s) {
+void launch_cg_current(const CgArgs& a, CgScal* host, hipStream_t s) {
   hipLaunchKernelGGL(k_cg_current, dim3(a.nb), dim3(NT), 0, s, a.m, a.bsrc, a.bsnk, a.x, a.part_rz);
-  hipLaunchKernelGGL(k_cg_currents, dim3(1), dim3(NT), 0, s, a);
+  hipLaunchKernelGGL(k_cg_currents, dim3(1), dim3(NT), 0, s, a, host);
 }
 
 }  // namespace nf
