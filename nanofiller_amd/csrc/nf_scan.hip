@@ -14,6 +14,7 @@ namespace nf {
 constexpr int SCAN_THREADS = 256;
 constexpr int SCAN_ITEMS = 8;
 constexpr int SCAN_TILE = SCAN_THREADS * SCAN_ITEMS;
+constexpr uint32_t SUMS_MAX = 2048;
 
 __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
   const int lane = threadIdx.x & (WAVE - 1);
@@ -44,17 +45,37 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* sm, ui
   return off + inc - v;
 }
 
-__global__ void __launch_bounds__(SCAN_THREADS) k_scan_tiles(const uint32_t* __restrict__ in,
-                                                             uint64_t n, uint32_t* __restrict__ sums) {
-  __shared__ uint32_t sm[SCAN_THREADS / WAVE];
-  const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE + (uint64_t)threadIdx.x * SCAN_ITEMS;
-  uint32_t s = 0;
+// The thread's eight elements, zero past the end.
+__device__ __forceinline__ void scan_load(const uint32_t* __restrict__ in, uint64_t base, uint64_t n, bool wide,
+                                          uint32_t v[SCAN_ITEMS]) {
+  if (wide && base + SCAN_ITEMS <= n) {
+    const uint4 a = *(const uint4*)(in + base), b = *(const uint4*)(in + base + 4);
+    v[0] = a.x;
+    v[1] = a.y;
+    v[2] = a.z;
+    v[3] = a.w;
+    v[4] = b.x;
+    v[5] = b.y;
+    v[6] = b.z;
+    v[7] = b.w;
+    return;
+  }
 #pragma unroll
   for (int k = 0; k < SCAN_ITEMS; ++k) {
     const uint64_t i = base + k;
-    const uint32_t v = in[i < n ? i : n - 1];  // clamped load, masked below
-    s += i < n ? v : 0u;
+    const uint32_t x = in[i < n ? i : n - 1];  // clamped load, masked below
+    v[k] = i < n ? x : 0u;
   }
+}
+
+__global__ void __launch_bounds__(SCAN_THREADS) k_scan_tiles(const uint32_t* __restrict__ in,
+                                                             uint64_t n, bool wide, uint32_t* __restrict__ sums) {
+  __shared__ uint32_t sm[SCAN_THREADS / WAVE];
+  const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE + (uint64_t)threadIdx.x * SCAN_ITEMS;
+  uint32_t v[SCAN_ITEMS], s = 0;
+  scan_load(in, base, n, wide, v);
+#pragma unroll
+  for (int k = 0; k < SCAN_ITEMS; ++k) s += v[k];
   uint32_t tot;
   block_excl_scan(s, sm, &tot);
   if (threadIdx.x == 0) sums[blockIdx.x] = tot;
@@ -79,29 +100,42 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_sums(uint32_t* __restrict
   if (threadIdx.x == 0) out[n] = carry;
 }
 
-__global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(const uint32_t* __restrict__ in,
-                                                             uint64_t n,
-                                                             const uint32_t* __restrict__ sums,
-                                                             uint32_t* __restrict__ out) {
-  __shared__ uint32_t sm[SCAN_THREADS / WAVE];
+// SUMMED: sums holds the exclusive prefix of the tile sums, else the sums.
+// (in and out may be one array: a thread reads its elements before it writes.)
+template <bool SUMMED>
+__global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(const uint32_t* in, uint64_t n, bool wide,
+                                                             const uint32_t* __restrict__ sums, uint32_t* out) {
+  __shared__ uint32_t sm[SCAN_THREADS / WAVE], sp[SCAN_THREADS / WAVE];
   const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE + (uint64_t)threadIdx.x * SCAN_ITEMS;
-  uint32_t v[SCAN_ITEMS];
-  uint32_t s = 0;
+  uint32_t v[SCAN_ITEMS], s = 0, before = 0;
+  scan_load(in, base, n, wide, v);
+  if (!SUMMED)
+    for (uint32_t t = threadIdx.x; t < blockIdx.x; t += SCAN_THREADS) before += sums[t];
+#pragma unroll
+  for (int k = 0; k < SCAN_ITEMS; ++k) s += v[k];
+  uint32_t tot, lead;
+  uint32_t run = block_excl_scan(s, sm, &tot);
+  if (SUMMED) {
+    lead = sums[blockIdx.x];
+  } else {
+    block_excl_scan(before, sp, &lead);
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = lead + tot;
+  }
+  run += lead;
 #pragma unroll
   for (int k = 0; k < SCAN_ITEMS; ++k) {
-    const uint64_t i = base + k;
-    const uint32_t x = in[i < n ? i : n - 1];
-    v[k] = i < n ? x : 0u;
-    s += v[k];
+    const uint32_t x = v[k];
+    v[k] = run;
+    run += x;
   }
-  uint32_t tot;
-  uint32_t run = block_excl_scan(s, sm, &tot) + sums[blockIdx.x];
+  if (wide && base + SCAN_ITEMS <= n) {
+    *(uint4*)(out + base) = make_uint4(v[0], v[1], v[2], v[3]);
+    *(uint4*)(out + base + 4) = make_uint4(v[4], v[5], v[6], v[7]);
+    return;
+  }
 #pragma unroll
-  for (int k = 0; k < SCAN_ITEMS; ++k) {
-    const uint64_t i = base + k;
-    if (i < n) out[i] = run;
-    run += v[k];
-  }
+  for (int k = 0; k < SCAN_ITEMS; ++k)
+    if (base + k < n) out[base + k] = v[k];
 }
 
 // Short arrays (the cells of a single packing): one workgroup of 1024
@@ -163,9 +197,14 @@ void scan_u32(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* tmp, hipS
     hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SCAN_THREADS), 0, s, tmp, 0u, out, (uint64_t)0);
     return;
   }
-  hipLaunchKernelGGL(k_scan_tiles, dim3(nt), dim3(SCAN_THREADS), 0, s, in, n, tmp);
+  const bool wide = (((uintptr_t)in | (uintptr_t)out) & 15u) == 0;
+  hipLaunchKernelGGL(k_scan_tiles, dim3(nt), dim3(SCAN_THREADS), 0, s, in, n, wide, tmp);
+  if (nt <= SUMS_MAX) {
+    hipLaunchKernelGGL(k_scan_apply<false>, dim3(nt), dim3(SCAN_THREADS), 0, s, in, n, wide, tmp, out);
+    return;
+  }
   hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SCAN_THREADS), 0, s, tmp, nt, out, n);
-  hipLaunchKernelGGL(k_scan_apply, dim3(nt), dim3(SCAN_THREADS), 0, s, in, n, tmp, out);
+  hipLaunchKernelGGL(k_scan_apply<true>, dim3(nt), dim3(SCAN_THREADS), 0, s, in, n, wide, tmp, out);
 }
 
 __global__ void k_fill_u32(uint32_t* __restrict__ p, uint32_t v, uint64_t n) {
