@@ -36,8 +36,8 @@ int contact_bounds(nf_handle* h, uint32_t n, const float4* P, const float4* D, f
   float v[3] = {0.0f, 0.0f, 0.0f};
   fill_u32(out, 0u, 4, h->stream);
   launch_rod_bounds(P, D, n, out, h->stream);
-  hipError_t e = hipMemcpyAsync(v, out, sizeof(v), hipMemcpyDeviceToHost, h->stream);
-  if (e == hipSuccess) e = sync_stream(h->stream, "rod bounds");
+  const HostPart part = {v, out, sizeof(v)};
+  hipError_t e = to_host(h, &part, 1);
   if (e == hipSuccess) e = hipGetLastError();
   dfree(h, out);
   if (e != hipSuccess) return fail(h, NF_E_HIP, std::string("rod bounds: ") + hipGetErrorString(e));
@@ -94,7 +94,8 @@ static int bin_rods(nf_handle* h, const float4* P, const float4* D, uint32_t n, 
   return NF_OK;
 }
 
-static int build_cell_list(nf_handle* h, double edge, double reach, bool half, int bx = 1) {
+// (scratch is in use until the caller has waited for the stream and frees it)
+static int build_cell_list(nf_handle* h, double edge, double reach, bool half, BinScratch* bs, int bx = 1) {
   ContactBuffers& c = h->cb;
   const nf_params& p = h->params[h->post_inst];
   const uint32_t n = c.n_rods;
@@ -114,7 +115,8 @@ static int build_cell_list(nf_handle* h, double edge, double reach, bool half, i
   }
   if (ncells > (1ull << 26)) return fail(h, NF_E_INVALID, "contact grid too large");
   c.ncells = (uint32_t)ncells;
-  std::vector<int4> st = build_stencil(c.ncell, p.box, reach, half, bx);
+  std::vector<int4>& st = h->contact_stencil;
+  st = build_stencil(c.ncell, p.box, reach, half, bx);
   c.st_n = (uint32_t)st.size();
   int rc = NF_OK;
 #define ALLOC(ptr, cnt) \
@@ -129,21 +131,12 @@ static int build_cell_list(nf_handle* h, double edge, double reach, bool half, i
 #undef ALLOC
   if (rc != NF_OK) return rc;
   HIPCHK(h, hipMemcpyAsync(c.stencil, st.data(), sizeof(int4) * st.size(), hipMemcpyHostToDevice, s));
-  BinScratch bs;
-  rc = bin_rods(h, P, D, n, c.ncell, scale, c.cP, c.cD, c.cid, c.cstart, c.ccount, c.chl, &bs);
-  if (rc != NF_OK) {
-    free_bin_scratch(h, &bs);
-    return rc;
-  }
-  const hipError_t e = sync_stream(s, "contact cell list");
-  free_bin_scratch(h, &bs);
-  if (e != hipSuccess) return fail(h, NF_E_HIP, std::string("contact cell list: ") + hipGetErrorString(e));
-  return NF_OK;
+  return bin_rods(h, P, D, n, c.ncell, scale, c.cP, c.cD, c.cid, c.cstart, c.ccount, c.chl, bs);
 }
 
 // Cell list of the cell-pair engine: cells of about one typical pair reach,
 // half stencil of the longest pair reach.
-int build_contact_cells(nf_handle* h) {
+static int contact_cells(nf_handle* h, BinScratch* bs) {
   ContactBuffers& c = h->cb;
   if (c.cP && c.cell_list == 1) return NF_OK;
   if (c.cP) {
@@ -164,8 +157,18 @@ int build_contact_cells(nf_handle* h) {
   double edge = (p.len_law == NF_LEN_LOGNORMAL ? p.len : (double)c.hl_max * 2.0) * REACH_PAD + Rmax;
   if (edge > reach) edge = reach;
   edge = default_cell_edge(edge, (double)c.n_rods / (p.box[0] * p.box[1] * p.box[2]), 1.0);
-  const int rc = build_cell_list(h, edge, reach, true);
+  const int rc = build_cell_list(h, edge, reach, true, bs);
   if (rc == NF_OK) c.cell_list = 1;
+  return rc;
+}
+
+int build_contact_cells(nf_handle* h) {
+  BinScratch bs;
+  int rc = contact_cells(h, &bs);
+  const hipError_t e = sync_stream(h->stream, "contact cell list");
+  free_bin_scratch(h, &bs);
+  if (rc == NF_OK && e != hipSuccess)
+    rc = fail(h, NF_E_HIP, std::string("contact cell list: ") + hipGetErrorString(e));
   return rc;
 }
 
@@ -277,15 +280,18 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, Co
   if (rc == NF_OK) rc = dalloc(h, &(ptr), (cnt));
   ALLOC(c.cnt, (uint64_t)n + 1);
   ALLOC(c.rowptr, (uint64_t)n + 1);
-  ALLOC(c.fill, std::max<uint64_t>(n, 1));
-  ALLOC(ctr, 8);  // pair tests, rechecks, max dd, tile bytes, append count, work counter, overflow
+  // pair tests, rechecks, max dd, tile bytes, append count, work counter, overflow; then the work queues
+  constexpr uint64_t CTR_WORDS = 16 + 2 * QWORDS;
+  ALLOC(ctr, CTR_WORDS / 2);
   ALLOC(tmp, scan_tmp_words((uint64_t)n + 1));
-  ALLOC(queues, 2 * QWORDS);
 #undef ALLOC
+  BinScratch bs;
+  PinnedScalars* pinned = pinned_scalars(h);
+  if (rc == NF_OK && !pinned) rc = fail(h, NF_E_NOMEM, "contacts: no pinned memory");
   auto free_scratch = [&]() {
+    free_bin_scratch(h, &bs);
     dfree(h, ctr);
     dfree(h, tmp);
-    dfree(h, queues);
     dfree(h, lrods);
     if (lown) {
       dfree(h, lcount);
@@ -301,13 +307,13 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, Co
   }
   hipEvent_t* ev = h->ev;
   hipEventRecord(ev[0], s);
-  fill_u32((uint32_t*)ctr, 0u, 16, s);
-  fill_u32(queues, 0u, 2 * QWORDS, s);
+  queues = (uint32_t*)(ctr + 8);
+  fill_u32((uint32_t*)ctr, 0u, CTR_WORDS, s);
   PairArgs a{};
   SegCrossArgs xa{};
   // ---- bin: centre cell list
   if (cells || way == WAY_LISTS) {
-    rc = build_contact_cells(h);
+    rc = contact_cells(h, &bs);
   } else {
     double edge = 0.0;
     int fine = 1;
@@ -316,7 +322,7 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, Co
     c.fp_fine = fine;
     xa.g = seg_grid(p.box, edge, (double)amax, gap, ew);
     const double rpad = (double)xa.g.r + 2.0 * (double)CELL_MARGIN;
-    rc = build_cell_list(h, edge, (double)hlmax * REACH_PAD + rpad, false, SEG_ROW);
+    rc = build_cell_list(h, edge, (double)hlmax * REACH_PAD + rpad, false, &bs, SEG_ROW);
     if (rc == NF_OK) c.cell_list = 2;
     xa.fine = fine;
     xa.rpad = (float)rpad;
@@ -472,8 +478,7 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, Co
       return rc;
     }
     if (attempt > 0) {
-      fill_u32((uint32_t*)ctr, 0u, 16, s);
-      fill_u32(queues, 0u, 2 * QWORDS, s);
+      fill_u32((uint32_t*)ctr, 0u, CTR_WORDS, s);
     }
     hipEventRecord(ev[1], s);
     if (cells) {
@@ -508,10 +513,10 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, Co
     hipEventRecord(ev[2], s);
     trace("contacts: %u rods, %s pass launched", n,
           cells ? "cell-pair" : (way == WAY_LISTS ? "crossing-list" : "footprint"));
-    uint32_t over = 0;
-    HIPCHK(h, hipMemcpyAsync(&total, (uint32_t*)(ctr + 4), sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    HIPCHK(h, hipMemcpyAsync(&over, (uint32_t*)(ctr + 6), sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    launch_to_pinned(ctr, sizeof(pinned->ctr), pinned->ctr, s);
     HIPCHK(h, sync_stream(s, "contact pair pass"));
+    total = (uint32_t)pinned->ctr[4];
+    const uint32_t over = (uint32_t)pinned->ctr[6];
     HIPCHK(h, hipGetLastError());
     if (over) {
       trace("contacts: more rods cross a cell than fit; another engine instead");
@@ -544,16 +549,15 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, Co
   // CSR over I: counts, scan, scatter, canonical row order
   hipEventRecord(ev[3], s);
   fill_u32(c.cnt, 0u, (uint64_t)n + 1, s);
-  fill_u32(c.fill, 0u, n, s);
   launch_csr_count(appI, total, c.cnt, s);
   scan_u32(c.cnt, c.rowptr, n, tmp, s);
-  launch_csr_scatter(appI, appJ, appG, appG64, appImg, total, c.rowptr, c.fill, c.J, c.gap, c.gap64,
+  launch_csr_scatter(appI, appJ, appG, appG64, appImg, total, c.rowptr, c.cnt, c.J, c.gap, c.gap64,
                      c.img, s);
   hipEventRecord(ev[4], s);
   launch_row_sort(c.rowptr, n, c.J, c.gap, c.gap64, c.img, s);
   launch_contact_area(P, D, n, c.rowptr, c.J, c.img, p.box, gap, c.area, s);
   hipEventRecord(ev[5], s);
-  HIPCHK(h, hipMemcpyAsync(h->cb_stats, ctr, sizeof(unsigned long long) * 6, hipMemcpyDeviceToHost, s));
+  std::copy(pinned->ctr, pinned->ctr + 6, h->cb_stats);
   HIPCHK(h, sync_stream(s, "contact list"));
   trace("contacts: %u recorded and sorted", total);
   HIPCHK(h, hipGetLastError());
@@ -742,17 +746,14 @@ int hist_run(nf_handle* h, const HistPlan& pl, const double* edges, double* dE,
   }
   // int64 and u64 share the layout; counts never reach 2^63
   const int64_t* src = (const int64_t*)dOut;
-  struct {
-    int64_t* dst;
-    size_t off, len;
-  } cp[4] = {{out_centre, 0, (size_t)nb},
-             {out_polar, (size_t)nb, (size_t)nb},
-             {pl.mutual ? out_mutual : nullptr, 2 * (size_t)nb, (size_t)nb},
-             {pl.npb ? out_phitheta : nullptr, 3 * (size_t)nb, (size_t)pl.npb * pl.ntb}};
-  for (auto& c : cp)
-    if (e == hipSuccess && c.dst)
-      e = hipMemcpyAsync(c.dst, src + c.off, sizeof(int64_t) * c.len, hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  auto part = [&](int64_t* dst, size_t off, size_t len) {
+    return HostPart{dst, src + off, dst ? sizeof(int64_t) * len : 0};
+  };
+  const HostPart parts[4] = {part(out_centre, 0, nb), part(out_polar, nb, nb),
+                             part(pl.mutual ? out_mutual : nullptr, 2 * (size_t)nb, nb),
+                             part(pl.npb ? out_phitheta : nullptr, 3 * (size_t)nb, (size_t)pl.npb * pl.ntb)};
+  const hipError_t w = to_host(h, parts, 4);  // (waits for the upload of `edges` too)
+  if (e == hipSuccess) e = w;
   if (e != hipSuccess) return fail(h, NF_E_HIP, std::string("histograms: ") + hipGetErrorString(e));
   return NF_OK;
 }
@@ -871,8 +872,8 @@ extern "C" int nf_centre_distance(nf_handle* h, int32_t bins, double width, int6
   launch_cent(cP, cid, cstart, ccount, dst, (uint32_t)runs.size(), n, nc, p.box, de2, bins, width,
               rf * rf * 1.00001f, part, out, s);
   std::vector<unsigned long long> hout((size_t)bins + 3);
-  e = hipMemcpyAsync(hout.data(), out, sizeof(unsigned long long) * hout.size(), hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = sync_stream(s, "centre distance");
+  const HostPart out_part = {hout.data(), out, sizeof(unsigned long long) * hout.size()};
+  e = to_host(h, &out_part, 1);
   if (e == hipSuccess) e = hipGetLastError();
   release();
   if (e != hipSuccess) return fail(h, NF_E_HIP, std::string("centre distance: ") + hipGetErrorString(e));

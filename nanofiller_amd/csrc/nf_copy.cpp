@@ -71,7 +71,10 @@ bool staged(nf_handle* h, const HostPart* parts, size_t n_parts, Issue issue, hi
     total += parts[i].bytes;
     padded += (parts[i].bytes + 255) & ~(size_t)255;
   }
-  if (total == 0) return true;
+  if (total == 0) {
+    *out = sync_stream(h->stream, "copy to the host");
+    return true;
+  }
   if (padded <= PIN_SMALL) {
     char* pin = pin_block(h, padded);
     if (!pin) return false;

@@ -16,6 +16,7 @@ namespace nf {
 struct PinnedScalars {
   RoundInfo ri;   // of the generation's last round
   CgScal cg[2];   // of the conductance solve's last two checks
+  unsigned long long ctr[8];  // counters of a contact pass; summary of a network build
 };
 }  // namespace nf
 
@@ -47,6 +48,7 @@ struct nf_handle {
   std::unordered_map<void*, size_t> allocs;
   std::multimap<size_t, void*> pool;
   size_t pool_bytes = 0;
+  std::vector<int4> contact_stencil;  // on its way to the device
   // blocks of 1 to 32 MB are cut from larger ones (one hipMalloc of that size
   // takes 0.3 ms, and a packing needs a dozen); given back with the handle
   struct Slab {

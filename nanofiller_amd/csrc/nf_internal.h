@@ -211,7 +211,6 @@ struct ContactBuffers {
   // contacts
   uint32_t* cnt = nullptr;     // N
   uint32_t* rowptr = nullptr;  // N + 1
-  uint32_t* fill = nullptr;    // N
   uint32_t* J = nullptr;
   float* gap = nullptr;
   double* gap64 = nullptr;
@@ -467,7 +466,7 @@ void launch_contact_area(const float4* P, const float4* D, uint32_t n, const uin
 // (rowptr from scan_u32 of the counts in between).
 void launch_csr_count(const uint32_t* I, uint64_t c, uint32_t* cnt, hipStream_t s);
 void launch_csr_scatter(const uint32_t* I, const uint32_t* J, const float* gap, const double* gap64,
-                        const int32_t* img, uint64_t c, const uint32_t* rowptr, uint32_t* fill,
+                        const int32_t* img, uint64_t c, const uint32_t* rowptr, uint32_t* cnt,
                         uint32_t* oJ, float* ogap, double* ogap64, int32_t* oimg, hipStream_t s);
 void launch_hist(const float4* P, const float4* D, uint32_t n, const uint32_t* rowptr,
                  const uint32_t* J, const double* edges_p, const double* edges_m,

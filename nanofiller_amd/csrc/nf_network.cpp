@@ -80,6 +80,8 @@ extern "C" int nf_network(nf_handle* h, nf_network_info* info) {
                  a.summary, a.tmp,     a.cg,      a.bsum};
     for (void* q : w) dfree(h, q);
   };
+  PinnedScalars* pinned = pinned_scalars(h);
+  if (rc == NF_OK && !pinned) rc = fail(h, NF_E_NOMEM, "network: no pinned memory");
   if (rc != NF_OK) {
     release_work();
     return rc;
@@ -88,9 +90,10 @@ extern "C" int nf_network(nf_handle* h, nf_network_info* info) {
   a.nrow = c.nrow;
   hipEventRecord(h->ev[0], s);
   launch_network_build(a, s);
-  unsigned long long sum[NET_SUMMARY] = {};
-  hipError_t e = hipMemcpyAsync(sum, a.summary, sizeof(sum), hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = sync_stream(s, "network build");
+  const unsigned long long* sum = pinned->ctr;
+  static_assert(NET_SUMMARY <= sizeof(pinned->ctr) / sizeof(pinned->ctr[0]), "summary");
+  launch_to_pinned(a.summary, sizeof(unsigned long long) * NET_SUMMARY, pinned->ctr, s);
+  hipError_t e = sync_stream(s, "network build");
   if (e == hipSuccess) e = hipGetLastError();
   if (e != hipSuccess) {
     release_work();

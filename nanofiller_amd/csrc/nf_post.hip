@@ -273,7 +273,8 @@ void launch_contact_area(const float4* P, const float4* D, uint32_t n, const uin
 }
 
 // CSR over I from the unsorted contact list (the pair pass appends in any
-// order; the row sort makes every row canonical afterwards).
+// order, the row sort makes every row canonical afterwards; a row's places are
+// taken from its count downwards).
 __global__ void k_csr_count(const uint32_t* __restrict__ I, uint64_t c, uint32_t* __restrict__ cnt) {
   for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < c;
        k += (uint64_t)gridDim.x * blockDim.x)
@@ -283,13 +284,13 @@ __global__ void k_csr_count(const uint32_t* __restrict__ I, uint64_t c, uint32_t
 __global__ void k_csr_scatter(const uint32_t* __restrict__ I, const uint32_t* __restrict__ J,
                               const float* __restrict__ gap, const double* __restrict__ gap64,
                               const int32_t* __restrict__ img, uint64_t c,
-                              const uint32_t* __restrict__ rowptr, uint32_t* __restrict__ fill,
+                              const uint32_t* __restrict__ rowptr, uint32_t* __restrict__ cnt,
                               uint32_t* __restrict__ oJ, float* __restrict__ ogap,
                               double* __restrict__ ogap64, int32_t* __restrict__ oimg) {
   for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < c;
        k += (uint64_t)gridDim.x * blockDim.x) {
     const uint32_t i = I[k];
-    const uint32_t pos = rowptr[i] + atomicAdd(&fill[i], 1u);
+    const uint32_t pos = rowptr[i] + atomicSub(&cnt[i], 1u) - 1u;
     oJ[pos] = J[k];
     ogap[pos] = gap[k];
     ogap64[pos] = gap64[k];
@@ -303,11 +304,11 @@ void launch_csr_count(const uint32_t* I, uint64_t c, uint32_t* cnt, hipStream_t 
 }
 
 void launch_csr_scatter(const uint32_t* I, const uint32_t* J, const float* gap, const double* gap64,
-                        const int32_t* img, uint64_t c, const uint32_t* rowptr, uint32_t* fill,
+                        const int32_t* img, uint64_t c, const uint32_t* rowptr, uint32_t* cnt,
                         uint32_t* oJ, float* ogap, double* ogap64, int32_t* oimg, hipStream_t s) {
   if (c == 0) return;
   hipLaunchKernelGGL(k_csr_scatter, dim3(grid_for(c, 256)), dim3(256), 0, s, I, J, gap, gap64, img, c,
-                     rowptr, fill, oJ, ogap, ogap64, oimg);
+                     rowptr, cnt, oJ, ogap, ogap64, oimg);
 }
 
 // ---------------------------------------------------------------------------

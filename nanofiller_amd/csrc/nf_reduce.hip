@@ -95,7 +95,11 @@ __global__ void k_red_degree(RedArgs a) {
   }
 }
 
-__global__ void k_red_mark(RedArgs a, uint32_t slot) {
+// (few blocks, one atomic each: 12 ns apiece on one address; one per wave had
+// taken 8 us for 200,000 rods, this takes 4)
+constexpr int MARK_THREADS = 1024, MARK_BLOCKS = 256;
+__global__ void __launch_bounds__(MARK_THREADS) k_red_mark(RedArgs a, uint32_t slot) {
+  __shared__ uint32_t sh[MARK_THREADS / WAVE];
   if (__hip_atomic_load(a.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
   uint32_t local = 0;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += gridDim.x * blockDim.x) {
@@ -109,9 +113,13 @@ __global__ void k_red_mark(RedArgs a, uint32_t slot) {
       ++local;
     }
   }
-  // one atomic per wave after the loop (all lanes converged)
-  const unsigned long long w = wave_sum_u64(local);
-  if ((threadIdx.x & (WAVE - 1)) == 0 && w) atomicAdd(&a.cnt[slot], (uint32_t)w);
+  const uint32_t w = (uint32_t)wave_sum_u64(local);
+  if (threadIdx.x % WAVE == 0) sh[threadIdx.x / WAVE] = w;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  uint32_t sum = 0;
+  for (int k = 0; k < MARK_THREADS / WAVE; ++k) sum += sh[k];
+  if (sum) atomicAdd(&a.cnt[slot], sum);
 }
 
 __global__ void k_red_propagate(RedArgs a, uint32_t slot) {
@@ -203,6 +211,7 @@ extern "C" int nf_reduce(nf_handle* h, int32_t min_cont, nf_reduce_info* info) {
   hipEvent_t* ev = h->ev;
   hipEventRecord(ev[0], s);
   const dim3 grid(red_grid(n)), block(RED_THREADS);
+  const dim3 mark_grid(std::min<uint32_t>(n / MARK_THREADS + 1u, MARK_BLOCKS));
   hipLaunchKernelGGL(k_red_init, grid, block, 0, s, a);
   hipLaunchKernelGGL(k_red_degree, grid, block, 0, s, a);
   uint32_t rounds = 0;
@@ -213,11 +222,11 @@ extern "C" int nf_reduce(nf_handle* h, int32_t min_cont, nf_reduce_info* info) {
   while (e == hipSuccess && !done && rounds <= n) {
     fill_u32(a.cnt, 0u, RED_BATCH, s);
     for (uint32_t b = 0; b < (uint32_t)RED_BATCH; ++b) {
-      hipLaunchKernelGGL(k_red_mark, grid, block, 0, s, a, b);
+      hipLaunchKernelGGL(k_red_mark, mark_grid, dim3(MARK_THREADS), 0, s, a, b);
       hipLaunchKernelGGL(k_red_propagate, grid, block, 0, s, a, b);
     }
-    e = hipMemcpyAsync(hc.data(), a.cnt, sizeof(uint32_t) * RED_BATCH, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = sync_stream(s, "reduce rounds");
+    const HostPart part = {hc.data(), a.cnt, sizeof(uint32_t) * RED_BATCH};
+    e = to_host(h, &part, 1);
     if (e == hipSuccess) e = hipGetLastError();
     for (uint32_t b = 0; b < (uint32_t)RED_BATCH && e == hipSuccess; ++b) {
       ++rounds;
@@ -243,8 +252,8 @@ extern "C" int nf_reduce(nf_handle* h, int32_t min_cont, nf_reduce_info* info) {
   if (e == hipSuccess && kept) {
     e = hipMemcpyAsync(P, oP, sizeof(float4) * kept, hipMemcpyDeviceToDevice, s);
     if (e == hipSuccess) e = hipMemcpyAsync(D, oD, sizeof(float4) * kept, hipMemcpyDeviceToDevice, s);
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(ids.data(), oid, sizeof(uint32_t) * kept, hipMemcpyDeviceToHost, s);
+    const HostPart part = {ids.data(), oid, sizeof(uint32_t) * kept};
+    if (e == hipSuccess) e = to_host(h, &part, 1);
   }
   hipEventRecord(ev[1], s);
   if (e == hipSuccess) e = sync_stream(s, "reduce");
