@@ -81,6 +81,15 @@ __device__ __forceinline__ double2 block_sum2(double v, double w, double2* sh) {
   return t;
 }
 
+// The block's place among the rows: each XCD, which takes every eighth block,
+// has a stretch of its own, so that the columns of its rows (unknowns are in
+// spatial order) are mostly in its stretch too and are fetched once, not by all
+// eight.
+__device__ __forceinline__ uint32_t row_block() {
+  const uint32_t x = blockIdx.x % 8u, q = gridDim.x / 8u, r = gridDim.x % 8u;
+  return x * q + min(x, r) + blockIdx.x / 8u;
+}
+
 // This thread's share of at most CG_MAX_BLOCKS block sums of an earlier
 // kernel: loads without a branch, so that they go out with the caller's.
 template <int NW = NT / WAVE>
@@ -231,9 +240,10 @@ __global__ void __launch_bounds__(NT) k_cg_init(CgArgs a) {
 // dependent loads (offsets, column, gather) bounds it, not the bytes: the first
 // eight entries and the block sums that beta needs are fetched side by side,
 // and every row of 262,000 is in flight at once.  178,000 unknowns with 3.9
-// entries a row: 7.2 us, and the update 5.8, where product, direction, update
+// entries a row: 6.8 us, and the update 4.5 (7.2 and 5.8 with blocks in launch
+// order, see row_block), where product, direction, update
 // and two scalars had been launches of 9.9, 3.5, 4.3 and 3.1 us each; 3120
-// iterations 64 -> 37..43 ms.  One or four lanes per row: 7.2, 8.7 us.
+// iterations 64 -> 36 ms.  One or four lanes per row: 7.2, 8.7 us (in launch order).
 constexpr int SPMV_LANES = 2, SPMV_AHEAD = 8 / SPMV_LANES;  // entries of a row fetched at once: 8
 constexpr int SPMV_NT = 512;
 constexpr int SPMV_ROWS = SPMV_NT / SPMV_LANES;
@@ -283,7 +293,8 @@ __global__ void __launch_bounds__(SPMV_NT) k_cg_spmv(CgArgs a, uint32_t it) {
   constexpr int NW = SPMV_NT / WAVE;
   __shared__ double sh[NW], sh_pq[NW];
   const uint32_t sub = threadIdx.x % SPMV_LANES;
-  uint32_t k = blockIdx.x * SPMV_ROWS + threadIdx.x / SPMV_LANES;
+  const uint32_t block = row_block();
+  uint32_t k = block * SPMV_ROWS + threadIdx.x / SPMV_LANES;
   SpmvRow row;
   const uint32_t done = a.scal->done;
   double old = a.scal->rz[(it + 1u) & 1u];
@@ -296,20 +307,21 @@ __global__ void __launch_bounds__(SPMV_NT) k_cg_spmv(CgArgs a, uint32_t it) {
   if (blockIdx.x == 0 && threadIdx.x == 0) a.scal->rz[it & 1u] = rz;
   double pq = spmv_row(a, k, sub, beta, row);
   // block-uniform loop over row groups, so the sums run with every lane
-  for (uint32_t k0 = (blockIdx.x + gridDim.x) * SPMV_ROWS; k0 < a.m; k0 += gridDim.x * SPMV_ROWS) {
+  for (uint32_t k0 = (block + gridDim.x) * SPMV_ROWS; k0 < a.m; k0 += gridDim.x * SPMV_ROWS) {
     k += gridDim.x * SPMV_ROWS;
     spmv_fetch(a, k, sub, row);
     pq += spmv_row(a, k, sub, beta, row);
   }
   const double t = block_sum<NW>(pq, sh_pq);
-  if (threadIdx.x == 0) a.part_pq[blockIdx.x] = t;
+  if (threadIdx.x == 0) a.part_pq[block] = t;
 }
 
 // x += alpha p, r -= alpha q, (z, p) = (D^-1 r, p); partials of r.z and r.r.
 __global__ void __launch_bounds__(NT) k_cg_update(CgArgs a, uint32_t it) {
   __shared__ double sh[NT / WAVE];
   __shared__ double2 sh2[NT / WAVE];
-  uint32_t k = blockIdx.x * NT + threadIdx.x;
+  const uint32_t block = row_block();
+  uint32_t k = block * NT + threadIdx.x;
   // the first elements are on their way while alpha is summed
   const uint32_t kr = min(k, a.m - 1u);
   const uint32_t done = a.scal->done;
@@ -340,8 +352,8 @@ __global__ void __launch_bounds__(NT) k_cg_update(CgArgs a, uint32_t it) {
   }
   const double2 t = block_sum2(rz, rr, sh2);
   if (threadIdx.x == 0) {
-    a.part_rz[blockIdx.x] = t.x;
-    a.part_rr[blockIdx.x] = t.y;
+    a.part_rz[block] = t.x;
+    a.part_rr[block] = t.y;
   }
 }
 
