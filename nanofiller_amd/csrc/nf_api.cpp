@@ -873,14 +873,10 @@ extern "C" int nf_set_option(nf_handle* h, int key, int64_t value) {
 // generation
 // ===========================================================================
 static int reset_generation(nf_handle* h) {
-  GenBuffers& b = h->gb;
-  HIPCHK(h, hipMemsetAsync(b.st, 0, sizeof(InstState) * b.n_inst, h->stream));
-  HIPCHK(h, hipMemsetAsync(b.ri, 0, sizeof(RoundInfo), h->stream));
-  fill_u32(b.ocount, 0u, b.total_cells, h->stream);
-  fill_u32((uint32_t*)b.ohl, 0u, b.total_cells, h->stream);
-  if (b.walk) fill_u32(b.fcountA, 0u, b.total_fine, h->stream);
+  h->gb.one_length = true;
+  for (const nf_params& p : h->params) h->gb.one_length = h->gb.one_length && p.len_law == NF_LEN_CONST;
+  launch_reset(h->gb, h->stream);
   HIPCHK(h, hipGetLastError());
-  HIPCHK(h, sync_stream(h->stream, "generation reset"));
   return NF_OK;
 }
 

@@ -44,6 +44,28 @@ __device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v, uint32_t* total) 
   return inc - v;
 }
 
+// Clears what a generation starts from.  A cell's longest rod: that of every
+// rod where all have one length.
+__global__ void __launch_bounds__(GEN_THREADS) k_reset(const InstDesc* __restrict__ desc, InstState* __restrict__ st,
+                                                       RoundInfo* __restrict__ ri, int n_inst,
+                                                       const uint32_t* __restrict__ cell_inst,
+                                                       uint32_t* __restrict__ ocount, float* __restrict__ ohl,
+                                                       float* __restrict__ phl, uint64_t ncells, bool one_length,
+                                                       uint32_t* __restrict__ fcount, uint64_t nfine) {
+  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (uint64_t)gridDim.x * blockDim.x;
+  for (uint64_t c = t; c < ncells; c += step) {
+    const float hl = one_length ? desc[cell_inst[c]].hl_max : 0.0f;
+    ocount[c] = 0u;
+    ohl[c] = hl;
+    phl[c] = hl;
+  }
+  for (uint64_t c = t; c < nfine; c += step) fcount[c] = 0u;
+  uint32_t* w = reinterpret_cast<uint32_t*>(st);
+  for (uint64_t k = t; k < (uint64_t)n_inst * (sizeof(InstState) / 4); k += step) w[k] = 0u;
+  w = reinterpret_cast<uint32_t*>(ri);
+  for (uint64_t k = t; k < sizeof(RoundInfo) / 4; k += step) w[k] = 0u;
+}
+
 // Plans the round: M per running instance, slot prefix, queue reset (the
 // first wave; lane l owns a contiguous chunk of instances), and clears the
 // per-cell proposal counts and longest proposals (the whole grid).
@@ -61,7 +83,7 @@ __global__ void __launch_bounds__(GEN_THREADS) k_ctl_begin(const InstDesc* __res
   for (uint64_t c = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; c < ncells;
        c += (uint64_t)gridDim.x * blockDim.x) {
     pcount[c] = 0u;
-    phl[c] = 0u;
+    if (phl != nullptr) phl[c] = 0u;
   }
   // and the lengths of the survivors' crossing lists
   for (uint64_t c = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; c < nfine; c += (uint64_t)gridDim.x * blockDim.x)
@@ -144,7 +166,7 @@ __global__ void __launch_bounds__(GEN_THREADS) k_gen(const InstDesc* __restrict_
     if (v == 1) {
       const uint32_t gc = d.cell_base + cell_of(d, r.P);
       srk[g] = atomicAdd(&pcount[gc], 1u);
-      atomicMax((unsigned int*)&phl[gc], __float_as_uint(r.P.w));
+      if (phl != nullptr) atomicMax((unsigned int*)&phl[gc], __float_as_uint(r.P.w));
       sP[g] = r.P;
       sD[g] = r.D;
       scell[g] = (int32_t)gc;
@@ -275,7 +297,7 @@ __global__ void __launch_bounds__(GEN_THREADS) k_commit(const InstDesc* __restri
         oR[2ull * dst] = P;
         oR[2ull * dst + 1u] = D;
       }
-      atomicMax((unsigned int*)&ohl[c], __float_as_uint(P.w));
+      if (ohl != nullptr) atomicMax((unsigned int*)&ohl[c], __float_as_uint(P.w));
     } else {
       // no slot: give the count back, so that once this kernel ends every
       // cell's count is at most its capacity (later passes of the other
@@ -360,6 +382,12 @@ static int gen_grid(uint64_t n) {
   return (int)b;
 }
 
+void launch_reset(GenBuffers& b, hipStream_t s) {
+  const uint64_t nfine = b.walk ? b.total_fine : 0;
+  hipLaunchKernelGGL(k_reset, dim3(gen_grid(std::max(b.total_cells, nfine))), dim3(GEN_THREADS), 0, s, b.desc, b.st, b.ri,
+                     b.n_inst, b.cell_inst, b.ocount, b.ohl, b.phl, b.total_cells, b.one_length, b.fcountA, nfine);
+}
+
 // One round.  ev (optional, 9 events) brackets the kernel classes.
 void launch_round(GenBuffers& b, int prec, int diag, hipStream_t s, hipEvent_t* ev) {
   const int n = b.n_inst;
@@ -367,13 +395,18 @@ void launch_round(GenBuffers& b, int prec, int diag, hipStream_t s, hipEvent_t* 
   // crossing lists, unless every pair within reach has to be tested
   const bool walk = b.walk && !b.tiles.test_all;
   const bool cells = b.cellwise || !walk;
+  // a cell's longest rod bounds the cell pairs only; of one length, the start's
+  // holds (an atomic per candidate at 30 G/s otherwise)
+  const bool track = cells && !b.one_length;
+  float* const phl = track ? b.phl : nullptr;
+  float* const ohl = track ? b.ohl : nullptr;
   hipLaunchKernelGGL(k_ctl_begin, dim3(gen_grid(std::max(b.total_cells, walk ? b.total_fine : 0))),
                      dim3(GEN_THREADS), 0, s, b.desc, b.st, b.ri, b.slot_base, b.queues, n, b.pcount,
-                     (uint32_t*)b.phl, (uint64_t)b.total_cells, b.fcountP, walk ? b.total_fine : (uint64_t)0);
+                     (uint32_t*)phl, (uint64_t)b.total_cells, b.fcountP, walk ? b.total_fine : (uint64_t)0);
   if (ev) (void)hipEventRecord(ev[1], s);
   hipLaunchKernelGGL(k_gen, dim3(gen_grid(b.T_cap + 1)), dim3(GEN_THREADS), 0, s, b.desc, b.st,
                      b.ri, b.slot_base, n, b.T_cap, b.sP, b.sD, b.scell, b.srk, b.surv, b.palive,
-                     b.pcount, b.phl);
+                     b.pcount, phl);
   if (ev) (void)hipEventRecord(ev[2], s);
   scan_u32(b.pcount, b.pstart, b.total_cells, b.scan_tmp, s);
   hipLaunchKernelGGL(k_scatter, dim3(gen_grid(b.T_cap)), dim3(GEN_THREADS), 0, s, b.ri, b.sP,
@@ -471,7 +504,7 @@ void launch_round(GenBuffers& b, int prec, int diag, hipStream_t s, hipEvent_t* 
   scan_u32(b.surv, b.srank, b.T_cap, b.scan_tmp, s);
   hipLaunchKernelGGL(k_commit, dim3(gen_grid(b.T_cap)), dim3(GEN_THREADS), 0, s, b.desc, b.st,
                      b.ri, b.slot_base, n, b.sP, b.sD, b.scell, b.surv, b.srank, b.bP, b.bD,
-                     b.ostart, b.ocount, b.ohl, b.oP, b.oD, b.oid, b.sdst, walk ? b.oR : (float4*)nullptr);
+                     b.ostart, b.ocount, ohl, b.oP, b.oD, b.oid, b.sdst, walk ? b.oR : (float4*)nullptr);
   if (walk) launch_enter(true, w, b.T_cap, s);
   if (ev) (void)hipEventRecord(ev[6], s);
   hipLaunchKernelGGL(k_ctl_end, dim3(1), dim3(WAVE), 0, s, b.desc, b.st, b.ri,

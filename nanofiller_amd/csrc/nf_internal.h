@@ -149,6 +149,7 @@ struct GenBuffers {
   uint32_t* ostart = nullptr;  // start slot of every cell
   uint32_t* ocount = nullptr;
   float* ohl = nullptr;        // max half length in the cell
+  bool one_length = false;     // every instance's rods have one length
   // accepted rods by id
   float4* bP = nullptr;
   float4* bD = nullptr;
@@ -398,6 +399,7 @@ size_t scan_tmp_words(uint64_t n);
 void fill_u32(uint32_t* p, uint32_t v, uint64_t n, hipStream_t s);
 
 // ---- launchers (nf_gen.hip) ----
+void launch_reset(GenBuffers& b, hipStream_t s);
 void launch_round(GenBuffers& b, int prec, int diag, hipStream_t s, hipEvent_t* ev);
 void launch_ctl_init(GenBuffers& b, hipStream_t s);
 
