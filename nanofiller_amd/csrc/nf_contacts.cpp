@@ -537,6 +537,7 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, Co
   c.n_contacts = total;
   c.cap_contacts = total;
   rc = NF_OK;
+  if (rc == NF_OK) rc = dalloc(h, &c.I, total);
   if (rc == NF_OK) rc = dalloc(h, &c.J, total);
   if (rc == NF_OK) rc = dalloc(h, &c.gap, total);
   if (rc == NF_OK) rc = dalloc(h, &c.gap64, total);
@@ -551,11 +552,11 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, Co
   fill_u32(c.cnt, 0u, (uint64_t)n + 1, s);
   launch_csr_count(appI, total, c.cnt, s);
   scan_u32(c.cnt, c.rowptr, n, tmp, s);
-  launch_csr_scatter(appI, appJ, appG, appG64, appImg, total, c.rowptr, c.cnt, c.J, c.gap, c.gap64,
+  launch_csr_scatter(appI, appJ, appG, appG64, appImg, total, c.rowptr, c.cnt, c.I, c.J, c.gap, c.gap64,
                      c.img, s);
   hipEventRecord(ev[4], s);
   launch_row_sort(c.rowptr, n, c.J, c.gap, c.gap64, c.img, s);
-  launch_contact_area(P, D, n, c.rowptr, c.J, c.img, p.box, gap, c.area, s);
+  launch_contact_area(P, D, total, c.I, c.J, c.img, p.box, gap, c.area, s);
   hipEventRecord(ev[5], s);
   std::copy(pinned->ctr, pinned->ctr + 6, h->cb_stats);
   HIPCHK(h, sync_stream(s, "contact list"));
@@ -739,7 +740,7 @@ int hist_run(nf_handle* h, const HistPlan& pl, const double* edges, double* dE,
   const InstDesc& d = h->desc[h->post_inst];
   const uint32_t n = h->n_rods[h->post_inst];
   if (e == hipSuccess && n) {
-    launch_hist(h->gb.bP + d.rod_off, h->gb.bD + d.rod_off, n, pl.mutual ? h->cb.rowptr : nullptr,
+    launch_hist(h->gb.bP + d.rod_off, h->gb.bD + d.rod_off, n, pl.mutual ? h->cb.n_contacts : 0, h->cb.I,
                 h->cb.J, dE, dE + (nb + 1), pl.npb ? dE + 2 * (nb + 1) : nullptr, nb, pl.npb, pl.ntb,
                 pl.axis, h->params[h->post_inst].box[pl.axis], pl.mu, dOut, s);
     e = hipGetLastError();

@@ -211,6 +211,7 @@ struct ContactBuffers {
   uint32_t ncells = 0;
   // contacts
   uint32_t* cnt = nullptr;     // N
+  uint32_t* I = nullptr;       // n_contacts: row of every contact
   uint32_t* rowptr = nullptr;  // N + 1
   uint32_t* J = nullptr;
   float* gap = nullptr;
@@ -461,16 +462,15 @@ void launch_row_sort(const uint32_t* rowptr, uint32_t n, uint32_t* J, float* gap
                      int32_t* img, hipStream_t s);
 // Contact area S (contact_area_f64) of every contact of the CSR, rod J at
 // its image; rlim is the contact gap.
-void launch_contact_area(const float4* P, const float4* D, uint32_t n, const uint32_t* rowptr,
-                         const uint32_t* J, const int32_t* img, const double box[3], double rlim,
-                         double* area, hipStream_t s);
+void launch_contact_area(const float4* P, const float4* D, uint64_t c, const uint32_t* I, const uint32_t* J,
+                         const int32_t* img, const double box[3], double rlim, double* area, hipStream_t s);
 // CSR over I from the unsorted contact list: per-row counts, then scatter
 // (rowptr from scan_u32 of the counts in between).
 void launch_csr_count(const uint32_t* I, uint64_t c, uint32_t* cnt, hipStream_t s);
 void launch_csr_scatter(const uint32_t* I, const uint32_t* J, const float* gap, const double* gap64,
                         const int32_t* img, uint64_t c, const uint32_t* rowptr, uint32_t* cnt,
-                        uint32_t* oJ, float* ogap, double* ogap64, int32_t* oimg, hipStream_t s);
-void launch_hist(const float4* P, const float4* D, uint32_t n, const uint32_t* rowptr,
+                        uint32_t* oI, uint32_t* oJ, float* ogap, double* ogap64, int32_t* oimg, hipStream_t s);
+void launch_hist(const float4* P, const float4* D, uint32_t n, uint64_t n_contacts, const uint32_t* I,
                  const uint32_t* J, const double* edges_p, const double* edges_m,
                  const double* edges_t, int nb, int npb, int ntb, int axis, double L,
                  const double* mu, unsigned long long* out, hipStream_t s);

@@ -244,32 +244,28 @@ void launch_row_sort(const uint32_t* rowptr, uint32_t n, uint32_t* J, float* gap
                      gap64, img);
 }
 
-// Contact area of every contact, one thread per row (rows are short).
-__global__ void k_contact_area(const float4* __restrict__ P, const float4* __restrict__ D, uint32_t n,
-                               const uint32_t* __restrict__ rowptr, const uint32_t* __restrict__ J,
+// Contact area of every contact, one thread per contact: a thread per row had
+// most lanes of a wave wait for the few rows that hold any (215,000 contacts of
+// 4M rods 104 us, now 24; 46,000 of 500,000 rods 23 and 7, 2,000 rods 11 and 4).
+__global__ void k_contact_area(const float4* __restrict__ P, const float4* __restrict__ D, uint64_t c,
+                               const uint32_t* __restrict__ I, const uint32_t* __restrict__ J,
                                const int32_t* __restrict__ img, double bx, double by, double bz,
                                double rlim, double* __restrict__ area) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const uint32_t b = rowptr[i], e = rowptr[i + 1];
-    if (b == e) continue;
-    const float4 P1 = P[i], D1 = D[i];
-    for (uint32_t k = b; k < e; ++k) {
-      const uint32_t j = J[k];
-      const int32_t m = img[k];
-      const double sx = (double)(int)(int8_t)(m & 0xFF) * bx;
-      const double sy = (double)(int)(int8_t)((m >> 8) & 0xFF) * by;
-      const double sz = (double)(int)(int8_t)((m >> 16) & 0xFF) * bz;
-      area[k] = contact_area_f64(P1, D1, P[j], D[j], sx, sy, sz, rlim);
-    }
+  for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < c; k += (uint64_t)gridDim.x * blockDim.x) {
+    const uint32_t i = I[k], j = J[k];
+    const int32_t m = img[k];
+    const double sx = (double)(int)(int8_t)(m & 0xFF) * bx;
+    const double sy = (double)(int)(int8_t)((m >> 8) & 0xFF) * by;
+    const double sz = (double)(int)(int8_t)((m >> 16) & 0xFF) * bz;
+    area[k] = contact_area_f64(P[i], D[i], P[j], D[j], sx, sy, sz, rlim);
   }
 }
 
-void launch_contact_area(const float4* P, const float4* D, uint32_t n, const uint32_t* rowptr,
-                         const uint32_t* J, const int32_t* img, const double box[3], double rlim,
-                         double* area, hipStream_t s) {
-  if (n == 0) return;
-  hipLaunchKernelGGL(k_contact_area, dim3(grid_for(n, 256)), dim3(256), 0, s, P, D, n, rowptr, J, img,
-                     box[0], box[1], box[2], rlim, area);
+void launch_contact_area(const float4* P, const float4* D, uint64_t c, const uint32_t* I, const uint32_t* J,
+                         const int32_t* img, const double box[3], double rlim, double* area, hipStream_t s) {
+  if (c == 0) return;
+  hipLaunchKernelGGL(k_contact_area, dim3(grid_for(c, 256)), dim3(256), 0, s, P, D, c, I, J, img, box[0], box[1],
+                     box[2], rlim, area);
 }
 
 // CSR over I from the unsorted contact list (the pair pass appends in any
@@ -285,12 +281,13 @@ __global__ void k_csr_scatter(const uint32_t* __restrict__ I, const uint32_t* __
                               const float* __restrict__ gap, const double* __restrict__ gap64,
                               const int32_t* __restrict__ img, uint64_t c,
                               const uint32_t* __restrict__ rowptr, uint32_t* __restrict__ cnt,
-                              uint32_t* __restrict__ oJ, float* __restrict__ ogap,
+                              uint32_t* __restrict__ oI, uint32_t* __restrict__ oJ, float* __restrict__ ogap,
                               double* __restrict__ ogap64, int32_t* __restrict__ oimg) {
   for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < c;
        k += (uint64_t)gridDim.x * blockDim.x) {
     const uint32_t i = I[k];
     const uint32_t pos = rowptr[i] + atomicSub(&cnt[i], 1u) - 1u;
+    oI[pos] = i;
     oJ[pos] = J[k];
     ogap[pos] = gap[k];
     ogap64[pos] = gap64[k];
@@ -305,10 +302,10 @@ void launch_csr_count(const uint32_t* I, uint64_t c, uint32_t* cnt, hipStream_t 
 
 void launch_csr_scatter(const uint32_t* I, const uint32_t* J, const float* gap, const double* gap64,
                         const int32_t* img, uint64_t c, const uint32_t* rowptr, uint32_t* cnt,
-                        uint32_t* oJ, float* ogap, double* ogap64, int32_t* oimg, hipStream_t s) {
+                        uint32_t* oI, uint32_t* oJ, float* ogap, double* ogap64, int32_t* oimg, hipStream_t s) {
   if (c == 0) return;
   hipLaunchKernelGGL(k_csr_scatter, dim3(grid_for(c, 256)), dim3(256), 0, s, I, J, gap, gap64, img, c,
-                     rowptr, cnt, oJ, ogap, ogap64, oimg);
+                     rowptr, cnt, oI, oJ, ogap, ogap64, oimg);
 }
 
 // ---------------------------------------------------------------------------
@@ -605,7 +602,8 @@ void launch_vdw(const float4* P, const float4* D, uint32_t n, const uint32_t* ro
 // 13-76) and statKernel_MUT_ANGLE_weightedFloat (inc/statKernel_MUT.h:
 // 26-131) with their uint32/float accumulators.  What a block adds to the
 // result bounds small packings, so there are few blocks: 300,000 rods in 1024
-// of 256 threads 29 + 25 us, in 256 of 1024 15 + 12 (4M: 69 + 73, 58 + 66).
+// of 256 threads 29 + 25 us, in 256 of 1024 15 + 12 (4M: 69 + 73, 58 + 66); the
+// mutual angles by contact instead of by row 6 (13).
 // ---------------------------------------------------------------------------
 constexpr int HIST_THREADS = 1024;
 constexpr int HIST_BLOCKS = 256;
@@ -678,28 +676,22 @@ __global__ void __launch_bounds__(HIST_THREADS) k_hist_rods(const float4* __rest
     if (h2[k]) atomicAdd(&out[3 * h.nb + k], (unsigned long long)h2[k]);
 }
 
-// Mutual angle of contact pairs: one thread per row I of the contact CSR.
-__global__ void __launch_bounds__(HIST_THREADS) k_hist_mut(const float4* __restrict__ D, uint32_t n,
-                                                           const uint32_t* __restrict__ rowptr,
+// Mutual angle of contact pairs, one thread per contact.
+__global__ void __launch_bounds__(HIST_THREADS) k_hist_mut(const float4* __restrict__ D, uint64_t c,
+                                                           const uint32_t* __restrict__ I,
                                                            const uint32_t* __restrict__ J,
                                                            HistArg h,
                                                            unsigned long long* __restrict__ out) {
   __shared__ uint32_t hm[HIST_MAX_BINS];
   for (int k = threadIdx.x; k < HIST_MAX_BINS; k += blockDim.x) hm[k] = 0;
   __syncthreads();
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const uint32_t b = rowptr[i], e = rowptr[i + 1];
-    if (b == e) continue;
-    const float4 a = D[i];
-    const double ax = a.x, ay = a.y, az = a.z;
+  for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < c; k += (uint64_t)gridDim.x * blockDim.x) {
+    const float4 a = D[I[k]], b = D[J[k]];
+    const double ax = a.x, ay = a.y, az = a.z, bx = b.x, by = b.y, bz = b.z;
     const double na = sqrt_cr((ax * ax + ay * ay) + az * az);
-    for (uint32_t k = b; k < e; ++k) {
-      const float4 c = D[J[k]];
-      const double bx = c.x, by = c.y, bz = c.z;
-      const double nbv = sqrt_cr((bx * bx + by * by) + bz * bz);
-      const double dv = fabs((ax * bx + ay * by) + az * bz) / (na * nbv);
-      atomicAdd(&hm[edge_bin(dv, h.em, h.nb)], 1u);
-    }
+    const double nbv = sqrt_cr((bx * bx + by * by) + bz * bz);
+    const double dv = fabs((ax * bx + ay * by) + az * bz) / (na * nbv);
+    atomicAdd(&hm[edge_bin(dv, h.em, h.nb)], 1u);
   }
   __syncthreads();
   for (int k = threadIdx.x; k < h.nb; k += blockDim.x)
@@ -707,7 +699,7 @@ __global__ void __launch_bounds__(HIST_THREADS) k_hist_mut(const float4* __restr
 }
 
 // out layout: [centre nb][polar nb][mutual nb][phitheta npb*ntb]
-void launch_hist(const float4* P, const float4* D, uint32_t n, const uint32_t* rowptr,
+void launch_hist(const float4* P, const float4* D, uint32_t n, uint64_t n_contacts, const uint32_t* I,
                  const uint32_t* J, const double* edges_p, const double* edges_m,
                  const double* edges_t, int nb, int npb, int ntb, int axis, double L,
                  const double* mu, unsigned long long* out, hipStream_t s) {
@@ -724,9 +716,9 @@ void launch_hist(const float4* P, const float4* D, uint32_t n, const uint32_t* r
   for (int a = 0; a < 3; ++a) h.mu[a] = mu[a];
   const int blocks = std::min(grid_for(n, HIST_THREADS), HIST_BLOCKS);
   hipLaunchKernelGGL(k_hist_rods, dim3(blocks), dim3(HIST_THREADS), 0, s, P, D, n, h, out);
-  if (rowptr)
-    hipLaunchKernelGGL(k_hist_mut, dim3(blocks), dim3(HIST_THREADS), 0, s, D, n, rowptr, J, h,
-                       out);
+  if (I && n_contacts)
+    hipLaunchKernelGGL(k_hist_mut, dim3(std::min(grid_for(n_contacts, HIST_THREADS), HIST_BLOCKS)), dim3(HIST_THREADS), 0,
+                       s, D, n_contacts, I, J, h, out);
 }
 
 // ---------------------------------------------------------------------------
