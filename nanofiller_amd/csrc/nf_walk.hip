@@ -529,7 +529,10 @@ __global__ void __launch_bounds__(WAVE, 4) k_walk(WalkArgs a) {
       float4 P2[4], D2[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const float4* e = rods + 2u * (ent[u] & ENT_MASK);
+        // contacts: each pair from the rod further on in the cell list, so the
+        // others need not be fetched (the probe's own line is at hand)
+        const uint32_t r = ent[u] & ENT_MASK;
+        const float4* e = rods + 2u * (CNT ? min(r, k) : r);
         P2[u] = e[0];
         D2[u] = e[1];
       }
@@ -553,7 +556,6 @@ __global__ void __launch_bounds__(WAVE, 4) k_walk(WalkArgs a) {
                  line_apart_from(u1, P2[u].x - P1.x, P2[u].y - P1.y, P2[u].z - P1.z, D1, D2[u], lb) < 0.0f;
         // same-round pass: only an earlier slot rejects the probe
         if (MODE == PM_GEN_NEW) may[u] = may[u] && __float_as_uint(D2[u].w) < slot;
-        // contacts: each pair from the rod further on in the cell list
         if (CNT) may[u] = may[u] && (ent[u] & ENT_MASK) < k;
       }
       if (CNT)
