@@ -11,8 +11,9 @@ FP64 re-check band; `value` is accepted rods/s over the timed steps.
 The same JSON line carries:
   * fp64_plain: the same packing by the plain FP64 path; identity of the two
     packings and of their contact lists;
-  * roofline: the reject-vs-accepted kernel, algorithmic tile bytes per launch
-    over its HIP-event time per launch (one extra, profiled generation);
+  * roofline: the reject-vs-accepted kernel, bytes of the list entries and rods
+    that it reads per launch over its HIP-event time (one extra, profiled
+    generation);
   * batch: 256 independent packings of uneven size (2k-200k rods) in one
     batched FP32 + recheck generation, against the same 256 packings made one
     at a time by the plain FP64 path, with identical packings;
@@ -50,7 +51,7 @@ K_OLD = nf.KERNEL_CLASSES.index("reject_old")
 K_NEW = nf.KERNEL_CLASSES.index("reject_new")
 
 
-TRAFFIC_SUMMARY = os.path.join(ROOT, "profiles", "k_pair_generate_cfg2_500k_hbm_counters.md")
+TRAFFIC_SUMMARY = os.path.join(ROOT, "profiles", "generate_500k_hbm_counters.md")
 VALU_SUMMARY = os.path.join(ROOT, "profiles", "pair_kernels_valu_counters.md")
 # VALU issue roof: a wave64 VALU instruction occupies a 16-lane SIMD for 4
 # cycles; 256 CUs x 4 SIMDs at the 2.4 GHz peak engine clock
@@ -65,7 +66,7 @@ def profiled_traffic():
 
     try:
         with open(TRAFFIC_SUMMARY) as f:
-            m = re.search(r"traffic_bytes_per_launch k_pair<0, 1>: (\d+)", f.read())
+            m = re.search(r"traffic_bytes_per_launch k_walk<0, 1>: (\d+)", f.read())
         return float(m.group(1)) if m else None
     except OSError:
         return None
@@ -170,9 +171,9 @@ def leg_main(a, out: dict) -> None:
         "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
         "frac": achieved / HBM_PEAK_GBS, "traffic": profiled_traffic(),
         "traffic_source": os.path.relpath(TRAFFIC_SUMMARY, ROOT),
-        "kernel": "k_pair<reject vs accepted, FP32+recheck>",
+        "kernel": "k_walk<reject vs accepted, FP32+recheck>",
         "bytes_per_launch": sp.tile_bytes / launches, "avg_launch_ms": k_old / launches,
-        "launches": launches, "valu": valu_roof("k_pair<0, 1> 500k", k_old / launches),
+        "launches": launches, "valu": valu_roof("k_walk<0, 1> 500k", k_old / launches),
     }
     out["extra"]["fp32_recheck"] = {
         "tile_options": tiles,
