@@ -729,7 +729,7 @@ int hist_prepare(nf_handle* h, const nf_hist_spec* spec, bool want_mutual, bool 
 
 int hist_run(nf_handle* h, const HistPlan& pl, const double* edges, double* dE,
              unsigned long long* dOut, int64_t* out_centre, int64_t* out_polar, int64_t* out_mutual,
-             int64_t* out_phitheta) {
+             int64_t* out_phitheta, bool may_allocate) {
   hipStream_t s = h->stream;
   const int nb = pl.nb;
   hipError_t e = hipMemcpyAsync(dE, edges, sizeof(double) * pl.n_edges, hipMemcpyHostToDevice, s);
@@ -753,7 +753,15 @@ int hist_run(nf_handle* h, const HistPlan& pl, const double* edges, double* dE,
   const HostPart parts[4] = {part(out_centre, 0, nb), part(out_polar, nb, nb),
                              part(pl.mutual ? out_mutual : nullptr, 2 * (size_t)nb, nb),
                              part(pl.npb ? out_phitheta : nullptr, 3 * (size_t)nb, (size_t)pl.npb * pl.ntb)};
-  const hipError_t w = to_host(h, parts, 4);  // (waits for the upload of `edges` too)
+  hipError_t w = hipSuccess;
+  if (may_allocate || h->pin) {
+    w = to_host(h, parts, 4);  // (waits for the upload of `edges` too)
+  } else {
+    for (const HostPart& q : parts)
+      if (w == hipSuccess && q.bytes) w = hipMemcpyAsync(q.dst, q.src, q.bytes, hipMemcpyDeviceToHost, s);
+    const hipError_t sy = sync_stream(s, "histograms");
+    if (w == hipSuccess) w = sy;
+  }
   if (e == hipSuccess) e = w;
   if (e != hipSuccess) return fail(h, NF_E_HIP, std::string("histograms: ") + hipGetErrorString(e));
   return NF_OK;
@@ -773,7 +781,7 @@ extern "C" int nf_histograms(nf_handle* h, const nf_hist_spec* spec, int64_t* ou
   rc = dalloc(h, &dE, pl.n_edges);
   if (rc == NF_OK) rc = dalloc(h, &dOut, pl.n_out);
   if (rc == NF_OK)
-    rc = hist_run(h, pl, edges, dE, dOut, out_centre, out_polar, out_mutual, out_phitheta);
+    rc = hist_run(h, pl, edges, dE, dOut, out_centre, out_polar, out_mutual, out_phitheta, true);
   dfree(h, dE);
   dfree(h, dOut);
   return rc;

@@ -183,6 +183,7 @@ struct OnDevice {
 }  // namespace
 
 hipError_t to_host(nf_handle* h, const HostPart* parts, size_t n_parts) {
+  std::lock_guard<std::mutex> lock(h->pin_mu);
   OnDevice on(h->device);
   hipError_t e = hipSuccess;
   const bool done = staged(h, parts, n_parts, [&](size_t i, size_t off, size_t bytes, char* to) {
@@ -197,6 +198,7 @@ hipError_t to_host(nf_handle* h, const HostPart* parts, size_t n_parts) {
 }
 
 hipError_t rods_to_host(nf_handle* h, const float4* P, const float4* D, uint32_t n, float* rods) {
+  std::lock_guard<std::mutex> lock(h->pin_mu);
   OnDevice on(h->device);
   const size_t rod = 8 * sizeof(float);
   const HostPart part = {rods, nullptr, n * rod};
@@ -223,6 +225,7 @@ hipError_t rods_to_host(nf_handle* h, const float4* P, const float4* D, uint32_t
 
 hipError_t rods_to_device(nf_handle* h, const float* rods, uint32_t n, float4* P, float4* D) {
   if (n == 0) return hipSuccess;
+  std::lock_guard<std::mutex> lock(h->pin_mu);
   OnDevice on(h->device);
   const size_t rod = 8 * sizeof(float);
   // slots of the block in turn, filled while the one before is on its way

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <map>
+#include <mutex>
 #include <string>
 #include <unordered_map>
 #include <vector>
@@ -61,7 +62,9 @@ struct nf_handle {
   uint64_t contact_hint = 0;                      // contacts found by the last call (append capacity)
   nf_network_info net_info = {};
   std::vector<uint32_t> reduce_ids;  // old id of every rod kept by the last nf_reduce
-  // pinned host memory of the handle, made when first needed (nf_copy.cpp)
+  // pinned host memory of the handle, made when first needed (nf_copy.cpp);
+  // pin_mu: two threads may read results of one handle at a time
+  std::mutex pin_mu;
   char* pin = nullptr;
   size_t pin_bytes = 0;
   hipEvent_t pin_ev[8] = {};
@@ -132,9 +135,10 @@ int hist_prepare(nf_handle* h, const nf_hist_spec* spec, bool want_mutual, bool 
                  double* edges, HistPlan* plan);
 // Uploads the edges to dE[n_edges], clears dOut[n_out], counts, and copies the
 // counts to the caller's host arrays (any may be NULL); waits for the stream.
+// Without may_allocate no memory is allocated, pinned memory neither.
 int hist_run(nf_handle* h, const HistPlan& pl, const double* edges, double* dE,
              unsigned long long* dOut, int64_t* out_centre, int64_t* out_polar, int64_t* out_mutual,
-             int64_t* out_phitheta);
+             int64_t* out_phitheta, bool may_allocate);
 
 template <class T>
 int dalloc(nf_handle* h, T** p, size_t count) {

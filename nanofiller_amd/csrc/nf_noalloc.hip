@@ -82,5 +82,5 @@ extern "C" int nf_histograms_noalloc(nf_handle* h, const nf_hist_spec* spec, int
   if (rc != NF_OK) return rc;
   return hist_run(h, pl, edges, (double*)(base + NOALLOC_EDGES_OFF),
                   (unsigned long long*)(base + NOALLOC_OUT_OFF), out_centre, out_polar, out_mutual,
-                  out_phitheta);
+                  out_phitheta, false);
 }

@@ -50,3 +50,20 @@ def test_arrays_of_several_sizes_arrive_whole(n, gap):
         sums = np.add.reduceat(net["val"], net["row_ptr"][:-1].astype(np.int64))[:n]
         diag = net["val"][net["col"] == np.repeat(np.arange(n + 2), np.diff(net["row_ptr"].astype(np.int64)))][:n]
         np.testing.assert_allclose(sums, 0.0, atol=1e-12 * np.abs(diag).max())
+
+
+def test_two_threads_read_one_packing():
+    from concurrent.futures import ThreadPoolExecutor
+
+    p = nf.normalize(nf.default_params(box=(4.0, 4.0, 4.0), n_rods=30000, len=0.2, radius=0.003, seed=11,
+                                       contact_gap=0.004))
+    with nf.Packing(p) as pk:
+        pk.generate()
+        rods = pk.rods()
+        c = pk.contacts(0.004)
+        gaps = pk.contact_gap64(c.n)
+        with ThreadPoolExecutor(2) as ex:
+            jobs = [(ex.submit(pk.rods), ex.submit(pk.contact_gap64, c.n)) for _ in range(20)]
+            for a, b in jobs:
+                np.testing.assert_array_equal(a.result().view(np.uint32), rods.view(np.uint32))
+                np.testing.assert_array_equal(b.result().view(np.uint64), gaps.view(np.uint64))
