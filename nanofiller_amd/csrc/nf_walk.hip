@@ -332,7 +332,7 @@ __global__ void __launch_bounds__(WAVE, 4) k_walk(WalkArgs a) {
     ln = a.cnt.ln;
     lb = -1.0f - ln.slack;
   }
-  unsigned long long bytes = 0;
+  uint32_t seen = 0;  // contacts: entries read
   bool started = false;
   uint32_t kills = 0;
   auto flush_queue = [&]() {
@@ -360,7 +360,7 @@ __global__ void __launch_bounds__(WAVE, 4) k_walk(WalkArgs a) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, WAVE));
     if (CNT) {
-      const unsigned long long wb = wave_sum_u64(bytes);
+      const unsigned long long wb = 36ull * wave_sum_u64(seen);
       if (lane == 0u) {
         if (wt) atomicAdd(&a.cnt.ctr[0], wt);
         if (wr) atomicAdd(&a.cnt.ctr[1], wr);
@@ -559,7 +559,7 @@ __global__ void __launch_bounds__(WAVE, 4) k_walk(WalkArgs a) {
         if (CNT) may[u] = may[u] && (ent[u] & ENT_MASK) < k;
       }
       if (CNT)
-        bytes += 36ull * min(m, 4u);
+        seen += min(m, 4u);
       else
         acc.tests += min(m, 4u);
       pos += 4u;
