@@ -144,7 +144,7 @@ __global__ void __launch_bounds__(GEN_THREADS) k_gen(const InstDesc* __restrict_
                                                      const InstState* __restrict__ st,
                                                      const RoundInfo* __restrict__ ri,
                                                      const uint32_t* __restrict__ slot_base,
-                                                     int n_inst, uint64_t T_cap,
+                                                     int n_inst,
                                                      float4* __restrict__ sP, float4* __restrict__ sD,
                                                      int32_t* __restrict__ scell,
                                                      uint32_t* __restrict__ srk,
@@ -153,11 +153,10 @@ __global__ void __launch_bounds__(GEN_THREADS) k_gen(const InstDesc* __restrict_
                                                      uint32_t* __restrict__ pcount,
                                                      float* __restrict__ phl) {
   const uint32_t T = ri->T;
-  for (uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; g <= T_cap;
-       g += (uint64_t)gridDim.x * blockDim.x) {
-    surv[g] = 0;
-    if (g < T_cap) palive[g] = 0;  // the survivors' scan reads all T_cap flags
-    if (g >= T) continue;
+  // (flags of all T slots: the scans read no further)
+  for (uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; g < T; g += (uint64_t)gridDim.x * blockDim.x) {
+    surv[g] = 0u;
+    palive[g] = 0u;
     const int inst = find_inst(slot_base, n_inst, (uint32_t)g);
     const InstDesc& d = desc[inst];
     const uint32_t slot = (uint32_t)g - slot_base[inst];
@@ -404,8 +403,8 @@ void launch_round(GenBuffers& b, int prec, int diag, hipStream_t s, hipEvent_t* 
                      dim3(GEN_THREADS), 0, s, b.desc, b.st, b.ri, b.slot_base, b.queues, n, b.pcount,
                      (uint32_t*)phl, (uint64_t)b.total_cells, b.fcountP, walk ? b.total_fine : (uint64_t)0);
   if (ev) (void)hipEventRecord(ev[1], s);
-  hipLaunchKernelGGL(k_gen, dim3(gen_grid(b.T_cap + 1)), dim3(GEN_THREADS), 0, s, b.desc, b.st,
-                     b.ri, b.slot_base, n, b.T_cap, b.sP, b.sD, b.scell, b.srk, b.surv, b.palive,
+  hipLaunchKernelGGL(k_gen, dim3(gen_grid(b.T_cap)), dim3(GEN_THREADS), 0, s, b.desc, b.st,
+                     b.ri, b.slot_base, n, b.sP, b.sD, b.scell, b.srk, b.surv, b.palive,
                      b.pcount, phl);
   if (ev) (void)hipEventRecord(ev[2], s);
   scan_u32(b.pcount, b.pstart, b.total_cells, b.scan_tmp, s);
@@ -470,7 +469,7 @@ void launch_round(GenBuffers& b, int prec, int diag, hipStream_t s, hipEvent_t* 
   // stage 2: survivors vs higher-priority survivors, over the survivors
   // compacted per cell (a cell's longest rod stays that of all its
   // proposals: a bound, as the stencil walk needs)
-  scan_u32(b.palive, b.aidx, b.T_cap, b.scan_tmp, s);
+  scan_u32(b.palive, b.aidx, b.T_cap, b.scan_tmp, s, &b.ri->T);
   hipLaunchKernelGGL(k_alive_scatter, dim3(gen_grid(std::max(b.T_cap, b.total_cells + 1))),
                      dim3(GEN_THREADS), 0, s, b.pstart, b.pP, b.pD, b.pslot, b.palive, b.aidx, b.aP,
                      b.aD, b.aslot, b.astart, b.acount, b.surv, (uint64_t)b.total_cells, walk ? b.aR : (float4*)nullptr);
@@ -501,7 +500,7 @@ void launch_round(GenBuffers& b, int prec, int diag, hipStream_t s, hipEvent_t* 
   }
   if (cells) launch_pair(PM_GEN_NEW, prec, a, s, &b.tiles);
   if (ev) (void)hipEventRecord(ev[5], s);
-  scan_u32(b.surv, b.srank, b.T_cap, b.scan_tmp, s);
+  scan_u32(b.surv, b.srank, b.T_cap, b.scan_tmp, s, &b.ri->T);
   hipLaunchKernelGGL(k_commit, dim3(gen_grid(b.T_cap)), dim3(GEN_THREADS), 0, s, b.desc, b.st,
                      b.ri, b.slot_base, n, b.sP, b.sD, b.scell, b.surv, b.srank, b.bP, b.bD,
                      b.ostart, b.ocount, ohl, b.oP, b.oD, b.oid, b.sdst, walk ? b.oR : (float4*)nullptr);

@@ -395,7 +395,8 @@ struct SegCrossArgs {
 };
 
 // ---- launchers (nf_scan.hip) ----
-void scan_u32(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* tmp, hipStream_t s);
+void scan_u32(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* tmp, hipStream_t s,
+              const uint32_t* limit = nullptr);
 size_t scan_tmp_words(uint64_t n);
 void fill_u32(uint32_t* p, uint32_t v, uint64_t n, hipStream_t s);
 

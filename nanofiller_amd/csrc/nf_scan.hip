@@ -68,9 +68,17 @@ __device__ __forceinline__ void scan_load(const uint32_t* __restrict__ in, uint6
   }
 }
 
-__global__ void __launch_bounds__(SCAN_THREADS) k_scan_tiles(const uint32_t* __restrict__ in,
-                                                             uint64_t n, bool wide, uint32_t* __restrict__ sums) {
+// Elements that count: all, or as many as the device says (limit).
+__device__ __forceinline__ uint64_t scan_length(uint64_t n, const uint32_t* limit) {
+  return limit != nullptr && *limit < n ? *limit : n;
+}
+
+__global__ void __launch_bounds__(SCAN_THREADS) k_scan_tiles(const uint32_t* __restrict__ in, uint64_t n,
+                                                             const uint32_t* limit, bool wide,
+                                                             uint32_t* __restrict__ sums) {
   __shared__ uint32_t sm[SCAN_THREADS / WAVE];
+  n = scan_length(n, limit);
+  if ((uint64_t)blockIdx.x * SCAN_TILE >= n) return;
   const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE + (uint64_t)threadIdx.x * SCAN_ITEMS;
   uint32_t v[SCAN_ITEMS], s = 0;
   scan_load(in, base, n, wide, v);
@@ -83,7 +91,9 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_tiles(const uint32_t* __r
 
 __global__ void __launch_bounds__(SCAN_THREADS) k_scan_sums(uint32_t* __restrict__ sums,
                                                             uint32_t nt, uint32_t* __restrict__ out,
-                                                            uint64_t n) {
+                                                            uint64_t n, const uint32_t* limit) {
+  n = scan_length(n, limit);
+  nt = min(nt, (uint32_t)((n + SCAN_TILE - 1) / SCAN_TILE));
   __shared__ uint32_t sm[SCAN_THREADS / WAVE];
   __shared__ uint32_t dummy[SCAN_THREADS];
   uint32_t carry = 0;
@@ -103,9 +113,15 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_sums(uint32_t* __restrict
 // SUMMED: sums holds the exclusive prefix of the tile sums, else the sums.
 // (in and out may be one array: a thread reads its elements before it writes.)
 template <bool SUMMED>
-__global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(const uint32_t* in, uint64_t n, bool wide,
-                                                             const uint32_t* __restrict__ sums, uint32_t* out) {
+__global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(const uint32_t* in, uint64_t n, const uint32_t* limit,
+                                                             bool wide, const uint32_t* __restrict__ sums,
+                                                             uint32_t* out) {
   __shared__ uint32_t sm[SCAN_THREADS / WAVE], sp[SCAN_THREADS / WAVE];
+  n = scan_length(n, limit);
+  if ((uint64_t)blockIdx.x * SCAN_TILE >= n) {
+    if (n == 0 && blockIdx.x == 0 && threadIdx.x == 0) out[0] = 0u;
+    return;
+  }
   const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE + (uint64_t)threadIdx.x * SCAN_ITEMS;
   uint32_t v[SCAN_ITEMS], s = 0, before = 0;
   scan_load(in, base, n, wide, v);
@@ -119,7 +135,7 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(const uint32_t* in,
     lead = sums[blockIdx.x];
   } else {
     block_excl_scan(before, sp, &lead);
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = lead + tot;
+    if (blockIdx.x == (n - 1) / SCAN_TILE && threadIdx.x == 0) out[n] = lead + tot;
   }
   run += lead;
 #pragma unroll
@@ -187,24 +203,27 @@ __global__ void __launch_bounds__(SCAN1_THREADS) k_scan_one(const uint32_t* __re
 size_t scan_tmp_words(uint64_t n) { return (size_t)((n + SCAN_TILE - 1) / SCAN_TILE) + 1; }
 
 // out[0..n) = exclusive prefix of in, out[n] = total.  in and out may alias.
-void scan_u32(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* tmp, hipStream_t s) {
+// limit (optional, device): a smaller n that only the device knows; what lies
+// past it is neither read (but by the one workgroup of a short array) nor
+// written to any purpose.
+void scan_u32(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* tmp, hipStream_t s, const uint32_t* limit) {
   if (n > 0 && n <= SCAN1_MAX) {
     hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(SCAN1_THREADS), 0, s, in, n, out);
     return;
   }
   const uint32_t nt = (uint32_t)((n + SCAN_TILE - 1) / SCAN_TILE);
   if (nt == 0) {
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SCAN_THREADS), 0, s, tmp, 0u, out, (uint64_t)0);
+    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SCAN_THREADS), 0, s, tmp, 0u, out, (uint64_t)0, nullptr);
     return;
   }
   const bool wide = (((uintptr_t)in | (uintptr_t)out) & 15u) == 0;
-  hipLaunchKernelGGL(k_scan_tiles, dim3(nt), dim3(SCAN_THREADS), 0, s, in, n, wide, tmp);
+  hipLaunchKernelGGL(k_scan_tiles, dim3(nt), dim3(SCAN_THREADS), 0, s, in, n, limit, wide, tmp);
   if (nt <= SUMS_MAX) {
-    hipLaunchKernelGGL(k_scan_apply<false>, dim3(nt), dim3(SCAN_THREADS), 0, s, in, n, wide, tmp, out);
+    hipLaunchKernelGGL(k_scan_apply<false>, dim3(nt), dim3(SCAN_THREADS), 0, s, in, n, limit, wide, tmp, out);
     return;
   }
-  hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SCAN_THREADS), 0, s, tmp, nt, out, n);
-  hipLaunchKernelGGL(k_scan_apply<true>, dim3(nt), dim3(SCAN_THREADS), 0, s, in, n, wide, tmp, out);
+  hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SCAN_THREADS), 0, s, tmp, nt, out, n, limit);
+  hipLaunchKernelGGL(k_scan_apply<true>, dim3(nt), dim3(SCAN_THREADS), 0, s, in, n, limit, wide, tmp, out);
 }
 
 __global__ void k_fill_u32(uint32_t* __restrict__ p, uint32_t v, uint64_t n) {
