@@ -911,6 +911,9 @@ static int milestone_check(nf_handle* h, size_t* next) {
   if (*next >= h->milestones.size()) return NF_OK;
   InstState st0{};
   HIPCHK(h, hipMemcpy(&st0, h->gb.st, sizeof(InstState), hipMemcpyDeviceToHost));
+  // out of room: the round's packing may hold rods that overlap (its lists of
+  // survivors were cut short), and the generation starts again, dumps included
+  if (st0.overflow != 0u) return NF_OK;
   const nf_params& p = h->params[0];
   const double PI = 3.14159265358979323846;
   const double vf = (double)st0.n_acc * PI * p.radius * p.radius * p.len / (p.box[0] * p.box[1] * p.box[2]) * 100.0;
