@@ -366,7 +366,8 @@ __global__ void __launch_bounds__(NT) k_cg_check(CgArgs a, uint32_t it, double t
     const double rr = block_sum(part_share(a.part_rr, a.nb), sh);
     if (threadIdx.x != 0) return;
     const double bb = it ? sc->bb : rr;
-    const double res = bb > 0.0 ? sqrt_cr((rr > 0.0 ? rr : 0.0) / bb) : 0.0;
+    // (a sum that is no number stays one: it compares false with zero)
+    const double res = bb > 0.0 ? sqrt_cr((rr < 0.0 ? 0.0 : rr) / bb) : 0.0;
     sc->bb = bb;
     sc->res = res;
     sc->done = res <= tol ? CG_CONVERGED : (res < __longlong_as_double(0x7FF0000000000000ll) ? 0u : CG_BROKEN);
