@@ -115,6 +115,15 @@ def build(force: bool = False, jobs: int = 8) -> str:
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError(f"band harness build failed\n{' '.join(cmd)}\n{r.stderr}")
+    # allocators that refuse, for the tests of memory limits (test only)
+    limits = os.path.join(ROOT, "tests", "native", "mem_limit.cpp")
+    llib = os.path.join(ROOT, "tests", "native", "libnf_mem_limit.so")
+    if os.path.exists(limits) and (force or _newer(llib, [limits])):
+        cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", limits, "-o", llib, "-L", "/opt/rocm/lib",
+               "-Wl,--no-as-needed", "-lamdhip64", "-ldl", "-Wl,-rpath,/opt/rocm/lib"]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode != 0:
+            raise RuntimeError(f"memory limit build failed\n{' '.join(cmd)}\n{r.stderr}")
     cli_src = os.path.join(CSRC, "nf_cli.cpp")
     if os.path.exists(cli_src) and (force or _newer(CLI, [cli_src, LIB])):
         cmd = ["g++", "-O2", "-std=c++17", "-I", os.path.join(ROOT, "include"), cli_src,

@@ -101,9 +101,13 @@ int dalloc_bytes(nf_handle* h, void** p, size_t bytes) {
     hipError_t e = q ? hipSuccess : hipMalloc(&q, cls);
     if (e != hipSuccess && !h->pool.empty()) {
       // give the cached blocks back and try once more
+      (void)hipGetLastError();
       trim_pool(h);
       e = hipMalloc(&q, cls);
     }
+    // a caller may do without the block: its next check of the runtime's last
+    // error must not find this one
+    if (e != hipSuccess) (void)hipGetLastError();
     if (e != hipSuccess)
       return fail(h, NF_E_NOMEM,
                   "hipMalloc of " + std::to_string(cls) + " bytes failed: " + hipGetErrorString(e));

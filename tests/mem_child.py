@@ -1,0 +1,79 @@
+"""Runs one scenario of test_gpu_memory_limits.py with the allocators of
+tests/native/mem_limit.cpp in front of the HIP runtime's, which have to be in
+place before the library is loaded: in a process of its own."""
+import ctypes as C
+import os
+import sys
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+sys.path.insert(0, os.path.dirname(HERE))
+M = C.CDLL(os.path.join(HERE, "native", "libnf_mem_limit.so"), mode=C.RTLD_GLOBAL)
+M.nfm_live.restype = M.nfm_peak.restype = C.c_size_t
+M.nfm_limit.argtypes = [C.c_size_t]
+NO_LIMIT = C.c_size_t(-1).value
+
+import numpy as np  # noqa: E402
+
+import nanofiller_amd as nf  # noqa: E402
+
+
+def params(n, box, **kw):
+    kw = dict(dict(len=1.0, radius=0.005, seed=3, contact_gap=0.004, max_rounds=40), **kw)
+    return nf.normalize(nf.default_params(box=(box,) * 3, n_rods=n, **kw))
+
+
+def flat(*arrays):
+    return b"".join(np.ascontiguousarray(a).tobytes() for a in arrays)
+
+
+def contacts(pk, gap=0.004):
+    c = pk.contacts(gap)
+    return flat(c.row_ptr, c.col, c.gap, c.image, pk.contact_gap64(c.n), pk.contact_area(c.n))
+
+
+def create_at_the_limit():
+    """A handle for which the crossing lists do not fit generates all the same."""
+    p = params(20000, 5.0)
+    with nf.Packing(p) as pk:
+        pk.generate()
+        want = flat(pk.rods())
+        full = M.nfm_peak()
+    for less in (1, full // 16, full // 8, full // 4):
+        M.nfm_limit(full - less)
+        with nf.Packing(p) as pk:
+            M.nfm_limit(NO_LIMIT)
+            pk.generate()
+            assert flat(pk.rods()) == want, less
+
+
+def contacts_at_the_limit():
+    """A call that runs out of memory says so, one that has enough is right,
+    and neither leaves anything behind for the next."""
+    p = params(20000, 4.0)
+    with nf.Packing(p) as pk:
+        pk.generate()
+        rods = pk.rods()
+        base = M.nfm_live()
+        want = contacts(pk)
+        full = M.nfm_peak() - base
+    fits = 0
+    for part in range(16, -1, -1):
+        with nf.Packing(p) as pk:
+            pk.set_rods(rods)
+            M.nfm_limit(M.nfm_live() + full * part // 16)
+            try:
+                assert contacts(pk) == want, part
+                fits += 1
+            except nf.NFError as e:
+                assert e.code == nf.NF_E_NOMEM, (part, e)
+            M.nfm_limit(NO_LIMIT)
+            assert contacts(pk) == want, part
+            pk.generate()
+            assert flat(pk.rods()) == flat(rods), part
+    assert 0 < fits
+
+
+if __name__ == "__main__":
+    print("[scenario]", sys.argv[1], flush=True)
+    globals()[sys.argv[1]]()
+    print("ok", flush=True)
