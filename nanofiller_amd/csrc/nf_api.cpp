@@ -1068,9 +1068,7 @@ static int generate_once(nf_handle* h, nf_gen_stats* stats, std::vector<std::pai
   }
   double kern[8] = {0};
   RoundInfo ri{};
-  PinnedScalars* pinned = pinned_scalars(h);
-  if (!pinned) return fail(h, NF_E_NOMEM, "generation: no pinned memory");
-  RoundInfo* ri_host = &pinned->ri;
+  RoundInfo* ri_host = &host_scalars(h)->ri;
   uint32_t max_rounds = 0;
   for (auto& p : h->params) max_rounds = std::max(max_rounds, p.max_rounds);
   const auto t0 = std::chrono::steady_clock::now();
@@ -1099,7 +1097,7 @@ static int generate_once(nf_handle* h, nf_gen_stats* stats, std::vector<std::pai
       }
       ++launched;
     }
-    launch_to_pinned(h->gb.ri, sizeof(RoundInfo), ri_host, h->stream);
+    if (e == hipSuccess) e = scalars_to_host(h, ri_host, h->gb.ri, sizeof(RoundInfo));
     if (e == hipSuccess) e = sync_stream(h->stream, "generation round");
     if (e != hipSuccess) break;
     ri = *ri_host;

@@ -35,11 +35,11 @@ extern "C" int nf_conductance(nf_handle* h, double tol, uint32_t max_iter, nf_co
   double *cval = nullptr, *dinv = nullptr, *bsrc = nullptr, *bsnk = nullptr, *x = nullptr,
          *r = nullptr, *pv = nullptr, *q = nullptr, *part = nullptr, *vdev = nullptr;
   double2* zp = nullptr;
-  CgScal* scal = nullptr;
+  CgScal *scal = nullptr, *verdicts = nullptr;
   uint32_t *acto = nullptr, *rlo = nullptr, *idxo = nullptr, *offo = nullptr;
   auto release = [&]() {
     void* ptrs[] = {flag, act, rl,   idx, off, tmp,  crow, ccol, cval, dinv, bsrc, bsnk,
-                    x,    r,   zp,   pv,  q,   part, vdev, scal, acto, rlo,  idxo, offo};
+                    x,    r,   zp,   pv,  q,   part, vdev, scal, acto, rlo,  idxo, offo, verdicts};
     for (void* p : ptrs) dfree(h, p);
   };
   const uint64_t n1 = (uint64_t)n + 1;
@@ -127,10 +127,13 @@ extern "C" int nf_conductance(nf_handle* h, double tol, uint32_t max_iter, nf_co
       release();
       return rc;
     }
-    PinnedScalars* pinned = pinned_scalars(h);
-    if (!pinned) {
-      release();
-      return fail(h, NF_E_NOMEM, "conductance: no pinned memory");
+    HostScalars* scalars = host_scalars(h);
+    if (!h->scal_pinned) {
+      ALLOC(verdicts, 2);
+      if (rc != NF_OK) {
+        release();
+        return rc;
+      }
     }
     launch_cs_fill(c.nrow, c.ncol, c.nval, n, act, idx, off, crow, ccol, cval, dinv, bsrc, bsnk, s);
     fill_u32(crow + m, nnz, 1, s);
@@ -139,21 +142,27 @@ extern "C" int nf_conductance(nf_handle* h, double tol, uint32_t max_iter, nf_co
     cg_grids(a);
     struct Check {
       uint32_t it;     // iterations before it
-      CgScal* host;    // pinned copy of the scalars
+      CgScal* host;    // copy of the scalars on the host
+      CgScal* out;     // where the kernel leaves it: there, or in device memory if the host has none pinned
       hipEvent_t done;
     };
-    Check slot[2] = {{0, &pinned->cg[0], h->ev[2]}, {0, &pinned->cg[1], h->ev[3]}};
+    CgScal* out0 = h->scal_pinned ? scalars->cg : verdicts;
+    Check slot[2] = {{0, &scalars->cg[0], out0, h->ev[2]}, {0, &scalars->cg[1], out0 + 1, h->ev[3]}};
+    auto fetch = [&](const Check& c) -> hipError_t {
+      return c.out == c.host ? hipSuccess : scalars_to_host(h, c.host, c.out, sizeof(CgScal));
+    };
     uint32_t pending = 0, newest = 0;
     hipEventRecord(h->ev[0], s);
     // queues what leads to the next check (init for the first) and the check, which leaves its verdict in c.host
     auto queue = [&](uint32_t it, uint32_t count, Check& c) -> hipError_t {
       if (count == 0)
-        launch_cg_init(a, tol, c.host, s);
+        launch_cg_init(a, tol, c.out, s);
       else
-        launch_cg_iterations(a, it, count, tol, c.host, s);
+        launch_cg_iterations(a, it, count, tol, c.out, s);
       c.it = it + count;
       ++pending;
-      return hipEventRecord(c.done, s);
+      const hipError_t e = fetch(c);
+      return e == hipSuccess ? hipEventRecord(c.done, s) : e;
     };
     uint32_t it = 0;
     CgScal hs{};
@@ -181,13 +190,15 @@ extern "C" int nf_conductance(nf_handle* h, double tol, uint32_t max_iter, nf_co
       }
     }
     const bool conv = hs.done == CG_CONVERGED;
-    launch_cg_current(a, pinned->cg, s);  // (after whatever is queued: both slots are free by then)
+    launch_cg_current(a, slot[0].out, s);  // (after whatever is queued: both slots are free by then)
     hipEventRecord(h->ev[1], s);
-    if (hipError_t e = sync_stream(s, "conductance currents"); e != hipSuccess) {
+    e = fetch(slot[0]);
+    if (e == hipSuccess) e = sync_stream(s, "conductance currents");
+    if (e != hipSuccess) {
       release();
       return fail(h, NF_E_HIP, std::string("conductance currents: ") + hipGetErrorString(e));
     }
-    hs = pinned->cg[0];
+    hs = scalars->cg[0];
     hipEventElapsedTime(&solve_ms, h->ev[0], h->ev[1]);
     out.iterations = it;
     out.converged = conv ? 1 : 0;

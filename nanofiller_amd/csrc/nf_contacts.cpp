@@ -286,8 +286,7 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, Co
   ALLOC(tmp, scan_tmp_words((uint64_t)n + 1));
 #undef ALLOC
   BinScratch bs;
-  PinnedScalars* pinned = pinned_scalars(h);
-  if (rc == NF_OK && !pinned) rc = fail(h, NF_E_NOMEM, "contacts: no pinned memory");
+  HostScalars* scalars = host_scalars(h);
   auto free_scratch = [&]() {
     free_bin_scratch(h, &bs);
     dfree(h, ctr);
@@ -513,10 +512,10 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, Co
     hipEventRecord(ev[2], s);
     trace("contacts: %u rods, %s pass launched", n,
           cells ? "cell-pair" : (way == WAY_LISTS ? "crossing-list" : "footprint"));
-    launch_to_pinned(ctr, sizeof(pinned->ctr), pinned->ctr, s);
+    HIPCHK(h, scalars_to_host(h, scalars->ctr, ctr, sizeof(scalars->ctr)));
     HIPCHK(h, sync_stream(s, "contact pair pass"));
-    total = (uint32_t)pinned->ctr[4];
-    const uint32_t over = (uint32_t)pinned->ctr[6];
+    total = (uint32_t)scalars->ctr[4];
+    const uint32_t over = (uint32_t)scalars->ctr[6];
     HIPCHK(h, hipGetLastError());
     if (over) {
       trace("contacts: more rods cross a cell than fit; another engine instead");
@@ -558,7 +557,7 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, Co
   launch_row_sort(c.rowptr, n, c.J, c.gap, c.gap64, c.img, s);
   launch_contact_area(P, D, total, c.I, c.J, c.img, p.box, gap, c.area, s);
   hipEventRecord(ev[5], s);
-  std::copy(pinned->ctr, pinned->ctr + 6, h->cb_stats);
+  std::copy(scalars->ctr, scalars->ctr + 6, h->cb_stats);
   HIPCHK(h, sync_stream(s, "contact list"));
   trace("contacts: %u recorded and sorted", total);
   HIPCHK(h, hipGetLastError());

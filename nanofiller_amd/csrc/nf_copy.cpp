@@ -257,23 +257,30 @@ hipError_t rods_to_device(nf_handle* h, const float* rods, uint32_t n, float4* P
   return e != hipSuccess ? e : w;
 }
 
-PinnedScalars* pinned_scalars(nf_handle* h) {
-  if (!h->pin_scal) {
+HostScalars* host_scalars(nf_handle* h) {
+  if (!h->scal) {
     void* p = nullptr;
-    if (hipHostMalloc(&p, sizeof(PinnedScalars), hipHostMallocDefault) != hipSuccess) {
-      (void)hipGetLastError();
-      return nullptr;
-    }
-    h->pin_scal = (PinnedScalars*)p;
+    h->scal_pinned = hipHostMalloc(&p, sizeof(HostScalars), hipHostMallocDefault) == hipSuccess;
+    if (!h->scal_pinned) (void)hipGetLastError();
+    h->scal = h->scal_pinned ? (HostScalars*)p : new HostScalars();
   }
-  return h->pin_scal;
+  return h->scal;
+}
+
+hipError_t scalars_to_host(nf_handle* h, void* dst, const void* src, size_t bytes) {
+  if (!h->scal_pinned) return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, h->stream);
+  launch_to_pinned(src, bytes, dst, h->stream);
+  return hipGetLastError();
 }
 
 void release_pinned(nf_handle* h) {
   for (auto& e : h->pin_ev)
     if (e) (void)hipEventDestroy(e);
   if (h->pin) (void)hipHostFree(h->pin);
-  if (h->pin_scal) (void)hipHostFree(h->pin_scal);
+  if (h->scal_pinned)
+    (void)hipHostFree(h->scal);
+  else
+    delete h->scal;
 }
 
 }  // namespace nf

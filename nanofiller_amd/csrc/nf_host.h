@@ -13,8 +13,9 @@
 #include "nf_internal.h"
 
 namespace nf {
-// Scalars that a queued kernel's result is awaited in.
-struct PinnedScalars {
+// Scalars that a queued kernel's result is awaited in: pinned, or plain memory
+// of a host that has none to pin.
+struct HostScalars {
   RoundInfo ri;   // of the generation's last round
   CgScal cg[2];   // of the conductance solve's last two checks
   unsigned long long ctr[8];  // counters of a contact pass; summary of a network build
@@ -68,7 +69,8 @@ struct nf_handle {
   char* pin = nullptr;
   size_t pin_bytes = 0;
   hipEvent_t pin_ev[8] = {};
-  nf::PinnedScalars* pin_scal = nullptr;
+  nf::HostScalars* scal = nullptr;
+  bool scal_pinned = false;
   float net_ms = 0.0f;  // device time of the last nf_network call
 };
 
@@ -95,7 +97,10 @@ hipError_t to_host(nf_handle* h, const HostPart* parts, size_t n_parts);
 // Rods as nf_get_rods gives and nf_set_rods takes them.
 hipError_t rods_to_host(nf_handle* h, const float4* P, const float4* D, uint32_t n, float* rods);
 hipError_t rods_to_device(nf_handle* h, const float* rods, uint32_t n, float4* P, float4* D);
-PinnedScalars* pinned_scalars(nf_handle* h);
+// The handle's scalars (never null), and device memory queued into them on the
+// handle's stream.
+HostScalars* host_scalars(nf_handle* h);
+hipError_t scalars_to_host(nf_handle* h, void* dst, const void* src, size_t bytes);
 void release_pinned(nf_handle* h);
 // Centre cell list of the contact rods (edge about one pair reach, sorted
 // stencil): built by the cell engine of nf_contacts, or on demand by the

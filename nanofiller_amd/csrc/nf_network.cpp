@@ -80,8 +80,7 @@ extern "C" int nf_network(nf_handle* h, nf_network_info* info) {
                  a.summary, a.tmp,     a.cg,      a.bsum};
     for (void* q : w) dfree(h, q);
   };
-  PinnedScalars* pinned = pinned_scalars(h);
-  if (rc == NF_OK && !pinned) rc = fail(h, NF_E_NOMEM, "network: no pinned memory");
+  HostScalars* scalars = host_scalars(h);
   if (rc != NF_OK) {
     release_work();
     return rc;
@@ -90,10 +89,10 @@ extern "C" int nf_network(nf_handle* h, nf_network_info* info) {
   a.nrow = c.nrow;
   hipEventRecord(h->ev[0], s);
   launch_network_build(a, s);
-  const unsigned long long* sum = pinned->ctr;
-  static_assert(NET_SUMMARY <= sizeof(pinned->ctr) / sizeof(pinned->ctr[0]), "summary");
-  launch_to_pinned(a.summary, sizeof(unsigned long long) * NET_SUMMARY, pinned->ctr, s);
-  hipError_t e = sync_stream(s, "network build");
+  const unsigned long long* sum = scalars->ctr;
+  static_assert(NET_SUMMARY <= sizeof(scalars->ctr) / sizeof(scalars->ctr[0]), "summary");
+  hipError_t e = scalars_to_host(h, scalars->ctr, a.summary, sizeof(unsigned long long) * NET_SUMMARY);
+  if (e == hipSuccess) e = sync_stream(s, "network build");
   if (e == hipSuccess) e = hipGetLastError();
   if (e != hipSuccess) {
     release_work();

@@ -31,6 +31,37 @@ def contacts(pk, gap=0.004):
     return flat(c.row_ptr, c.col, c.gap, c.image, pk.contact_gap64(c.n), pk.contact_area(c.n))
 
 
+def everything(pk):
+    out = [flat(pk.rods()) if pk.generate() else b"", contacts(pk)]
+    h = pk.histograms(bins=16)
+    out.append(flat(h["centre"], h["polar"], h["mutual"]))
+    out.append(flat(pk.centre_distance(16, 0.02)["counts"]))
+    net = pk.network()[1]
+    out.append(flat(net["labels"], net["row_ptr"], net["col"], net["val"]))
+    # (rounded differently from run to run: the order of the unknowns is not fixed)
+    info, v = pk.conductance(tol=1e-12, max_iter=50000, potentials=True)
+    assert info["converged"] == 1 and info["unknowns"] > 100
+    out.append(flat(pk.reduce(2)[1]))
+    return out, info["conductance"], v
+
+
+def no_pinned_memory():
+    p = params(3000, 2.5, tunnel_lambda=0.002)
+    want = everything_of(p)
+    M.nfm_pinned(0)
+    got = everything_of(p)
+    M.nfm_pinned(1)
+    for k, (a, b) in enumerate(zip(got[0], want[0])):
+        assert a == b, k
+    assert abs(got[1] - want[1]) <= 1e-8 * want[1]
+    np.testing.assert_allclose(got[2], want[2], rtol=0, atol=1e-8)
+
+
+def everything_of(p):
+    with nf.Packing(p) as pk:
+        return everything(pk)
+
+
 def create_at_the_limit():
     """A handle for which the crossing lists do not fit generates all the same."""
     p = params(20000, 5.0)

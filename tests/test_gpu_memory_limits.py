@@ -1,5 +1,5 @@
 """The library where memory runs out: device allocations refused from a given
-total on (tests/mem_child.py)."""
+total on, pinned host memory refused altogether (tests/mem_child.py)."""
 import os
 import subprocess
 import sys
@@ -19,3 +19,7 @@ def _run(scenario):
 @pytest.mark.parametrize("scenario", ["create_at_the_limit", "contacts_at_the_limit"])
 def test_a_refused_allocation_leaves_nothing_behind(scenario):
     _run(scenario)
+
+
+def test_results_without_pinned_memory():
+    _run("no_pinned_memory")
