@@ -49,23 +49,43 @@ constexpr size_t POOL_CAP = (size_t)16 << 30;  // freed bytes kept per handle
 
 constexpr size_t SLAB_FROM = (size_t)1 << 20, SLAB_TO = (size_t)32 << 20, SLAB_LARGEST = (size_t)256 << 20;
 
-static bool in_slab(const nf_handle* h, const void* p) {
-  for (const auto& s : h->slabs)
-    if ((const char*)p >= s.p && (const char*)p < s.p + s.size) return true;
-  return false;
+static nf_handle::Slab* slab_of(nf_handle* h, const void* p) {
+  for (auto& s : h->slabs)
+    if ((const char*)p >= s.p && (const char*)p < s.p + s.size) return &s;
+  return nullptr;
 }
 
-// A block cut from the newest slab, or from a new one twice its size; null if
-// there is no memory for one.
+// Takes the blocks of a slab without one in use out of the pool.
+static void clear_slab(nf_handle* h, nf_handle::Slab& s) {
+  for (auto it = h->pool.begin(); it != h->pool.end();) {
+    if ((char*)it->second < s.p || (char*)it->second >= s.p + s.size) {
+      ++it;
+      continue;
+    }
+    h->pool_bytes -= it->first;
+    it = h->pool.erase(it);
+  }
+  s.used = 0;
+}
+
+// A block cut from the newest slab, from one whose blocks are all free, or
+// from a new one twice the newest's size; null if there is no memory for one.
 static void* slab_block(nf_handle* h, size_t cls) {
   if (h->slabs.empty() || h->slabs.back().size - h->slabs.back().used < cls) {
-    const size_t size = h->slabs.empty() ? SLAB_TO : std::min(2 * h->slabs.back().size, SLAB_LARGEST);
-    void* p = nullptr;
-    if (hipMalloc(&p, size) != hipSuccess) {
-      (void)hipGetLastError();
-      return nullptr;
+    auto idle = std::find_if(h->slabs.begin(), h->slabs.end(),
+                             [&](const nf_handle::Slab& s) { return s.live == 0 && s.size >= cls; });
+    if (idle != h->slabs.end()) {
+      clear_slab(h, *idle);
+      std::rotate(idle, idle + 1, h->slabs.end());
+    } else {
+      const size_t size = h->slabs.empty() ? SLAB_TO : std::min(2 * h->slabs.back().size, SLAB_LARGEST);
+      void* p = nullptr;
+      if (hipMalloc(&p, size) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+      }
+      h->slabs.push_back({(char*)p, size, 0, 0});
     }
-    h->slabs.push_back({(char*)p, size, 0});
   }
   auto& s = h->slabs.back();
   void* q = s.p + s.used;
@@ -73,10 +93,20 @@ static void* slab_block(nf_handle* h, size_t cls) {
   return q;
 }
 
-// Gives the pool's blocks back to the device, but for those cut from slabs.
+// Gives the pool's blocks back to the device: those of their own, and the
+// slabs without a block in use.
 static void trim_pool(nf_handle* h) {
+  for (size_t k = 0; k < h->slabs.size();) {
+    if (h->slabs[k].live != 0) {
+      ++k;
+      continue;
+    }
+    clear_slab(h, h->slabs[k]);
+    (void)hipFree(h->slabs[k].p);
+    h->slabs.erase(h->slabs.begin() + k);
+  }
   for (auto it = h->pool.begin(); it != h->pool.end();) {
-    if (in_slab(h, it->second)) {
+    if (slab_of(h, it->second)) {
       ++it;
       continue;
     }
@@ -99,7 +129,7 @@ int dalloc_bytes(nf_handle* h, void** p, size_t bytes) {
   } else {
     if (cls >= SLAB_FROM && cls <= SLAB_TO) q = slab_block(h, cls);
     hipError_t e = q ? hipSuccess : hipMalloc(&q, cls);
-    if (e != hipSuccess && !h->pool.empty()) {
+    if (e != hipSuccess && (!h->pool.empty() || !h->slabs.empty())) {
       // give the cached blocks back and try once more
       (void)hipGetLastError();
       trim_pool(h);
@@ -112,6 +142,7 @@ int dalloc_bytes(nf_handle* h, void** p, size_t bytes) {
       return fail(h, NF_E_NOMEM,
                   "hipMalloc of " + std::to_string(cls) + " bytes failed: " + hipGetErrorString(e));
   }
+  if (auto* s = slab_of(h, q)) ++s->live;
   h->allocs[q] = cls;
   *p = q;
   return NF_OK;
@@ -184,7 +215,9 @@ void dfree(nf_handle* h, void* p) {
   const size_t cls = it->second;
   h->allocs.erase(it);
   if (h->stream) (void)hipStreamSynchronize(h->stream);
-  if (h->pool_bytes + cls > POOL_CAP && !in_slab(h, p)) {
+  if (auto* s = slab_of(h, p)) {
+    --s->live;
+  } else if (h->pool_bytes + cls > POOL_CAP) {
     (void)hipFree(p);
     return;
   }
@@ -787,7 +820,7 @@ extern "C" void nf_destroy(nf_handle* h) {
   release_gen(h);
   trim_pool(h);
   for (auto& kv : h->allocs)
-    if (!in_slab(h, kv.first)) (void)hipFree(kv.first);
+    if (!slab_of(h, kv.first)) (void)hipFree(kv.first);
   for (auto& s : h->slabs) (void)hipFree(s.p);
   for (auto& e : h->ev)
     if (e) (void)hipEventDestroy(e);

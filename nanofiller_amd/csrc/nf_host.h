@@ -52,10 +52,12 @@ struct nf_handle {
   size_t pool_bytes = 0;
   std::vector<int4> contact_stencil;  // on its way to the device
   // blocks of 1 to 32 MB are cut from larger ones (one hipMalloc of that size
-  // takes 0.3 ms, and a packing needs a dozen); given back with the handle
+  // takes 0.3 ms, and a packing needs a dozen); one without a block in use
+  // serves other sizes, or goes back to the device where memory runs out
   struct Slab {
     char* p;
     size_t size, used;
+    uint32_t live;  // blocks in use
   };
   std::vector<Slab> slabs;
   unsigned long long cb_stats[6] = {0, 0, 0, 0, 0, 0};  // contact pair tests, rechecks, max dd bits

@@ -11,6 +11,7 @@ M = C.CDLL(os.path.join(HERE, "native", "libnf_mem_limit.so"), mode=C.RTLD_GLOBA
 M.nfm_live.restype = M.nfm_peak.restype = C.c_size_t
 M.nfm_limit.argtypes = [C.c_size_t]
 NO_LIMIT = C.c_size_t(-1).value
+SLAB = 256 << 20  # the largest that blocks are cut from
 
 import numpy as np  # noqa: E402
 
@@ -102,6 +103,30 @@ def contacts_at_the_limit():
             pk.generate()
             assert flat(pk.rods()) == flat(rods), part
     assert 0 < fits
+
+
+def another_instance():
+    """What the calls on one instance held is there for the next one's; a slab
+    that the handle's own blocks share stays."""
+    ps = [params(2000000, 34.0, contact_gap=0.03), params(3000000, 40.0, stream=1)]
+    with nf.Packing(ps) as pk:
+        pk.generate()
+        pk.select(1)
+        want = contacts(pk)
+        alone = M.nfm_peak()
+    assert M.nfm_live() == 0
+    with nf.Packing(ps) as pk:
+        pk.generate()
+        own = M.nfm_live()
+        pk.contacts(0.03)
+        pk.network()
+        held = M.nfm_live() - own
+        assert held > 3 * SLAB, held
+        pk.select(1)
+        M.nfm_limit(alone + SLAB)
+        assert contacts(pk) == want
+        M.nfm_limit(NO_LIMIT)
+    assert M.nfm_live() == 0
 
 
 if __name__ == "__main__":

@@ -23,3 +23,7 @@ def test_a_refused_allocation_leaves_nothing_behind(scenario):
 
 def test_results_without_pinned_memory():
     _run("no_pinned_memory")
+
+
+def test_memory_of_one_instance_serves_the_next():
+    _run("another_instance")
