@@ -116,6 +116,8 @@ static void trim_pool(nf_handle* h) {
   }
 }
 
+static bool shed_lists(nf_handle* h);
+
 int dalloc_bytes(nf_handle* h, void** p, size_t bytes) {
   *p = nullptr;
   if (bytes == 0) bytes = 16;
@@ -131,6 +133,11 @@ int dalloc_bytes(nf_handle* h, void** p, size_t bytes) {
     hipError_t e = q ? hipSuccess : hipMalloc(&q, cls);
     if (e != hipSuccess && (!h->pool.empty() || !h->slabs.empty())) {
       // give the cached blocks back and try once more
+      (void)hipGetLastError();
+      trim_pool(h);
+      e = hipMalloc(&q, cls);
+    }
+    if (e != hipSuccess && shed_lists(h)) {
       (void)hipGetLastError();
       trim_pool(h);
       e = hipMalloc(&q, cls);
@@ -603,7 +610,7 @@ void nf::release_contacts(nf_handle* h) {
 // them (desc: to be uploaded afterwards).
 constexpr uint32_t LIST_CAP_MAX = 8192;
 constexpr uint64_t LIST_ENTRIES_MAX = (uint64_t)1 << 32;  // 16 GiB
-static int layout_lists(nf_handle* h) {
+static void free_lists(nf_handle* h) {
   GenBuffers& b = h->gb;
   void* old[] = {b.fcountA, b.fcountP, b.flistA, b.flistP, b.oR, b.aR};
   for (void* p : old) dfree(h, p);
@@ -611,6 +618,12 @@ static int layout_lists(nf_handle* h) {
   b.oR = b.aR = nullptr;
   b.total_fine = b.total_listA = b.total_listP = 0;
   b.walk = b.cellwise = false;
+}
+
+static int layout_lists(nf_handle* h) {
+  GenBuffers& b = h->gb;
+  free_lists(h);
+  bool walk = false;
   for (InstDesc& d : h->desc) {
     FineGrid& g = d.fine;
     if (!g.on) {
@@ -634,9 +647,9 @@ static int layout_lists(nf_handle* h) {
     b.total_fine += cells;
     b.total_listA += cells * g.capA;
     b.total_listP += cells * g.capP;
-    b.walk = true;
+    walk = true;
   }
-  if (!b.walk) return NF_OK;
+  if (!walk) return NF_OK;
   int rc = dalloc(h, &b.fcountA, b.total_fine);
   if (rc == NF_OK) rc = dalloc(h, &b.fcountP, b.total_fine);
   if (rc == NF_OK) rc = dalloc(h, &b.flistA, b.total_listA);
@@ -648,7 +661,24 @@ static int layout_lists(nf_handle* h) {
     for (InstDesc& d : h->desc) d.fine.on = 0u;
     return layout_lists(h);
   }
+  b.walk = rc == NF_OK;  // (not before: shed_lists)
   return rc;
+}
+
+static void drop_graph(nf_handle* h);
+
+// Memory has run out: the lists give theirs to the call that needs it, and the
+// generations that follow go without (a third of a large handle's memory, up to
+// 16 GiB).  False if there are none, or a pass is using them.
+static bool nf::shed_lists(nf_handle* h) {
+  GenBuffers& b = h->gb;
+  if (!b.walk || h->lists_in_use) return false;
+  for (InstDesc& d : h->desc) d.fine.on = 0u;
+  free_lists(h);
+  b.cellwise = true;
+  drop_graph(h);
+  trace("out of memory: crossing lists given back");
+  return hipMemcpy(b.desc, h->desc.data(), sizeof(InstDesc) * h->desc.size(), hipMemcpyHostToDevice) == hipSuccess;
 }
 
 extern "C" int nf_create_batch(const nf_params* ps, int n, nf_handle** out) {
@@ -997,6 +1027,7 @@ static int relayout_old(nf_handle* h, const std::vector<uint32_t>& caps) {
     off += (uint64_t)d.ncells * d.cap;
   }
   if (off > 0xFFFFFFF0ull) return fail(h, NF_E_INVALID, "cell slots exceed the 32-bit index space");
+  free_lists(h);  // laid out anew below
   dfree(h, b.oP);
   dfree(h, b.oD);
   dfree(h, b.oid);

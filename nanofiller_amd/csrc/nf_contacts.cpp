@@ -273,6 +273,10 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, Co
   float4* lrods = nullptr;
   uint32_t *lcount = nullptr, *llist = nullptr;
   bool lown = false;  // the lists are this pass's own (else the generation's, idle here)
+  struct ListUse {
+    nf_handle* h;
+    ~ListUse() { h->lists_in_use = false; }
+  } list_use{h};
   unsigned long long* ctr = nullptr;
   uint32_t* tmp = nullptr;
   uint32_t* queues = nullptr;
@@ -367,10 +371,11 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, Co
   } else if (way == WAY_LISTS) {
     WalkContacts& w = wa.cnt;
     const uint64_t entries = (uint64_t)w.g.ncells * w.fine.capA;
-    rc = dalloc(h, &lrods, 2 * (uint64_t)n);
+    rc = dalloc(h, &lrods, 2 * (uint64_t)n);  // (before the look at the lists: it may cost them)
     if (h->gb.walk && h->gb.total_fine >= w.g.ncells && h->gb.total_listA >= entries) {
       lcount = h->gb.fcountA;  // cleared again before the next generation
       llist = h->gb.flistA;
+      h->lists_in_use = true;
     } else {
       lown = true;
       if (rc == NF_OK) rc = dalloc(h, &lcount, w.g.ncells);

@@ -44,6 +44,7 @@ struct nf_handle {
   std::vector<std::pair<uint32_t, uint32_t>> planned_list;  // and entries per crossing list (accepted, survivors)
   std::vector<double> milestones;  // volume fractions (percent) of the state dumps, ascending
   std::string milestone_dir;       // where nf_generate writes them
+  bool lists_in_use = false;       // a contact pass keeps its entries in the generation's lists
   bool generated = false;
   // device memory: live blocks (pointer -> size-class bytes) and a pool of
   // freed blocks by size class, reused by later calls of the same handle

@@ -129,6 +129,27 @@ def another_instance():
     assert M.nfm_live() == 0
 
 
+def lists_make_room():
+    """Crossing lists of the generation give way to a call that needs their
+    memory; the next generation makes the same packing."""
+    p = params(400000, 16.0, len_law=nf.NF_LEN_LOGNORMAL, len_sigma=0.3, len_min=0.3, len_max=3.0)
+    engine = {nf.NF_OPT_CONTACT_ENGINE: nf.NF_ENGINE_CELLS}
+    with nf.Packing(p, engine) as pk:
+        pk.generate()
+        rods = flat(pk.rods())
+        want = contacts(pk)
+    with nf.Packing(p, engine) as pk:
+        pk.generate()
+        M.nfm_limit(M.nfm_live() + (2 << 20))
+        assert contacts(pk) == want
+        pk.generate()
+        assert flat(pk.rods()) == rods
+        assert contacts(pk) == want
+        M.nfm_limit(NO_LIMIT)
+        pk.generate()
+        assert flat(pk.rods()) == rods
+
+
 if __name__ == "__main__":
     print("[scenario]", sys.argv[1], flush=True)
     globals()[sys.argv[1]]()

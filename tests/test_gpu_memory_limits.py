@@ -27,3 +27,7 @@ def test_results_without_pinned_memory():
 
 def test_memory_of_one_instance_serves_the_next():
     _run("another_instance")
+
+
+def test_lists_give_way():
+    _run("lists_make_room")
