@@ -105,16 +105,17 @@ def build(force: bool = False, jobs: int = 8) -> str:
         if r.returncode != 0:
             raise RuntimeError(f"link failed\n{' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
         os.replace(tmp, LIB)
-    # host build of the pair predicates for the CPU test suite (test only)
-    harness = os.path.join(ROOT, "tests", "native", "band_harness.cpp")
-    hlib = os.path.join(ROOT, "tests", "native", "libnf_band.so")
-    if os.path.exists(harness) and (force or _newer(hlib, [harness, os.path.join(CSRC, "nf_common.h"),
-                                                           os.path.join(CSRC, "nf_seg.h")])):
-        cmd = [hipcc(), "--offload-host-only", "-x", "hip", "-O2", "-fPIC", "-shared", "-std=c++17",
-               "-ffp-contract=off", "-I", os.path.join(ROOT, "include"), harness, "-o", hlib]
-        r = subprocess.run(cmd, capture_output=True, text=True)
-        if r.returncode != 0:
-            raise RuntimeError(f"band harness build failed\n{' '.join(cmd)}\n{r.stderr}")
+    # host builds of the pair predicates for the CPU test suite (test only)
+    for name in ("band", "line"):
+        harness = os.path.join(ROOT, "tests", "native", f"{name}_harness.cpp")
+        hlib = os.path.join(ROOT, "tests", "native", f"libnf_{name}.so")
+        deps = [harness] + [os.path.join(CSRC, h) for h in ("nf_common.h", "nf_seg.h", "nf_line.h")]
+        if os.path.exists(harness) and (force or _newer(hlib, deps)):
+            cmd = [hipcc(), "--offload-host-only", "-x", "hip", "-O2", "-fPIC", "-shared", "-std=c++17",
+                   "-ffp-contract=off", "-I", os.path.join(ROOT, "include"), harness, "-o", hlib]
+            r = subprocess.run(cmd, capture_output=True, text=True)
+            if r.returncode != 0:
+                raise RuntimeError(f"{name} harness build failed\n{' '.join(cmd)}\n{r.stderr}")
     # allocators that refuse, for the tests of memory limits (test only)
     limits = os.path.join(ROOT, "tests", "native", "mem_limit.cpp")
     llib = os.path.join(ROOT, "tests", "native", "libnf_mem_limit.so")

@@ -73,7 +73,45 @@ NF_HD float line_apart(const LineSide& p, const LineSide& q, float b) {
   return fmaf(t, t, fmaf(c, c, b));
 }
 
-// The same with the origin at the first rod's centre, whose moment is then
+// A staging slot's side of the cell-pair engine's filter: its line, or, where
+// every pair within reach is tested (ALL), its centre (u), the reach part rq
+// (mx) and rq^2 - |centre|^2 (b).
+struct SlotSide {
+  LineSide l;
+  float b;  // -1 - slack; a slot without a rod is apart from everything
+};
+
+// (x, y, z), hl, D: the rod's centre from the common origin, half length and
+// direction; without `valid` whatever memory held, NaN included.
+template <bool ALL>
+NF_HD SlotSide slot_side(const LineFilter& f, float x, float y, float z, float hl, float4 D, bool valid) {
+  SlotSide q;
+  x = valid ? x : 0.0f;
+  y = valid ? y : 0.0f;
+  z = valid ? z : 0.0f;
+  if (ALL) {
+    const float r = valid ? (hl * 1.000001f) * 1.000006f : 0.0f;
+    q.l = LineSide{x, y, z, r, 0.0f, 0.0f};
+    q.b = valid ? fmaf(r, r, -fmaf(z, z, fmaf(y, y, x * x))) : -3e38f;
+  } else {
+    D.x = valid ? D.x : 0.0f;
+    D.y = valid ? D.y : 0.0f;
+    D.z = valid ? D.z : 0.0f;
+    q.l = line_side(f, x, y, z, D);
+    q.b = valid ? -1.0f - f.slack : 3e38f;
+  }
+  return q;
+}
+
+// Negative when the pair may be cut.  (f, h): the probe's line (direction,
+// moment), or 2 (P - o), 2 rp and |P - o|^2 - rp^2 - slack.
+template <bool ALL>
+NF_HD float slot_apart(const float4 f, const float2 h, const SlotSide& q) {
+  if (ALL) return h.x - fmaf(f.w, q.l.mx, fmaf(f.z, q.l.uz, fmaf(f.y, q.l.uy, fmaf(f.x, q.l.ux, q.b))));
+  return line_apart(LineSide{f.x, f.y, f.z, f.w, h.x, h.y}, q.l, q.b);
+}
+
+// line_apart with the origin at the first rod's centre, whose moment is then
 // zero: u1s its direction times scale, (x, y, z) the second rod's centre.
 NF_HD float line_apart_from(const float3 u1s, float x, float y, float z, const float4 D1, const float4 D2, float b) {
   const float mx = fmaf(y, D2.z, -(z * D2.y)), my = fmaf(z, D2.x, -(x * D2.z)), mz = fmaf(x, D2.y, -(y * D2.x));

@@ -417,39 +417,17 @@ struct Filter {
   LineFilter ln;  // nf_line.h (every pair: slack 64 u S^2, see process_cell)
 };
 
-// A slot's side of the filter: its line, or, where every pair within reach is
-// tested, its centre (u), the reach part rq (mx) and rq^2 - |centre|^2 (b).
-struct SlotPre {
-  LineSide l;
-  float b;  // -1 - slack; an unfilled slot is apart from everything
-};
-
 // Shifts a pair's verdict into the word: 1 when the lines may come within the
 // cut distance, or (every pair) the centres within reach.
 template <bool ALL>
-__device__ __forceinline__ uint32_t may_cut(const float4 f, const float2 h, const SlotPre& q, uint32_t word) {
-  float d;
-  if (ALL)
-    d = h.x - fmaf(f.w, q.l.mx, fmaf(f.z, q.l.uz, fmaf(f.y, q.l.uy, fmaf(f.x, q.l.ux, q.b))));
-  else
-    d = line_apart(LineSide{f.x, f.y, f.z, f.w, h.x, h.y}, q.l, q.b);
-  return __builtin_amdgcn_alignbit(word, __float_as_uint(d), 31u);
+__device__ __forceinline__ uint32_t may_cut(const float4 f, const float2 h, const SlotSide& q, uint32_t word) {
+  return __builtin_amdgcn_alignbit(word, __float_as_uint(slot_apart<ALL>(f, h, q)), 31u);
 }
 
 template <bool ALL>
-__device__ __forceinline__ SlotPre slot_pre(const float4 P, const float4 D, const float3 sh, const Filter& F,
-                                            bool valid) {
-  SlotPre q;
-  const float x = (P.x + sh.x) - F.o.x, y = (P.y + sh.y) - F.o.y, z = (P.z + sh.z) - F.o.z;
-  if (ALL) {
-    const float r = (P.w * 1.000001f) * 1.000006f;
-    q.l = LineSide{valid ? x : 0.0f, valid ? y : 0.0f, valid ? z : 0.0f, r, 0.0f, 0.0f};
-    q.b = valid ? fmaf(r, r, -fmaf(z, z, fmaf(y, y, x * x))) : -3e38f;
-  } else {
-    q.l = line_side(F.ln, x, y, z, D);
-    q.b = valid ? -1.0f - F.ln.slack : 3e38f;
-  }
-  return q;
+__device__ __forceinline__ SlotSide slot_pre(const float4 P, const float4 D, const float3 sh, const Filter& F,
+                                             bool valid) {
+  return slot_side<ALL>(F.ln, (P.x + sh.x) - F.o.x, (P.y + sh.y) - F.o.y, (P.z + sh.z) - F.o.z, P.w, D, valid);
 }
 
 // Appends the pairs of one word of probes (bit k: probe base + k) with the
@@ -482,7 +460,7 @@ __device__ __forceinline__ void push_pairs(const PairArgs& a, const CellGeom& g,
 // allows (half-stencil passes).
 template <int MODE, int PREC, bool ALL, bool TWO>
 __device__ __forceinline__ void probe_loop(const PairArgs& a, const CellGeom& g, PairLds& L, uint32_t nprobe,
-                                           const SlotPre& Q0, const SlotPre& Q1, unsigned long long keep0,
+                                           const SlotSide& Q0, const SlotSide& Q1, unsigned long long keep0,
                                            unsigned long long keep1, uint32_t& qn, uint32_t& q2n, Acc& acc) {
   constexpr bool ORD = (MODE == PM_CNT || MODE == PM_GEN_NEW);
   const uint32_t lane = threadIdx.x;
@@ -697,7 +675,7 @@ __device__ void process_cell(const PairArgs& a, const CellGeom& g, uint32_t gc, 
       L.bX[lane + WAVE] = x1;
       L.bM[lane + WAVE] = m1;
       const float3 s0 = shift_f32(g, m0), s1 = shift_f32(g, m1);
-      const SlotPre Q0 = slot_pre<ALL>(p0, d0, s0, F, v0), Q1 = slot_pre<ALL>(p1, d1, s1, F, v1);
+      const SlotSide Q0 = slot_pre<ALL>(p0, d0, s0, F, v0), Q1 = slot_pre<ALL>(p1, d1, s1, F, v1);
       unsigned long long keep0 = ~0ull, keep1 = ~0ull;
       if (MODE == PM_CNT || MODE == PM_GEN_NEW) {
         keep0 = ordered(src0, m0, ps + pb);
