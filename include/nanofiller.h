@@ -482,11 +482,14 @@ enum {
                                 1 << shift work items (-1: by the cell's cost)         */
   NF_OPT_SPLIT_MIN = 13,     /* probes per work item of a dealt cell, at least
                                 (0: by the cell's cost; either option set: 1 and 32)   */
-  NF_OPT_TEST_ALL_PAIRS = 14 /* 1: the generation passes test every pair within reach,
+  NF_OPT_TEST_ALL_PAIRS = 14,/* 1: the generation passes test every pair within reach,
                                 so that the pair-test count is the oracle's;
                                 0 (default): pairs whose lines stay apart are left out
                                 and a proposal leaves its stencil walk once an accepted
                                 rod cuts it (same decisions, fewer tests)               */
+  NF_OPT_CROSSING_LISTS = 15 /* generation: 1 (default): instances whose rods suit it
+                                test their pairs over lists of the rods that cross each
+                                cell; 0: every instance over cell pairs (same packing)  */
 };
 /* Candidate pairs of nf_contacts.  Both give the same contact list.
  * FOOTPRINT: each rod binned into the fine cells its capsule (radius

@@ -391,8 +391,9 @@ void launch_reset(GenBuffers& b, hipStream_t s) {
 void launch_round(GenBuffers& b, int prec, int diag, hipStream_t s, hipEvent_t* ev) {
   const int n = b.n_inst;
   if (ev) (void)hipEventRecord(ev[0], s);
-  // crossing lists, unless every pair within reach has to be tested
-  const bool walk = b.walk && !b.tiles.test_all;
+  // crossing lists, unless they are switched off or every pair within reach has
+  // to be tested
+  const bool walk = b.walk && b.tiles.lists && !b.tiles.test_all;
   const bool cells = b.cellwise || !walk;
   // a cell's longest rod bounds the cell pairs only; of one length, the start's
   // holds (an atomic per candidate at 30 G/s otherwise)

@@ -130,6 +130,7 @@ struct PairTiles {
   int32_t part_shift = -1; // work items per dense cell (reject vs accepted), as a shift
   uint32_t split_min = 0;  // probes per part of a split cell, at least
   uint32_t test_all = 0;   // reject vs accepted: cut proposals stay in the walk (every pair within reach tested)
+  uint32_t lists = 1;      // crossing lists where an instance has them (NF_OPT_CROSSING_LISTS)
 };
 
 struct GenBuffers {
