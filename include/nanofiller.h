@@ -478,8 +478,10 @@ enum {
    * depend on it; nanofiller_amd/autotune.py picks it per workload): */
   NF_OPT_WAVES_OLD = 10,     /* waves per CU, reject vs accepted (0: default 16)     */
   NF_OPT_WAVES_NEW = 11,     /* waves per CU, reject vs same-round (0: default 16)   */
-  NF_OPT_PART_SHIFT = 12,    /* reject vs accepted: a dense cell is dealt over at most
-                                1 << shift work items (-1: by the cell's cost)         */
+  NF_OPT_PART_SHIFT = 12,    /* reject vs accepted over cell pairs (without effect on
+                                instances with crossing lists, as SPLIT_MIN is): a
+                                dense cell is dealt over at most 1 << shift work items
+                                (-1: by the cell's cost)                               */
   NF_OPT_SPLIT_MIN = 13,     /* probes per work item of a dealt cell, at least
                                 (0: by the cell's cost; either option set: 1 and 32)   */
   NF_OPT_TEST_ALL_PAIRS = 14,/* 1: the generation passes test every pair within reach,

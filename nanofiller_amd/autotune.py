@@ -15,12 +15,12 @@ alone - so tuning changes speed only; the tests check that.
 Launch shape (--tiles): per workload (the 20k-, 500k-, 4M- and 8M-rod
 packings and the 256-packing batch), the generation cell edge as a factor of
 the library's default (single packings without a set cell size), the waves
-per CU of the reject-vs-accepted and same-round passes, and for launches
-with few cells per wave the split of a dense cell (work items as a shift,
-and the probes per item at least), by one pass of coordinate descent over
-the generation time from the library's defaults, keeping a change for a
-gain over 2%.  The batch's launches have a million cells, so only its wave
-counts are tuned.  The packing does not depend on any of these
+per CU of the reject-vs-accepted and same-round passes, and where the passes
+run over cell pairs the split of a dense cell (work items as a shift, and the
+probes per item at least; the passes over crossing lists have no such split),
+by one pass of coordinate descent over the generation time from the library's
+defaults, keeping a change for a gain over 2%.  The packing does not depend
+on any of these
 (test_tile_shape_does_not_change_packing, test_cell_size_does_not_change_packing).
 
 Usage: python -m nanofiller_amd.autotune [--factors 0.7,0.85,1,1.2,1.4]
@@ -70,15 +70,17 @@ def _gen_ms(params, tiles: dict, repeats: int) -> float:
 def tile_workloads() -> dict:
     """The workloads the launch shape is tuned on: parameters, keys tuned,
     repeats."""
-    launch = ["waves_old", "waves_new", "part_shift", "split_min"]
+    waves = ["waves_old", "waves_new"]
     return {
-        # the 20k case keeps its 1 um cells (the reference's domain grid)
-        "20k": (configs.cfg1(NF_PREC_FP32_RECHECK), launch, 3),
-        "500k": (configs.cfg2(NF_PREC_FP32_RECHECK, tuned=False), ["cell_factor"] + launch, 5),
-        "4M": (configs.cfg4(NF_PREC_FP32_RECHECK, tuned=False), ["cell_factor"] + launch, 3),
-        "8M": (configs.cfg5(NF_PREC_FP32_RECHECK, tuned=False), ["cell_factor", "waves_old", "waves_new"], 1),
-        # per-bucket cell factors (tune()); its launches hold a million cells
-        "batch256": (configs.cfg3(NF_PREC_FP32_RECHECK), ["waves_old", "waves_new"], 1),
+        # over crossing lists; the 20k case keeps its 1 um cells (the
+        # reference's domain grid)
+        "20k": (configs.cfg1(NF_PREC_FP32_RECHECK), waves, 3),
+        "500k": (configs.cfg2(NF_PREC_FP32_RECHECK, tuned=False), ["cell_factor"] + waves, 5),
+        # over cell pairs
+        "4M": (configs.cfg4(NF_PREC_FP32_RECHECK, tuned=False), ["cell_factor"] + waves + ["part_shift", "split_min"], 3),
+        "8M": (configs.cfg5(NF_PREC_FP32_RECHECK, tuned=False), ["cell_factor"] + waves, 1),
+        # per-bucket cell factors (tune())
+        "batch256": (configs.cfg3(NF_PREC_FP32_RECHECK), waves, 1),
     }
 
 

@@ -464,7 +464,7 @@ void launch_round(GenBuffers& b, int prec, int diag, hipStream_t s, hipEvent_t* 
   w.surv = b.surv;
   w.diag = diag;
   w.qctr = b.queues + Q_WALK_OLD * QWORDS;
-  if (walk) launch_walk(PM_GEN_OLD, prec, w, s);
+  if (walk) launch_walk(PM_GEN_OLD, prec, w, s, &b.tiles);
   if (cells) launch_pair(PM_GEN_OLD, prec, a, s, &b.tiles);
   if (ev) (void)hipEventRecord(ev[4], s);
   // stage 2: survivors vs higher-priority survivors, over the survivors
@@ -497,7 +497,7 @@ void launch_round(GenBuffers& b, int prec, int diag, hipStream_t s, hipEvent_t* 
   w.qctr = b.queues + Q_WALK_NEW * QWORDS;
   if (walk) {
     launch_enter(false, w, b.T_cap, s);
-    launch_walk(PM_GEN_NEW, prec, w, s);
+    launch_walk(PM_GEN_NEW, prec, w, s, &b.tiles);
   }
   if (cells) launch_pair(PM_GEN_NEW, prec, a, s, &b.tiles);
   if (ev) (void)hipEventRecord(ev[5], s);

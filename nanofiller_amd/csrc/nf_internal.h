@@ -420,7 +420,7 @@ uint32_t pair_items_max(uint64_t ncells);
 // Enters the round's accepted rods (rods: candidate slots) or the survivors
 // of the first pass in their lists.
 void launch_enter(bool accepted, const WalkArgs& a, uint64_t rods, hipStream_t s);
-void launch_walk(int mode, int prec, const WalkArgs& a, hipStream_t s);
+void launch_walk(int mode, int prec, const WalkArgs& a, hipStream_t s, const PairTiles* t = nullptr);
 void launch_enter_contacts(const WalkArgs& a, hipStream_t s);
 
 // ---- launchers (nf_seg.hip) ----

@@ -625,8 +625,12 @@ void launch_enter_contacts(const WalkArgs& a, hipStream_t s) {
   hipLaunchKernelGGL(k_enter_contacts, dim3(enter_grid(a.cnt.n)), dim3(ENTER_THREADS), 0, s, a);
 }
 
-void launch_walk(int mode, int prec, const WalkArgs& a, hipStream_t s) {
-  const dim3 grid(pair_grid(mode)), block(WAVE);
+// (whole blocks per XCD: the walk deals its chunks to eighths of the grid)
+void launch_walk(int mode, int prec, const WalkArgs& a, hipStream_t s, const PairTiles* t) {
+  uint32_t waves = t ? (mode == PM_GEN_OLD ? t->waves_old : t->waves_new) : 0u;
+  if (waves == 0u || waves > 16u) waves = 16u;
+  const uint32_t blocks = (uint32_t)(pair_grid(mode) / 16) * waves;
+  const dim3 grid((blocks + 7u) / 8u * 8u), block(WAVE);
   if (mode == PM_CNT) {
     if (prec == NF_PREC_FP64)
       hipLaunchKernelGGL((k_walk<PM_CNT, NF_PREC_FP64>), grid, block, 0, s, a);
