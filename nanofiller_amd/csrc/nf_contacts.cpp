@@ -806,83 +806,129 @@ extern "C" int nf_centre_distance(nf_handle* h, int32_t bins, double width, int6
   hipStream_t s = h->stream;
   const float4* P = h->gb.bP + h->desc[h->post_inst].rod_off;
   const float4* D = h->gb.bD + h->desc[h->post_inst].rod_off;
-  // grid: edge just over rmax and the stencil's margin (half stencil of +-1
-  // cells; at rmax itself a box of whole edges has cells two away in it, three
-  // times the candidates), finer when crowded
-  const double edge = default_cell_edge(rmax + 1.01 * (double)CELL_MARGIN, (double)n / (p.box[0] * p.box[1] * p.box[2]), 1.0);
+  const double density = (double)n / (p.box[0] * p.box[1] * p.box[2]);
   int32_t nc[3];
-  double scale[3];
-  uint64_t ncells = 1;
-  for (int a = 0; a < 3; ++a) {
-    double k = std::floor(p.box[a] / edge);
-    if (k < 1.0) k = 1.0;
-    if (k > 1024.0) k = 1024.0;
-    nc[a] = (int32_t)k;
-    scale[a] = (double)nc[a] / p.box[a];
-    ncells *= (uint64_t)nc[a];
-  }
-  if (ncells > (1ull << 26)) return fail(h, NF_E_INVALID, "statistics grid too large");
-  // the half stencil as runs of cells along x
-  std::vector<int4> st = build_stencil(nc, p.box, rmax, true);
-  std::sort(st.begin(), st.end(), [](const int4& a, const int4& b) {
-    return a.z != b.z ? a.z < b.z : (a.y != b.y ? a.y < b.y : a.x < b.x);
-  });
-  std::vector<int4> runs;
-  for (const int4& o : st) {
-    if (!runs.empty() && runs.back().z == o.y && runs.back().w == o.z && runs.back().y + 1 == o.x)
-      runs.back().y = o.x;
-    else
-      runs.push_back(make_int4(o.x, o.x, o.y, o.z));
-  }
+  auto cells_of = [&](double edge) {
+    uint64_t c = 1;
+    for (int a = 0; a < 3; ++a) {
+      nc[a] = (int32_t)std::min(std::max(std::floor(p.box[a] / edge), 1.0), 1024.0);
+      c *= (uint64_t)nc[a];
+    }
+    return c;
+  };
+  if (cells_of(default_cell_edge(rmax, density, 1.0)) > (1ull << 26))
+    return fail(h, NF_E_INVALID, "statistics grid too large");
   std::vector<double> e2(bins + 1);
   for (int k = 0; k <= bins; ++k) e2[k] = ((double)k * width) * ((double)k * width);
   float4* cP = nullptr;
   float4* cD = nullptr;
-  uint32_t *cid = nullptr, *cstart = nullptr, *ccount = nullptr;
+  uint32_t *cid = nullptr, *cstart = nullptr, *ccount = nullptr, *cells = nullptr;
   float* chl = nullptr;
   int4* dst = nullptr;
   double* de2 = nullptr;
   unsigned long long *out = nullptr, *part = nullptr;
   int rc = NF_OK;
   const uint64_t n1 = std::max<uint64_t>(n, 1);
+  BinScratch bs;
+  std::vector<int4> runs;
+  uint64_t ncells = 0;
+  auto release_grid = [&]() {
+    void* w[] = {cstart, ccount, chl, dst};
+    for (void* q : w) dfree(h, q);
+    free_bin_scratch(h, &bs);
+    cstart = ccount = nullptr;
+    chl = nullptr;
+    dst = nullptr;
+  };
+  // the rods on cells of `edge`, and the half stencil as runs of cells along x
+  auto layout = [&](double edge) -> int {
+    release_grid();
+    ncells = cells_of(edge);
+    double scale[3];
+    for (int a = 0; a < 3; ++a) scale[a] = (double)nc[a] / p.box[a];
+    std::vector<int4> st = build_stencil(nc, p.box, rmax, true);
+    std::sort(st.begin(), st.end(), [](const int4& a, const int4& b) {
+      return a.z != b.z ? a.z < b.z : (a.y != b.y ? a.y < b.y : a.x < b.x);
+    });
+    runs.clear();
+    for (const int4& o : st) {
+      if (!runs.empty() && runs.back().z == o.y && runs.back().w == o.z && runs.back().y + 1 == o.x)
+        runs.back().y = o.x;
+      else
+        runs.push_back(make_int4(o.x, o.x, o.y, o.z));
+    }
+    int r = dalloc(h, &cstart, ncells + 1);
+    if (r == NF_OK) r = dalloc(h, &ccount, ncells);
+    if (r == NF_OK) r = dalloc(h, &chl, ncells);
+    if (r == NF_OK) r = dalloc(h, &dst, runs.size());
+    if (r != NF_OK) return r;
+    const hipError_t u = hipMemcpyAsync(dst, runs.data(), sizeof(int4) * runs.size(), hipMemcpyHostToDevice, s);
+    if (u != hipSuccess) return fail(h, NF_E_HIP, std::string("statistics upload: ") + hipGetErrorString(u));
+    return bin_rods(h, P, D, n, nc, scale, cP, cD, cid, cstart, ccount, chl, &bs);
+  };
   if (rc == NF_OK) rc = dalloc(h, &cP, n1);
   if (rc == NF_OK) rc = dalloc(h, &cD, n1);
   if (rc == NF_OK) rc = dalloc(h, &cid, n1);
-  if (rc == NF_OK) rc = dalloc(h, &cstart, ncells + 1);
-  if (rc == NF_OK) rc = dalloc(h, &ccount, ncells);
-  if (rc == NF_OK) rc = dalloc(h, &chl, ncells);
-  if (rc == NF_OK) rc = dalloc(h, &dst, runs.size());
   if (rc == NF_OK) rc = dalloc(h, &part, (size_t)CENT_BLOCKS * (bins + 3));
   if (rc == NF_OK) rc = dalloc(h, &de2, (size_t)bins + 1);
   if (rc == NF_OK) rc = dalloc(h, &out, (size_t)bins + 3);
-  BinScratch bs;
   auto release = [&]() {
-    void* w[] = {cP, cD, cid, cstart, ccount, chl, dst, de2, part, out};
+    (void)sync_stream(s, "centre distance");
+    release_grid();
+    void* w[] = {cP, cD, cid, cells, de2, part, out};
     for (void* q : w) dfree(h, q);
-    free_bin_scratch(h, &bs);
   };
   if (rc != NF_OK) {
     release();
     return rc;
   }
-  hipError_t e = hipMemcpyAsync(dst, runs.data(), sizeof(int4) * runs.size(), hipMemcpyHostToDevice, s);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(de2, e2.data(), sizeof(double) * e2.size(), hipMemcpyHostToDevice, s);
+  hipError_t e = hipMemcpyAsync(de2, e2.data(), sizeof(double) * e2.size(), hipMemcpyHostToDevice, s);
   if (e != hipSuccess) {
     release();
     return fail(h, NF_E_HIP, std::string("statistics upload: ") + hipGetErrorString(e));
   }
-  fill_u32((uint32_t*)out, 0u, 2 * ((uint64_t)bins + 3), s);
-  rc = bin_rods(h, P, D, n, nc, scale, cP, cD, cid, cstart, ccount, chl, &bs);
-  if (rc != NF_OK) {
-    (void)sync_stream(s, "centre distance");
-    release();
-    return rc;
+  // grid: edge just over rmax and the stencil's margin (half stencil of +-1
+  // cells; at rmax itself a box of whole edges has cells two away in it, three
+  // times the candidates), finer when crowded.  Where that makes many cells,
+  // wide enough for 16 rods a cell, so that a run of three fills a wave's 64
+  // lanes: 300,000 rods within 0.05 um of each other 29 ms on cells of that edge
+  // (most of them empty), with 4, 8, 16, 24 rods a cell 0.27, 0.20, 0.155, 0.175
+  // ms; 1M rods within 0.13 um 6.9 and 0.78, 0.53, 0.39, 0.44 ms.  17,500 cells
+  // for 2,000 rods take 80 us, with the look at their crowding below 75-98;
+  // 23,000 for 20,000 rods 110, 97-111.
+  const double near_edge = default_cell_edge(rmax + 1.01 * (double)CELL_MARGIN, density, 1.0);
+  double edge = near_edge;
+  if (density > 0.0 && cells_of(near_edge) > 16384) edge = std::max(near_edge, std::cbrt(16.0 / density));
+  rc = layout(edge);
+  double mean = (double)n / (double)std::max<uint64_t>(ncells, 1);  // rods in a cell that holds any
+  if (rc == NF_OK && edge > near_edge) {
+    // Widened cells suit rods that are spread out: where a rod shares its cell
+    // with four times the others that it would in an even packing (agglomerates
+    // three times as dense as the mean reach two), cells for 16 of the rods as
+    // they lie, and the empty ones, most then, are left out by a list.
+    HostScalars* scalars = host_scalars(h);
+    fill_u32((uint32_t*)out, 0u, 2, s);
+    launch_cent_crowd(ccount, ncells, out, s);
+    e = scalars_to_host(h, scalars->ctr, out, sizeof(unsigned long long));
+    if (e == hipSuccess) e = sync_stream(s, "centre distance");
+    const double crowd = (double)scalars->ctr[0] / (double)n1;
+    if (e == hipSuccess && crowd > 4.0 * (mean + 1.0)) {
+      const double cell = p.box[0] * p.box[1] * p.box[2] / (double)ncells;
+      rc = layout(std::max(near_edge, std::cbrt(16.0 * cell / crowd)));
+      mean = std::max(16.0, crowd * p.box[0] * p.box[1] * p.box[2] / (double)ncells / cell);
+      if (rc == NF_OK) rc = dalloc(h, &cells, std::min<uint64_t>(n1, ncells) + 1);
+      if (rc == NF_OK) launch_cent_cells(ccount, ncells, cells, s);
+    }
   }
+  if (rc != NF_OK || e != hipSuccess) {
+    release();
+    return rc != NF_OK ? rc : fail(h, NF_E_HIP, std::string("centre distance: ") + hipGetErrorString(e));
+  }
+  fill_u32((uint32_t*)out, 0u, 2 * ((uint64_t)bins + 3), s);
   const double Lmax = std::max(p.box[0], std::max(p.box[1], p.box[2]));
   const float ew = (float)(5.9604644775390625e-8 * (Lmax + rmax) * 1.01);
   const float rf = (float)rmax + 8.0f * ew;
-  launch_cent(cP, cid, cstart, ccount, dst, (uint32_t)runs.size(), n, nc, p.box, de2, bins, width,
+  launch_cent(cP, cid, cstart, ccount, cells, dst, (uint32_t)runs.size(), mean, nc, p.box, de2, bins, width,
               rf * rf * 1.00001f, part, out, s);
   std::vector<unsigned long long> hout((size_t)bins + 3);
   const HostPart out_part = {hout.data(), out, sizeof(unsigned long long) * hout.size()};

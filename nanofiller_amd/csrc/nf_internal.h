@@ -482,8 +482,14 @@ void launch_selftest_pairs(const float* ra, const float* rb, const double* sh, u
                            int32_t* out_within, hipStream_t s);
 constexpr int CENT_BINS_MAX = 1024;
 constexpr int CENT_BLOCKS = 2048;  // part holds CENT_BLOCKS x (bins + 3) words
+// out (cleared): the rods' sum of the rods in their cells (each itself included).
+void launch_cent_crowd(const uint32_t* count, uint64_t ncells, unsigned long long* out, hipStream_t s);
+// cells[0]: how many cells hold rods; cells[1..]: those cells, in any order.
+void launch_cent_cells(const uint32_t* count, uint64_t ncells, uint32_t* cells, hipStream_t s);
+// cells: launch_cent_cells' list, or null for every cell; mean: rods in a cell that holds any.
 void launch_cent(const float4* P, const uint32_t* X, const uint32_t* start, const uint32_t* count,
-                 const int4* runs, uint32_t n_runs, uint32_t n, const int32_t nc[3], const double box[3],
+                 const uint32_t* cells, const int4* runs, uint32_t n_runs, double mean, const int32_t nc[3],
+                 const double box[3],
                  const double* e2, int bins, double width, float r2f, unsigned long long* part,
                  unsigned long long* out, hipStream_t s);
 void launch_vdw(const float4* P, const float4* D, uint32_t n, const uint32_t* rowptr,

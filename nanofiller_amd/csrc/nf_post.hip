@@ -344,6 +344,7 @@ struct CentArg {
   const uint32_t* X;  // rod ids
   const uint32_t* start;
   const uint32_t* count;
+  const uint32_t* cells;  // their number, then the cells that hold rods; null: every cell
   const int4* runs;  // first and last x offset, y and z offset
   uint32_t n_runs, chunks, chunk;  // a cell's rods in `chunks` shares of `chunk` at a time
   int32_t nc[3];
@@ -414,9 +415,11 @@ __global__ void __launch_bounds__(CENT_THREADS) k_cent(const float4* __restrict_
   CentAcc acc = {0ull, 0ull, 0ull};
   uint32_t qn = 0u;
   const uint32_t per_cell = a.n_runs * a.chunks;
-  const uint64_t items = (uint64_t)a.nc[0] * (uint64_t)a.nc[1] * (uint64_t)a.nc[2] * per_cell;
+  const uint64_t items =
+      (a.cells ? (uint64_t)uni_u32(a.cells[0]) : (uint64_t)a.nc[0] * (uint64_t)a.nc[1] * (uint64_t)a.nc[2]) * per_cell;
   for (uint64_t t = blockIdx.x * (CENT_THREADS / WAVE) + wave; t < items; t += gridDim.x * (CENT_THREADS / WAVE)) {
-    const uint32_t cell = uni_u32((uint32_t)(t / per_cell)), part_of = uni_u32((uint32_t)(t % per_cell));
+    const uint32_t at = uni_u32((uint32_t)(t / per_cell)), part_of = uni_u32((uint32_t)(t % per_cell));
+    const uint32_t cell = a.cells ? uni_u32(a.cells[at + 1u]) : at;
     const uint32_t c = part_of % a.chunks;
     const int4 run = a.runs[part_of / a.chunks];
     const uint32_t pc = uni_u32(a.count[cell]), ps = uni_u32(a.start[cell]);
@@ -498,14 +501,57 @@ __global__ void __launch_bounds__(CENT_THREADS) k_cent_total(const unsigned long
   if (s) atomicAdd(&out[k], s);
 }
 
+// Rods in their cells, summed over the rods.
+__global__ void __launch_bounds__(CENT_THREADS) k_cent_crowd(const uint32_t* __restrict__ count, uint64_t ncells,
+                                                             unsigned long long* __restrict__ out) {
+  unsigned long long s = 0;
+  for (uint64_t c = (uint64_t)blockIdx.x * CENT_THREADS + threadIdx.x; c < ncells; c += (uint64_t)gridDim.x * CENT_THREADS)
+    s += (unsigned long long)count[c] * count[c];
+  s = wave_sum_u64(s);
+  if (threadIdx.x % WAVE == 0 && s) atomicAdd(out, s);
+}
+
+void launch_cent_crowd(const uint32_t* count, uint64_t ncells, unsigned long long* out, hipStream_t s) {
+  hipLaunchKernelGGL(k_cent_crowd, dim3(std::min(grid_for(ncells, 4 * CENT_THREADS), 64)), dim3(CENT_THREADS), 0, s, count,
+                     ncells, out);
+}
+
+// The cells that hold rods: a block takes the places of its own with one atomic.
+__global__ void __launch_bounds__(CENT_THREADS) k_cent_cells(const uint32_t* __restrict__ count, uint64_t ncells,
+                                                             uint32_t* __restrict__ cells) {
+  __shared__ uint32_t sh[CENT_THREADS / WAVE], base;
+  const uint32_t lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+  for (uint64_t c0 = (uint64_t)blockIdx.x * CENT_THREADS; c0 < ncells; c0 += (uint64_t)gridDim.x * CENT_THREADS) {
+    const uint64_t c = c0 + threadIdx.x;
+    const bool some = c < ncells && count[c] != 0u;
+    const unsigned long long m = __ballot(some);
+    if (lane == 0) sh[wave] = (uint32_t)__popcll(m);
+    __syncthreads();
+    uint32_t before = 0, all = 0;
+    for (uint32_t w = 0; w < CENT_THREADS / WAVE; ++w) {
+      before += w < wave ? sh[w] : 0u;
+      all += sh[w];
+    }
+    if (threadIdx.x == 0 && all) base = atomicAdd(&cells[0], all);
+    __syncthreads();
+    if (some) cells[1u + base + before + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = (uint32_t)c;
+  }
+}
+
+void launch_cent_cells(const uint32_t* count, uint64_t ncells, uint32_t* cells, hipStream_t s) {
+  fill_u32(cells, 0u, 1, s);
+  hipLaunchKernelGGL(k_cent_cells, dim3(grid_for(ncells, CENT_THREADS)), dim3(CENT_THREADS), 0, s, count, ncells, cells);
+}
+
 void launch_cent(const float4* P, const uint32_t* X, const uint32_t* start, const uint32_t* count,
-                 const int4* runs, uint32_t n_runs, uint32_t n, const int32_t nc[3], const double box[3],
-                 const double* e2, int bins, double width, float r2f, unsigned long long* part,
+                 const uint32_t* cells, const int4* runs, uint32_t n_runs, double mean, const int32_t nc[3],
+                 const double box[3], const double* e2, int bins, double width, float r2f, unsigned long long* part,
                  unsigned long long* out, hipStream_t s) {
   CentArg a;
   a.X = X;
   a.start = start;
   a.count = count;
+  a.cells = cells;
   a.runs = runs;
   a.n_runs = n_runs;
   for (int d = 0; d < 3; ++d) {
@@ -518,10 +564,12 @@ void launch_cent(const float4* P, const uint32_t* X, const uint32_t* start, cons
   a.inv_width = (float)(1.0 / width);
   // shares of 32 probes, of fewer where cells and runs alone leave the chip idle
   const uint64_t cr = (uint64_t)nc[0] * nc[1] * nc[2] * n_runs;
-  const uint64_t mean = (uint64_t)n / ((uint64_t)nc[0] * nc[1] * nc[2]) + 1;
+  const uint64_t rods = (uint64_t)mean + 1;
   a.chunk = 32;
-  while (a.chunk > 4 && cr * ((mean + a.chunk - 1) / a.chunk) < 16384) a.chunk /= 2;
-  a.chunks = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((mean + a.chunk - 1) / a.chunk, 65536 / std::min<uint64_t>(cr, 65536)));
+  while (a.chunk > 4 && cr * ((rods + a.chunk - 1) / a.chunk) < 16384) a.chunk /= 2;
+  // (a list's cells are few among cr)
+  const uint64_t most = cells ? 64 : 65536 / std::min<uint64_t>(cr, 65536);
+  a.chunks = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((rods + a.chunk - 1) / a.chunk, most));
   const int blocks = std::min(grid_for(cr * a.chunks, CENT_THREADS / WAVE), CENT_BLOCKS);
   hipLaunchKernelGGL(k_cent, dim3(blocks), dim3(CENT_THREADS), 0, s, P, a, part);
   const uint32_t words = (uint32_t)bins + 3;
