@@ -434,21 +434,33 @@ std::vector<int4> build_stencil(const int32_t nc[3], const double box[3], double
 // Which packings: entering a rod costs some seven device-scope atomics, the
 // cell-pair engine a number of staged pairs that grows with crowding (rods
 // per excluded volume), with the spread of the lengths (its cells are as wide
-// as the longest) and with the rounds.  Whole generations of constant-length
-// rods at 0.5 / 1 / 1.5 rods per excluded volume, cells of one reach against
-// lists: 200,000 rods 0.97 / 1.53 / 2.03 against 0.94 / 1.32 / 1.79 ms, 1M
-// 1.77 / 2.86 / 4.40 against 2.21 / 3.26 / 4.38 ms, 4M 4.7 / 7.9 / 12.6
-// against 7.1 / 10.7 / 15.1 ms; at 0.25 200,000 rods 0.55 against 0.62 ms.
-// Log-normal lengths, 1M rods: 3.2 / 6.8 / 11.6 against 2.4 / 3.5 / 4.5 ms.
-//
-// peak: densest point over the mean.
+// as the longest), with the rounds and, where every pair that the filter leaves
+// is evaluated in FP64, with the precision.  Rods of one length take the lists
+// from this many per excluded volume on; whole generations, cells of one reach
+// against lists, at 0.31 / 0.52 / 0.83 / 1.25 / 1.66 / 2.1 / 2.7 in ms:
+//   FP32   100,000  .30 .60 .83 1.08 1.40 1.67 2.51    .31 .48 .71  .90 1.12 1.40 1.91
+//          300,000  .40 .81 1.29 1.52 2.03 2.52 3.88   .44 .78 1.10 1.31 1.74 2.08 2.89
+//          450,000  .48 .95 1.48 1.80 2.49 3.01 5.08   .57 .99 1.37 1.70 2.19 2.65 3.71
+//          1M       .80 1.38 2.20 2.75 4.12 5.41 8.44  1.08 1.81 2.40 3.08 4.18 5.06 6.82
+//          4M       2.63 4.01 6.17 8.54 13.0 17.9 30.6 4.15 6.50 8.62 11.4 15.0 18.1 23.9
+//   FP64   700,000  .82 1.82 3.00 3.35 4.91 5.82 8.65  .82 1.29 1.82 2.28 3.02 3.55 4.97
+//          1M       1.00 2.01 3.28 3.87 5.64 6.96 10.7 1.07 1.81 2.39 3.04 4.11 4.98 6.75
+//          1.5M     1.25 2.42 3.87 4.83 7.00 8.78 14.4 1.57 2.52 3.47 4.33 5.77 7.15 9.47
+//          2.5M     1.82 3.20 5.17 6.80 10.1 13.3 20.6 2.76 4.16 5.65 7.30 9.74 11.8 15.5
+//          4M       2.68 4.46 7.10 9.53 14.4 18.8 31.6 4.15 6.49 8.55 11.4 14.9 18.3 23.8
+// Log-normal lengths take them always: at 0.3 / 1 / 2.1 100,000 rods .42 1.37 2.59
+// against .32 .85 1.32 ms, 4M 7.2 21.1 54.7 against 4.4 10.9 19.0.
+static double lists_from(uint32_t n, bool fp64) {
+  if (fp64) return n <= 700000u ? 0.0 : n <= 1000000u ? 0.4 : n <= 2000000u ? 0.65 : n <= 3000000u ? 1.55 : 1.9;
+  return n <= 100000u ? 0.0 : n <= 300000u ? 0.4 : n <= 500000u ? 0.75 : n <= 1000000u ? 1.65 : 2.05;
+}
+
+// An instance's crossing lists.  peak: densest point over the mean.
 static void plan_fine(const nf_params& p, InstDesc& d, double peak) {
   FineGrid& g = d.fine;
   const double V = p.box[0] * p.box[1] * p.box[2];
   const double crowd = (double)p.n_rods * excluded_volume(p.len, p.radius) / V;
-  if (p.len_law == NF_LEN_CONST &&
-      ((p.n_rods > 300000u && crowd < 1.6) || (p.n_rods > 100000u && crowd < 0.4)))
-    return;
+  if (p.len_law == NF_LEN_CONST && crowd < lists_from(p.n_rods, p.precision == NF_PREC_FP64)) return;
   const double r = 0.50001 * (double)d.R_max + 16.0 * (double)d.ew;
   double E = 1.5 * std::cbrt(V / (double)p.n_rods);
   E = std::min(std::max(E, p.len / 16.0), p.len / 1.5);

@@ -1,0 +1,39 @@
+"""Packings on both sides of the size and crowding from which rods of one length
+take crossing lists, in both precisions: the same packing over lists or cells,
+and the grid that state files name."""
+import numpy as np
+import pytest
+
+import nanofiller_amd as nf
+
+pytestmark = pytest.mark.gpu
+
+EXCLUDED = 0.5 * np.pi * 0.01 + 2.0 * np.pi * 1e-4 + 4.0 / 3.0 * np.pi * 1e-6  # of 1 um rods, 5 nm radius
+COUNTERS = ("n_accepted", "rounds", "status", "candidates", "proposals", "rejected_old", "rejected_new")
+
+
+def _params(n, crowd, prec):
+    edge = (n * EXCLUDED / crowd) ** (1.0 / 3.0)
+    return nf.normalize(nf.default_params(box=(edge,) * 3, n_rods=n, len=1.0, radius=0.005, seed=13, max_rounds=30,
+                                          precision=prec))
+
+
+@pytest.mark.parametrize("n,crowd,prec", [
+    (100001, 0.35, 1), (250000, 0.45, 1), (310000, 0.7, 1), (310000, 0.8, 1), (600000, 1.6, 1), (600000, 1.7, 1),
+    (1100000, 1.9, 1), (1100000, 2.2, 1), (600000, 0.1, 0), (800000, 0.35, 0), (800000, 0.5, 0), (1200000, 0.6, 0),
+    (1200000, 0.7, 0), (2200000, 1.4, 0), (2200000, 1.6, 0)])
+def test_same_packing_over_lists_and_cells(n, crowd, prec, tmp_path):
+    p = _params(n, crowd, prec)
+    got = []
+    for options in (None, {nf.NF_OPT_CROSSING_LISTS: 0}):
+        with nf.Packing(p, options) as pk:
+            got.append((pk.generate()[0], pk.rods()))
+            if options is None and n < 400000:
+                pk.save_state(str(tmp_path / "s.bin"))
+    for k in COUNTERS:
+        assert getattr(got[0][0], k) == getattr(got[1][0], k), k
+    assert got[0][0].rejected_new > 0
+    np.testing.assert_array_equal(got[0][1].view(np.uint32), got[1][1].view(np.uint32))
+    if n < 400000:
+        reach = p.len * 1.000001 + 2.0 * p.radius
+        assert nf.read_state_header(str(tmp_path / "s.bin"))["ext"] == (int(p.box[0] / (0.85 * reach)),) * 3
