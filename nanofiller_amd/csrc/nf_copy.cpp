@@ -29,7 +29,7 @@ constexpr size_t PIN_SMALL = 256u << 10, PIN_LARGE = 8u << 20;
 constexpr int SLOTS = 8;                       // chunks of the large block
 constexpr size_t THREADS_FROM = 8u << 20;      // bytes from which helpers copy
 constexpr int HELPERS = 4;
-constexpr size_t PLAIN_TO = 768u << 10;        // bytes up to which plain copies may be quicker (to_host)
+constexpr size_t PLAIN_TO = 768u << 10;        // bytes of one array up to which a plain copy is quicker (to_host)
 
 // The handle's pinned block, at least `bytes` of it (at most PIN_LARGE); null
 // if the host has no pinned memory left.
@@ -197,13 +197,13 @@ hipError_t to_host(nf_handle* h, const HostPart* parts, size_t n_parts) {
       if (parts[i].bytes) e = hipMemcpy(parts[i].dst, parts[i].src, parts[i].bytes, hipMemcpyDeviceToHost);
     return e;
   };
-  // Where nothing is queued that a copy would have to wait for, plain copies of
-  // little are back sooner.  One array, staged and plain: 80 bytes 26 and 14 us,
-  // 24 KB 27 and 10 (in some processes 31), 74 KB 26 and 12, 310 KB 45 and 24,
-  // 960 KB 73 and 51 (into fresh memory 173 and 159), 2.2 MB 90 and 134; four
-  // arrays of 250 KB together 52 and 59, of 620 KB 82 and 73, of 1.9 MB 98 and 114.
-  const bool little = total <= PLAIN_TO && (some == 1 || total > PIN_SMALL);
-  if (little && hipStreamQuery(h->stream) == hipSuccess) return plain();
+  // Where nothing is queued that a copy would have to wait for, a plain copy of
+  // one short array is back sooner.  Staged and plain, into memory in use / never
+  // touched: 72 bytes 28 and 13 us; 24 KB 25 / 28 and 28 / 32; 164 KB 28 / 60 and
+  // 16 / 43; 310 KB 42 / 80 and 23 / 74; 960 KB 68 / 219 and 49 / 211; 2.2 MB 84 /
+  // 451 and 132 / 586.  Several arrays share the staging: four of 480 KB together
+  // 75 / 134 and 71 / 150.
+  if (some == 1 && total <= PLAIN_TO && hipStreamQuery(h->stream) == hipSuccess) return plain();
   const bool done = staged(h, parts, n_parts, [&](size_t i, size_t off, size_t bytes, char* to) {
     launch_to_pinned((const char*)parts[i].src + off, bytes, to, h->stream);
     return hipGetLastError();
