@@ -287,6 +287,11 @@ double nf::excluded_volume(double L, double a) {
   return 0.5 * PI * D * L * L + 2.0 * PI * D * D * L + (4.0 * PI / 3.0) * D * D * D;
 }
 
+RodMean nf::rod_mean(const nf_handle* h, int inst) {
+  if (!h->generated && h->given[inst].radius > 0.0) return h->given[inst];
+  return {h->params[inst].len, h->params[inst].radius};
+}
+
 extern "C" int nf_params_normalize(nf_params* p) {
   for (int d = 0; d < 3; ++d) {
     if (!(p->box[d] > 0.0)) return fail(nullptr, NF_E_INVALID, "box edges must be > 0");
@@ -842,6 +847,7 @@ extern "C" int nf_create_batch(const nf_params* ps, int n, nf_handle** out) {
     return fail(nullptr, NF_E_HIP, std::string("upload failed: ") + hipGetErrorString(e));
   }
   h->n_rods.assign(n, 0);
+  h->given.assign(n, RodMean{0.0, 0.0});
   h->planned_cap.resize(n);
   h->planned_list.resize(n);
   for (int i = 0; i < n; ++i) {
@@ -1240,6 +1246,7 @@ static int generate_once(nf_handle* h, nf_gen_stats* stats, std::vector<std::pai
     }
   }
   h->generated = true;
+  h->given.assign(h->given.size(), RodMean{0.0, 0.0});
   h->cb.valid = false;
   h->cb.net_valid = false;
   h->cb.nd_valid = false;
@@ -1262,8 +1269,11 @@ extern "C" int nf_set_rods(nf_handle* h, int inst, const float* rods, uint32_t n
   if (!h || inst < 0 || inst >= (int)h->params.size()) return fail(h, NF_E_INVALID, "bad instance");
   if (n > h->desc[inst].n_target) return fail(h, NF_E_CAPACITY, "more rods than the instance target");
   if (n && !rods) return fail(h, NF_E_INVALID, "null rods");
+  RodMean sum = {0.0, 0.0};
   for (uint32_t i = 0; i < n; ++i) {
     const float* r = rods + 8 * (size_t)i;
+    sum.len += r[6];
+    sum.radius += r[7];
     if (!(r[6] > 0.0f) || !(r[7] > 0.0f)) return fail(h, NF_E_INVALID, "rod length and radius must be > 0");
     for (int a = 0; a < 3; ++a)
       if (!(r[a] >= 0.0f && r[a] < (float)h->params[inst].box[a]))
@@ -1272,6 +1282,7 @@ extern "C" int nf_set_rods(nf_handle* h, int inst, const float* rods, uint32_t n
   const uint32_t off = h->desc[inst].rod_off;
   HIPCHK(h, rods_to_device(h, rods, n, h->gb.bP + off, h->gb.bD + off));
   h->n_rods[inst] = n;
+  h->given[inst] = n ? RodMean{sum.len / n, sum.radius / n} : RodMean{0.0, 0.0};
   h->generated = false;
   h->cb.valid = false;
   h->cb.net_valid = false;

@@ -218,7 +218,7 @@ static bool contact_fine(nf_handle* h, uint32_t n, float dev, double gap, double
   const nf_params& p = h->params[h->post_inst];
   if (n == 0 || !(dev <= 1e-3f)) return false;
   const double V = p.box[0] * p.box[1] * p.box[2];
-  const double typ = p.len_law == NF_LEN_LOGNORMAL ? p.len : 2.0 * (double)c.hl_max;
+  const double typ = p.len_law == NF_LEN_LOGNORMAL ? rod_mean(h, h->post_inst).len : 2.0 * (double)c.hl_max;
   double E = std::min(std::max(1.5 * std::cbrt(V / (double)n), typ / 16.0), typ / 1.5);
   *g = seg_grid(p.box, E, (double)c.a_max, gap, ew);
   if (4.0 * (double)g->r > E) {
@@ -583,24 +583,37 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, Co
   return NF_OK;
 }
 
-// Crossing lists where they are the faster way.  A whole call, home cells
-// against lists, MI355X: 20,000 rods 0.41 / 0.35 ms (a home cell's work runs on
-// one wave, and there are few), 2,000 0.46 / 0.30; 100,000 rods of one length
-// 0.41 / 0.47, 1M 1.0 / 1.2, 4M 3.1 / 3.9 (entering pays an atomic per rod and
-// cell); at two to four rods per excluded volume 200,000 0.81 / 0.74, 500,000
-// 1.28 / 1.25, 800,000 1.72 / 1.96.  Log-normal lengths, one rod per excluded
-// volume, 300,000 rods 0.73 / 0.64, 600,000 0.97 / 0.90, 1M 1.24 / 1.25; at a
-// quarter 0.49 / 0.52.  In FP64 home cells evaluate every candidate in full,
-// the lists only what the line filter leaves: 800,000 rods at one to four per
-// excluded volume 3.5..7.2 / 1.5..3.4, 600,000 at a half 0.75 / 1.0 ms.
+// Crossing lists where they are the faster way: home cells run a cell's work on
+// one wave, which leaves the chip idle on small packings, and evaluate every
+// candidate in FP64 in full; the lists pay an atomic per rod and cell entered.
+// Whole calls, home cells against lists, in us (rods in thousands):
+//   one length, FP32, at 0.5 / 1 / 2 / 3 rods per excluded volume
+//     20   281 276 296 448    222 232 251 276      200   372 438 495 646     428 472 542 588
+//     40   292 292 288 457    283 302 325 391      400   475 533 702 937     515 583 699 829
+//     60   311 310 312 472    310 347 379 411      600   583 687 805 1109    598 708 934 1114
+//     100  313 324 332 499    361 399 441 495      4000  2.2 3.0 3.7 5.6 ms  2.7 3.3 4.8 6.0
+//   log-normal lengths, FP32
+//     60   354 452 532 368    324 355 393 408      1500  1.1 1.5 2.0 2.3 ms  1.2 1.45 1.9 2.3
+//     100  365 454 554 387    359 393 447 484      2500  1.6 2.3 3.1 3.7     1.9 2.5 3.2 4.0
+//     400  543 720 903 872    542 609 702 799      4000  2.4 3.4 4.6 5.8     2.9 3.5 4.7 5.6
+//   one length, FP64
+//     60   318 336 386 622    313 343 381 407      400   558 748 1202 1872   506 573 679 804
+//     100  321 397 517 831    352 390 449 483      1000  910 1463 2516 3942  770 959 1302 1649
+//     200  419 559 761 1184   419 467 534 584      8000  5.6 10.1 18.4 ms    5.2 6.6 9.7
+//   log-normal lengths, FP64
+//     100  356 531 724 628    360 390 437 489      8000  6.0 10.2 16.7 ms    5.6 7.0 9.5
+// At a quarter and less, home cells from 80,000 rods on in all of them.
 static bool lists_suit(const nf_handle* h, int prec) {
   const nf_params& p = h->params[h->post_inst];
   const uint32_t n = h->n_rods[h->post_inst];
-  const double crowd = (double)n * excluded_volume(p.len, p.radius) / (p.box[0] * p.box[1] * p.box[2]);
-  if (n <= 60000u) return true;
-  if (p.len_law == NF_LEN_LOGNORMAL && crowd >= 0.4 && n <= 800000u) return true;
-  if (prec == NF_PREC_FP64) return crowd >= 0.8 && n <= 1000000u;
-  return crowd >= 1.8 && n <= 400000u;
+  const RodMean m = rod_mean(h, h->post_inst);
+  const double crowd = (double)n * excluded_volume(m.len, m.radius) / (p.box[0] * p.box[1] * p.box[2]);
+  const bool mixed = p.len_law == NF_LEN_LOGNORMAL;
+  if (n <= 30000u) return true;
+  if (prec == NF_PREC_FP64)
+    return n <= 60000u || crowd >= 0.95 || (crowd >= 0.48 && (mixed || n >= 200000u));
+  if (mixed) return n <= 60000u || (n <= 150000u && crowd >= 0.48) || (n <= 1500000u && crowd >= 0.8);
+  return (n <= 60000u && crowd < 0.75) || (n <= 500000u && crowd >= 2.6);
 }
 
 int contacts_run(nf_handle* h, double gap, uint64_t* n_out, int prec, unsigned long long*) {

@@ -22,6 +22,14 @@ struct HostScalars {
 };
 }  // namespace nf
 
+namespace nf {
+// Mean length and radius of an instance's rods, what the choice of an engine
+// goes by.
+struct RodMean {
+  double len, radius;
+};
+}  // namespace nf
+
 // Options of nf_set_option() (declared in nanofiller.h).
 struct nf_handle {
   std::vector<nf_params> params;
@@ -40,6 +48,7 @@ struct nf_handle {
   int post_inst = 0;  // instance that contacts, statistics, network, reduce, writers, state files and expand use
   int device = 0;
   std::vector<uint32_t> n_rods;  // current rod count per instance
+  std::vector<nf::RodMean> given;  // of the rods that nf_set_rods gave (radius 0: none did)
   std::vector<uint32_t> planned_cap;  // cell slots per instance as planned (NF_OPT_SLOT_SCALE scales them)
   std::vector<std::pair<uint32_t, uint32_t>> planned_list;  // and entries per crossing list (accepted, survivors)
   std::vector<double> milestones;  // volume fractions (percent) of the state dumps, ascending
@@ -114,6 +123,8 @@ int build_contact_cells(nf_handle* h);
 // generation's bounds after nf_generate, else reduced on the device.
 int contact_bounds(nf_handle* h, uint32_t n, const float4* P, const float4* D, float* hlmax, float* amax,
                    float* dev = nullptr);
+// Of the rods as given, or as the instance's parameters draw them.
+RodMean rod_mean(const nf_handle* h, int inst);
 // Mean excluded volume of two isotropic capsules of length L and radius a.
 double excluded_volume(double L, double a);
 // Default cell edge for a typical pair reach and a mean rod density.
