@@ -848,6 +848,7 @@ extern "C" int nf_create_batch(const nf_params* ps, int n, nf_handle** out) {
   }
   h->n_rods.assign(n, 0);
   h->given.assign(n, RodMean{0.0, 0.0});
+  h->short_gap.assign(n, HUGE_VAL);
   h->planned_cap.resize(n);
   h->planned_list.resize(n);
   for (int i = 0; i < n; ++i) {
@@ -1247,6 +1248,7 @@ static int generate_once(nf_handle* h, nf_gen_stats* stats, std::vector<std::pai
   }
   h->generated = true;
   h->given.assign(h->given.size(), RodMean{0.0, 0.0});
+  h->short_gap.assign(h->short_gap.size(), HUGE_VAL);
   h->cb.valid = false;
   h->cb.net_valid = false;
   h->cb.nd_valid = false;
@@ -1283,6 +1285,7 @@ extern "C" int nf_set_rods(nf_handle* h, int inst, const float* rods, uint32_t n
   HIPCHK(h, rods_to_device(h, rods, n, h->gb.bP + off, h->gb.bD + off));
   h->n_rods[inst] = n;
   h->given[inst] = n ? RodMean{sum.len / n, sum.radius / n} : RodMean{0.0, 0.0};
+  h->short_gap[inst] = HUGE_VAL;
   h->generated = false;
   h->cb.valid = false;
   h->cb.net_valid = false;

@@ -524,6 +524,7 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, Co
     HIPCHK(h, hipGetLastError());
     if (over) {
       trace("contacts: more rods cross a cell than fit; another engine instead");
+      if (way == WAY_LISTS) h->short_gap[h->post_inst] = gap;
       free_all();
       return 1;
     }
@@ -619,8 +620,9 @@ static bool lists_suit(const nf_handle* h, int prec) {
 int contacts_run(nf_handle* h, double gap, uint64_t* n_out, int prec, unsigned long long*) {
   if (h->opt_contact_engine == NF_ENGINE_CELLS) return contacts_pass(h, gap, n_out, prec, WAY_CELLS);
   int rc = 1;
-  // (home cells or fine cells asked for by size are the footprint pass's)
-  if (h->opt_footprint_fine == 0 && h->opt_footprint_occ == 0 && lists_suit(h, prec))
+  // (home cells or fine cells asked for by size are the footprint pass's; lists
+  // that were too short for these rods at this gap or a smaller one still are)
+  if (h->opt_footprint_fine == 0 && h->opt_footprint_occ == 0 && gap < h->short_gap[h->post_inst] && lists_suit(h, prec))
     rc = contacts_pass(h, gap, n_out, prec, WAY_LISTS);
   if (rc == 1) rc = contacts_pass(h, gap, n_out, prec, WAY_SEG);
   if (rc == 1) rc = contacts_pass(h, gap, n_out, prec, WAY_CELLS);

@@ -51,6 +51,9 @@ struct nf_handle {
   std::vector<nf::RodMean> given;  // of the rods that nf_set_rods gave (radius 0: none did)
   std::vector<uint32_t> planned_cap;  // cell slots per instance as planned (NF_OPT_SLOT_SCALE scales them)
   std::vector<std::pair<uint32_t, uint32_t>> planned_list;  // and entries per crossing list (accepted, survivors)
+  // contact gap from which the crossing lists are too short for the instance's
+  // present rods (infinite: not found out)
+  std::vector<double> short_gap;
   std::vector<double> milestones;  // volume fractions (percent) of the state dumps, ascending
   std::string milestone_dir;       // where nf_generate writes them
   bool lists_in_use = false;       // a contact pass keeps its entries in the generation's lists

@@ -264,6 +264,7 @@ extern "C" int nf_reduce(nf_handle* h, int32_t min_cont, nf_reduce_info* info) {
   // and radius bounds of the handle still hold); every contact-derived
   // result refers to the old ids
   h->n_rods[h->post_inst] = kept;
+  h->short_gap[h->post_inst] = HUGE_VAL;
   release_contacts(h);
   h->reduce_ids.swap(ids);
   if (info) {

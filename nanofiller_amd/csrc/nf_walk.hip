@@ -111,16 +111,19 @@ __device__ __forceinline__ void enter(const FineGrid& g, uint32_t* __restrict__ 
                                       uint32_t* overflow, uint32_t bit) {
   const uint32_t sub = threadIdx.x & (ENTER_LANES - 1);
   uint32_t ord = 0;
+  bool over = false;
   crossed_cells(g, P, D, [&](uint32_t cell, uint32_t image) {
-    if ((ord++ & (ENTER_LANES - 1)) != sub) return;
+    if ((ord++ & (ENTER_LANES - 1)) != sub || over) return;
     const uint32_t gc = g.base + cell;
     const uint32_t at = atomicAdd(&count[gc], 1u);
     if (at < cap) {
       list[off + (uint64_t)cell * cap + at] = idx | image << ENT_BITS;
     } else {
       // no room: the instance stops and the host generates it again with
-      // longer lists; readers take at most cap entries of a list
-      atomicOr(overflow, bit);
+      // longer lists (a contact pass takes another way); readers take at most
+      // cap entries of a list, and what is not entered any more does not count
+      over = true;
+      if ((__hip_atomic_load(overflow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bit) == 0u) atomicOr(overflow, bit);
     }
   });
 }
@@ -289,6 +292,7 @@ __global__ void __launch_bounds__(WAVE, 4) k_walk(WalkArgs a) {
   __shared__ WalkLds L;
   constexpr bool CNT = MODE == PM_CNT;
   if (!CNT && wuni(a.ri->T) == 0u) return;
+  if (CNT && wuni(*a.cnt.overflow) != 0u) return;  // a list was too short: another engine's pass
   if (MODE == PM_GEN_OLD && wuni(a.ri->old) == 0u) return;
   const uint32_t lane = threadIdx.x;
   const uint32_t total = CNT ? a.cnt.n : wuni(a.prStart[a.ncells]);
