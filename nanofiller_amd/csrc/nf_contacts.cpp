@@ -284,8 +284,10 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, Co
   if (rc == NF_OK) rc = dalloc(h, &(ptr), (cnt));
   ALLOC(c.cnt, (uint64_t)n + 1);
   ALLOC(c.rowptr, (uint64_t)n + 1);
-  // pair tests, rechecks, max dd, tile bytes, append count, work counter, overflow; then the work queues
-  constexpr uint64_t CTR_WORDS = 16 + 2 * QWORDS;
+  // pair tests, rechecks, max dd, tile bytes, append count, work counter, overflow; then, on lines of their
+  // own (the waves that have ended add to the counters' line, 12 ns each, and a wave that takes its next item
+  // must not wait behind them), the work queues
+  constexpr uint64_t CTR_LINE = 2 * QSTRIDE, CTR_WORDS = CTR_LINE + 2 * QWORDS;
   ALLOC(ctr, CTR_WORDS / 2);
   ALLOC(tmp, scan_tmp_words((uint64_t)n + 1));
 #undef ALLOC
@@ -310,7 +312,7 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, Co
   }
   hipEvent_t* ev = h->ev;
   hipEventRecord(ev[0], s);
-  queues = (uint32_t*)(ctr + 8);
+  queues = (uint32_t*)ctr + CTR_LINE;
   fill_u32((uint32_t*)ctr, 0u, CTR_WORDS, s);
   PairArgs a{};
   SegCrossArgs xa{};
