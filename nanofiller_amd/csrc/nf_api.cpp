@@ -1271,11 +1271,8 @@ extern "C" int nf_set_rods(nf_handle* h, int inst, const float* rods, uint32_t n
   if (!h || inst < 0 || inst >= (int)h->params.size()) return fail(h, NF_E_INVALID, "bad instance");
   if (n > h->desc[inst].n_target) return fail(h, NF_E_CAPACITY, "more rods than the instance target");
   if (n && !rods) return fail(h, NF_E_INVALID, "null rods");
-  RodMean sum = {0.0, 0.0};
   for (uint32_t i = 0; i < n; ++i) {
     const float* r = rods + 8 * (size_t)i;
-    sum.len += r[6];
-    sum.radius += r[7];
     if (!(r[6] > 0.0f) || !(r[7] > 0.0f)) return fail(h, NF_E_INVALID, "rod length and radius must be > 0");
     for (int a = 0; a < 3; ++a)
       if (!(r[a] >= 0.0f && r[a] < (float)h->params[inst].box[a]))
@@ -1284,7 +1281,15 @@ extern "C" int nf_set_rods(nf_handle* h, int inst, const float* rods, uint32_t n
   const uint32_t off = h->desc[inst].rod_off;
   HIPCHK(h, rods_to_device(h, rods, n, h->gb.bP + off, h->gb.bD + off));
   h->n_rods[inst] = n;
-  h->given[inst] = n ? RodMean{sum.len / n, sum.radius / n} : RodMean{0.0, 0.0};
+  // (of some thousand rods: sums over all of 200,000 took 40 us)
+  RodMean sum = {0.0, 0.0};
+  const uint32_t step = n / 1024u + 1u;
+  uint32_t seen = 0;
+  for (uint32_t i = 0; i < n; i += step, ++seen) {
+    sum.len += rods[8 * (size_t)i + 6];
+    sum.radius += rods[8 * (size_t)i + 7];
+  }
+  h->given[inst] = n ? RodMean{sum.len / seen, sum.radius / seen} : RodMean{0.0, 0.0};
   h->short_gap[inst] = HUGE_VAL;
   h->generated = false;
   h->cb.valid = false;
