@@ -652,7 +652,7 @@ extern "C" int nf_get_contacts(nf_handle* h, uint32_t* row_ptr, uint32_t* col, f
                              {col, c.J, col ? sizeof(uint32_t) * nc : 0},
                              {gap, c.gap, gap ? sizeof(float) * nc : 0},
                              {image, c.img, image ? sizeof(int32_t) * nc : 0}};
-  HIPCHK(h, to_host(h, parts, 4));
+  HIPCHK(h, results_to_host(h, parts, 4));
   return NF_OK;
 }
 
@@ -662,7 +662,7 @@ extern "C" int nf_get_contact_gap64(nf_handle* h, double* gap64, uint64_t cap) {
   if (!c.valid) return fail(h, NF_E_STATE, "no contacts computed");
   if (cap < c.n_contacts) return fail(h, NF_E_CAPACITY, "buffer too small");
   const HostPart part = {gap64, c.gap64, gap64 ? sizeof(double) * c.n_contacts : 0};
-  HIPCHK(h, to_host(h, &part, 1));
+  HIPCHK(h, results_to_host(h, &part, 1));
   return NF_OK;
 }
 
@@ -672,7 +672,7 @@ extern "C" int nf_get_contact_area(nf_handle* h, double* area, uint64_t cap) {
   if (!c.valid) return fail(h, NF_E_STATE, "no contacts computed");
   if (cap < c.n_contacts) return fail(h, NF_E_CAPACITY, "buffer too small");
   const HostPart part = {area, c.area, area ? sizeof(double) * c.n_contacts : 0};
-  HIPCHK(h, to_host(h, &part, 1));
+  HIPCHK(h, results_to_host(h, &part, 1));
   return NF_OK;
 }
 

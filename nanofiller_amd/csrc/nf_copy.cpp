@@ -29,7 +29,7 @@ constexpr size_t PIN_SMALL = 256u << 10, PIN_LARGE = 8u << 20;
 constexpr int SLOTS = 8;                       // chunks of the large block
 constexpr size_t THREADS_FROM = 8u << 20;      // bytes from which helpers copy
 constexpr int HELPERS = 4;
-constexpr size_t PLAIN_TO = 768u << 10;        // bytes of one array up to which a plain copy is quicker (to_host)
+constexpr size_t PLAIN_TO = 768u << 10;        // bytes of one result up to which a plain copy is quicker
 
 // The handle's pinned block, at least `bytes` of it (at most PIN_LARGE); null
 // if the host has no pinned memory left.
@@ -183,34 +183,49 @@ struct OnDevice {
 
 }  // namespace
 
+namespace {
+
+hipError_t plain(const HostPart* parts, size_t n_parts) {
+  hipError_t e = hipSuccess;
+  for (size_t i = 0; i < n_parts && e == hipSuccess; ++i)
+    if (parts[i].bytes) e = hipMemcpy(parts[i].dst, parts[i].src, parts[i].bytes, hipMemcpyDeviceToHost);
+  return e;
+}
+
+}  // namespace
+
 hipError_t to_host(nf_handle* h, const HostPart* parts, size_t n_parts) {
   std::lock_guard<std::mutex> lock(h->pin_mu);
   OnDevice on(h->device);
   hipError_t e = hipSuccess;
-  size_t some = 0, total = 0;
-  for (size_t i = 0; i < n_parts; ++i) {
-    some += parts[i].bytes ? 1 : 0;
-    total += parts[i].bytes;
-  }
-  auto plain = [&]() {
-    for (size_t i = 0; i < n_parts && e == hipSuccess; ++i)
-      if (parts[i].bytes) e = hipMemcpy(parts[i].dst, parts[i].src, parts[i].bytes, hipMemcpyDeviceToHost);
-    return e;
-  };
-  // Where nothing is queued that a copy would have to wait for, a plain copy of
-  // one short array is back sooner.  Staged and plain, into memory in use / never
-  // touched: 72 bytes 28 and 13 us; 24 KB 25 / 28 and 28 / 32; 164 KB 28 / 60 and
-  // 16 / 43; 310 KB 42 / 80 and 23 / 74; 960 KB 68 / 219 and 49 / 211; 2.2 MB 84 /
-  // 451 and 132 / 586.  Several arrays share the staging: four of 480 KB together
-  // 75 / 134 and 71 / 150.
-  if (some == 1 && total <= PLAIN_TO && hipStreamQuery(h->stream) == hipSuccess) return plain();
   const bool done = staged(h, parts, n_parts, [&](size_t i, size_t off, size_t bytes, char* to) {
     launch_to_pinned((const char*)parts[i].src + off, bytes, to, h->stream);
     return hipGetLastError();
   }, &e);
   if (done) return e;
   e = sync_stream(h->stream, "copy to the host");
-  return plain();
+  return e == hipSuccess ? plain(parts, n_parts) : e;
+}
+
+// A plain copy of one short array is back sooner than a staged one where nothing
+// has been queued.  Staged and plain, into memory in use / never touched: 72
+// bytes 28 and 13 us; 24 KB 25 / 28 and 28 / 32; 164 KB 28 / 60 and 16 / 43; 310 KB
+// 42 / 80 and 23 / 74; 960 KB 68 / 219 and 49 / 211; 2.2 MB 84 / 451 and 132 /
+// 586.  Several arrays share the staging: four of 480 KB together 75 / 134 and
+// 71 / 150.  Behind kernels and device copies of the same call it had cost 30 us
+// (nf_reduce of 200,000 rods 290 -> 325).
+hipError_t results_to_host(nf_handle* h, const HostPart* parts, size_t n_parts) {
+  size_t some = 0, total = 0;
+  for (size_t i = 0; i < n_parts; ++i) {
+    some += parts[i].bytes ? 1 : 0;
+    total += parts[i].bytes;
+  }
+  if (some == 1 && total <= PLAIN_TO && hipStreamQuery(h->stream) == hipSuccess) {
+    std::lock_guard<std::mutex> lock(h->pin_mu);
+    OnDevice on(h->device);
+    return plain(parts, n_parts);
+  }
+  return to_host(h, parts, n_parts);
 }
 
 hipError_t rods_to_host(nf_handle* h, const float4* P, const float4* D, uint32_t n, float* rods) {

@@ -109,6 +109,8 @@ struct HostPart {
   size_t bytes;
 };
 hipError_t to_host(nf_handle* h, const HostPart* parts, size_t n_parts);
+// The same for results of an earlier call (usually nothing is queued).
+hipError_t results_to_host(nf_handle* h, const HostPart* parts, size_t n_parts);
 // Rods as nf_get_rods gives and nf_set_rods takes them.
 hipError_t rods_to_host(nf_handle* h, const float4* P, const float4* D, uint32_t n, float* rods);
 hipError_t rods_to_device(nf_handle* h, const float* rods, uint32_t n, float4* P, float4* D);

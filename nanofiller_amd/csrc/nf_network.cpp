@@ -145,6 +145,6 @@ extern "C" int nf_get_network(nf_handle* h, uint32_t* labels, uint32_t* row_ptr,
                              {row_ptr, c.nrow, row_ptr ? sizeof(uint32_t) * ((size_t)n + 3) : 0},
                              {col, c.ncol, col ? sizeof(uint32_t) * c.nnz : 0},
                              {val, c.nval, val ? sizeof(double) * c.nnz : 0}};
-  HIPCHK(h, to_host(h, parts, 4));
+  HIPCHK(h, results_to_host(h, parts, 4));
   return NF_OK;
 }

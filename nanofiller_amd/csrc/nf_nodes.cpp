@@ -246,7 +246,7 @@ extern "C" int nf_get_nodes(nf_handle* h, uint32_t* rod, double* t, uint64_t cap
   if (c.nd_nodes == 0) return NF_OK;
   const HostPart parts[2] = {{rod, c.nd_node_rod, rod ? sizeof(uint32_t) * c.nd_nodes : 0},
                              {t, c.nd_node_t, t ? sizeof(double) * c.nd_nodes : 0}};
-  HIPCHK(h, to_host(h, parts, 2));
+  HIPCHK(h, results_to_host(h, parts, 2));
   return NF_OK;
 }
 
@@ -262,7 +262,7 @@ extern "C" int nf_get_segments(nf_handle* h, uint32_t* na, uint32_t* nb, double*
                              {nb, c.nd_seg_b, nb ? sizeof(uint32_t) * m : 0},
                              {L, c.nd_seg_L, L ? sizeof(double) * m : 0},
                              {A, c.nd_seg_A, A ? sizeof(double) * m : 0}};
-  HIPCHK(h, to_host(h, parts, 4));
+  HIPCHK(h, results_to_host(h, parts, 4));
   return NF_OK;
 }
 
@@ -279,7 +279,7 @@ extern "C" int nf_get_node_edges(nf_handle* h, uint32_t* na, uint32_t* nb, uint3
   const HostPart parts[3] = {{na, c.nd_ce_a, na ? sizeof(uint32_t) * m : 0},
                              {nb, c.nd_ce_b, nb ? sizeof(uint32_t) * m : 0},
                              {contact, c.nd_ce_k, contact ? sizeof(uint32_t) * m : 0}};
-  HIPCHK(h, to_host(h, parts, 3));
+  HIPCHK(h, results_to_host(h, parts, 3));
   return NF_OK;
 }
 
@@ -296,6 +296,6 @@ extern "C" int nf_get_node_electrodes(nf_handle* h, uint32_t* node, double* gap,
   const HostPart parts[3] = {{node, c.nd_cel_node, node ? sizeof(uint32_t) * m : 0},
                              {gap, c.nd_cel_gap, gap ? sizeof(double) * m : 0},
                              {side, c.nd_cel_side, side ? sizeof(int32_t) * m : 0}};
-  HIPCHK(h, to_host(h, parts, 3));
+  HIPCHK(h, results_to_host(h, parts, 3));
   return NF_OK;
 }
