@@ -34,10 +34,20 @@ namespace nf {
 
 constexpr int PAIR_THREADS = WAVE;
 
+// Largest of the lanes' values, which are not negative, in every lane (uniform).
+// Without shuffles: their lane addresses, six registers that live through the
+// kernel, had been spilled and fetched again for every cell.
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, WAVE));
-  return v;
+  auto step = [&](int w) { v = fmaxf(v, __int_as_float(w)); };
+#define NF_DPP(CTRL, ROWS) __builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xF, false)
+  step(NF_DPP(0xB1, 0xF));   // lane ^ 1
+  step(NF_DPP(0x4E, 0xF));   // lane ^ 2
+  step(NF_DPP(0x141, 0xF));  // the other quad of eight lanes
+  step(NF_DPP(0x140, 0xF));  // the other eight of a row of 16
+  step(NF_DPP(0x142, 0xA));  // row before, into rows 1 and 3
+  step(NF_DPP(0x143, 0xC));  // rows 0 and 1, into rows 2 and 3
+#undef NF_DPP
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
 __device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
@@ -430,18 +440,25 @@ __device__ __forceinline__ SlotSide slot_pre(const float4 P, const float4 D, con
   return slot_side<ALL>(F.ln, (P.x + sh.x) - F.o.x, (P.y + sh.y) - F.o.y, (P.z + sh.z) - F.o.z, P.w, D, valid);
 }
 
-// Appends the pairs of one word of probes (bit k: probe base + k) with the
-// lane's slot to the first queue, screening 64 at a time when enough wait.
-template <int MODE, int PREC>
-__device__ __forceinline__ void push_pairs(const PairArgs& a, const CellGeom& g, PairLds& L, uint32_t word,
-                                           uint32_t base, uint32_t slot, uint32_t& qn, uint32_t& q2n, Acc& acc) {
+// Appends the pairs of a word of probes per slot of the lane (bit k: probe base
+// + k; m1: the second slot) to the first queue, screening 64 at a time when
+// enough wait.
+template <int MODE, int PREC, bool TWO>
+__device__ __forceinline__ void push_pairs(const PairArgs& a, const CellGeom& g, PairLds& L, uint32_t m0, uint32_t m1,
+                                           uint32_t base, uint32_t& qn, uint32_t& q2n, Acc& acc) {
+  const uint32_t lane = threadIdx.x;
   for (;;) {
-    const bool f = word != 0u;
+    const bool f0 = m0 != 0u, f = TWO ? (m0 | m1) != 0u : f0;
     const unsigned long long m = __ballot(f);
     if (m == 0ull) return;
-    const uint32_t k = base + (uint32_t)__builtin_ctz(word | 0x80000000u);
-    word &= word - 1u;
-    if (f) L.qE[qn + lane_prefix(m)] = k | (slot << 8);
+    const uint32_t w = TWO && !f0 ? m1 : m0;
+    const uint32_t k = base + (uint32_t)__builtin_ctz(w | 0x80000000u);
+    const uint32_t code = k | ((TWO && !f0 ? lane + (uint32_t)WAVE : lane) << 8);
+    if (TWO && !f0)
+      m1 &= m1 - 1u;
+    else
+      m0 &= m0 - 1u;
+    if (f) L.qE[qn + lane_prefix(m)] = code;
     qn += (uint32_t)__popcll(m);
     if (qn >= (uint32_t)WAVE) {
       __syncthreads();
@@ -463,7 +480,6 @@ __device__ __forceinline__ void probe_loop(const PairArgs& a, const CellGeom& g,
                                            const SlotSide& Q0, const SlotSide& Q1, unsigned long long keep0,
                                            unsigned long long keep1, uint32_t& qn, uint32_t& q2n, Acc& acc) {
   constexpr bool ORD = (MODE == PM_CNT || MODE == PM_GEN_NEW);
-  const uint32_t lane = threadIdx.x;
   for (uint32_t w = 0; w < nprobe; w += 32u) {
     uint32_t m0 = 0u, m1 = 0u;
     // the first probe ends in bit 0
@@ -487,8 +503,7 @@ __device__ __forceinline__ void probe_loop(const PairArgs& a, const CellGeom& g,
       m0 &= (uint32_t)(keep0 >> w);
       m1 &= (uint32_t)(keep1 >> w);
     }
-    push_pairs<MODE, PREC>(a, g, L, m0, w, lane, qn, q2n, acc);
-    if (TWO) push_pairs<MODE, PREC>(a, g, L, m1, w, lane + WAVE, qn, q2n, acc);
+    push_pairs<MODE, PREC, TWO>(a, g, L, m0, m1, w, qn, q2n, acc);
   }
 }
 
@@ -589,15 +604,17 @@ __device__ void process_cell(const PairArgs& a, const CellGeom& g, uint32_t gc, 
   const int c0 = (int)(lc % (uint32_t)g.nc[0]);
   const int c1 = (int)((lc / (uint32_t)g.nc[0]) % (uint32_t)g.nc[1]);
   const int c2 = (int)(lc / ((uint32_t)g.nc[0] * (uint32_t)g.nc[1]));
-  // the filter's origin (the home cell's centre), scale and slack
+  // the filter's origin (the home cell's centre), scale and slack (scalars)
   Filter F;
-  F.o = make_float3(((float)c0 + 0.5f) * g.edge[0], ((float)c1 + 0.5f) * g.edge[1], ((float)c2 + 0.5f) * g.edge[2]);
+  F.o = make_float3(unif(((float)c0 + 0.5f) * g.edge[0]), unif(((float)c1 + 0.5f) * g.edge[1]),
+                    unif(((float)c2 + 0.5f) * g.edge[2]));
   const float Smax = 0.51f * (g.edge[0] + g.edge[1] + g.edge[2]) + 2.0f * CELL_MARGIN +
                      2.00002f * (g.hl_max + g.R_max + 16.0f * g.ew);
   if (ALL)
     F.ln = LineFilter{0.0f, 64.0f * U32 * Smax * Smax};
   else
     F.ln = line_filter(g.R_max, g.ew, Smax);
+  F.ln = LineFilter{unif(F.ln.scale), unif(F.ln.slack)};
 
   for (uint32_t pb = cg * csz; pb < pc; pb += ncg * csz) {
     const uint32_t G = min(csz, pc - pb);
@@ -610,7 +627,7 @@ __device__ void process_cell(const PairArgs& a, const CellGeom& g, uint32_t gc, 
     const bool have = inrange;
     // probes still in the walk, as a wave-uniform mask
     unsigned long long pmask = __ballot(have);
-    const float chunk_hl = unif(wave_max(have ? P1.w : 0.0f));
+    const float chunk_hl = wave_max(have ? P1.w : 0.0f);
     if (sp == 0u) acc.bytes += (unsigned long long)G * 36ull;
     const float rr_chunk = (chunk_hl + g.hl_max) * 1.000001f + g.R_max + CELL_MARGIN;
     const float rr_chunk2 = rr_chunk * rr_chunk;
