@@ -49,9 +49,12 @@ constexpr size_t POOL_CAP = (size_t)16 << 30;  // freed bytes kept per handle
 
 constexpr size_t SLAB_FROM = (size_t)1 << 20, SLAB_TO = (size_t)32 << 20, SLAB_LARGEST = (size_t)256 << 20;
 
+constexpr size_t SMALL_TO = (size_t)128 << 10, SMALL_SLAB = (size_t)1 << 20;
+
 static nf_handle::Slab* slab_of(nf_handle* h, const void* p) {
-  for (auto& s : h->slabs)
-    if ((const char*)p >= s.p && (const char*)p < s.p + s.size) return &s;
+  for (auto& kind : h->slabs)
+    for (auto& s : kind)
+      if ((const char*)p >= s.p && (const char*)p < s.p + s.size) return &s;
   return nullptr;
 }
 
@@ -69,25 +72,28 @@ static void clear_slab(nf_handle* h, nf_handle::Slab& s) {
 }
 
 // A block cut from the newest slab, from one whose blocks are all free, or
-// from a new one twice the newest's size; null if there is no memory for one.
+// from a new one (of large blocks twice the newest's size); null if there is no
+// memory for one.
 static void* slab_block(nf_handle* h, size_t cls) {
-  if (h->slabs.empty() || h->slabs.back().size - h->slabs.back().used < cls) {
-    auto idle = std::find_if(h->slabs.begin(), h->slabs.end(),
-                             [&](const nf_handle::Slab& s) { return s.live == 0 && s.size >= cls; });
-    if (idle != h->slabs.end()) {
+  const bool small = cls <= SMALL_TO;
+  auto& slabs = h->slabs[small ? 0 : 1];
+  if (slabs.empty() || slabs.back().size - slabs.back().used < cls) {
+    auto idle =
+        std::find_if(slabs.begin(), slabs.end(), [&](const nf_handle::Slab& s) { return s.live == 0 && s.size >= cls; });
+    if (idle != slabs.end()) {
       clear_slab(h, *idle);
-      std::rotate(idle, idle + 1, h->slabs.end());
+      std::rotate(idle, idle + 1, slabs.end());
     } else {
-      const size_t size = h->slabs.empty() ? SLAB_TO : std::min(2 * h->slabs.back().size, SLAB_LARGEST);
+      const size_t size = small ? SMALL_SLAB : (slabs.empty() ? SLAB_TO : std::min(2 * slabs.back().size, SLAB_LARGEST));
       void* p = nullptr;
       if (hipMalloc(&p, size) != hipSuccess) {
         (void)hipGetLastError();
         return nullptr;
       }
-      h->slabs.push_back({(char*)p, size, 0, 0});
+      slabs.push_back({(char*)p, size, 0, 0});
     }
   }
-  auto& s = h->slabs.back();
+  auto& s = slabs.back();
   void* q = s.p + s.used;
   s.used += cls;
   return q;
@@ -96,15 +102,16 @@ static void* slab_block(nf_handle* h, size_t cls) {
 // Gives the pool's blocks back to the device: those of their own, and the
 // slabs without a block in use.
 static void trim_pool(nf_handle* h) {
-  for (size_t k = 0; k < h->slabs.size();) {
-    if (h->slabs[k].live != 0) {
-      ++k;
-      continue;
+  for (auto& slabs : h->slabs)
+    for (size_t k = 0; k < slabs.size();) {
+      if (slabs[k].live != 0) {
+        ++k;
+        continue;
+      }
+      clear_slab(h, slabs[k]);
+      (void)hipFree(slabs[k].p);
+      slabs.erase(slabs.begin() + k);
     }
-    clear_slab(h, h->slabs[k]);
-    (void)hipFree(h->slabs[k].p);
-    h->slabs.erase(h->slabs.begin() + k);
-  }
   for (auto it = h->pool.begin(); it != h->pool.end();) {
     if (slab_of(h, it->second)) {
       ++it;
@@ -129,9 +136,9 @@ int dalloc_bytes(nf_handle* h, void** p, size_t bytes) {
     h->pool.erase(it);
     h->pool_bytes -= cls;
   } else {
-    if (cls >= SLAB_FROM && cls <= SLAB_TO) q = slab_block(h, cls);
+    if (cls <= SMALL_TO || (cls >= SLAB_FROM && cls <= SLAB_TO)) q = slab_block(h, cls);
     hipError_t e = q ? hipSuccess : hipMalloc(&q, cls);
-    if (e != hipSuccess && (!h->pool.empty() || !h->slabs.empty())) {
+    if (e != hipSuccess) {
       // give the cached blocks back and try once more
       (void)hipGetLastError();
       trim_pool(h);
@@ -870,7 +877,8 @@ extern "C" void nf_destroy(nf_handle* h) {
   trim_pool(h);
   for (auto& kv : h->allocs)
     if (!slab_of(h, kv.first)) (void)hipFree(kv.first);
-  for (auto& s : h->slabs) (void)hipFree(s.p);
+  for (auto& slabs : h->slabs)
+    for (auto& s : slabs) (void)hipFree(s.p);
   for (auto& e : h->ev)
     if (e) (void)hipEventDestroy(e);
   release_pinned(h);

@@ -64,15 +64,16 @@ struct nf_handle {
   std::multimap<size_t, void*> pool;
   size_t pool_bytes = 0;
   std::vector<int4> contact_stencil;  // on its way to the device
-  // blocks of 1 to 32 MB are cut from larger ones (one hipMalloc of that size
-  // takes 0.3 ms, and a packing needs a dozen); one without a block in use
+  // blocks of 1 to 32 MB are cut from larger ones (a hipMalloc of that size and
+  // its hipFree take 0.3 ms, and a packing needs a dozen), those up to 128 KB from
+  // ones of 1 MB (1.7 us each for two to three dozen); one without a block in use
   // serves other sizes, or goes back to the device where memory runs out
   struct Slab {
     char* p;
     size_t size, used;
     uint32_t live;  // blocks in use
   };
-  std::vector<Slab> slabs;
+  std::vector<Slab> slabs[2];  // of small blocks, of large ones
   unsigned long long cb_stats[6] = {0, 0, 0, 0, 0, 0};  // contact pair tests, rechecks, max dd bits
   float cb_ms[4] = {0, 0, 0, 0};                  // contact kernel times: bin, pair pass, CSR build, row sort
   uint64_t contact_hint = 0;                      // contacts found by the last call (append capacity)

@@ -150,6 +150,27 @@ def lists_make_room():
         assert flat(pk.rods()) == rods
 
 
+def small_handles():
+    """A small packing's handle takes a few allocations, not one per array, and
+    gives them back."""
+    M.nfm_calls.restype = C.c_long
+    p = params(2000, 3.0)
+    for _ in range(3):
+        before = M.nfm_calls()
+        with nf.Packing(p) as pk:
+            assert M.nfm_calls() - before <= 10, M.nfm_calls() - before
+            pk.generate()
+            contacts(pk)
+            pk.network()
+            after = M.nfm_calls()
+            for _ in range(3):
+                pk.generate()
+                contacts(pk)
+                pk.network()
+            assert M.nfm_calls() == after
+        assert M.nfm_live() == 0
+
+
 if __name__ == "__main__":
     print("[scenario]", sys.argv[1], flush=True)
     globals()[sys.argv[1]]()

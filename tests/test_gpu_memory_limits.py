@@ -31,3 +31,7 @@ def test_memory_of_one_instance_serves_the_next():
 
 def test_lists_give_way():
     _run("lists_make_room")
+
+
+def test_small_handles_take_few_allocations():
+    _run("small_handles")
