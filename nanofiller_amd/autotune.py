@@ -89,7 +89,7 @@ def tune_tiles(names=None, log=print) -> dict:
     for name, (params, keys, reps) in tile_workloads().items():
         if names and name not in names:
             continue
-        cur = {k: v for k, v in TILE_DEFAULTS.items() if k in keys or k in TILE_KEYS}
+        cur = {k: v for k, v in TILE_DEFAULTS.items() if k in keys}
         cur_ms = _gen_ms(params, cur, reps)
         tried = {json.dumps(cur, sort_keys=True): cur_ms}
         log(f"{name}: defaults {cur_ms:.2f} ms")
@@ -103,7 +103,7 @@ def tune_tiles(names=None, log=print) -> dict:
                 log(f"{name}: {k}={v} {t:.2f} ms")
                 if t < cur_ms * 0.98:
                     cur, cur_ms = trial, t
-        d0 = {k: v for k, v in TILE_DEFAULTS.items() if k in keys or k in TILE_KEYS}
+        d0 = {k: v for k, v in TILE_DEFAULTS.items() if k in keys}
         out[name] = dict(cur, ms=cur_ms, ms_defaults=tried[json.dumps(d0, sort_keys=True)],
                          tried={kk: vv for kk, vv in tried.items()})
         log(f"{name}: {cur} {cur_ms:.2f} ms")
