@@ -11,15 +11,15 @@ FP64 re-check band; `value` is accepted rods/s over the timed steps.
 The same JSON line carries:
   * fp64_plain: the same packing by the plain FP64 path; identity of the two
     packings and of their contact lists;
-  * roofline: the reject-vs-accepted kernel, bytes of the list entries and rods
-    that it reads per launch over its HIP-event time (one extra, profiled
-    generation);
+  * roofline: the reject-vs-accepted kernel, its VALU issue (counted wave
+    instructions per launch over its HIP-event time in one extra, profiled
+    generation), and its HBM traffic beside it;
   * batch: 256 independent packings of uneven size (2k-200k rods) in one
     batched FP32 + recheck generation, against the same 256 packings made one
     at a time by the plain FP64 path, with identical packings;
   * contacts: 4,000,000 rods in a 50 um cube: contact list by the footprint
     engine (FP32 + recheck, and FP64) and by the cell-pair engine, three
-    64-bin int64 histograms, contact-kernel HBM and VALU-issue rooflines;
+    64-bin int64 histograms, contact-kernel VALU-issue and HBM rooflines;
   * network: 8,000,000 rods in a 40 um cube: contacts, components and the
     FP64 Kirchhoff matrix;
   * cpu_baseline: the C oracle on a bounded sample of the headline workload.
@@ -102,16 +102,24 @@ def profiled_valu(key: str):
         return None
 
 
-def valu_roof(key: str, ms_per_launch: float):
-    """VALU-issue roofline of a kernel: its counted wave instructions at 4
-    cycles each spread over every SIMD, against its measured time."""
+def pair_roofline(kernel: str, key: str, ms: float, traffic=None, traffic_file=None, **more) -> dict:
+    """Roofline of a pair kernel: VALU issue, which bounds it (its counted wave
+    instructions per launch against one per SIMD every 4 cycles, at its
+    measured time `ms`), and beside it what it moves to and from HBM (counted
+    as well).  Bytes that the kernel asks for but L2 serves are in `more`, and
+    are held against no peak."""
+    peak = SIMDS * CLOCK_HZ / VALU_CYCLES / 1e9
     n = profiled_valu(key)
-    if n is None or ms_per_launch <= 0:
-        return None
-    issue_ms = n * VALU_CYCLES / SIMDS / CLOCK_HZ * 1e3
-    return {"bound": "valu", "instructions_per_launch": n, "issue_ms": issue_ms,
-            "launch_ms": ms_per_launch, "frac": issue_ms / ms_per_launch,
-            "source": os.path.relpath(VALU_SUMMARY, ROOT)}
+    rate = n / (ms * 1e-3) / 1e9 if n is not None and ms > 0 else None
+    out = {"bound": "valu", "achieved": rate, "peak": peak, "unit": "G wave instructions/s",
+           "frac": rate / peak if rate is not None else None, "kernel": kernel,
+           "instructions_per_launch": n, "launch_ms": ms, "source": os.path.relpath(VALU_SUMMARY, ROOT)}
+    if traffic_file is not None:
+        gbs = traffic / (ms * 1e-3) / 1e9 if traffic is not None and ms > 0 else None
+        out["hbm"] = {"bytes_per_launch": traffic, "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                      "frac": gbs / HBM_PEAK_GBS if gbs is not None else None,
+                      "source": os.path.relpath(traffic_file, ROOT)}
+    return {**out, **more}
 
 
 def log(msg: str) -> None:
@@ -163,18 +171,12 @@ def leg_main(a, out: dict) -> None:
         sp = pk.generate()[0]
     launches = max(sp.rounds_launched, 1)
     k_old = sp.kern_ms[K_OLD]
-    achieved = (sp.tile_bytes / launches) / (k_old / launches * 1e-3) / 1e9 if k_old > 0 else 0.0
     log(f"profiled: reject_old {k_old:.3f} ms over {launches} launches, "
         f"reject_new {sp.kern_ms[K_NEW]:.3f} ms")
     out.update(value=rods_s, ms_per_step=ms_step, n_rods=p32.n_rods)
-    out["roofline"] = {
-        "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-        "frac": achieved / HBM_PEAK_GBS, "traffic": profiled_traffic(),
-        "traffic_source": os.path.relpath(TRAFFIC_SUMMARY, ROOT),
-        "kernel": "k_walk<reject vs accepted, FP32+recheck>",
-        "bytes_per_launch": sp.tile_bytes / launches, "avg_launch_ms": k_old / launches,
-        "launches": launches, "valu": valu_roof("k_walk<0, 1> 500k", k_old / launches),
-    }
+    out["roofline"] = pair_roofline(
+        "k_walk<reject vs accepted, FP32+recheck>", "k_walk<0, 1> 500k", k_old / launches,
+        profiled_traffic(), TRAFFIC_SUMMARY, list_bytes_per_launch=sp.tile_bytes / launches, launches=launches)
     out["extra"]["fp32_recheck"] = {
         "tile_options": tiles,
         "accepted_rods_per_s": rods_s, "ms_per_step": ms_step,
@@ -362,12 +364,7 @@ def leg_contacts(a, out: dict) -> None:
         cs64 = pk.contact_stats()
     gen_prof = profiled_generation(p, configs.tile_options("4M"))
     km = cs["kernel_ms"]
-    # the algorithmic bytes of the contact pass: N * 32 B * 14 tiles (27-cell
-    # stencil with Newton's third law) + C * 12 B (I, J, gap)
-    alg_bytes = st.n_accepted * 32 * 14 + c32.n * 12
-    alg_achieved = alg_bytes / (km["pairs"] * 1e-3) / 1e9 if km["pairs"] > 0 else 0.0
-    alg_cells = alg_bytes / (csc["kernel_ms"]["pairs"] * 1e-3) / 1e9 if csc["kernel_ms"]["pairs"] > 0 else 0.0
-    log(f"contacts: {c32.n} pairs, footprint pass {km['pairs']:.3f} ms ({alg_achieved:.0f} GB/s), "
+    log(f"contacts: {c32.n} pairs, footprint pass {km['pairs']:.3f} ms, "
         f"cell-pair pass {csc['kernel_ms']['pairs']:.3f} ms; FP64 pass {cs64['kernel_ms']['pairs']:.3f} ms")
     out["extra"]["contacts"] = {
         "workload": "4,000,000 rods, 50 um cube, l 1 um, d 10 nm, uniform, vMF(+x, 2), gap <= 2 nm",
@@ -376,19 +373,13 @@ def leg_contacts(a, out: dict) -> None:
         "contacts": int(c32.n), "contacts_call_ms": t_c * 1e3, "kernel_ms": km, "engine": eng,
         "pair_tests": cs["pair_tests"], "rechecks": cs["rechecks"],
         "streamed_bytes": cs["tile_bytes"],
-        "pair_kernel_roofline": {"bound": "hbm", "achieved": alg_achieved, "peak": HBM_PEAK_GBS,
-                                  "unit": "GB/s", "frac": alg_achieved / HBM_PEAK_GBS,
-                                  "algorithmic_bytes_per_pass": alg_bytes,
-                                  "traffic": profiled_contact_traffic(),
-                                  "traffic_source": os.path.relpath(CONTACT_TRAFFIC_SUMMARY, ROOT),
-                                  "kernel": "k_seg_cross (footprint engine, FP32+recheck)",
-                                  "valu": valu_roof("k_seg_cross 4M", km["pairs"])},
+        "pair_kernel_roofline": pair_roofline("k_seg_cross (footprint engine, FP32+recheck)", "k_seg_cross 4M",
+                                              km["pairs"], profiled_contact_traffic(), CONTACT_TRAFFIC_SUMMARY),
         "cell_engine": {"contacts_call_ms": t_cc * 1e3, "kernel_ms": csc["kernel_ms"],
                         "pairs_within_reach": csc["pair_tests"], "streamed_bytes": csc["tile_bytes"],
                         "identical_list": bool(same_contacts(c32, cc)),
-                        "roofline": {"bound": "hbm", "achieved": alg_cells, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                                     "frac": alg_cells / HBM_PEAK_GBS,
-                                     "valu": valu_roof("k_pair<2, 1> 4M", csc["kernel_ms"]["pairs"])}},
+                        "roofline": pair_roofline("k_pair<contacts> (cell-pair engine, FP32+recheck)",
+                                                  "k_pair<2, 1> 4M", csc["kernel_ms"]["pairs"])},
         "max_abs_d32_d64_um": dd_contacts,
         "generation_profile": gen_prof,
         "fp64_contacts_call_ms": t_c64 * 1e3, "fp64_kernel_ms": cs64["kernel_ms"],
