@@ -52,9 +52,6 @@ static double contact_reach(const ContactBuffers& c) {
   return ((double)c.hl_max + (double)c.hl_max) * REACH_PAD + Rmax;
 }
 
-// Centre cell list of the contact rods on cells of about `edge`, with the
-// stencil of every cell within `reach` of a home block of bx cells along x
-// (half, bx = 1: each cell pair once).
 // Scratch of bin_rods, given back by the caller once the stream has
 // synchronized.
 struct BinScratch {
@@ -94,7 +91,10 @@ static int bin_rods(nf_handle* h, const float4* P, const float4* D, uint32_t n, 
   return NF_OK;
 }
 
-// (scratch is in use until the caller has waited for the stream and frees it)
+// Centre cell list of the contact rods on cells of about `edge`, with the
+// stencil of every cell within `reach` of a home block of bx cells along x
+// (half, bx = 1: each cell pair once).  The scratch is in use until the
+// caller has waited for the stream and frees it.
 static int build_cell_list(nf_handle* h, double edge, double reach, bool half, BinScratch* bs, int bx = 1) {
   ContactBuffers& c = h->cb;
   const nf_params& p = h->params[h->post_inst];

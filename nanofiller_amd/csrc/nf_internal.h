@@ -448,12 +448,12 @@ void launch_bin_rods(const BinPlan& bp, const float4* P, const float4* D, uint32
                      const double scale[3], uint32_t* M, uint32_t* scan_tmp, float4* tP, float4* tD,
                      uint32_t* tid, float4* oP, float4* oD, uint32_t* oid, uint32_t* start, uint32_t* count,
                      float* hl, hipStream_t s);
-// out[0..2] (cleared): largest half length, radius and |u|^2 - 1 of the rods, as
-// the bits of non-negative floats.
 // bytes (a multiple of 4) of device memory to pinned host memory.
 void launch_to_pinned(const void* src, size_t bytes, void* dst, hipStream_t s);
 // rods[2 i], rods[2 i + 1]: rod i as eight floats (centre, direction, length, radius).
 void launch_pack_rods(const float4* P, const float4* D, uint32_t n, float4* rods, hipStream_t s);
+// out[0..2] (cleared): largest half length, radius and |u|^2 - 1 of the rods, as
+// the bits of non-negative floats.
 void launch_rod_bounds(const float4* P, const float4* D, uint32_t n, uint32_t* out, hipStream_t s);
 void launch_expand_flags(const float4* P, uint32_t n, int k, double L, double B, uint32_t* below, uint32_t* above,
                          hipStream_t s);

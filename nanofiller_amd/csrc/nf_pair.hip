@@ -472,8 +472,9 @@ __device__ __forceinline__ void push_pairs(const PairArgs& a, const CellGeom& g,
 // the slots (one each, or two when the batch fills the second half), the
 // probes read from LDS by all lanes at once.  A lane gathers the verdicts of
 // 32 probes in one word per slot and only then turns to the pairs that
-// passed, so the loop is 13 VALU instructions per 64 pairs without a branch,
-// ballot or queue write.  keep0, keep1: the pairs that the pass's ordering
+// passed, so the loop is 12 VALU instructions per 64 pairs (6 with the centre
+// filter of ALL) without a branch, ballot or queue write.  keep0, keep1: the
+// pairs that the pass's ordering
 // allows (half-stencil passes).
 template <int MODE, int PREC, bool ALL, bool TWO>
 __device__ __forceinline__ void probe_loop(const PairArgs& a, const CellGeom& g, PairLds& L, uint32_t nprobe,

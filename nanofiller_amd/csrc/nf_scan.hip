@@ -3,10 +3,12 @@
 // Replaces the thrust::inclusive_scan / exclusive_scan calls of the
 // reference (src/get_contact_arrays.cu:101, src/conductivity.cu:495,
 // src/adjacency_graph.cu:79) and its in-block work-efficient scan
-// (inc/sort.h:103-154).  Three passes (tile sums, scan of tile sums, tile
-// rescan) with 2048-element tiles, 256 threads x 8 items, or for arrays of
-// at most 16384 one pass of one workgroup; fixed launch shape for a given
-// n, so the passes can be captured in a HIP graph.
+// (inc/sort.h:103-154).  Tiles of 2048 elements, 256 threads x 8
+// items.  Two passes (tile sums; tile scan, each workgroup adding up the sums
+// before its own) for up to 2048 tiles, three (the tile sums scanned between
+// them) beyond, and for arrays of at most 16384 one pass of one workgroup;
+// fixed launch shape for a given n, so the passes can be captured in a HIP
+// graph.
 #include "nf_internal.h"
 
 namespace nf {
@@ -155,8 +157,8 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_apply(const uint32_t* in,
 }
 
 // Short arrays (the cells of a single packing): one workgroup of 1024
-// threads walks the array in tiles of 4096 with a running carry, one launch
-// instead of three.
+// threads walks the array in tiles of 4096 with a running carry, in one
+// launch.
 constexpr int SCAN1_THREADS = 1024;
 constexpr int SCAN1_ITEMS = 4;
 constexpr uint64_t SCAN1_MAX = 16384;

@@ -151,6 +151,8 @@ __device__ __forceinline__ bool last_round(const WalkArgs& a, const InstDesc& d,
 
 // Rods accepted by this round's commit, found among the survivors of the
 // first pass: these are in cell order, so that neighbouring lanes' atomics
+// and stores fall into the same few lists.  In the last round nothing is
+// entered (last_round).
 __global__ void __launch_bounds__(ENTER_THREADS) k_enter_accepted(WalkArgs a) {
   const uint32_t total = a.prStart[a.ncells];
   for (uint64_t t = (uint64_t)blockIdx.x * ENTER_THREADS + threadIdx.x; t < (uint64_t)total * ENTER_LANES;
