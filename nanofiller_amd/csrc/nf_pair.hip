@@ -474,8 +474,7 @@ __device__ __forceinline__ void push_pairs(const PairArgs& a, const CellGeom& g,
 // 32 probes in one word per slot and only then turns to the pairs that
 // passed, so the loop is 12 VALU instructions per 64 pairs (6 with the centre
 // filter of ALL) without a branch, ballot or queue write.  keep0, keep1: the
-// pairs that the pass's ordering
-// allows (half-stencil passes).
+// pairs that the pass's ordering allows (half-stencil passes).
 template <int MODE, int PREC, bool ALL, bool TWO>
 __device__ __forceinline__ void probe_loop(const PairArgs& a, const CellGeom& g, PairLds& L, uint32_t nprobe,
                                            const SlotSide& Q0, const SlotSide& Q1, unsigned long long keep0,
