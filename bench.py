@@ -53,9 +53,13 @@ K_NEW = nf.KERNEL_CLASSES.index("reject_new")
 
 TRAFFIC_SUMMARY = os.path.join(ROOT, "profiles", "generate_500k_hbm_counters.md")
 VALU_SUMMARY = os.path.join(ROOT, "profiles", "pair_kernels_valu_counters.md")
-# VALU issue roof: a wave64 VALU instruction occupies a 16-lane SIMD for 4
-# cycles; 256 CUs x 4 SIMDs at the 2.4 GHz peak engine clock
-SIMDS, VALU_CYCLES, CLOCK_HZ = 1024, 4, 2.4e9
+# VALU issue: 256 CUs x 4 SIMDs at the 2.4 GHz peak engine clock.  FP32 adds,
+# multiplies and FMAs and 32-bit integer adds and logic of vector registers
+# take a SIMD 2 cycles (measured 870-1090 G wave instructions/s), compares,
+# selects, shifts, min/max, FP64 and whatever reads a scalar register 4
+# (530-590): the roof is the first, and the share at 4 cycles each is an upper
+# bound of the time that issue takes, which a kernel of FMAs passes.
+SIMDS, VALU_CYCLES, VALU_CYCLES_MOST, CLOCK_HZ = 1024, 2, 4, 2.4e9
 
 
 def profiled_traffic():
@@ -103,16 +107,17 @@ def profiled_valu(key: str):
 
 
 def pair_roofline(kernel: str, key: str, ms: float, traffic=None, traffic_file=None, **more) -> dict:
-    """Roofline of a pair kernel: VALU issue, which bounds it (its counted wave
-    instructions per launch against one per SIMD every 4 cycles, at its
-    measured time `ms`), and beside it what it moves to and from HBM (counted
-    as well).  Bytes that the kernel asks for but L2 serves are in `more`, and
-    are held against no peak."""
+    """Roofline of a pair kernel: VALU issue (its counted wave instructions per
+    launch against one per SIMD every 2 cycles, at its measured time `ms`), and
+    beside it what it moves to and from HBM (counted as well).  Bytes that the
+    kernel asks for but L2 serves are in `more`, held against no peak."""
     peak = SIMDS * CLOCK_HZ / VALU_CYCLES / 1e9
     n = profiled_valu(key)
     rate = n / (ms * 1e-3) / 1e9 if n is not None and ms > 0 else None
     out = {"bound": "valu", "achieved": rate, "peak": peak, "unit": "G wave instructions/s",
-           "frac": rate / peak if rate is not None else None, "kernel": kernel,
+           "frac": rate / peak if rate is not None else None,
+           "frac_at_4_cycles": rate / peak * VALU_CYCLES_MOST / VALU_CYCLES if rate is not None else None,
+           "kernel": kernel,
            "instructions_per_launch": n, "launch_ms": ms, "source": os.path.relpath(VALU_SUMMARY, ROOT)}
     if traffic_file is not None:
         gbs = traffic / (ms * 1e-3) / 1e9 if traffic is not None and ms > 0 else None
