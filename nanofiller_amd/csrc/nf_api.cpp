@@ -450,21 +450,37 @@ std::vector<int4> build_stencil(const int32_t nc[3], const double box[3], double
 // is evaluated in FP64, with the precision.  Rods of one length take the lists
 // from this many per excluded volume on; whole generations, cells of one reach
 // against lists, at 0.31 / 0.52 / 0.83 / 1.25 / 1.66 / 2.1 / 2.7 in ms:
-//   FP32   100,000  .30 .60 .83 1.08 1.40 1.67 2.51    .31 .48 .71  .90 1.12 1.40 1.91
-//          300,000  .40 .81 1.29 1.52 2.03 2.52 3.88   .44 .78 1.10 1.31 1.74 2.08 2.89
-//          450,000  .48 .95 1.48 1.80 2.49 3.01 5.08   .57 .99 1.37 1.70 2.19 2.65 3.71
-//          1M       .80 1.38 2.20 2.75 4.12 5.41 8.44  1.08 1.81 2.40 3.08 4.18 5.06 6.82
-//          4M       2.63 4.01 6.17 8.54 13.0 17.9 30.6 4.15 6.50 8.62 11.4 15.0 18.1 23.9
-//   FP64   700,000  .82 1.82 3.00 3.35 4.91 5.82 8.65  .82 1.29 1.82 2.28 3.02 3.55 4.97
-//          1M       1.00 2.01 3.28 3.87 5.64 6.96 10.7 1.07 1.81 2.39 3.04 4.11 4.98 6.75
-//          1.5M     1.25 2.42 3.87 4.83 7.00 8.78 14.4 1.57 2.52 3.47 4.33 5.77 7.15 9.47
-//          2.5M     1.82 3.20 5.17 6.80 10.1 13.3 20.6 2.76 4.16 5.65 7.30 9.74 11.8 15.5
-//          4M       2.68 4.46 7.10 9.53 14.4 18.8 31.6 4.15 6.49 8.55 11.4 14.9 18.3 23.8
+//   FP32   100,000  .30 .61 .82 1.08 1.40 1.87 2.85    .32 .51 .74  .90 1.14 1.59 2.28
+//          300,000  .41 .82 1.27 1.50 2.06 2.64 4.07   .46 .80 1.11 1.36 1.77 2.26 3.10
+//          450,000  .45 .93 1.50 1.76 2.44 3.26 5.28   .59 1.01 1.40 1.71 2.22 2.71 3.96
+//          1M       .77 1.33 2.14 2.75 4.09 5.69 9.49  1.10 1.83 2.47 3.14 4.25 5.34 7.21
+//          4M       2.43 3.84 5.83 8.50 12.9 20.0 31.1 4.14 6.60 8.68 11.6 15.1 19.0 24.5
+//          8M       6.63 7.55 9.93 15.7 21.5 32.8 59.2 10.2 12.0 16.1 21.2 27.3 33.9 48.6
+//   FP64   700,000  .83 1.81 2.96 3.40 4.87 6.26 9.86  .82 1.34 1.84 2.31 3.08 3.78 5.18
+//          1M       .97 2.02 3.25 3.86 5.67 7.49 12.0  1.09 1.81 2.46 3.09 4.18 5.31 7.12
+//          1.5M     1.27 2.39 3.82 4.82 7.13 9.63 15.5 1.60 2.58 3.46 4.36 5.86 7.49 9.79
+//          2.5M     1.80 3.17 5.11 6.86 10.1 14.2 21.8 2.77 4.21 5.71 7.34 9.87 12.2 15.8
+//          4M       2.60 4.45 6.88 9.71 14.4 21.3 32.8 4.13 6.53 8.65 11.5 14.8 19.0 24.3
+//          8M       6.97 7.73 10.7 16.6 22.5 33.6 59.0 9.69 11.7 15.8 21.1 27.0 33.8 47.7
+// Dense places cost the cells more and take more rounds, so above 300,000 rods
+// the line falls with the densest place over the mean: of 16 agglomerates, FP32,
+// peak 3 (2.8 over the mean) 4M rods at 1.66 / 2.0 11.8 / 16.7 against 12.8 /
+// 16.0 ms, 8M at 2.0 32.8 against 31.8; peak 8 (6.6) 1M at 0.9 / 1.3 3.8 / 5.6
+// against 3.5 / 4.8, 4M at 0.9 / 1.3 / 1.7 11.1 / 14.9 / 20.8 against 11.8 / 14.0
+// / 18.5; FP64, 4M, peak 3 at 1.3 / 1.66 9.9 / 13.6 against 10.2 / 12.7, peak 8
+// at 0.9 13.2 against 11.5.  At peak 20 (16) the lists, as long everywhere as in
+// the densest place, take 2.5 GB at 4M rods and lose again: 29 against 41 ms at
+// 1.3, where 1M rods still take 11.0 against 7.9.
 // Log-normal lengths take them always: at 0.3 / 1 / 2.1 100,000 rods .42 1.37 2.59
 // against .32 .85 1.32 ms, 4M 7.2 21.1 54.7 against 4.4 10.9 19.0.
-static double lists_from(uint32_t n, bool fp64) {
-  if (fp64) return n <= 700000u ? 0.0 : n <= 1000000u ? 0.4 : n <= 2000000u ? 0.65 : n <= 3000000u ? 1.55 : 1.9;
-  return n <= 100000u ? 0.0 : n <= 300000u ? 0.4 : n <= 500000u ? 0.75 : n <= 1000000u ? 1.65 : 2.05;
+static double lists_from(uint32_t n, bool fp64, double dense) {
+  double c = 0.0;
+  if (fp64)
+    c = n <= 700000u ? 0.0 : n <= 1000000u ? 0.4 : n <= 2000000u ? 0.65 : n <= 3000000u ? 1.55 : 1.9;
+  else
+    c = n <= 100000u ? 0.0 : n <= 300000u ? 0.4 : n <= 500000u ? 0.75 : n <= 1000000u ? 1.65 : 2.05;
+  if (n <= 300000u || (n > 1000000u && dense > 10.0)) return c;
+  return c / (1.0 + 0.1 * (std::min(dense, 10.0) - 1.0));
 }
 
 // An instance's crossing lists.  peak: densest point over the mean.
@@ -472,7 +488,13 @@ static void plan_fine(const nf_params& p, InstDesc& d, double peak) {
   FineGrid& g = d.fine;
   const double V = p.box[0] * p.box[1] * p.box[2];
   const double crowd = (double)p.n_rods * excluded_volume(p.len, p.radius) / V;
-  if (p.len_law == NF_LEN_CONST && crowd < lists_from(p.n_rods, p.precision == NF_PREC_FP64)) return;
+  // densest place over the mean: of agglomerates that overlap less than they may
+  double dense = peak;
+  if (p.den_law == NF_DEN_AGGLOM) {
+    const double blobs = p.n_agg * std::pow(2.0 * M_PI, 1.5) * p.agg_sigma * p.agg_sigma * p.agg_sigma / V;
+    dense /= 1.0 + (peak - 1.0) * std::min(blobs, 1.0);
+  }
+  if (p.len_law == NF_LEN_CONST && crowd < lists_from(p.n_rods, p.precision == NF_PREC_FP64, dense)) return;
   const double r = 0.50001 * (double)d.R_max + 16.0 * (double)d.ew;
   double E = 1.5 * std::cbrt(V / (double)p.n_rods);
   E = std::min(std::max(E, p.len / 16.0), p.len / 1.5);

@@ -37,3 +37,20 @@ def test_same_packing_over_lists_and_cells(n, crowd, prec, tmp_path):
     if n < 400000:
         reach = p.len * 1.000001 + 2.0 * p.radius
         assert nf.read_state_header(str(tmp_path / "s.bin"))["ext"] == (int(p.box[0] / (0.85 * reach)),) * 3
+
+
+@pytest.mark.parametrize("n,crowd,peak,sigma,prec", [
+    (1100000, 1.7, 3.0, 0.05, 1), (1100000, 1.8, 3.0, 0.05, 1), (320000, 0.5, 8.0, 0.05, 1),
+    (1100000, 0.6, 8.0, 0.05, 0), (400000, 0.6, 3.0, 0.5, 1)])
+def test_same_packing_in_agglomerates(n, crowd, peak, sigma, prec):
+    p = _params(n, crowd, prec)
+    p = nf.normalize(nf.default_params(box=tuple(p.box), n_rods=n, len=1.0, radius=0.005, seed=13, max_rounds=30,
+                                       precision=prec, den_law=nf.NF_DEN_AGGLOM, n_agg=16, agg_peak=peak,
+                                       agg_sigma=sigma * p.box[0]))
+    got = []
+    for options in (None, {nf.NF_OPT_CROSSING_LISTS: 0}):
+        with nf.Packing(p, options) as pk:
+            got.append((pk.generate()[0], pk.rods()))
+    for k in COUNTERS:
+        assert getattr(got[0][0], k) == getattr(got[1][0], k), k
+    np.testing.assert_array_equal(got[0][1].view(np.uint32), got[1][1].view(np.uint32))
