@@ -483,18 +483,13 @@ static double lists_from(uint32_t n, bool fp64, double dense) {
   return c / (1.0 + 0.1 * (std::min(dense, 10.0) - 1.0));
 }
 
-// An instance's crossing lists.  peak: densest point over the mean.
+// An instance's crossing lists.  peak: densest point over the background or the
+// mean, a bound that cell capacities follow; d.dense has it over the mean.
 static void plan_fine(const nf_params& p, InstDesc& d, double peak) {
   FineGrid& g = d.fine;
   const double V = p.box[0] * p.box[1] * p.box[2];
   const double crowd = (double)p.n_rods * excluded_volume(p.len, p.radius) / V;
-  // densest place over the mean: of agglomerates that overlap less than they may
-  double dense = peak;
-  if (p.den_law == NF_DEN_AGGLOM) {
-    const double blobs = p.n_agg * std::pow(2.0 * M_PI, 1.5) * p.agg_sigma * p.agg_sigma * p.agg_sigma / V;
-    dense /= 1.0 + (peak - 1.0) * std::min(blobs, 1.0);
-  }
-  if (p.len_law == NF_LEN_CONST && crowd < lists_from(p.n_rods, p.precision == NF_PREC_FP64, dense)) return;
+  if (p.len_law == NF_LEN_CONST && crowd < lists_from(p.n_rods, p.precision == NF_PREC_FP64, d.dense)) return;
   const double r = 0.50001 * (double)d.R_max + 16.0 * (double)d.ew;
   double E = 1.5 * std::cbrt(V / (double)p.n_rods);
   E = std::min(std::max(E, p.len / 16.0), p.len / 1.5);
@@ -581,6 +576,12 @@ static int plan_instance(const nf_params& p, InstDesc& d, std::vector<double>& a
   }
   const double Lmax = std::max(p.box[0], std::max(p.box[1], p.box[2]));
   d.ew = (float)(5.9604644775390625e-8 * (Lmax + reach) * 1.01);
+  double dense = peak;
+  if (p.den_law == NF_DEN_AGGLOM) {  // the mean, as if no two agglomerates overlapped
+    const double blobs = p.n_agg * std::pow(2.0 * M_PI, 1.5) * p.agg_sigma * p.agg_sigma * p.agg_sigma / V;
+    dense /= 1.0 + (peak - 1.0) * std::min(blobs, 1.0);
+  }
+  d.dense = (float)dense;
   plan_fine(p, d, peak);
   auto cells_of = [&](double edge, int32_t nc[3]) {
     uint64_t c = 1;

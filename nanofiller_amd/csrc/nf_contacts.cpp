@@ -605,7 +605,17 @@ static int contacts_pass(nf_handle* h, double gap, uint64_t* n_out, int prec, Co
 //     200  419 559 761 1184   419 467 534 584      8000  5.6 10.1 18.4 ms    5.2 6.6 9.7
 //   log-normal lengths, FP64
 //     100  356 531 724 628    360 390 437 489      8000  6.0 10.2 16.7 ms    5.6 7.0 9.5
-// At a quarter and less, home cells from 80,000 rods on in all of them.
+// At a quarter and less, home cells from 80,000 rods on in all of them; at 2.4,
+// FP32, one length, 100,000 and 400,000 rods 521 and 1000 against 531 and 930.
+// A home cell in a dense place holds one wave up, or has to be done again in
+// parts: of 16 agglomerates with peak 3 (2.8 over the mean) both ways are within
+// 6 % where these lines differ from the uniform ones, with peaks 8 (6.6) / 20 (16)
+//   one length, FP32, 60,000 rods at 0.8 / 1.3 440 / 486, 505 / 522 against 429 /
+//   451, 430 / 456; 400,000 at 1.9 / 2.4 838 / 1109, 916 / 971 against 868 / 940,
+//   894 / 867; FP64, 100,000 at 0.85 587, 686 against 497, 481
+//   log-normal, FP32, 200,000 at 0.42 / 0.6 709 / 701, 1795 / 2064 against 556 /
+//   584, 568 / 596; 800,000 1093 / 1168, 3036 / 3644 against 1002 / 1066, 1056 /
+//   1131
 static bool lists_suit(const nf_handle* h, int prec) {
   const nf_params& p = h->params[h->post_inst];
   const uint32_t n = h->n_rods[h->post_inst];
@@ -613,10 +623,14 @@ static bool lists_suit(const nf_handle* h, int prec) {
   const double crowd = (double)n * excluded_volume(m.len, m.radius) / (p.box[0] * p.box[1] * p.box[2]);
   const bool mixed = p.len_law == NF_LEN_LOGNORMAL;
   if (n <= 30000u) return true;
+  if (h->desc[h->post_inst].dense >= 4.0f) {
+    if (n <= 60000u) return true;
+    if (mixed ? crowd >= 0.4 && n <= 800000u : crowd >= (prec == NF_PREC_FP64 ? 0.8 : 2.0) && n <= 400000u) return true;
+  }
   if (prec == NF_PREC_FP64)
-    return n <= 60000u || crowd >= 0.95 || (crowd >= 0.48 && (mixed || n >= 200000u));
+    return n <= 60000u || crowd >= 0.95 || (crowd >= 0.48 && n >= 200000u) || (crowd >= 0.4 && mixed);
   if (mixed) return n <= 60000u || (n <= 150000u && crowd >= 0.48) || (n <= 1500000u && crowd >= 0.8);
-  return (n <= 60000u && crowd < 0.75) || (n <= 500000u && crowd >= 2.6);
+  return (n <= 60000u && crowd < 0.75) || (n <= 500000u && crowd >= (n < 150000u ? 2.6 : 2.3));
 }
 
 int contacts_run(nf_handle* h, double gap, uint64_t* n_out, int prec, unsigned long long*) {

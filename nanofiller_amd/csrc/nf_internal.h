@@ -52,7 +52,7 @@ struct InstDesc {
   float ew;               // FP32 bound on a centre-difference component error
   float hl_max;           // max half length of any rod of this instance
   float R_max;            // max hard-core distance
-  uint32_t pad;
+  float dense;            // densest place over the mean density, of the parameters
   FineGrid fine;
 };
 

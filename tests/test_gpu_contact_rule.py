@@ -35,8 +35,10 @@ def _compare(p, rods, gap):
 @pytest.mark.parametrize("prec", [nf.NF_PREC_FP64, nf.NF_PREC_FP32_RECHECK])
 @pytest.mark.parametrize("n,crowd,law", [
     (30000, 1.0, "const"), (30001, 1.0, "const"), (60000, 0.7, "const"), (60000, 0.8, "const"), (100000, 2.4, "const"),
+    (160000, 2.2, "const"), (160000, 2.4, "const"),
     (100000, 2.8, "const"), (210000, 0.4, "const"), (210000, 0.6, "const"), (100000, 0.9, "const"), (100000, 1.1, "const"),
-    (60000, 0.3, "logn"), (61000, 0.3, "logn"), (140000, 0.5, "logn"), (160000, 0.5, "logn"), (160000, 1.0, "logn")])
+    (60000, 0.3, "logn"), (61000, 0.3, "logn"), (100000, 0.44, "logn"), (140000, 0.5, "logn"),
+    (160000, 0.5, "logn"), (160000, 1.0, "logn")])
 def test_generated_rods(n, crowd, law, prec):
     _compare(nf.normalize(nf.default_params(box=(_edge(n, crowd),) * 3, n_rods=n, len=1.0, radius=0.005, seed=17,
                                             contact_gap=0.002, precision=prec, max_rounds=30,
@@ -58,3 +60,15 @@ def test_given_rods_unlike_the_parameters(law, length, prec):
     p = nf.normalize(nf.default_params(box=box, n_rods=n, len=1.0, radius=0.005, contact_gap=0.001, precision=prec,
                                        **(LOGN if law == "logn" else {})))
     _compare(p, rods, 0.001)
+
+
+@pytest.mark.parametrize("prec", [nf.NF_PREC_FP64, nf.NF_PREC_FP32_RECHECK])
+@pytest.mark.parametrize("n,crowd,peak,law", [(60000, 0.9, 8.0, "const"), (61000, 0.9, 8.0, "const"),
+                                              (100000, 2.1, 8.0, "const"), (200000, 0.5, 20.0, "logn"),
+                                              (60000, 0.9, 3.0, "const")])
+def test_agglomerates(n, crowd, peak, law, prec):
+    b = _edge(n, crowd)
+    _compare(nf.normalize(nf.default_params(box=(b,) * 3, n_rods=n, len=1.0, radius=0.005, seed=19, contact_gap=0.002,
+                                            precision=prec, max_rounds=30, den_law=nf.NF_DEN_AGGLOM, n_agg=16,
+                                            agg_peak=peak, agg_sigma=b / 20, **(LOGN if law == "logn" else {}))),
+             None, 0.002)
