@@ -20,13 +20,13 @@
 // list and reported in the one cell that holds the midpoint of its closest
 // points (nf_seg.h's rule).
 //
-// What bounds them: the walk is VALU issue and the latency of its fetches
-// (144 of a launch's 250 us issue on 32 jamming packings; 96% of its lines come
-// from L2), entering is the rate of device-scope atomics, about 30 G/s.  Whole generations on MI355X, cell-pair engine with
-// the line filter against this: 500,000 log-normal rods in agglomerates 3.24
-// -> 1.95 ms, 20,000 rods in FP64 on 1 um cells 3.6 -> 1.4 ms, 32 uneven
-// packings, some past jamming, 155 -> 63 ms.  Which packings take the lists:
-// plan_fine (nf_api.cpp).
+// What bounds them: the walk is VALU issue and the latency of its fetches (at
+// most 144 of a launch's 250 us issue on 32 jamming packings; 96% of its lines
+// come from L2), entering is the rate of device-scope atomics, about 30 G/s.
+// Whole generations on MI355X, cell-pair engine with the line filter against
+// this: 500,000 log-normal rods in agglomerates 3.24 -> 1.95 ms, 20,000 rods in
+// FP64 on 1 um cells 3.6 -> 1.4 ms, 32 uneven packings, some past jamming, 155 ->
+// 63 ms.  Which packings take the lists: plan_fine (nf_api.cpp).
 #include "nf_internal.h"
 #include "nf_line.h"
 
